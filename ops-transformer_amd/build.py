@@ -27,6 +27,9 @@ SOURCES = [
     "grouped_gemm_i8_int32.hip",
     "grouped_gemm_i8_dequant.hip",
     "grouped_gemm_i8_swiglu.hip",
+    "grouped_gemm_i8_int32_tail.hip",
+    "grouped_gemm_i8_dequant_tail.hip",
+    "grouped_gemm_i8_swiglu_tail.hip",
     "grouped_matmul_swiglu_quant.hip",
     "grouped_matmul_v4.hip",
     "grouped_matmul_finalize_routing.hip",
@@ -48,7 +51,8 @@ COMMON_FLAGS = [
 
 # The translation units that hold the LDS-DMA kernels (grouped_gemm_i8_kernels.h instantiated per epilogue): their device
 # assembly goes through the guards below whenever they are compiled.
-RING_SOURCES = ("grouped_gemm_i8_int32.hip", "grouped_gemm_i8_dequant.hip", "grouped_gemm_i8_swiglu.hip")
+RING_SOURCES = ("grouped_gemm_i8_int32.hip", "grouped_gemm_i8_dequant.hip", "grouped_gemm_i8_swiglu.hip",
+                "grouped_gemm_i8_int32_tail.hip", "grouped_gemm_i8_dequant_tail.hip", "grouped_gemm_i8_swiglu_tail.hip")
 
 # The LDS-DMA loads of grouped_gemm_i8_kernels.h set m0 in an inline-assembly statement and count outstanding loads by hand,
 # which leans on how this compiler schedules around such statements.  The kernels were validated (bit-exact suites on

@@ -18,14 +18,15 @@
 //
 // This file: the scheduling kernel, the requantisation kernel, planning and the launch sequence.  The GEMM kernels
 // themselves are in grouped_gemm_i8_kernels.h and are instantiated by one translation unit per epilogue:
-//   StreamGemmKernel  the fast path (K a multiple of 128; K-contiguous, blocked or row-major [K, N] weights).  Persistent
+//   StreamGemmKernel  the fast path (K a multiple of 16; K-contiguous, blocked or row-major [K, N] weights).  Persistent
 //                     workgroups; operands go global -> LDS with global_load_lds_dwordx4 into a ring of 2..4 stages of
 //                     128 k-bytes (192-row tiles: two activation and three weight stages), so several stages of weights
 //                     are in flight per CU with no staging registers, and the ring already holds the next tile's first
 //                     steps while the current tile's epilogue runs.
 //   MixedGemmKernel   the same body twice, once per run of the table with a stage geometry of its own (pulled tiles of
 //                     192 and 256 rows).
-//   GenericGemmKernel byte-wise loader for K not a multiple of 128 and channel counts off the 16-byte grid: correct, slow.
+//   GenericGemmKernel byte-wise loader for K off the 16-byte grid or below 128 and, with the other two weight layouts,
+//                     channel counts off theirs: correct, slow.
 // LDS rows are XOR-swizzled in 16-byte chunks so that the 16 lanes the LDS serves per clock (64 banks) never collide,
 // for the DMA writes as well as for the MFMA operand reads.
 #include "grouped_gemm_i8.h"
@@ -336,7 +337,7 @@ uint64_t* SpanBufferFor(Epilogue epi, int grid, int tileM) {
 }
 
 namespace {
-// The DMA ring needs whole 128-byte k steps, 16-byte aligned bases, 32-bit offsets inside one expert's weights and one of
+// The DMA ring needs at least one 128-byte k step, rows and bases on the 16-byte grid, 32-bit offsets inside one expert's weights and one of
 // the three weight layouts it knows: K-contiguous rows per channel, the blocked layout, or row-major [K, N].
 bool StreamOk(const Problem& p) {
     // blocked: whole 32-channel blocks; row-major: whole 16-byte chunks (per half of a SwiGLU tile)
@@ -345,7 +346,7 @@ bool StreamOk(const Problem& p) {
                           : (p.N % grain == 0 && (p.epilogue != Epilogue::kSwiglu || (p.N / 2) % grain == 0));
     // One expert's weights must hold at least the kilobyte (64 lanes x 16 bytes) that a drained workgroup's idle issue
     // slots keep re-reading from the start of its last tile's expert: smaller experts go to the byte-wise kernel.
-    return layoutOk && p.K % 128 == 0 && reinterpret_cast<uintptr_t>(p.x) % kChunk == 0 &&
+    return layoutOk && p.K % kChunk == 0 && p.K >= 128 && reinterpret_cast<uintptr_t>(p.x) % kChunk == 0 &&
            reinterpret_cast<uintptr_t>(p.w) % kChunk == 0 && p.N * p.K < (1ll << 31) && p.N * p.K >= 64 * kChunk;
 }
 
@@ -391,9 +392,11 @@ Plan MakePlan(const Problem& p) {
     // (the issue side then never runs more than one tile ahead, which is what the two-tile look-ahead of the draw
     // covers) and more than 64 rows; the handful-of-rows tiles of a decode step keep their fixed shares.
     // OPAPI_GEMM_PULL=0 / 1 switches it off / on for every shape with eight k-steps.
-    plan.pullTiles = StreamOk(p) && p.K / 128 >= 8 && plan.tileM > 64 && plan.maxTiles < (1ll << 31);
+    const int64_t kSteps = (p.K + 127) / 128;
+    plan.pullTiles = StreamOk(p) && kSteps >= 8 && plan.tileM > 64 && plan.maxTiles < (1ll << 31);
     if (const char* env = std::getenv("OPAPI_GEMM_PULL")) {
-        plan.pullTiles = StreamOk(p) && p.K / 128 >= 8 && plan.maxTiles < (1ll << 31) && std::atoi(env) != 0;
+        const int64_t kSteps = (p.K + 127) / 128;
+    plan.pullTiles = StreamOk(p) && kSteps >= 8 && plan.maxTiles < (1ll << 31) && std::atoi(env) != 0;
     }
     plan.wavesM = plan.tileM >= 64 && StreamOk(p) ? 2 : 1;
     plan.subTilesM = (plan.tileM / 32 + plan.wavesM - 1) / plan.wavesM;
@@ -498,19 +501,22 @@ hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStrea
                                                static_cast<uintptr_t>(rowBegin) * static_cast<uintptr_t>(p.N / 2) * 4);
         }
         if (p.K > 0) {
-            const bool fast = StreamOk(p);
+            const bool fast = StreamOk(p), tail = p.K % 128 != 0;
             opapi::KernelTimer timer(p.epilogue == Epilogue::kSwiglu ? "gmm_swiglu"
                                      : p.epilogue != Epilogue::kDequant ? "gmm_int32"
                                      : p.combineIndex != nullptr ? "gmm_combine" : "gmm_dequant", stream);
             switch (p.epilogue) {
                 case Epilogue::kInt32:
-                    e = fast ? LaunchRingInt32(plan, ka, sched, stream) : LaunchGenericInt32(plan, ka, sched, stream);
+                    e = !fast ? LaunchGenericInt32(plan, ka, sched, stream) : tail ? LaunchRingTailInt32(plan, ka, sched, stream)
+                         : LaunchRingInt32(plan, ka, sched, stream);
                     break;
                 case Epilogue::kDequant:
-                    e = fast ? LaunchRingDequant(plan, ka, sched, stream) : LaunchGenericDequant(plan, ka, sched, stream);
+                    e = !fast ? LaunchGenericDequant(plan, ka, sched, stream) : tail ? LaunchRingTailDequant(plan, ka, sched, stream)
+                         : LaunchRingDequant(plan, ka, sched, stream);
                     break;
                 case Epilogue::kSwiglu:
-                    e = fast ? LaunchRingSwiglu(plan, ka, sched, stream) : LaunchGenericSwiglu(plan, ka, sched, stream);
+                    e = !fast ? LaunchGenericSwiglu(plan, ka, sched, stream) : tail ? LaunchRingTailSwiglu(plan, ka, sched, stream)
+                         : LaunchRingSwiglu(plan, ka, sched, stream);
                     break;
             }
             if (e != hipSuccess) return e;

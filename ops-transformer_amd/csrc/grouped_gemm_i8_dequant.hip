@@ -4,7 +4,7 @@
 namespace gemm {
 
 hipError_t LaunchRingDequant(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream) {
-    return LaunchStreamShape<Epilogue::kDequant>(plan, args, sched, stream);
+    return LaunchStreamShape<Epilogue::kDequant, false>(plan, args, sched, stream);
 }
 
 hipError_t LaunchGenericDequant(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream) {

@@ -4,7 +4,7 @@
 namespace gemm {
 
 hipError_t LaunchRingInt32(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream) {
-    return LaunchStreamShape<Epilogue::kInt32>(plan, args, sched, stream);
+    return LaunchStreamShape<Epilogue::kInt32, false>(plan, args, sched, stream);
 }
 
 hipError_t LaunchGenericInt32(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream) {

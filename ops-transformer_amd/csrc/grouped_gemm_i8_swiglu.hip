@@ -4,7 +4,7 @@
 namespace gemm {
 
 hipError_t LaunchRingSwiglu(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream) {
-    return LaunchStreamShape<Epilogue::kSwiglu>(plan, args, sched, stream);
+    return LaunchStreamShape<Epilogue::kSwiglu, false>(plan, args, sched, stream);
 }
 
 hipError_t LaunchGenericSwiglu(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream) {
