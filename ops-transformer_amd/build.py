@@ -30,6 +30,8 @@ SOURCES = [
     "grouped_gemm_i8_int32_tail.hip",
     "grouped_gemm_i8_dequant_tail.hip",
     "grouped_gemm_i8_swiglu_tail.hip",
+    "grouped_gemm_i8_slim_plain.hip",
+    "grouped_gemm_i8_slim_swiglu.hip",
     "grouped_matmul_swiglu_quant.hip",
     "grouped_matmul_v4.hip",
     "grouped_matmul_finalize_routing.hip",
@@ -52,7 +54,8 @@ COMMON_FLAGS = [
 # The translation units that hold the LDS-DMA kernels (grouped_gemm_i8_kernels.h instantiated per epilogue): their device
 # assembly goes through the guards below whenever they are compiled.
 RING_SOURCES = ("grouped_gemm_i8_int32.hip", "grouped_gemm_i8_dequant.hip", "grouped_gemm_i8_swiglu.hip",
-                "grouped_gemm_i8_int32_tail.hip", "grouped_gemm_i8_dequant_tail.hip", "grouped_gemm_i8_swiglu_tail.hip")
+                "grouped_gemm_i8_int32_tail.hip", "grouped_gemm_i8_dequant_tail.hip", "grouped_gemm_i8_swiglu_tail.hip",
+                "grouped_gemm_i8_slim_plain.hip", "grouped_gemm_i8_slim_swiglu.hip")
 
 # The LDS-DMA loads of grouped_gemm_i8_kernels.h set m0 in an inline-assembly statement and count outstanding loads by hand,
 # which leans on how this compiler schedules around such statements.  The kernels were validated (bit-exact suites on
@@ -109,7 +112,7 @@ def check_lds_dma_assembly(asm_path):
 def check_ring_kernel_codegen(asm_path):
     """Second build-time guard on the device assembly of the GEMM kernel units, for three properties of the generated code
     that the kernels' speed and exactness rest on and that a compiler can change without any test noticing at once:
-      * no LDS-ring kernel (StreamGemmKernel, MixedGemmKernel) uses scratch memory -- a spilled register is reloaded inside the tile loop;
+      * no LDS-ring kernel (StreamGemmKernel, MixedGemmKernel, SlimGemmKernel) uses scratch memory -- a spilled register is reloaded inside the tile loop;
       * no generic (flat) memory instruction: one still in flight makes the compiler drain vmcnt, DMAs included, in
         front of every LDS read;
       * no mixed-precision multiply-add (v_fma_mix*, v_mad_mix*): that is a product and its fp16 conversion merged into
@@ -125,7 +128,7 @@ def check_ring_kernel_codegen(asm_path):
     checked = 0
     for block in text.split(".amdhsa_kernel ")[1:]:
         name = block.split()[0]
-        if "StreamGemmKernel" not in name and "MixedGemmKernel" not in name:
+        if not any(ring in name for ring in ("StreamGemmKernel", "MixedGemmKernel", "SlimGemmKernel")):
             continue
         fields = dict(l.split()[:2] for l in block.split(".end_amdhsa_kernel")[0].splitlines()[1:] if len(l.split()) >= 2)
         if int(fields.get(".amdhsa_private_segment_fixed_size", "0")) != 0:

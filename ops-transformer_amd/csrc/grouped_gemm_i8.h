@@ -53,6 +53,12 @@ struct Problem {
     float* quantScaleOut = nullptr;  // [M]
 };
 
+// Limits of the kernels for a handful of rows per group (grouped_gemm_i8_slim.h): channels per tile (kSwiglu: half of them
+// activated), groups, and rows (the prefix table in LDS holds 16-bit entries).
+constexpr int kSlimTileN = 128;
+constexpr int kSlimMaxGroups = 512;
+constexpr int64_t kSlimMaxRows = 65535;
+
 // Tile shape chosen from the static shape (M, groups); fixed for the lifetime of a plan.
 struct Plan {
     int tileM = 0;          // rows per workgroup tile (multiple of 32)
@@ -62,6 +68,7 @@ struct Plan {
     int32_t maxMTiles = 0;  // upper bound on m-tiles over all groups (M / tileM + groups)
     int32_t tilesN = 0;
     bool pullTiles = false; // LDS-ring kernels: workgroups draw their tiles from counters instead of walking fixed shares
+    bool slim = false;      // a handful of rows per group: the kernels of grouped_gemm_i8_slim.h, without a scheduling kernel
     int64_t bandRows = 0;   // kSwiglu: rows of S held in the workspace at a time (M when the launch runs as one band)
     uint64_t offSched = 0, offRowMax = 0, offS = 0;
     uint64_t workspaceBytes = 0;

@@ -31,6 +31,7 @@
 // for the DMA writes as well as for the MFMA operand reads.
 #include "grouped_gemm_i8.h"
 
+#include <cmath>
 #include <mutex>
 #include <vector>
 
@@ -225,9 +226,9 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
 // ---------------------------------------------------------------------------------------------- requantisation
 struct RequantArgs {
     const float* s;          // [rows of the band, halfN]: row r of the problem at index r - rowBegin
-    const float* rowMax;     // [tilesN][M] partial max |S|
-    int32_t tilesN;
-    int64_t M;
+    const float* rowMax;     // partial max |S|: entry t of row r at r * maxRowStride + t * maxStride, t < partials
+    int32_t partials;
+    int64_t maxRowStride, maxStride;
     const int32_t* sched;
     int8_t* y;               // [M, halfN]
     float* yScale;           // [M]
@@ -261,7 +262,7 @@ __global__ __launch_bounds__(256) void RequantKernel(RequantArgs a) {
         }
     }
     float mx = 0.0f;
-    for (int t = threadIdx.x & 63; t < a.tilesN; t += 64) mx = fmaxf(mx, a.rowMax[static_cast<int64_t>(t) * a.M + row]);
+    for (int t = threadIdx.x & 63; t < a.partials; t += 64) mx = fmaxf(mx, a.rowMax[row * a.maxRowStride + t * a.maxStride]);
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
     const float ys = __fdiv_rn(mx, 127.0f);
@@ -352,6 +353,48 @@ bool StreamOk(const Problem& p) {
 
 uint64_t Align256(uint64_t v) { return (v + 255) / 256 * 256; }
 
+// S, the fp32 SwiGLU result that the requantisation reads back, is held for a band of rows at a time: at most 512 MiB of it
+// (OPAPI_SWIGLU_WORKSPACE_MB=<n> sets another limit).
+uint64_t SwigluWorkspaceCap() {
+    if (const char* env = std::getenv("OPAPI_SWIGLU_WORKSPACE_MB")) {
+        const long long mb = std::atoll(env);
+        if (mb > 0) return static_cast<uint64_t>(mb) << 20;
+    }
+    return 512ull << 20;
+}
+
+// Rows that hold nearly every group of a router's choice whole: group sizes spread like a Poisson variable around their
+// mean, so the mean plus 2.5 standard deviations.
+double RowsOfNearlyEveryGroup(double meanRows) { return meanRows + 2.5 * std::sqrt(meanRows) + 1.0; }
+
+// Share of the CUs' time that `tiles` like tiles use in whole rounds of one tile per CU.
+double RoundEfficiency(int64_t tiles) {
+    const int64_t cus = DeviceCuCount();
+    return static_cast<double>(tiles) / static_cast<double>((tiles + cus - 1) / cus * cus);
+}
+
+// Rows per tile of the kernels for a handful of rows per group, or 0 where they are not the ones to run.  A tile has to hold
+// nearly every group whole, since a second tile reads the group's weights again.  At 64 rows the LDS-ring kernel's 64-row
+// tile, twice as many channels wide, moves less per weight byte: gate/up of 31 rows each for 128 experts, hidden 4096,
+// intermediate 1536, takes it 280 us against 300; it is left where its tiles fill the machine's rounds worse by more than
+// that (a down projection of 128 of them: 115 us against 78).
+// A forced tile height (OPAPI_GEMM_TILE_M) or tile order (OPAPI_GEMM_PULL) means the kernels those belong to.
+int SlimTileRows(const Problem& p, double meanRows) {
+    if (!StreamOk(p) || !(p.wKMajor || p.wNz) || p.groups > kSlimMaxGroups || p.M > kSlimMaxRows || p.groupListKind == GroupListKind::kSparse ||
+        p.combineIndex != nullptr || p.bias != nullptr || std::getenv("OPAPI_GEMM_TILE_M") != nullptr ||
+        std::getenv("OPAPI_GEMM_PULL") != nullptr) {
+        return 0;
+    }
+    if (p.epilogue == Epilogue::kSwiglu && static_cast<uint64_t>(p.M) * static_cast<uint64_t>(p.N / 2) * 4 > SwigluWorkspaceCap()) return 0;
+    const double want = RowsOfNearlyEveryGroup(meanRows);
+    if (want <= 16.0) return 16;
+    if (want <= 32.0) return 32;
+    if (want > 64.0) return 0;
+    const int64_t cols = p.epilogue == Epilogue::kSwiglu ? p.N / 2 : p.N;
+    const int64_t wide = p.epilogue == Epilogue::kSwiglu ? kTileN / 2 : kTileN, slim = wide * kSlimTileN / kTileN;
+    return RoundEfficiency(p.groups * ((cols + slim - 1) / slim)) > 1.06 * RoundEfficiency(p.groups * ((cols + wide - 1) / wide)) ? 64 : 0;
+}
+
 }  // namespace
 
 Plan MakePlan(const Problem& p) {
@@ -367,6 +410,24 @@ Plan MakePlan(const Problem& p) {
     // their extra rows with a shallower activation ring, which costs less than that round.
     const double meanRows = p.expectedRowsPerGroup > 0 ? static_cast<double>(p.expectedRowsPerGroup)
                                                        : static_cast<double>(p.M) / static_cast<double>(groups);
+    if (const int slimRows = SlimTileRows(p, meanRows)) {
+        plan.slim = true;
+        plan.tileM = slimRows;
+        const int64_t slimCols = p.epilogue == Epilogue::kSwiglu ? kSlimTileN / 2 : kSlimTileN;
+        plan.tilesN = static_cast<int32_t>((cols + slimCols - 1) / slimCols);
+        plan.maxMTiles = static_cast<int32_t>(p.M / slimRows + (groups < p.M ? groups : p.M));
+        plan.maxTiles = (static_cast<int64_t>(plan.maxMTiles) * plan.tilesN + kXcds - 1) / kXcds * kXcds;
+        uint64_t off = Align256(kQueueHeaderInts * 4);
+        if (p.epilogue == Epilogue::kSwiglu) {
+            plan.offRowMax = off;
+            off += Align256(static_cast<uint64_t>(p.M) * static_cast<uint64_t>(plan.tilesN) * 16);
+            plan.bandRows = p.M;
+            plan.offS = off;
+            off += Align256(static_cast<uint64_t>(p.M) * static_cast<uint64_t>(p.N / 2) * 4);
+        }
+        plan.workspaceBytes = off;
+        return plan;
+    }
     const double rounds = static_cast<double>(groups) * plan.tilesN / DeviceCuCount();
     const double want = meanRows * (rounds <= 24.0 ? 1.5 : 1.25);
     if (StreamOk(p)) {
@@ -376,8 +437,10 @@ Plan MakePlan(const Problem& p) {
             if (static_cast<double>(s) >= want) { plan.tileM = s; break; }
         }
         // A handful of rows per group (decode): the 64-row shape, whose eight waves keep more of the weight stream in
-        // flight than the four of the 32-row shape (measured 0.3 - 0.7 % faster on both GEMMs of a 64-token step).
-        if (plan.tileM < 64) plan.tileM = 64;
+        // flight than the four of the 32-row shape (measured 0.3 - 0.7 % faster on both GEMMs of a 64-token step).  It
+        // also serves groups of more rows while it holds nearly all of them whole: 44 rows each for 128 experts, hidden
+        // 4096, intermediate 1536, took 341 / 180 us (gate/up, down) with 96-row tiles, 287 / 155 us with these.
+        if (plan.tileM < 64 || RowsOfNearlyEveryGroup(meanRows) <= 64.0) plan.tileM = 64;
         // tuning override: OPAPI_GEMM_TILE_M=<one of the shapes above>
         if (const char* env = std::getenv("OPAPI_GEMM_TILE_M")) {
             const int forced = std::atoi(env);
@@ -410,16 +473,11 @@ Plan MakePlan(const Problem& p) {
     if (p.epilogue == Epilogue::kSwiglu) {
         plan.offRowMax = off;
         off += Align256(static_cast<uint64_t>(p.M) * 4 * static_cast<uint64_t>(plan.tilesN));
-        // S, the fp32 SwiGLU result that the requantisation reads back, is held for one band of rows at a time: at most
-        // 512 MiB of it (OPAPI_SWIGLU_WORKSPACE_MB=<n> sets another limit), in whole m-tiles, at least one.  A launch
-        // whose S fits runs as one band; a taller one runs schedule, GEMM and requantisation once per band.  A band of
-        // 512 MiB is at least 4096 tiles, sixteen rounds of the machine, whatever the shape: measured against a single
-        // band on 1.9 GB of S it costs nothing (halving the limit twice costs 2 % and 7 % of the pass).
-        uint64_t capBytes = 512ull << 20;
-        if (const char* env = std::getenv("OPAPI_SWIGLU_WORKSPACE_MB")) {
-            const long long mb = std::atoll(env);
-            if (mb > 0) capBytes = static_cast<uint64_t>(mb) << 20;
-        }
+        // S is held for one band of rows at a time, in whole m-tiles, at least one.  A launch whose S fits the limit runs as
+        // one band; a taller one runs schedule, GEMM and requantisation once per band.  A band of 512 MiB is at least 4096
+        // tiles, sixteen rounds of the machine, whatever the shape: measured against a single band on 1.9 GB of S it
+        // costs nothing (halving the limit twice costs 2 % and 7 % of the pass).
+        const uint64_t capBytes = SwigluWorkspaceCap();
         const uint64_t rowBytes = static_cast<uint64_t>(p.N / 2) * 4;
         int64_t bandRows = rowBytes > 0 ? static_cast<int64_t>(capBytes / rowBytes) / plan.tileM * plan.tileM : p.M;
         if (bandRows < plan.tileM) bandRows = plan.tileM;
@@ -492,7 +550,7 @@ hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStrea
         const int64_t rowEnd = rowBegin + bandRows < p.M ? rowBegin + bandRows : p.M;
         sa.rowBegin = rowBegin;
         sa.rowEnd = rowEnd;
-        {
+        if (!plan.slim) {
             opapi::KernelTimer timer("gmm_schedule", stream);
             hipLaunchKernelGGL(ScheduleKernel, dim3(1), dim3(1024), 0, stream, sa);
         }
@@ -501,11 +559,15 @@ hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStrea
                                                static_cast<uintptr_t>(rowBegin) * static_cast<uintptr_t>(p.N / 2) * 4);
         }
         if (p.K > 0) {
-            const bool fast = StreamOk(p), tail = p.K % 128 != 0;
+            const bool fast = !plan.slim && StreamOk(p), tail = p.K % 128 != 0;
             opapi::KernelTimer timer(p.epilogue == Epilogue::kSwiglu ? "gmm_swiglu"
                                      : p.epilogue != Epilogue::kDequant ? "gmm_int32"
                                      : p.combineIndex != nullptr ? "gmm_combine" : "gmm_dequant", stream);
-            switch (p.epilogue) {
+            if (plan.slim) {
+                if (p.epilogue == Epilogue::kInt32) ka.scale = nullptr;  // raw accumulators
+                const SlimList list{p.groupList, sa.groupListIsInt64, sa.isCount, p.groups, sched + kHdrCoveredRows};
+                e = swiglu ? LaunchSlimSwiglu(plan, ka, list, stream) : LaunchSlimPlain(plan, ka, list, stream);
+            } else switch (p.epilogue) {
                 case Epilogue::kInt32:
                     e = !fast ? LaunchGenericInt32(plan, ka, sched, stream) : tail ? LaunchRingTailInt32(plan, ka, sched, stream)
                          : LaunchRingInt32(plan, ka, sched, stream);
@@ -522,7 +584,8 @@ hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStrea
             if (e != hipSuccess) return e;
         }
         if (swiglu) {
-            RequantArgs ra{sBuf, rowMax, plan.tilesN, p.M, sched, p.quantOut, p.quantScaleOut, static_cast<int32_t>(p.N / 2),
+            RequantArgs ra{sBuf, rowMax, plan.slim ? 4 * plan.tilesN : plan.tilesN, plan.slim ? 4 * plan.tilesN : 1,
+                           plan.slim ? 1 : p.M, sched, p.quantOut, p.quantScaleOut, static_cast<int32_t>(p.N / 2),
                            rowBegin};
             opapi::KernelTimer timer("gmm_requant", stream);
             hipLaunchKernelGGL(RequantKernel, dim3(static_cast<unsigned>(rowEnd - rowBegin)), dim3(256), 0, stream, ra);

@@ -37,7 +37,7 @@ struct KernelArgs {
     int32_t scaleDtype;
     const float* rowScale;
     float* sOut;
-    float* rowMax;  // [tilesN][M] partial max |S| per n-tile
+    float* rowMax;  // partial max |S|: [tilesN][M], one per n-tile; grouped_gemm_i8_slim.h: [M][4 tilesN], one per wave
     // scatter-add mode of the fp32 kDequant epilogue (Problem::combineIndex)
     const void* combineIndex;
     int32_t combineIndexIsInt64;
@@ -55,6 +55,15 @@ struct KernelArgs {
     int32_t pullTiles;
 };
 
+// The group list (cumsum or counts) as the kernels of grouped_gemm_i8_slim.h read it.
+struct SlimList {
+    const void* list;
+    int32_t isInt64;
+    int32_t isCount;
+    int32_t groups;
+    int32_t* coveredRows;  // written by workgroup 0: rows covered by the list (the requantisation reads it)
+};
+
 // Defined in grouped_gemm_i8.hip.
 int DeviceCuCount();
 uint64_t* SpanBufferFor(Epilogue epi, int grid, int tileM);
@@ -67,6 +76,8 @@ hipError_t LaunchRingSwiglu(const Plan& plan, const KernelArgs& args, const int3
 hipError_t LaunchRingTailInt32(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream);
 hipError_t LaunchRingTailDequant(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream);
 hipError_t LaunchRingTailSwiglu(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream);
+hipError_t LaunchSlimPlain(const Plan& plan, const KernelArgs& args, const SlimList& list, hipStream_t stream);
+hipError_t LaunchSlimSwiglu(const Plan& plan, const KernelArgs& args, const SlimList& list, hipStream_t stream);
 hipError_t LaunchGenericInt32(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream);
 hipError_t LaunchGenericDequant(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream);
 hipError_t LaunchGenericSwiglu(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream);

@@ -1,0 +1,95 @@
+"""The grouped GEMM kernels for a handful of rows per expert (no scheduling kernel, a prefix table per workgroup) against
+the CPU oracle: int32, bf16 and fp16 outputs bit-exact, SwiGLU-quant within one LSB."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# rows of each group, K, N (even; SwiGLU halves it).  The mean picks the tile (16, 32 or 64 rows); few tiles pick the deep ring.
+CASES = {
+    "one_token_two_experts": ([0, 1, 0, 0, 1, 0], 1024, 512),                       # deep, 16-row tile, idle groups
+    "one_row_k_one_step": ([1], 128, 256),                                            # a tile of one k-step
+    "tile16_edges": ([16, 0, 15, 1, 17, 3, 2, 0, 1, 5] * 2, 256, 704),                # either side of 16 rows, partial n-tile
+    "tile16_many_groups": ([(i * 7) % 5 for i in range(512)], 144, 192),              # the widest group list, K off the grid
+    "tile16_many_tiles": ([2, 0, 3, 1, 6, 4, 1, 1] * 24, 128, 2112),                  # workgroups walk several one-step tiles
+    "tile16_long": ([4] * 40, 2064, 1088),
+    "tile32_deep": ([32, 11, 33, 0], 1136, 288),
+    "tile32": ([20, 0, 31, 32, 33, 9, 18, 14] * 6, 384, 1344),
+    "tile64_deep": ([64, 40, 65, 20], 640, 224),
+    "tile64": ([64, 30, 65, 0, 40, 63, 12, 33, 49, 31] * 4, 272, 1600),
+    "skewed": ([150, 0, 1, 0, 0, 2, 0, 0, 1, 0, 3, 0, 0, 0, 1, 0] * 4, 512, 576),     # several m-tiles of one group
+}
+
+
+def _to_nz(w_dev):
+    E, N, K = w_dev.shape
+    return w_dev.view(E, N // 32, 32, K // 16, 16).permute(0, 1, 3, 4, 2).contiguous()
+
+
+@pytest.mark.parametrize("layout", ["kmajor", "nd", "nz"])
+@pytest.mark.parametrize("name", list(CASES))
+def test_against_oracle(aclnn, oracle, dev, name, layout):
+    sizes, K, N = CASES[name]
+    sizes = np.array(sizes, np.int64)
+    rng = np.random.default_rng(len(name) + K)
+    E, M = len(sizes), int(sizes.sum())
+    tail = 3                                      # rows beyond the list stay untouched
+    x = rng.integers(-127, 128, (M + tail, K)).astype(np.int8)
+    wt = rng.integers(-127, 128, (E, N, K)).astype(np.int8)
+    cumsum = np.cumsum(sizes)
+    scale = rng.uniform(1e-3, 1e-2, (E, N)).astype(np.float32)
+    pt = rng.uniform(0.01, 0.1, M + tail).astype(np.float32)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    w_dev = t(wt)
+    if layout == "nz":
+        wkw, wv, w = dict(weight_nz=(_to_nz(w_dev), "nz5d")), None, None
+    else:
+        w = w_dev.transpose(1, 2) if layout == "kmajor" else w_dev.transpose(1, 2).contiguous()
+        wkw, wv = {}, [w]
+    xd, ptd = t(x), t(pt)
+    acc_ref = oracle.grouped_matmul_i32(x, wt, cumsum, w_trans=True)
+    for values, kind, dtype in ((cumsum, 0, torch.int64), (sizes, 1, torch.int32)):
+        acc = torch.full((M + tail, N), -7, dtype=torch.int32, device=dev)
+        aclnn.grouped_matmul_v4([xd], wv, group_list=t(values).to(dtype), split_item=3, group_type=0, group_list_type=kind,
+                                out=[acc], **wkw)
+        torch.cuda.synchronize()
+        assert np.array_equal(acc.cpu().numpy()[:M], acc_ref[:M]) and bool((acc[M:] == -7).all())
+    for dtype, code in ((torch.bfloat16, oracle.DT_BF16), (torch.float16, oracle.DT_F16)):
+        y = torch.zeros((M + tail, N), dtype=dtype, device=dev)
+        aclnn.grouped_matmul_v4([xd], wv, scale=[t(scale)], per_token_scale=[ptd], group_list=t(cumsum), split_item=3,
+                                group_type=0, out=[y], **wkw)
+        ref = oracle.grouped_matmul_dequant(x, wt, scale, pt, cumsum, w_trans=True, out_dtype=code)
+        torch.cuda.synchronize()
+        got = y.view(torch.int16).cpu().numpy().view(np.uint16)
+        assert np.array_equal(got[:M], ref[:M]) and not got[M:].any(), dtype
+    # 16-bit channel scales are read in the epilogue instead of by DMA
+    s16 = t(scale).bfloat16()
+    y = aclnn.grouped_matmul_v4([xd], wv, scale=[s16], per_token_scale=[ptd], group_list=t(cumsum), split_item=3, group_type=0,
+                                output_dtype=torch.bfloat16, **wkw)[0]
+    ref = oracle.grouped_matmul_dequant(x, wt, s16.view(torch.int16).cpu().numpy().view(np.uint16), pt, cumsum, w_trans=True,
+                                        scale_dtype=oracle.DT_BF16, out_dtype=oracle.DT_BF16)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.view(torch.int16).cpu().numpy().view(np.uint16)[:M], ref[:M])
+    q = torch.full((M + tail, N // 2), 77, dtype=torch.int8, device=dev)
+    qs = torch.zeros(M + tail, device=dev)
+    aclnn.grouped_matmul_swiglu_quant(xd, w, t(cumsum), t(scale), ptd, out=(q, qs), **wkw)
+    torch.cuda.synchronize()
+    q_ref, qs_ref = oracle.grouped_matmul_swiglu_quant(x, wt, scale, pt, cumsum, w_trans=True)
+    diff = np.abs(q.cpu().numpy()[:M].astype(np.int32) - q_ref[:M].astype(np.int32))
+    assert diff.max() <= 1 and (diff != 0).mean() < 1e-3 and bool((q[M:] == 77).all())
+    np.testing.assert_allclose(qs.cpu().numpy()[:M], qs_ref[:M], rtol=1e-5)
+
+
+@pytest.mark.parametrize("kind,values", [(0, [30, 0, 30, 0, 30]), (0, [12, 5, 40, -7, 9]), (1, [30, 30, 30, 30, 30]),
+                                         (1, [-5, 40, 1, 0, 2000000000])])
+def test_malformed_lists_stay_in_bounds(aclnn, dev, kind, values):
+    M, K, N = 30, 256, 192
+    g = torch.Generator(device=dev).manual_seed(1)
+    x = torch.randint(-127, 128, (M, K), dtype=torch.int8, device=dev, generator=g)
+    w = torch.randint(-127, 128, (5, N, K), dtype=torch.int8, device=dev, generator=g)
+    guard = torch.full((M + 64, N), -7, dtype=torch.int32, device=dev)
+    aclnn.grouped_matmul_v4([x], [w.transpose(1, 2)], group_list=torch.tensor(values, dtype=torch.int64, device=dev),
+                            split_item=3, group_type=0, group_list_type=kind, out=[guard[:M]])
+    torch.cuda.synchronize()
+    assert bool((guard[M:] == -7).all())
