@@ -62,6 +62,7 @@ RING_SOURCES = ("grouped_gemm_i8_int32.hip", "grouped_gemm_i8_dequant.hip", "gro
 # the GPU) with the compiler named here; another one has to be validated again before its build is trusted:
 # OPAPI_ALLOW_UNVALIDATED_COMPILER=1 lets the build through so that the suites can be run.
 VALIDATED_COMPILERS = ("roc-7.2.0",)
+LDS_DMA_LOADS = ("global_load_lds_dwordx4", "global_load_lds_dword")  # operand chunks, scales
 
 
 def compiler_version():
@@ -85,7 +86,7 @@ def check_compiler():
 
 def check_lds_dma_assembly(asm_path):
     """Build-time guard on the device assembly of the GEMM kernel units: every instruction that writes m0 must be the
-    `s_mov_b32 m0, sN` of an LDS-DMA statement, i.e. be followed at once by its global_load_lds_dwordx4, and every such
+    `s_mov_b32 m0, sN` of an LDS-DMA statement, i.e. be followed at once by its global_load_lds_dword[x4], and every such
     load must be preceded by its own m0 write.  A compiler that puts anything between the two, or writes m0 for a
     purpose of its own inside these kernels, fails the build instead of producing kernels that read stale tiles."""
     lines = [l.split(";")[0].strip() for l in open(asm_path)]
@@ -96,7 +97,7 @@ def check_lds_dma_assembly(asm_path):
         writes_m0 = len(fields) > 1 and fields[1] == "m0" and not fields[0].startswith(("s_cmp", "s_bitcmp"))
         if writes_m0:
             nxt = lines[i + 1] if i + 1 < len(lines) else ""
-            if fields[0] != "s_mov_b32" or not nxt.startswith("global_load_lds_dwordx4"):
+            if fields[0] != "s_mov_b32" or nxt.split(" ")[0] not in LDS_DMA_LOADS:
                 raise RuntimeError("%s: m0 is written outside an LDS-DMA pair: '%s' followed by '%s'" % (asm_path, l, nxt))
             pairs += 1
         if l.startswith("global_load_lds_"):
