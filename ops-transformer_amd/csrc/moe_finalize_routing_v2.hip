@@ -171,10 +171,20 @@ __global__ __launch_bounds__(256) void FinalizeKernel(FinalizeArgs a, int scaleI
     }
 }
 
-// The common case -- no bias, at most kMaxK experts per token, 16-byte packets, one packet per lane -- with every load of a
-// token's K row indices and weights loaded up front (wave-uniform loads) and the K row packets requested two at a time,
-// one pair ahead of the sum, which runs in ascending k with the same separate multiply and add as the general kernel
-// (bit-identical results).  The general kernel makes 2 K dependent memory round trips per lane, this one K / 2 + 1.
+// The common case -- no bias, at most 8 experts per token, 16-byte packets, one packet per lane -- with a token's K row
+// indices and weights loaded up front (wave-uniform loads) and the K row packets requested two at a time, one pair ahead
+// of the sum, which runs in ascending k with the same separate multiply and add as the general kernel (bit-identical
+// results).  The general kernel makes 2 K dependent memory round trips per lane, this one K / 2 + 1.
+//
+// What bounds it is the memory system, as long as the sum stays straight-line code: with a case distinction around every
+// load and every term (index in range? first term? skip input?) the instructions did.  All of them are wave-uniform, so
+// they are settled in front of the sum: what it starts from (the skip inputs, zero, or its first term), and whether every
+// index is in range.  Where one is not -- a dropped row -- its load goes to the token's first row, which is in the cache
+// anyway, and its term is discarded by a select.  kMaxK is the next of 2, 4, 6, 8 at or above topK, so that few experts
+// per token cost no loads for absent ones.
+// Measured before and now: 4096 tokens of 7168 bf16, top-8 out of capacity slots with a fifth of the rows dropped, plus a
+// skip input: 139 -> 116 us (4.3 TB/s of rows, seed and result); 16384 x 4096, top-2: 94 -> 65 us (6.2 TB/s); 2047 x 4096,
+// top-8, with a skip input: 39 -> 34 us; 4096 x 7168, top-8, nothing else: 101 - 104 us, as before.
 template <typename Codec, int kVec, int kMaxK>
 __global__ __launch_bounds__(256) void FinalizeBatchedKernel(FinalizeArgs a, int scaleIsF32) {
     using P = Packet<Codec, kVec>;
@@ -192,6 +202,9 @@ __global__ __launch_bounds__(256) void FinalizeBatchedKernel(FinalizeArgs a, int
     constexpr int dataIsF16 = Codec::kRoundEveryOp ? 1 : 0;
     const int topK = a.topK;
 
+    P p1{}, p2{};
+    if (a.x1 != nullptr) p1 = static_cast<const P*>(a.x1)[token * packets + pk];
+    if (a.x2 != nullptr) p2 = static_cast<const P*>(a.x2)[token * packets + pk];
     int64_t d[kMaxK];
     float s[kMaxK];
 #pragma unroll
@@ -204,92 +217,64 @@ __global__ __launch_bounds__(256) void FinalizeBatchedKernel(FinalizeArgs a, int
             if (a.scales != nullptr) s[k] = ScaleAt(a.scales, token * topK + k, scaleIsF32, dataIsF16);
         }
     }
-    // The plain call -- exactly kMaxK experts per token, every index in range, no skip inputs -- as straight-line code:
-    // the general form below spends more instructions on its (wave-uniform) case distinctions than on the sum, and at
-    // sixteen bytes per lane that, not the memory system, was what bounded the kernel.
-    bool plain = topK == kMaxK && a.x1 == nullptr && a.x2 == nullptr;
+    // -1 marks a dropped row in the drop/pad arrangements; any other out-of-range index is ignored for safety
+    uint32_t valid = 0;
+    int first = kMaxK;      // the first term of the sum, and its row
+    int64_t firstRow = 0;
 #pragma unroll
-    for (int k = 0; k < kMaxK; ++k) plain = plain && d[k] >= 0 && d[k] < a.expandedRows;
-    if (plain) {
-        const P* const x = static_cast<const P*>(a.expandedX) + pk;
+    for (int k = kMaxK - 1; k >= 0; --k) {
+        if (d[k] < 0 || d[k] >= a.expandedRows) continue;
+        valid |= 1u << k;
+        first = k;
+        firstRow = d[k];
+    }
+    float acc[kVec];
+    if (a.x1 != nullptr && a.x2 != nullptr) {
+#pragma unroll
+        for (int i = 0; i < kVec; ++i) acc[i] = Codec::Round(__fadd_rn(Codec::Load(p1.v[i]), Codec::Load(p2.v[i])));
+    } else {  // an absent packet is all zero bits
+        const P& only = a.x1 != nullptr ? p1 : p2;
+#pragma unroll
+        for (int i = 0; i < kVec; ++i) acc[i] = __fadd_rn(Codec::Load(only.v[i]), 0.0f);
+    }
+    // without skip inputs the first term is the sum itself (adding it to zero would lose the sign of a negative zero),
+    // unless a dropped row came before it, which counts as zero
+    const bool replaces = a.x1 == nullptr && a.x2 == nullptr && !(skipsAllowed && first > 0);
+    const P* const x = static_cast<const P*>(a.expandedX) + pk;
+    auto sum = [&](auto allTag) __attribute__((always_inline)) {
+        constexpr bool kAll = decltype(allTag)::value;
+        auto rowOf = [&](int k) __attribute__((always_inline)) {
+            return x[(kAll || ((valid >> k) & 1u) != 0 ? d[k] : firstRow) * packets];
+        };
         P row[2][2];
-        row[0][0] = x[d[0] * packets];
-        row[0][1] = x[d[1] * packets];
-        float acc[kVec];
+        row[0][0] = rowOf(0);
+        row[0][1] = rowOf(1);
 #pragma unroll
         for (int k0 = 0; k0 < kMaxK; k0 += 2) {
             const int cur = (k0 >> 1) & 1;
             if (k0 + 2 < kMaxK) {
-                row[cur ^ 1][0] = x[d[k0 + 2] * packets];
-                row[cur ^ 1][1] = x[d[k0 + 3 < kMaxK ? k0 + 3 : k0 + 2] * packets];
+                row[cur ^ 1][0] = rowOf(k0 + 2);
+                row[cur ^ 1][1] = rowOf(k0 + 3);
             }
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int k = k0 + j;
-                if (k >= kMaxK) continue;
+                const bool counts = kAll || ((valid >> k) & 1u) != 0;
+                const bool starts = replaces && (kAll ? k == 0 : k == first);
 #pragma unroll
                 for (int i = 0; i < kVec; ++i) {
                     const float t = Codec::Round(__fmul_rn(Codec::Load(row[cur][j].v[i]), s[k]));
-                    acc[i] = k == 0 ? t : Codec::Round(__fadd_rn(acc[i], t));
+                    const float added = Codec::Round(__fadd_rn(acc[i], t));
+                    if (kAll && k > 0) acc[i] = added;
+                    else acc[i] = starts ? t : counts ? added : acc[i];
                 }
             }
-        }
-        static_cast<P*>(a.out)[token * packets + pk] = PackPacket<Codec, kVec>(acc);
-        return;
-    }
-    P p1{}, p2{};
-    if (a.x1 != nullptr) p1 = static_cast<const P*>(a.x1)[token * packets + pk];
-    if (a.x2 != nullptr) p2 = static_cast<const P*>(a.x2)[token * packets + pk];
-    // row packets travel in pairs, the next pair requested before the current one is added
-    P row[2][2];
-    auto request = [&](int k0, int slot) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int k = k0 + j;
-            const bool valid = k < kMaxK && k < topK && d[k < kMaxK ? k : 0] >= 0 && d[k < kMaxK ? k : 0] < a.expandedRows;
-            if (valid) row[slot][j] = static_cast<const P*>(a.expandedX)[d[k] * packets + pk];
         }
     };
-    request(0, 0);
-    float acc[kVec];
-    bool init = false;
-    if (a.x1 != nullptr && a.x2 != nullptr) {
-#pragma unroll
-        for (int i = 0; i < kVec; ++i) acc[i] = Codec::Round(__fadd_rn(Codec::Load(p1.v[i]), Codec::Load(p2.v[i])));
-        init = true;
-    } else if (a.x1 != nullptr || a.x2 != nullptr) {
-        const P& only = a.x1 != nullptr ? p1 : p2;
-#pragma unroll
-        for (int i = 0; i < kVec; ++i) acc[i] = __fadd_rn(Codec::Load(only.v[i]), 0.0f);
-        init = true;
-    }
-#pragma unroll
-    for (int k0 = 0; k0 < kMaxK; k0 += 2) {
-        if (k0 + 2 < kMaxK) request(k0 + 2, ((k0 >> 1) + 1) & 1);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int k = k0 + j;
-            if (k >= topK) continue;
-            if (d[k] < 0 || d[k] >= a.expandedRows) {
-                if (skipsAllowed && !init) {
-#pragma unroll
-                    for (int i = 0; i < kVec; ++i) acc[i] = 0.0f;
-                    init = true;
-                }
-                continue;
-            }
-#pragma unroll
-            for (int i = 0; i < kVec; ++i) {
-                const float t = Codec::Round(__fmul_rn(Codec::Load(row[(k0 >> 1) & 1][j].v[i]), s[k]));
-                acc[i] = init ? Codec::Round(__fadd_rn(acc[i], t)) : t;
-            }
-            init = true;
-        }
-    }
-    P o;
-#pragma unroll
-    for (int i = 0; i < kVec; ++i) o.v[i] = Codec::Store(init ? acc[i] : 0.0f);
-    static_cast<P*>(a.out)[token * packets + pk] = o;
+    static_assert(kMaxK % 2 == 0, "row packets travel in pairs");
+    if (valid == (1u << kMaxK) - 1u) sum(std::true_type{});
+    else if (valid != 0) sum(std::false_type{});
+    static_cast<P*>(a.out)[token * packets + pk] = PackPacket<Codec, kVec>(acc);
 }
 
 class FinalizeExecutor : public aclOpExecutor {
@@ -304,8 +289,11 @@ class FinalizeExecutor : public aclOpExecutor {
         const int64_t packets = args.hidden / kVec;
         if (kVec > 1 && args.bias == nullptr && args.topK <= 8 && packets > 64) {
             const unsigned slices = static_cast<unsigned>((packets + 255) / 256);
-            hipLaunchKernelGGL((FinalizeBatchedKernel<Codec, kVec, 8>), dim3(static_cast<unsigned>(args.tokens * slices)),
-                               dim3(256), 0, stream, args, scaleIsF32);
+            const dim3 grid(static_cast<unsigned>(args.tokens * slices));
+            if (args.topK <= 2) hipLaunchKernelGGL((FinalizeBatchedKernel<Codec, kVec, 2>), grid, dim3(256), 0, stream, args, scaleIsF32);
+            else if (args.topK <= 4) hipLaunchKernelGGL((FinalizeBatchedKernel<Codec, kVec, 4>), grid, dim3(256), 0, stream, args, scaleIsF32);
+            else if (args.topK <= 6) hipLaunchKernelGGL((FinalizeBatchedKernel<Codec, kVec, 6>), grid, dim3(256), 0, stream, args, scaleIsF32);
+            else hipLaunchKernelGGL((FinalizeBatchedKernel<Codec, kVec, 8>), grid, dim3(256), 0, stream, args, scaleIsF32);
             return;
         }
         if (packets <= 64) {

@@ -161,3 +161,23 @@ def test_wide_rows_without_bias(aclnn, oracle, dev, dtype, K, seeds, mode):
     assert np.array_equal(got_np, ref)
     if mode in (1, 3) and seeds == "none":
         assert (got.float().cpu().numpy()[1] == 0).all()     # every term dropped and no seed: zeros
+
+
+@pytest.mark.parametrize("K", [2, 4, 5, 6, 7])
+@pytest.mark.parametrize("seeds", ["none", "x1"])
+@pytest.mark.parametrize("mode", [2, 3])
+def test_experts_per_token_between_the_kernel_variants(aclnn, oracle, dev, K, seeds, mode):
+    """The batched kernel is built for 2, 4, 6 and 8 experts per token: each exactly met, and the counts that leave one of
+    its terms absent, with and without dropped rows, on rows that end inside a workgroup's slice."""
+    rng = np.random.default_rng(10 * K + mode)
+    T, H, E, C = 11, 2056, 5, 9
+    ex, idx, x1, _, _, scales, _ = _case(rng, T, K, H, E, seeds == "x1", False, False, mode, C)
+    if mode == 3:
+        idx[0], idx[K] = -1, 3                    # token 0: first term dropped; token 1: only its first term kept
+        idx[K + 1:2 * K] = -1
+    enc, to_dev, code = _to_dtype(oracle, "bf16", dev)
+    ref = oracle.moe_finalize_routing_v2(enc(ex), idx, enc(x1), None, None, enc(scales), None, drop_pad_mode=mode,
+                                         dtype=code, scale_dtype=code)
+    got = aclnn.moe_finalize_routing_v2(to_dev(enc(ex)), torch.from_numpy(idx).to(dev), to_dev(enc(x1)), None, None,
+                                        to_dev(enc(scales)), None, drop_pad_mode=mode)
+    assert np.array_equal(got.view(torch.int16).cpu().numpy().view(np.uint16), ref)
