@@ -312,18 +312,22 @@ def moe_init_routing_quant_v2(x, expert_idx, quant_mode, scale=None, offset=None
     T, H = x.shape
     K = expert_idx.shape[1]
     dev = x.device
+    # The operator writes every element of its outputs, padding slots included, unless there is nothing to route or a
+    # smooth scale leaves out rows whose expert id is none of its rows: only then do the outputs have to start at zero.
+    # (A fill is a launch of its own: 5 us each at decode sizes, 11 us for the rows of a 2047-token call.)
+    fresh = torch.zeros if scale is not None or T * K == 0 else torch.empty
     if drop_pad_mode == 1:
-        expanded_x = torch.zeros((expert_num, expert_capacity, H), dtype=torch.int8, device=dev)
+        expanded_x = fresh((expert_num, expert_capacity, H), dtype=torch.int8, device=dev)
         rows = expert_num * expert_capacity
         count_flag, before_flag = 0, expert_tokens_before_capacity_flag
     else:
         rows = T * K if active_num == 0 else min(T * K, active_num)
-        expanded_x = torch.zeros((rows, H), dtype=torch.int8, device=dev)
+        expanded_x = fresh((rows, H), dtype=torch.int8, device=dev)
         count_flag, before_flag = expert_tokens_count_or_cumsum_flag, False
     row_idx = torch.empty((T * K,), dtype=torch.int32, device=dev)
-    counts = torch.zeros((expert_num,), dtype=torch.int32, device=dev) if count_flag else None
-    before = torch.zeros((expert_num,), dtype=torch.int32, device=dev) if before_flag else None
-    dyn = torch.zeros((rows,), dtype=torch.float32, device=dev) if quant_mode == 1 else None
+    counts = fresh((expert_num,), dtype=torch.int32, device=dev) if count_flag else None
+    before = fresh((expert_num,), dtype=torch.int32, device=dev) if before_flag else None
+    dyn = fresh((rows,), dtype=torch.float32, device=dev) if quant_mode == 1 else None
     h = _Handles()
     try:
         args = [h.tensor(x), h.tensor(expert_idx), h.tensor(scale), h.tensor(offset), active_num, expert_capacity,
@@ -366,10 +370,14 @@ def moe_init_routing_v3(x, expert_idx, scale=None, expert_num=0, expert_tokens_n
     if out is not None:
         expanded_x, row_idx, counts, expanded_scale = out
     else:
-        expanded_x = torch.zeros((T * K, H), dtype=torch.int8 if quant_mode == 1 else x.dtype, device=dev)
+        # As in moe_init_routing_quant_v2; a range of experts leaves the rows of the others unwritten, and key/value
+        # counts what lies behind their last pair.
+        fresh = (torch.zeros if active_expert_range is not None or expert_tokens_num_type == 2 or T * K == 0 or
+                 (quant_mode == 1 and scale is not None) else torch.empty)
+        expanded_x = fresh((T * K, H), dtype=torch.int8 if quant_mode == 1 else x.dtype, device=dev)
         row_idx = torch.empty((T * K,), dtype=torch.int32, device=dev)
-        counts = torch.zeros((expert_num, 2) if expert_tokens_num_type == 2 else (end - start,), dtype=torch.int64, device=dev)
-        expanded_scale = (torch.zeros((T * K,), dtype=torch.float32, device=dev)
+        counts = fresh((expert_num, 2) if expert_tokens_num_type == 2 else (end - start,), dtype=torch.int64, device=dev)
+        expanded_scale = (fresh((T * K,), dtype=torch.float32, device=dev)
                           if (scale is not None or quant_mode == 1) else None)
     h = _Handles()
     try:

@@ -432,3 +432,31 @@ def test_decode_sized_calls_sort_and_gather_in_one_launch(aclnn, oracle, dev, T,
             ex_r, ri_r, cnt_r, es_r = oracle.moe_init_routing_v3(x, idx, scale, E, rng_, 1, row_idx_type)
             assert np.array_equal(ri, ri_r) and np.array_equal(cnt, cnt_r) and np.array_equal(es, es_r)
             assert np.array_equal(ex.view(np.uint8), ex_r.view(np.uint8))
+
+
+@pytest.mark.parametrize("T,K,H,dtype_name", [
+    (3, 2, 8, "bf16"), (5, 4, 4096, "f32"), (5, 4, 4104, "f16"), (4, 8, 8192, "bf16"), (4, 3, 8200, "bf16"),
+    (2, 64, 16384, "f16"),       # the widest row and the most experts per token of the packet kernel
+    (2, 65, 64, "bf16"), (2, 4, 16392, "bf16"), (3, 4, 4100, "bf16")])  # one past either, and no whole packets
+def test_dynamic_quant_row_widths(aclnn, oracle, dev, T, K, H, dtype_name):
+    """Dynamic quantisation without a smooth scale at the widths where its kernels change hands (4096 elements per packet
+    of a workgroup, up to four packets), through both operators, on outputs that do not start at zero."""
+    rng = np.random.default_rng(T * 3 + H)
+    E = 70
+    xt, bits, idx, code = _quant_v2_inputs(rng, T, K, E, H, dtype_name, oracle)
+    x, i = xt.to(dev), torch.from_numpy(idx).to(dev)
+    for kw in (dict(expert_tokens_count_or_cumsum_flag=2), dict(expert_tokens_count_or_cumsum_flag=1, active_num=T),
+               dict(drop_pad_mode=1, expert_capacity=max(1, T // 2), expert_tokens_before_capacity_flag=True)):
+        torch.full((64 << 20,), 77, dtype=torch.int8, device=dev)  # what the allocator hands out next is not zero
+        got = aclnn.moe_init_routing_quant_v2(x, i, 1, None, None, expert_num=E, **kw)
+        want = oracle.moe_init_routing_quant_v2(
+            bits, idx, 1, None, None, active_num=kw.get("active_num", 0), expert_capacity=kw.get("expert_capacity", 0),
+            expert_num=E, drop_pad_mode=kw.get("drop_pad_mode", 0), count_flag=kw.get("expert_tokens_count_or_cumsum_flag", 0),
+            before_capacity_flag=kw.get("expert_tokens_before_capacity_flag", False), dtype=code)
+        for g, w, name in zip(got, want, ("expandedX", "expandedRowIdx", "countOrCumsum", "beforeCapacity", "dynScale")):
+            assert _same(g, w), (kw, name)
+    for mode, rng_ in ((0, None), (1, None), (2, None), (1, (10, 40))):
+        got = aclnn.moe_init_routing_v3(x, i, expert_num=E, expert_tokens_num_type=mode, quant_mode=1, active_expert_range=rng_)
+        want = oracle.moe_init_routing_v3_quant(bits, idx, None, E, rng_, mode, 1, dtype=code)
+        for g, w in zip(got, want):
+            assert np.array_equal(g.cpu().numpy(), w)
