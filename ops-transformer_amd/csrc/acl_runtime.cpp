@@ -8,6 +8,7 @@
 #include <mutex>
 #include <new>
 
+#include "opapi_descriptor.h"
 #include "opapi_profile.h"
 
 namespace {
@@ -337,6 +338,17 @@ aclnnStatus aclDestroyIntArray(const aclIntArray* array) {
 aclnnStatus aclDestroyAclOpExecutor(aclOpExecutor* executor) {
     delete executor;
     return ACLNN_SUCCESS;
+}
+
+aclTensor* opapiCreateTensorPacked(const int64_t* packed) {
+    if (packed == nullptr || packed[0] < 0 || packed[0] > 8) return nullptr;
+    const uint64_t nd = static_cast<uint64_t>(packed[0]);
+    const int64_t* const dims = packed + 3;
+    return aclCreateTensor(dims, nd, static_cast<aclDataType>(packed[1]), dims + nd, 0, ACL_FORMAT_ND, dims, nd,
+                           reinterpret_cast<void*>(static_cast<uintptr_t>(packed[2])));
+}
+void opapiDestroyTensors(const aclTensor* const* tensors, uint64_t count) {
+    for (uint64_t i = 0; tensors != nullptr && i < count; ++i) delete tensors[i];
 }
 
 const char* aclGetRecentErrMsg(void) { return g_lastError.c_str(); }

@@ -704,3 +704,15 @@ def test_strided_inputs_are_staged_in_the_workspace(aclnn):
     args[0] = T(aclnn, (16, 256), I8, strides=[512, 1]).h                # x
     code, ws = _status(aclnn, "aclnnGroupedMatmulSwigluQuant", args)
     assert code == 0 and ws == (own + 255) // 256 * 256 + 16 * 256
+
+
+@pytest.mark.parametrize("dims", [0, 1, 3, 8])
+def test_packed_descriptors(aclnn, dims):
+    """Descriptors of torch tensors, views with strides of their own among them, up to eight dimensions."""
+    t = torch.zeros((2,) * dims, dtype=torch.bool).permute(*reversed(range(dims)))
+    handles = aclnn._Handles()
+    assert handles.tensor(t) and handles.tensor(t) and handles.tensor(None) is None
+    handles.close()
+    handles.close()
+    with pytest.raises(MemoryError):
+        aclnn.tensor_of(torch.zeros((1,) * 9))
