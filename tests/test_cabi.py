@@ -12,6 +12,7 @@ import os
 import re
 
 import pytest
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 NULLPTR, INVALID = 161001, 161002
@@ -709,7 +710,7 @@ def test_strided_inputs_are_staged_in_the_workspace(aclnn):
 @pytest.mark.parametrize("dims", [0, 1, 3, 8])
 def test_packed_descriptors(aclnn, dims):
     """Descriptors of torch tensors, views with strides of their own among them, up to eight dimensions."""
-    t = torch.zeros((2,) * dims, dtype=torch.bool).permute(*reversed(range(dims)))
+    t = torch.zeros((2,) * dims, dtype=torch.bool).permute(tuple(reversed(range(dims))))
     handles = aclnn._Handles()
     assert handles.tensor(t) and handles.tensor(t) and handles.tensor(None) is None
     handles.close()
