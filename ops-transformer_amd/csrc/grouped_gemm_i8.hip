@@ -378,6 +378,10 @@ double RoundEfficiency(int64_t tiles) {
 // tile, twice as many channels wide, moves less per weight byte: gate/up of 31 rows each for 128 experts, hidden 4096,
 // intermediate 1536, takes it 280 us against 300; it is left where its tiles fill the machine's rounds worse by more than
 // that (a down projection of 128 of them: 115 us against 78).
+// Groups of any size take the 64-row tiles where all of them are at most one round of the machine: taller and wider tiles
+// would leave it idle (64 rows each for 8 experts, hidden 1024, intermediate 1024: 64 and 32 tiles of 96 x 256 take 18.8 and
+// 16.7 us plus 4.8 us each for their table; 256 and 128 of these 12.6 and 11.3 us), and a group's m-tiles, side by side on
+// one XCD, share its weights through L2.
 // A forced tile height (OPAPI_GEMM_TILE_M) or tile order (OPAPI_GEMM_PULL) means the kernels those belong to.
 int SlimTileRows(const Problem& p, double meanRows) {
     if (!StreamOk(p) || !(p.wKMajor || p.wNz) || p.groups > kSlimMaxGroups || p.M > kSlimMaxRows || p.groupListKind == GroupListKind::kSparse ||
@@ -389,9 +393,10 @@ int SlimTileRows(const Problem& p, double meanRows) {
     const double want = RowsOfNearlyEveryGroup(meanRows);
     if (want <= 16.0) return 16;
     if (want <= 32.0) return 32;
-    if (want > 64.0) return 0;
     const int64_t cols = p.epilogue == Epilogue::kSwiglu ? p.N / 2 : p.N;
     const int64_t wide = p.epilogue == Epilogue::kSwiglu ? kTileN / 2 : kTileN, slim = wide * kSlimTileN / kTileN;
+    if (p.groups * static_cast<int64_t>(std::ceil(want / 64.0)) * ((cols + slim - 1) / slim) <= DeviceCuCount()) return 64;
+    if (want > 64.0) return 0;
     return RoundEfficiency(p.groups * ((cols + slim - 1) / slim)) > 1.06 * RoundEfficiency(p.groups * ((cols + wide - 1) / wide)) ? 64 : 0;
 }
 

@@ -18,6 +18,7 @@ CASES = {
     "tile32": ([20, 0, 31, 32, 33, 9, 18, 14] * 6, 384, 1344),
     "tile64_deep": ([64, 40, 65, 20], 640, 224),
     "tile64": ([64, 30, 65, 0, 40, 63, 12, 33, 49, 31] * 4, 272, 1600),
+    "tile64_one_round": ([100, 64, 0, 65, 130, 290], 400, 448),                      # taller groups, but few tiles in all
     "skewed": ([150, 0, 1, 0, 0, 2, 0, 0, 1, 0, 3, 0, 0, 0, 1, 0] * 4, 512, 576),     # several m-tiles of one group
 }
 
