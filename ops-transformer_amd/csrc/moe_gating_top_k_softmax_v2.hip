@@ -14,6 +14,8 @@
 
 #include <hip/hip_fp16.h>
 
+#include <type_traits>
+
 #include "aclnnop/aclnn_moe_gating_top_k_softmax_v2.h"
 
 namespace {
@@ -192,6 +194,110 @@ __global__ __launch_bounds__(kWave * kWaves) void GatingTopKKernel(GatingArgs a)
     }
 }
 
+// Rows of up to 512 columns with at most 64 picks (every router in use): one wave per row, four independent rows per
+// workgroup, the keys in registers (column lane + 64 i in register i), the picks in lane j of the wave.  What bounds it is
+// the latency of one row, k dependent rounds of arg-max: the general kernel goes through LDS for the scan and for twelve
+// shuffles in every round; here a round is four rotations inside a row of sixteen lanes, four lane reads and a ballot.
+// Sums run in the same order as there, so results are the same bits.
+// 2047 rows of 128 fp32 logits, 8 picks: 10.9 -> 5.6 us; 23 rows: 6.2 -> 5.2 us.
+constexpr int kGatingRowsPerBlock = 4;
+constexpr int kWaveCols = 512;
+constexpr int kWavePicks = 64;
+
+__device__ __forceinline__ uint32_t WaveMaxUniform(uint32_t v) {
+    auto ror = [](uint32_t u, auto ctl) __attribute__((always_inline)) {
+        return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(u), decltype(ctl)::value, 0xF, 0xF, true));
+    };
+    v = max(v, ror(v, std::integral_constant<int, 0x128>{}));  // row_ror:8
+    v = max(v, ror(v, std::integral_constant<int, 0x124>{}));
+    v = max(v, ror(v, std::integral_constant<int, 0x122>{}));
+    v = max(v, ror(v, std::integral_constant<int, 0x121>{}));
+    const int i = static_cast<int>(v);
+    return max(max(static_cast<uint32_t>(__builtin_amdgcn_readlane(i, 0)), static_cast<uint32_t>(__builtin_amdgcn_readlane(i, 16))),
+               max(static_cast<uint32_t>(__builtin_amdgcn_readlane(i, 32)), static_cast<uint32_t>(__builtin_amdgcn_readlane(i, 48))));
+}
+
+template <typename Codec, int kPer>
+__global__ __launch_bounds__(kWave * kGatingRowsPerBlock) void GatingTopKWaveKernel(GatingArgs a) {
+    const int lane = threadIdx.x % kWave;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * kGatingRowsPerBlock + threadIdx.x / kWave;
+    if (row >= a.rows) return;
+    const typename Codec::Storage* x = static_cast<const typename Codec::Storage*>(a.x) + row * a.cols;
+    float v[kPer];
+    uint32_t keys[kPer];
+    float localMax = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int c = lane + kWave * i;
+        v[i] = c < a.cols ? Codec::Load(x[c]) : -INFINITY;
+        if (c < a.cols) localMax = fmaxf(localMax, v[i]);
+    }
+    if (a.renorm == 0) {
+        const float rowMax = BlockMax<1>(localMax, nullptr);
+        float localSum = 0.f;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            if (lane + kWave * i >= a.cols) continue;
+            v[i] = expf(v[i] - rowMax);
+            localSum += v[i];
+        }
+        const float sum = BlockSum<1>(localSum, nullptr);
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int c = lane + kWave * i;
+            if (c >= a.cols) continue;
+            v[i] = v[i] / sum;
+            if (a.softmaxOut != nullptr) a.softmaxOut[row * a.cols + c] = v[i];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) keys[i] = lane + kWave * i < a.cols ? KeyOf(v[i]) : 0u;
+
+    uint32_t pickKey = 0;
+    int32_t pickIdx = 0;
+    for (int j = 0; j < a.k; ++j) {
+        uint32_t best = keys[0];
+        int32_t at = lane < a.cols ? lane : INT32_MAX;  // absent columns lose to a key of zero as well
+#pragma unroll
+        for (int i = 1; i < kPer; ++i) {
+            if (keys[i] > best) {  // equal keys: the lower column stays
+                best = keys[i];
+                at = lane + kWave * i;
+            }
+        }
+        const uint32_t top = WaveMaxUniform(best);
+        const uint64_t holders = __ballot(best == top);
+        int32_t idx;
+        if ((holders & (holders - 1)) == 0) {
+            idx = __builtin_amdgcn_readlane(at, __ffsll(static_cast<unsigned long long>(holders)) - 1);
+        } else {  // equal values: the lowest column
+            idx = best == top ? at : INT32_MAX;
+            for (int d = 32; d > 0; d >>= 1) idx = min(idx, __shfl_xor(idx, d));
+            idx = __builtin_amdgcn_readfirstlane(idx);
+        }
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            if (idx == lane + kWave * i) keys[i] = 0u;
+        }
+        if (lane == j) {
+            pickKey = top;
+            pickIdx = idx;
+        }
+    }
+
+    const bool done = a.finished != nullptr && a.finished[row] != 0;
+    float y = ValueOf(pickKey);
+    if (a.renorm != 0) {
+        const float top = ValueOf(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(pickKey))));
+        y = lane < a.k ? expf(y - top) : 0.f;
+        y = y / BlockSum<1>(y, nullptr);
+    }
+    if (lane < a.k) {
+        static_cast<typename Codec::Storage*>(a.y)[row * a.k + lane] = Codec::Store(y);
+        a.expertIdx[row * a.k + lane] = done ? a.cols : pickIdx;
+    }
+}
+
 class GatingExecutor : public aclOpExecutor {
    public:
     GatingArgs args{};
@@ -215,8 +321,21 @@ class GatingExecutor : public aclOpExecutor {
         return hipGetLastError();
     }
 
+    template <typename Codec, int kPer>
+    hipError_t LaunchWaves(hipStream_t stream) const {
+        const unsigned blocks = static_cast<unsigned>((args.rows + kGatingRowsPerBlock - 1) / kGatingRowsPerBlock);
+        hipLaunchKernelGGL((GatingTopKWaveKernel<Codec, kPer>), dim3(blocks), dim3(kWave * kGatingRowsPerBlock), 0, stream, args);
+        return hipGetLastError();
+    }
+
     template <typename Codec>
     hipError_t LaunchForWidth(hipStream_t stream) const {
+        if (args.cols <= kWaveCols && args.k <= kWavePicks) {
+            if (args.cols <= 64) return LaunchWaves<Codec, 1>(stream);
+            if (args.cols <= 128) return LaunchWaves<Codec, 2>(stream);
+            if (args.cols <= 256) return LaunchWaves<Codec, 4>(stream);
+            return LaunchWaves<Codec, 8>(stream);
+        }
         if (args.cols <= 512) return Launch<Codec, 1>(stream);
         if (args.cols <= 4096) return Launch<Codec, 4>(stream);
         return Launch<Codec, 16>(stream);

@@ -110,3 +110,21 @@ def test_router_feeds_the_ffn_chain(pkg, aclnn, oracle, dev):
     counts = np.bincount(idx.cpu().numpy().reshape(-1), minlength=cfg.experts)
     assert np.array_equal(np.cumsum(counts), ffn.cumsum.cpu().numpy())
     np.testing.assert_allclose(wgt.sum(-1).cpu().numpy(), 1.0, rtol=1e-5)
+
+
+@pytest.mark.parametrize("cols", [1, 63, 64, 65, 127, 130, 257, 511, 512, 513])
+def test_many_equal_values(aclnn, dev, cols):
+    """Columns either side of a wave's registers, one to sixty-five picks, values that repeat, -inf and NaN among them: the
+    picks are the first k of a stable descending sort (a positive NaN sorts above +inf, a negative one below -inf)."""
+    rng = np.random.default_rng(cols)
+    x = rng.integers(-3, 4, (7, cols)).astype(np.float32)
+    x[1, ::3] = -np.inf
+    x[2, ::5] = np.inf
+    x[3] = 0.0
+    x[4, cols // 2] = np.nan
+    u = x.view(np.uint32).astype(np.int64)
+    key = np.where(u & 0x80000000, 0xffffffff - u, u | 0x80000000)
+    order = np.argsort(-key, axis=1, kind="stable")
+    for k in sorted({1, min(8, cols), min(64, cols), min(65, cols), cols}):
+        _, idx, _ = aclnn.moe_gating_top_k_softmax_v2(torch.from_numpy(x).to(dev), k, renorm=1)
+        assert np.array_equal(idx.cpu().numpy(), order[:, :k])
