@@ -215,6 +215,7 @@ __global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, Sli
     const bool hasRowScale = a.rowScale != nullptr;
     const bool hasScale = a.scale != nullptr;
     const bool scaleByDma = hasScale && a.scaleDtype == 0;
+    const bool splitLines = !kNz && a.K % 128 != 0;
 
     // ---- issue side
     const uint32_t ldsBase = LdsAddress(lds);
@@ -287,10 +288,19 @@ __global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, Sli
         for (int q = 0; q < Cfg::kSlotsA; ++q) {
             DmaToLdsAddr16<false>(issBaseA + kOff, offA[q], dst + ((wave + 4 * q) % Cfg::kInstrA) * 1024);
         }
+        // Every weight byte is used once per m-tile: past the caches.  Not so the lines: rows that do not start on one
+        // have their 128 bytes of a k-step in two, each wanted again by the next step (K 2880 / 1440, 37 rows each for 32
+        // experts: 68.8 -> 64.6 us gate/up, 41.8 -> 39.0 us down).
+        if (splitLines) {
 #pragma unroll
-        for (int q = 0; q < Cfg::kSlotsB; ++q) {
-            // every weight byte is used once per m-tile: past the caches
-            DmaToLdsAddr16<true>(issBaseB + kOffW, offB[q], dst + Cfg::kStageA + (wave + 4 * q) * 1024);
+            for (int q = 0; q < Cfg::kSlotsB; ++q) {
+                DmaToLdsAddr16<false>(issBaseB + kOffW, offB[q], dst + Cfg::kStageA + (wave + 4 * q) * 1024);
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < Cfg::kSlotsB; ++q) {
+                DmaToLdsAddr16<true>(issBaseB + kOffW, offB[q], dst + Cfg::kStageA + (wave + 4 * q) * 1024);
+            }
         }
         issSlot = issSlot + 1 == kStages ? 0 : issSlot + 1;
         issK = issK + 1 == kSteps ? 0 : issK + 1;  // back at kStart after a tile's kSteps
