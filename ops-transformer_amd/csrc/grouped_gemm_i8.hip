@@ -434,7 +434,11 @@ Plan MakePlan(const Problem& p) {
         return plan;
     }
     const double rounds = static_cast<double>(groups) * plan.tilesN / DeviceCuCount();
-    const double want = meanRows * (rounds <= 24.0 ? 1.5 : 1.25);
+    double want = meanRows * (rounds <= 24.0 ? 1.5 : 1.25);
+    // Without the SwiGLU epilogue 160 rows are enough where they hold nearly every group: their activation ring is a stage deeper than
+    // that of 192 (128 rows each, K 1536 x N 4096, 128 experts: 233 -> 221 us; K 2048 x N 7168, 256 experts: 853 / 795).
+    // The SwiGLU operator has it the other way round: 379 us with 192 rows, 418 with 160 (N 3072, K 4096, 128 experts).
+    if (p.epilogue != Epilogue::kSwiglu && want > 160.0 && RowsOfNearlyEveryGroup(meanRows) <= 160.0) want = 160.0;
     if (StreamOk(p)) {
         static const int kShapes[] = {32, 64, 96, 128, 160, 192, 256};
         plan.tileM = 256;
