@@ -332,10 +332,11 @@ def moe_init_routing_quant_v2(x, expert_idx, quant_mode, scale=None, offset=None
     T, H = x.shape
     K = expert_idx.shape[1]
     dev = x.device
-    # The operator writes every element of its outputs, padding slots included, unless there is nothing to route or a
-    # smooth scale leaves out rows whose expert id is none of its rows: only then do the outputs have to start at zero.
+    # The operator writes every element of its outputs, padding slots included, unless there is nothing to route, rows
+    # have no columns (the kernel that writes their scales is not launched), or a smooth scale leaves out rows whose expert
+    # id is none of its rows: only then do the outputs have to start at zero.
     # (A fill is a launch of its own: 5 us each at decode sizes, 11 us for the rows of a 2047-token call.)
-    fresh = torch.zeros if scale is not None or T * K == 0 else torch.empty
+    fresh = torch.zeros if scale is not None or T * K * H == 0 else torch.empty
     if drop_pad_mode == 1:
         expanded_x = fresh((expert_num, expert_capacity, H), dtype=torch.int8, device=dev)
         rows = expert_num * expert_capacity
@@ -392,7 +393,7 @@ def moe_init_routing_v3(x, expert_idx, scale=None, expert_num=0, expert_tokens_n
     else:
         # As in moe_init_routing_quant_v2; a range of experts leaves the rows of the others unwritten, and key/value
         # counts what lies behind their last pair.
-        fresh = (torch.zeros if active_expert_range is not None or expert_tokens_num_type == 2 or T * K == 0 or
+        fresh = (torch.zeros if active_expert_range is not None or expert_tokens_num_type == 2 or T * K * H == 0 or
                  (quant_mode == 1 and scale is not None) else torch.empty)
         expanded_x = fresh((T * K, H), dtype=torch.int8 if quant_mode == 1 else x.dtype, device=dev)
         row_idx = torch.empty((T * K,), dtype=torch.int32, device=dev)

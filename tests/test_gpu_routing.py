@@ -460,3 +460,26 @@ def test_dynamic_quant_row_widths(aclnn, oracle, dev, T, K, H, dtype_name):
         want = oracle.moe_init_routing_v3_quant(bits, idx, None, E, rng_, mode, 1, dtype=code)
         for g, w in zip(got, want):
             assert np.array_equal(g.cpu().numpy(), w)
+
+
+@pytest.fixture
+def dirty_memory(monkeypatch):
+    """torch.empty hands out 77s and NaNs: an output element that nothing writes shows."""
+    empty = torch.empty
+
+    def dirty(*args, **kw):
+        t = empty(*args, **kw)
+        return t.fill_(float("nan") if t.is_floating_point() else 77)
+    monkeypatch.setattr(torch, "empty", dirty)
+
+
+@pytest.mark.parametrize("drop_pad", [0, 1])
+def test_dynamic_quant_of_a_row_without_columns(aclnn, dev, dirty_memory, drop_pad):
+    """H = 0 (accepted for a single row: an empty matrix of more rows does not count as contiguous): there is nothing to
+    quantise, and the row's scale is that of an all-zero row."""
+    x, idx = torch.zeros((1, 0), dtype=torch.bfloat16, device=dev), torch.zeros((1, 1), dtype=torch.int32, device=dev)
+    _, _, _, _, scale = aclnn.moe_init_routing_quant_v2(x, idx, 1, expert_num=1, drop_pad_mode=drop_pad, expert_capacity=drop_pad)
+    assert scale.tolist() == [0.0]
+    if not drop_pad:
+        _, _, counts, scale = aclnn.moe_init_routing_v3(x, idx, expert_num=4, expert_tokens_num_type=1, quant_mode=1)
+        assert scale.tolist() == [0.0] and counts.tolist() == [1, 0, 0, 0]
