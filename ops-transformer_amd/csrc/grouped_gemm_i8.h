@@ -61,7 +61,7 @@ constexpr int64_t kSlimMaxRows = 65535;
 
 // Tile shape chosen from the static shape (M, groups); fixed for the lifetime of a plan.
 struct Plan {
-    int tileM = 0;          // rows per workgroup tile (multiple of 32)
+    int tileM = 0;          // rows per workgroup tile (multiple of 32; slim: 16, 32 or 64, the lowest that the kernel may take)
     int wavesM = 1;         // 1 or 2 wave rows
     int subTilesM = 1;      // 32-row MFMA tiles per wave
     int64_t maxTiles = 0;   // launch bound on workgroups

@@ -374,7 +374,8 @@ double RoundEfficiency(int64_t tiles) {
 }
 
 // Rows per tile of the kernels for a handful of rows per group, or 0 where they are not the ones to run.  A tile has to hold
-// nearly every group whole, since a second tile reads the group's weights again.  At 64 rows the LDS-ring kernel's 64-row
+// nearly every group whole, since a second tile reads the group's weights again.  This is the height for groups that spread
+// like a Poisson variable; the kernel takes taller tiles where the list it finds is more uneven than that.  At 64 rows the LDS-ring kernel's 64-row
 // tile, twice as many channels wide, moves less per weight byte: gate/up of 31 rows each for 128 experts, hidden 4096,
 // intermediate 1536, takes it 280 us against 300; it is left where its tiles fill the machine's rounds worse by more than
 // that (a down projection of 128 of them: 115 us against 78).
@@ -574,7 +575,8 @@ hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStrea
                                      : p.combineIndex != nullptr ? "gmm_combine" : "gmm_dequant", stream);
             if (plan.slim) {
                 if (p.epilogue == Epilogue::kInt32) ka.scale = nullptr;  // raw accumulators
-                const SlimList list{p.groupList, sa.groupListIsInt64, sa.isCount, p.groups, sched + kHdrCoveredRows};
+                const SlimList list{p.groupList, sa.groupListIsInt64, sa.isCount, p.groups, plan.tileM == 16 ? 0 : plan.tileM == 32 ? 1 : 2,
+                                    sched + kHdrCoveredRows};
                 e = swiglu ? LaunchSlimSwiglu(plan, ka, list, stream) : LaunchSlimPlain(plan, ka, list, stream);
             } else switch (p.epilogue) {
                 case Epilogue::kInt32:

@@ -61,6 +61,7 @@ struct SlimList {
     int32_t isInt64;
     int32_t isCount;
     int32_t groups;
+    int32_t minHeight;     // lowest tiles to consider, as log2(rows / 16)
     int32_t* coveredRows;  // written by workgroup 0: rows covered by the list (the requantisation reads it)
 };
 

@@ -11,7 +11,8 @@
 //     64 tokens  (127, 2.4 GB)                               255 -> 254                       139 -> 125 (6.4 TB/s)
 //   hidden 4096, intermediate 14336, 8 experts, top-2, 64 tokens     178 -> 168               113 -> 77
 // The split:
-//   * A tile is 16 / 32 / 64 rows x 128 channels, a workgroup four waves of 32 channels on v_mfma_i32_16x16x64_i8, one
+//   * A tile is 16 / 32 / 64 rows x 128 channels (the lowest that holds the mean group nearly whole, or a taller one where
+//     the list at hand needs it: SlimGroupTable), a workgroup four waves of 32 channels on v_mfma_i32_16x16x64_i8, one
 //     workgroup per CU with a ring of six to eight stages of 16 KB of weights.  (Two workgroups per CU with half the ring
 //     each measured the same within 1 % on everything but launches of few tiles, where they lose up to 15 %.)  Half the
 //     channels of the 256-wide tiles: twice the tiles, so the last round of a launch leaves less of the machine idle.
@@ -35,6 +36,8 @@ namespace {
 constexpr int kSlimThreads = 256;
 constexpr int kSlimCols = kSlimTileN;     // channels per tile
 constexpr int kSlimTable = kSlimMaxGroups;
+constexpr int kSlimTableBytes = 3328;     // prefix, first row and rows of every group (16 bits each), four totals per wave
+static_assert(3 * kSlimTable * 2 + 16 * 4 <= kSlimTableBytes && kSlimTableBytes % 256 == 0, "the table in front of the ring");
 
 template <int kMi, int kStages>
 struct SlimCfg {
@@ -46,9 +49,8 @@ struct SlimCfg {
     static constexpr int kSlotsB = kStageB / 1024 / 4;
     static constexpr int kPerWave = kSlotsA + kSlotsB;
     static constexpr int kScaleFloats = kSlimCols + 64;    // per tile: channel scales, then row scales
-    static constexpr int kOffScales = kStages * (kStageA + kStageB);
-    static constexpr int kOffTable = kOffScales + kStages * kScaleFloats * 4;
-    static constexpr int kLdsBytes = kOffTable + 3 * kSlimTable * 2 + 64;
+    static constexpr int kOffScales = kSlimTableBytes + kStages * (kStageA + kStageB);  // the ring is behind the table
+    static constexpr int kLdsBytes = kOffScales + kStages * kScaleFloats * 4;
     static_assert(kSlotsA + kSlotsB <= 8 && (kStages - 2) * kPerWave <= 63, "vmcnt is a 6-bit counter");
     static_assert(kLdsBytes <= kLdsBudget, "LDS of one workgroup");
 };
@@ -72,6 +74,31 @@ __device__ __forceinline__ float MaxOver16(float v) {
     return fmaxf(v, ror(v, std::integral_constant<int, 0x121>{}));
 }
 
+// Relative cost of a tile of 16, 32 or 64 rows: its weights are the same, but a taller one leaves the ring fewer stages (64
+// tokens evenly over 128 experts, hidden 4096, intermediate 1536: 247 / 251 / 262 us gate/up).  A launch costs its rounds of
+// tiles times that.  What speaks for a taller tile is groups that need several of the lower ones; how many there are is known
+// here and not to the planner, which has only the mean.  Kernel time on the planner's height and on the one chosen here, and
+// the ring kernel's 64-row tiles beside them (1024 rows, all on eight of 256 experts, hidden 7168, intermediate 2048,
+// 16-row tiles planned): 143 -> 64 us, ring 67; popularity falling as rank^-1.2, 128 tokens: gate/up 347 -> 275, ring 308;
+// 512 tokens (32 rows planned): 630 -> 555, ring 689.
+__device__ constexpr uint32_t kSlimTileCost[3] = {50, 51, 62};
+
+// Inclusive sum over the wave, without LDS: inside the rows of sixteen lanes, then the rows' totals into those behind them.
+// (As six shuffles, three of these sums put 0.5 us more into the head of every launch.)
+__device__ __forceinline__ int32_t WaveInclusiveSum(int32_t v) {
+    auto add = [&](auto ctl, auto rows) __attribute__((always_inline)) {
+        v += __builtin_amdgcn_update_dpp(0, v, decltype(ctl)::value, decltype(rows)::value, 0xF, false);
+    };
+    using All = std::integral_constant<int, 0xF>;
+    add(std::integral_constant<int, 0x111>{}, All{});  // row_shr:1, 2, 4, 8
+    add(std::integral_constant<int, 0x112>{}, All{});
+    add(std::integral_constant<int, 0x114>{}, All{});
+    add(std::integral_constant<int, 0x118>{}, All{});
+    add(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // row_bcast:15 into rows 1 and 3
+    add(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 struct SlimTile {
     int32_t valid;
     int32_t group;
@@ -79,91 +106,120 @@ struct SlimTile {
     int32_t rows;
     int32_t tileN;
     int32_t part;  // of the tile's four 32-channel columns, this workgroup computes (4 >> cut) from part * (4 >> cut) on
+    int32_t shared;  // its weights are another m-tile's as well
+    int32_t kStart;  // k-step that its walk starts from
 };
+
+// The table of a launch, in LDS: m-tiles of groups 0 .. g, first row and rows of group g.
+struct SlimGroups {
+    uint16_t* incl;
+    uint16_t* start;
+    uint16_t* rows;
+};
+
+// Workgroup-wide: the group list becomes the prefix table.  Thread t owns groups 2t and 2t + 1.  Boundaries are clamped into
+// [0, M] and the prefix saturates, so that a malformed list cannot push an access out of bounds.  Returns the tile height,
+// as log2(rows / 16): the lowest from sl.minHeight on unless a taller one is the cheaper for this list.
+__device__ __forceinline__ int SlimGroupTable(const KernelArgs& a, const SlimList& sl, char* const lds, const SlimGroups& table) {
+    int32_t* const waveTotal = reinterpret_cast<int32_t*>(lds + 3 * kSlimTable * 2);  // [4][4]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g0 = 2 * tid, g1 = g0 + 1;
+    // entries g0 - 1, g0 and g1 in one round trip (indices clamped into the list)
+    int32_t vPrev, v0, v1;
+    {
+        const int last = sl.groups - 1;
+        const int iPrev = min(max(g0 - 1, 0), last), i0 = min(g0, last), i1 = min(g1, last);
+        auto clamped = [&](int64_t v) { return static_cast<int32_t>(v < 0 ? 0 : (v > a.M ? a.M : v)); };
+        if (sl.isInt64) {
+            const int64_t* const p = static_cast<const int64_t*>(sl.list);
+            const int64_t w0 = p[iPrev], w1 = p[i0], w2 = p[i1];
+            vPrev = clamped(w0);
+            v0 = clamped(w1);
+            v1 = clamped(w2);
+        } else {
+            const int32_t* const p = static_cast<const int32_t*>(sl.list);
+            const int32_t w0 = p[iPrev], w1 = p[i0], w2 = p[i1];
+            vPrev = clamped(w0);
+            v0 = clamped(w1);
+            v1 = clamped(w2);
+        }
+    }
+    // a wave's sums to the workgroup's: slot is the wave's of four totals that it leaves for the others
+    auto leaveTotal = [&](int32_t inclusive, int slot) __attribute__((always_inline)) {
+        if (lane == 63) waveTotal[4 * slot + wave] = inclusive;
+    };
+    auto wavesBefore = [&](int slot, int waves) __attribute__((always_inline)) {
+        const int4 t = *reinterpret_cast<const int4*>(waveTotal + 4 * slot);
+        return (waves > 0 ? t.x : 0) + (waves > 1 ? t.y : 0) + (waves > 2 ? t.z : 0) + (waves > 3 ? t.w : 0);
+    };
+    int32_t b0 = 0, e0 = 0, b1 = 0, e1 = 0;
+    if (sl.isCount) {
+        const int32_t c0 = g0 < sl.groups ? v0 : 0, c1 = g1 < sl.groups ? v1 : 0;
+        // counts may add up to more than M: 256 x 2 x 65535 still fits
+        const int32_t incl = WaveInclusiveSum(c0 + c1);
+        leaveTotal(incl, 3);
+        __syncthreads();
+        const int32_t before = incl - c0 - c1 + wavesBefore(3, wave);
+        b0 = min(before, a.M);
+        e0 = min(before + c0, a.M);
+        b1 = e0;
+        e1 = min(before + c0 + c1, a.M);
+    } else {
+        b0 = g0 > 0 ? vPrev : 0;
+        e0 = v0;
+        b1 = e0;
+        e1 = v1;
+    }
+    const int32_t r0 = g0 < sl.groups ? max(e0 - b0, 0) : 0, r1 = g1 < sl.groups ? max(e1 - b1, 0) : 0;
+    // m-tiles of 16, 32 and 64 rows
+    auto mTiles = [](int32_t rows, int height) { return (rows + (16 << height) - 1) >> (4 + height); };
+    int32_t incl[3];
+#pragma unroll
+    for (int h = 0; h < 3; ++h) {
+        incl[h] = WaveInclusiveSum(mTiles(r0, h) + mTiles(r1, h));
+        leaveTotal(incl[h], h);
+    }
+    __syncthreads();
+    auto all = [&](int h) __attribute__((always_inline)) { return static_cast<uint32_t>(min(__builtin_amdgcn_readfirstlane(wavesBefore(h, 4)), 65535)); };
+    const uint32_t total[3] = {all(0), all(1), all(2)};
+    int height = sl.minHeight;
+    if ((height == 0 ? total[0] : total[1]) != total[2] && height < 2) {
+        const uint32_t grid = gridDim.x;
+        auto cost = [&](int h) __attribute__((always_inline)) { return (total[h] * a.tilesN + grid - 1) / grid * kSlimTileCost[h]; };
+        const uint32_t cost16 = cost(0), cost32 = cost(1), cost64 = cost(2);
+        if (height == 0 && cost32 < cost16) height = 1;
+        if (cost64 < (height == 0 ? cost16 : cost32)) height = 2;
+    }
+    const int32_t mt1 = height == 0 ? mTiles(r1, 0) : height == 1 ? mTiles(r1, 1) : mTiles(r1, 2);
+    const int32_t incl1 = (height == 0 ? incl[0] : height == 1 ? incl[1] : incl[2]) + wavesBefore(height, wave);
+    table.incl[g0] = static_cast<uint16_t>(min(incl1 - mt1, 65535));
+    table.incl[g1] = static_cast<uint16_t>(min(incl1, 65535));
+    table.start[g0] = static_cast<uint16_t>(b0);
+    table.start[g1] = static_cast<uint16_t>(b1);
+    table.rows[g0] = static_cast<uint16_t>(r0);
+    table.rows[g1] = static_cast<uint16_t>(r1);
+    if (blockIdx.x == 0 && (g0 == sl.groups - 1 || g1 == sl.groups - 1)) {
+        *sl.coveredRows = g1 == sl.groups - 1 ? max(e1, b1) : max(e0, b0);
+    }
+    __syncthreads();
+    return height;
+}
 
 // kNz: weights in the blocked layout instead of K-contiguous channels.
 template <int kMi, int kStages, bool kSwiglu, bool kNz>
-__global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, SlimList sl) {
+__device__ __forceinline__ void SlimGemmBody(const KernelArgs& a, const SlimGroups& table, char* const lds, uint64_t& spanTiles) {
     using Cfg = SlimCfg<kMi, kStages>;
-    extern __shared__ __attribute__((aligned(16))) char lds[];
-    const uint64_t spanStart = a.wgSpans != nullptr ? __builtin_amdgcn_s_memrealtime() : 0;
-    uint64_t spanTiles = 0;
-    uint16_t* const tabIncl = reinterpret_cast<uint16_t*>(lds + Cfg::kOffTable);  // m-tiles of groups 0 .. g
-    uint16_t* const tabStart = tabIncl + kSlimTable;                              // first row of group g
-    uint16_t* const tabRows = tabStart + kSlimTable;
-    int32_t* const waveTotal = reinterpret_cast<int32_t*>(tabRows + kSlimTable);  // [8]
+    const uint16_t* const tabIncl = table.incl;
+    const uint16_t* const tabStart = table.start;
+    const uint16_t* const tabRows = table.rows;
+    char* const ringBase = lds + kSlimTableBytes;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15;
     const int quad = lane >> 4;
 
-    // ---- group list -> prefix table.  Thread t owns groups 2t and 2t + 1.  Boundaries are clamped into [0, M] and made
-    // monotonic, and the prefix saturates, so that a malformed list cannot push an access out of bounds.
-    {
-        const int g0 = 2 * tid, g1 = g0 + 1;
-        // entries g0 - 1, g0 and g1 in one round trip (indices clamped into the list)
-        int32_t vPrev, v0, v1;
-        {
-            const int last = sl.groups - 1;
-            const int iPrev = min(max(g0 - 1, 0), last), i0 = min(g0, last), i1 = min(g1, last);
-            auto clamped = [&](int64_t v) { return static_cast<int32_t>(v < 0 ? 0 : (v > a.M ? a.M : v)); };
-            if (sl.isInt64) {
-                const int64_t* const p = static_cast<const int64_t*>(sl.list);
-                const int64_t w0 = p[iPrev], w1 = p[i0], w2 = p[i1];
-                vPrev = clamped(w0);
-                v0 = clamped(w1);
-                v1 = clamped(w2);
-            } else {
-                const int32_t* const p = static_cast<const int32_t*>(sl.list);
-                const int32_t w0 = p[iPrev], w1 = p[i0], w2 = p[i1];
-                vPrev = clamped(w0);
-                v0 = clamped(w1);
-                v1 = clamped(w2);
-            }
-        }
-        auto exclusive = [&](int32_t v, int slot) -> int32_t {  // over the 256 threads
-            int32_t inc = v;
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const int32_t below = __shfl_up(inc, d, 64);
-                if (lane >= d) inc += below;
-            }
-            if (lane == 63) waveTotal[4 * slot + wave] = inc;
-            __syncthreads();
-            int32_t base = 0;
-            for (int w = 0; w < wave; ++w) base += waveTotal[4 * slot + w];
-            return base + inc - v;
-        };
-        int32_t b0 = 0, e0 = 0, b1 = 0, e1 = 0;
-        if (sl.isCount) {
-            const int32_t c0 = g0 < sl.groups ? v0 : 0, c1 = g1 < sl.groups ? v1 : 0;
-            // counts may add up to more than M: 256 x 2 x 65535 still fits
-            const int32_t before = exclusive(c0 + c1, 0);
-            b0 = min(before, a.M);
-            e0 = min(before + c0, a.M);
-            b1 = e0;
-            e1 = min(before + c0 + c1, a.M);
-        } else {
-            b0 = g0 > 0 ? vPrev : 0;
-            e0 = v0;
-            b1 = e0;
-            e1 = v1;
-        }
-        const int32_t r0 = g0 < sl.groups ? max(e0 - b0, 0) : 0, r1 = g1 < sl.groups ? max(e1 - b1, 0) : 0;
-        const int32_t m0 = (r0 + Cfg::kRows - 1) / Cfg::kRows, m1 = (r1 + Cfg::kRows - 1) / Cfg::kRows;
-        const int32_t before = exclusive(m0 + m1, 1);
-        tabIncl[g0] = static_cast<uint16_t>(min(before + m0, 65535));
-        tabIncl[g1] = static_cast<uint16_t>(min(before + m0 + m1, 65535));
-        tabStart[g0] = static_cast<uint16_t>(b0);
-        tabStart[g1] = static_cast<uint16_t>(b1);
-        tabRows[g0] = static_cast<uint16_t>(r0);
-        tabRows[g1] = static_cast<uint16_t>(r1);
-        if (blockIdx.x == 0 && (g0 == sl.groups - 1 || g1 == sl.groups - 1)) {
-            *sl.coveredRows = g1 == sl.groups - 1 ? max(e1, b1) : max(e0, b0);
-        }
-        __syncthreads();
-    }
     // ---- this workgroup's tiles: the list of (group, n-tile, m-tile) is cut into eight contiguous shares, one per XCD,
     // which the workgroups of an XCD walk side by side: the m-tiles of a group follow each other at one n-tile and share
     // its weights through L2, the n-tiles of a group share its rows.
@@ -179,6 +235,14 @@ __global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, Sli
     const int64_t xcdFirst = (blockIdx.x % kXcds) * perXcd;
     const int64_t xcdTiles = min(perXcd, totalTiles - xcdFirst);  // may be negative: nothing to do
     const int32_t slots = gridDim.x / kXcds, slot = blockIdx.x / kXcds;
+    const int kSteps = (a.K + 127) / 128;  // K off the step grid: the last step overlaps the one before (see kTail of StreamGemmBody)
+    // Every workgroup walks its tiles' k-steps from a start of its own and wraps (integer sums do not depend on the order):
+    // with rows a multiple of 4096 bytes apart the memory channel depends on the k offset alone, and workgroups at the
+    // same k-step would all queue on the same channels.  The m-tiles of a group have to meet in L2 instead: their start is
+    // that of the weight block they share.  (Not so where rows do not start on a cache line: they are spread over the
+    // channels as they are, and 320 rows at most for 32 experts, K 2880, take 96.6 us with a common start, 94.1 without.)
+    const bool splitLines = !kNz && a.K % 128 != 0;
+    const int32_t ownStart = static_cast<int32_t>((blockIdx.x * 7u + blockIdx.x / kXcds) % static_cast<unsigned>(kSteps));
     auto tileAt = [&](int32_t n) __attribute__((always_inline)) -> SlimTile {
         const int64_t local = slot + static_cast<int64_t>(n) * slots;
         SlimTile t{};
@@ -200,6 +264,8 @@ __global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, Sli
         t.group = g;
         t.tileN = idx / mTiles;
         t.part = logicalPart & ((1 << cut) - 1);
+        t.shared = mTiles > 1;
+        t.kStart = t.shared && !splitLines ? static_cast<int32_t>((g * 5u + t.tileN * 7u) % static_cast<unsigned>(kSteps)) : ownStart;
         t.rowBase = __builtin_amdgcn_readfirstlane(tabStart[g]) + mIn * Cfg::kRows;
         t.rows = min(Cfg::kRows, __builtin_amdgcn_readfirstlane(tabRows[g]) - mIn * Cfg::kRows);
         return t;
@@ -207,21 +273,15 @@ __global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, Sli
 
     SlimTile cur = tileAt(0);
     if (!cur.valid) return;
-    const int kSteps = (a.K + 127) / 128;  // K off the step grid: the last step overlaps the one before (see kTail of StreamGemmBody)
-    // Every workgroup walks its tiles' k-steps from a start of its own and wraps (integer sums do not depend on the order):
-    // with rows a multiple of 4096 bytes apart the memory channel depends on the k offset alone, and workgroups at the
-    // same k-step would all queue on the same channels.
-    const int kStart = static_cast<int>((blockIdx.x * 7u + blockIdx.x / kXcds) % static_cast<unsigned>(kSteps));
     const bool hasRowScale = a.rowScale != nullptr;
     const bool hasScale = a.scale != nullptr;
     const bool scaleByDma = hasScale && a.scaleDtype == 0;
-    const bool splitLines = !kNz && a.K % 128 != 0;
 
     // ---- issue side
     const uint32_t ldsBase = LdsAddress(lds);
     SlimTile iss = cur;
     int32_t issNo = 0;
-    int issStep = 0, issK = kStart, issSlot = 0, issScaleSlot = 0;
+    int issStep = 0, issK = cur.kStart, issSlot = 0, issScaleSlot = 0;
     bool drained = false;
     const char* issBaseA = nullptr;
     const char* issBaseB = nullptr;
@@ -283,15 +343,18 @@ __global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, Sli
         }
         const int kOff = drained ? 0 : min(issK * 128, a.K - 128);
         const int64_t kOffW = static_cast<int64_t>(kOff) * (kNz ? 32 : 1);
-        const uint32_t dst = ldsBase + issSlot * (Cfg::kStageA + Cfg::kStageB);
+        const uint32_t dst = ldsBase + kSlimTableBytes + issSlot * (Cfg::kStageA + Cfg::kStageB);
 #pragma unroll
         for (int q = 0; q < Cfg::kSlotsA; ++q) {
             DmaToLdsAddr16<false>(issBaseA + kOff, offA[q], dst + ((wave + 4 * q) % Cfg::kInstrA) * 1024);
         }
-        // Every weight byte is used once per m-tile: past the caches.  Not so the lines: rows that do not start on one
+        // The weights of a group with one m-tile are used once: past the caches.  Not so those that other m-tiles want as
+        // well, at about the same time on the same XCD: past the caches every m-tile fetched them from HBM (512 tokens of 256
+        // experts, top-8, popularity falling as rank^-1.2, hidden 7168, intermediate 2048, on 32-row tiles: 700 -> 630 us
+        // gate/up, 414 -> 336 us down).  And rows that do not start on a line
         // have their 128 bytes of a k-step in two, each wanted again by the next step (K 2880 / 1440, 37 rows each for 32
         // experts: 68.8 -> 64.6 us gate/up, 41.8 -> 39.0 us down).
-        if (splitLines) {
+        if (splitLines || iss.shared) {
 #pragma unroll
             for (int q = 0; q < Cfg::kSlotsB; ++q) {
                 DmaToLdsAddr16<false>(issBaseB + kOffW, offB[q], dst + Cfg::kStageA + (wave + 4 * q) * 1024);
@@ -303,12 +366,13 @@ __global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, Sli
             }
         }
         issSlot = issSlot + 1 == kStages ? 0 : issSlot + 1;
-        issK = issK + 1 == kSteps ? 0 : issK + 1;  // back at kStart after a tile's kSteps
+        issK = issK + 1 == kSteps ? 0 : issK + 1;
         if (++issStep == kSteps) {
             issStep = 0;
             const SlimTile next = tileAt(issNo + 1);
             if (next.valid) {
                 iss = next;
+                issK = next.kStart;
                 ++issNo;
                 issScaleSlot = issScaleSlot + 1 == kStages ? 0 : issScaleSlot + 1;
                 setupIssue(iss);
@@ -329,12 +393,12 @@ __global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, Sli
 
     int ring = 0, scaleSlot = 0;
     int32_t curNo = 0;
-    int curK = kStart;
     v4i acc[kMi][2];
     // weight rows of the wave's two 16-channel blocks: neighbours, or an activated block and its linear partner
     const int bRow0 = kSwiglu ? 16 * wave : 32 * wave;
     const int bRow1 = kSwiglu ? kSlimCols / 2 + 16 * wave : 32 * wave + 16;
     while (true) {
+        int curK = cur.kStart;
 #pragma unroll
         for (int mi = 0; mi < kMi; ++mi) acc[mi][0] = acc[mi][1] = v4i{0, 0, 0, 0};
 #pragma unroll 1
@@ -343,9 +407,9 @@ __global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, Sli
             // scales in flight only make that stricter); the barrier: for every wave, and the stage before is no longer read
             WaitVmcnt<(kStages - 2) * Cfg::kPerWave>();
             __syncthreads();
-            const char* const A = lds + ring * (Cfg::kStageA + Cfg::kStageB);
+            const char* const A = ringBase + ring * (Cfg::kStageA + Cfg::kStageB);
             const char* const B = A + Cfg::kStageA;
-            const uint32_t bAddr = ldsBase + ring * (Cfg::kStageA + Cfg::kStageB) + Cfg::kStageA;
+            const uint32_t bAddr = ldsBase + kSlimTableBytes + ring * (Cfg::kStageA + Cfg::kStageB) + Cfg::kStageA;
             const int covered = curK + 1 == kSteps ? kSteps * 128 - a.K : 0;  // leading k of this stage that another one has
             curK = curK + 1 == kSteps ? 0 : curK + 1;
             v4i bf[2][2], af[2][kMi];
@@ -481,15 +545,29 @@ __global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, Sli
     }
     // the drained slots' DMAs write this workgroup's LDS: none may be outstanding when it is given to another
     WaitVmcnt<0>();
+}
+
+// The three tile heights with as many stages as LDS holds.
+template <bool kSwiglu, bool kNz>
+__global__ __launch_bounds__(kSlimThreads) void SlimGemmKernel(KernelArgs a, SlimList sl) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const uint64_t spanStart = a.wgSpans != nullptr ? __builtin_amdgcn_s_memrealtime() : 0;
+    uint64_t spanTiles = 0;
+    uint16_t* const entries = reinterpret_cast<uint16_t*>(lds);
+    const SlimGroups table{entries, entries + kSlimTable, entries + 2 * kSlimTable};
+    const int height = SlimGroupTable(a, sl, lds, table);
+    if (height == 0) SlimGemmBody<1, 8, kSwiglu, kNz>(a, table, lds, spanTiles);
+    else if (height == 1) SlimGemmBody<2, 7, kSwiglu, kNz>(a, table, lds, spanTiles);
+    else SlimGemmBody<4, 6, kSwiglu, kNz>(a, table, lds, spanTiles);
     WriteSpan(a, spanStart, spanTiles);
 }
 
-template <int kMi, int kStages, bool kSwiglu, bool kNz>
+template <bool kSwiglu, bool kNz>
 hipError_t LaunchSlimKernel(const Plan& plan, const KernelArgs& args, const SlimList& list, hipStream_t stream) {
-    using Cfg = SlimCfg<kMi, kStages>;
-    auto kernel = SlimGemmKernel<kMi, kStages, kSwiglu, kNz>;
+    constexpr int kLdsBytes = std::max({SlimCfg<1, 8>::kLdsBytes, SlimCfg<2, 7>::kLdsBytes, SlimCfg<4, 6>::kLdsBytes});
+    auto kernel = SlimGemmKernel<kSwiglu, kNz>;
     static std::atomic<uint64_t> optedIn{0};
-    const hipError_t attr = opapi::EnsureDynamicLds(reinterpret_cast<const void*>(kernel), Cfg::kLdsBytes, optedIn);
+    const hipError_t attr = opapi::EnsureDynamicLds(reinterpret_cast<const void*>(kernel), kLdsBytes, optedIn);
     if (attr != hipSuccess) return attr;
     int64_t grid = DeviceCuCount();
     if (grid > 4 * plan.maxTiles) grid = 4 * plan.maxTiles;  // a tile may be cut in four
@@ -497,24 +575,15 @@ hipError_t LaunchSlimKernel(const Plan& plan, const KernelArgs& args, const Slim
     if (grid < kXcds) grid = kXcds;
     KernelArgs launchArgs = args;
     launchArgs.wgSpans = SpanBufferFor(kSwiglu ? Epilogue::kSwiglu : args.scale == nullptr ? Epilogue::kInt32 : Epilogue::kDequant,
-                                       static_cast<int>(grid), Cfg::kRows);
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kSlimThreads), Cfg::kLdsBytes, stream, launchArgs, list);
+                                       static_cast<int>(grid), plan.tileM);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kSlimThreads), kLdsBytes, stream, launchArgs, list);
     return hipGetLastError();
-}
-
-template <bool kSwiglu, bool kNz>
-hipError_t LaunchSlimShape(const Plan& plan, const KernelArgs& args, const SlimList& list, hipStream_t stream) {
-    switch (plan.tileM) {  // as many stages as LDS holds
-        case 16: return LaunchSlimKernel<1, 8, kSwiglu, kNz>(plan, args, list, stream);
-        case 32: return LaunchSlimKernel<2, 7, kSwiglu, kNz>(plan, args, list, stream);
-        default: return LaunchSlimKernel<4, 6, kSwiglu, kNz>(plan, args, list, stream);
-    }
 }
 
 template <bool kSwiglu>
 hipError_t LaunchSlimLayout(const Plan& plan, const KernelArgs& args, const SlimList& list, hipStream_t stream) {
-    if (args.wNz) return LaunchSlimShape<kSwiglu, true>(plan, args, list, stream);
-    return LaunchSlimShape<kSwiglu, false>(plan, args, list, stream);
+    if (args.wNz) return LaunchSlimKernel<kSwiglu, true>(plan, args, list, stream);
+    return LaunchSlimKernel<kSwiglu, false>(plan, args, list, stream);
 }
 
 }  // namespace
