@@ -447,10 +447,11 @@ Plan MakePlan(const Problem& p) {
             if (static_cast<double>(s) >= want) { plan.tileM = s; break; }
         }
         // A handful of rows per group (decode): the 64-row shape, whose eight waves keep more of the weight stream in
-        // flight than the four of the 32-row shape (measured 0.3 - 0.7 % faster on both GEMMs of a 64-token step).  It
-        // also serves groups of more rows while it holds nearly all of them whole: 44 rows each for 128 experts, hidden
-        // 4096, intermediate 1536, took 341 / 180 us (gate/up, down) with 96-row tiles, 287 / 155 us with these.
-        if (plan.tileM < 64 || RowsOfNearlyEveryGroup(meanRows) <= 64.0) plan.tileM = 64;
+        // flight than the four of the 32-row shape (measured 0.3 - 0.7 % faster on both GEMMs of a 64-token step).
+        // Not beyond the means that ask for it, although it would hold nearly all of evenly chosen groups of up to 45 rows:
+        // 45 rows each for 128 experts, hidden 4096, intermediate 1536, take 358 / 185 us (gate/up, down) with 96-row
+        // tiles and 295 / 158 us with these, but with popularity falling as rank^-1.2 293 / 163 and 366 / 179.
+        if (plan.tileM < 64) plan.tileM = 64;
         // tuning override: OPAPI_GEMM_TILE_M=<one of the shapes above>
         if (const char* env = std::getenv("OPAPI_GEMM_TILE_M")) {
             const int forced = std::atoi(env);

@@ -717,3 +717,17 @@ def test_packed_descriptors(aclnn, dims):
     handles.close()
     with pytest.raises(MemoryError):
         aclnn.tensor_of(torch.zeros((1,) * 9))
+
+
+def test_tile_height_leaves_room_for_uneven_groups(aclnn, monkeypatch):
+    """45 rows each on average: 96-row tiles, since a router's groups are less even than their mean.  The workspace holds a
+    table entry for every m-tile that the height allows."""
+    def workspace():
+        code, ws = _status(aclnn, "aclnnGroupedMatmulV4", _gmm_args(aclnn, M=45 * 128, K=1536, N=4096, E=128))
+        assert code == 0
+        return ws
+    chosen, of_height = workspace(), {}
+    for rows in (64, 96):
+        monkeypatch.setenv("OPAPI_GEMM_TILE_M", str(rows))
+        of_height[rows] = workspace()
+    assert chosen == of_height[96] != of_height[64]
