@@ -62,6 +62,7 @@ constexpr int64_t kSlimMaxRows = 65535;
 // Tile shape chosen from the static shape (M, groups); fixed for the lifetime of a plan.
 struct Plan {
     int tileM = 0;          // rows per workgroup tile (multiple of 32; slim: 16, 32 or 64, the lowest that the kernel may take)
+    int lowTileM = 0;       // a lower height that the scheduling kernel may choose instead (0: none)
     int wavesM = 1;         // 1 or 2 wave rows
     int subTilesM = 1;      // 32-row MFMA tiles per wave
     int64_t maxTiles = 0;   // launch bound on workgroups

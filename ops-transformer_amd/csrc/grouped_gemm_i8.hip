@@ -48,6 +48,7 @@ struct SchedArgs {
     int32_t groupListIsInt64;
     int32_t isCount;  // 0 cumsum, 1 counts, 2 sparse (expert id, count) pairs
     int32_t tileM;
+    int32_t mayLower;  // 1: m-tiles of kLowTileM rows instead where they leave at most an eighth of the groups a small last one
     int32_t maxMTiles;
     int64_t M;
     int64_t rowBegin, rowEnd;  // only rows in [rowBegin, rowEnd) get tiles (one band of a launch that runs in row bands)
@@ -145,19 +146,24 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
     begin = begin < a.rowBegin ? a.rowBegin : (begin > a.rowEnd ? a.rowEnd : begin);
     end = end < a.rowBegin ? a.rowBegin : (end > a.rowEnd ? a.rowEnd : end);
     const int32_t rows = t < a.groups ? static_cast<int32_t>(end - begin) : 0;
-    const int32_t tiles = (rows + a.tileM - 1) / a.tileM;
+    int32_t tileM = a.tileM;
+    if (a.mayLower) {
+        const int32_t last = rows % kLowTileM;
+        if (__syncthreads_count(last > 0 && last <= kSmallRows) * 8 <= a.groups) tileM = kLowTileM;
+    }
+    const int32_t tiles = (rows + tileM - 1) / tileM;
     // big and small m-tiles of this group (with tiles of at most kSmallRows rows every m-tile is small; otherwise only
     // a group's last, partly filled m-tile can be) and the cost of the big ones; two packed prefix sums give every
     // group the positions of its m-tiles in the two runs of the table, and the launch the totals
-    const bool allSmall = a.tileM <= kSmallRows;
-    const int32_t lastRows = tiles > 0 ? rows - (tiles - 1) * a.tileM : 0;
+    const bool allSmall = tileM <= kSmallRows;
+    const int32_t lastRows = tiles > 0 ? rows - (tiles - 1) * tileM : 0;
     const int32_t smallCount = allSmall ? tiles : (tiles > 0 && lastRows <= kSmallRows ? 1 : 0);
     const int32_t bigCount = tiles - smallCount;
     int32_t bigCost = 0;
     if (bigCount > 0) {
         const bool lastIsBig = smallCount == 0;
         const int32_t lastSub = (lastRows + 31) >> 5;
-        bigCost = (bigCount - (lastIsBig ? 1 : 0)) * max(a.tileM >> 5, kSmallCost) + (lastIsBig ? max(lastSub, kSmallCost) : 0);
+        bigCost = (bigCount - (lastIsBig ? 1 : 0)) * max(tileM >> 5, kSmallCost) + (lastIsBig ? max(lastSub, kSmallCost) : 0);
     }
     const uint64_t countsInc = inclusiveScan64(static_cast<uint64_t>(tiles) | (static_cast<uint64_t>(bigCount) << 32));
     const uint64_t costInc = inclusiveScan64(static_cast<uint64_t>(bigCost) | (static_cast<uint64_t>(tiles > 0 ? 1 : 0) << 32));
@@ -205,7 +211,7 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
     const int32_t wideBands = totalMTiles >= 2 * totals[3] ? kGroupM : 1;
     if (t < kQueueHeaderInts) {
         a.sched[t] = t == 0 ? nBig : t == 1 ? nSmall : t == 2 ? nSmall * kSmallCost : t == 3 ? totals[2] : t == 4 ? wideBands
-                   : t == 5 ? (allSmall ? wideBands : 1) : t == kHdrCoveredRows ? sCovered : 0;
+                   : t == 5 ? (allSmall ? wideBands : 1) : t == kHdrCoveredRows ? sCovered : t == kHdrTileM ? tileM : 0;
     }
     int4* const mTileTable = reinterpret_cast<int4*>(a.sched + kQueueHeaderInts + kQueueCounterInts);
     for (int32_t m = t; m < totalMTiles; m += 1024) {
@@ -215,11 +221,11 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
             if (scan[mid] > m) hi = mid; else lo = mid;
         }
         const int32_t inGroup = m - (hi > 0 ? scan[hi - 1] : 0);
-        const int32_t tileRows = min(a.tileM, sRows[hi] - inGroup * a.tileM);
+        const int32_t tileRows = min(tileM, sRows[hi] - inGroup * tileM);
         const bool small = allSmall || tileRows <= kSmallRows;
         const int32_t pos = small ? nBig + sSmallBefore[hi] + (allSmall ? inGroup : 0) : sBigBefore[hi] + inGroup;
         const int32_t limit = small ? nBig + nSmall : nBig;
-        if (pos < limit) mTileTable[pos] = make_int4(hi, sRowStart[hi] + inGroup * a.tileM, tileRows, 0);
+        if (pos < limit) mTileTable[pos] = make_int4(hi, sRowStart[hi] + inGroup * tileM, tileRows, 0);
     }
 }
 
@@ -436,10 +442,18 @@ Plan MakePlan(const Problem& p) {
     }
     const double rounds = static_cast<double>(groups) * plan.tilesN / DeviceCuCount();
     double want = meanRows * (rounds <= 24.0 ? 1.5 : 1.25);
-    // Without the SwiGLU epilogue 160 rows are enough where they hold nearly every group: their activation ring is a stage deeper than
-    // that of 192 (128 rows each, K 1536 x N 4096, 128 experts: 233 -> 221 us; K 2048 x N 7168, 256 experts: 853 / 795).
+    // Without the SwiGLU epilogue 160 rows are better where they hold nearly every group: their activation ring is a stage deeper
+    // than that of 192 (K 2048 x N 7168, 64 experts of 128 rows: 232 -> 218 us; K 1536 x N 4096, 128 experts of 112 rows:
+    // 220 -> 207).  Groups that spread more than a router's even choice leave many small m-tiles, which the 192-row kernel
+    // runs in a geometry of their own (the same shapes, popularity falling as rank^-0.6: 254 us against 276 with 160 rows;
+    // 229 / 251): the scheduling kernel decides, where it knows the groups.  A workgroup that walks a few tiles only does
+    // not repay the change of geometry, however uneven the groups (K 1024 x N 1024, 128 experts, two rounds of tiles:
+    // 85 us with 192 rows, 73 with 160; K 1440 x N 2880, 32 experts, a round and a half: 95 / 82; K 1536 x N 4096, 60
+    // experts, four rounds: 141 / 144), nor is there one below eight k-steps.
     // The SwiGLU operator has it the other way round: 379 us with 192 rows, 418 with 160 (N 3072, K 4096, 128 experts).
-    if (p.epilogue != Epilogue::kSwiglu && want > 160.0 && RowsOfNearlyEveryGroup(meanRows) <= 160.0) want = 160.0;
+    const int64_t kSteps = (p.K + 127) / 128;
+    const bool lowHolds = p.epilogue != Epilogue::kSwiglu && want > kLowTileM && RowsOfNearlyEveryGroup(meanRows) <= kLowTileM;
+    if (lowHolds) want = rounds > 4.0 && kSteps >= 8 ? 192.0 : kLowTileM;
     if (StreamOk(p)) {
         static const int kShapes[] = {32, 64, 96, 128, 160, 192, 256};
         plan.tileM = 256;
@@ -466,15 +480,14 @@ Plan MakePlan(const Problem& p) {
     // (the issue side then never runs more than one tile ahead, which is what the two-tile look-ahead of the draw
     // covers) and more than 64 rows; the handful-of-rows tiles of a decode step keep their fixed shares.
     // OPAPI_GEMM_PULL=0 / 1 switches it off / on for every shape with eight k-steps.
-    const int64_t kSteps = (p.K + 127) / 128;
     plan.pullTiles = StreamOk(p) && kSteps >= 8 && plan.tileM > 64 && plan.maxTiles < (1ll << 31);
     if (const char* env = std::getenv("OPAPI_GEMM_PULL")) {
-        const int64_t kSteps = (p.K + 127) / 128;
-    plan.pullTiles = StreamOk(p) && kSteps >= 8 && plan.maxTiles < (1ll << 31) && std::atoi(env) != 0;
+        plan.pullTiles = StreamOk(p) && kSteps >= 8 && plan.maxTiles < (1ll << 31) && std::atoi(env) != 0;
     }
+    if (lowHolds && plan.tileM == 192 && plan.pullTiles && std::getenv("OPAPI_GEMM_TILE_M") == nullptr) plan.lowTileM = kLowTileM;
     plan.wavesM = plan.tileM >= 64 && StreamOk(p) ? 2 : 1;
     plan.subTilesM = (plan.tileM / 32 + plan.wavesM - 1) / plan.wavesM;
-    const int64_t maxMTiles = p.M / plan.tileM + groups;
+    const int64_t maxMTiles = p.M / (plan.lowTileM > 0 ? plan.lowTileM : plan.tileM) + groups;
     plan.maxMTiles = static_cast<int32_t>(maxMTiles);
     // round up so that every XCD's share [xcd * ceil(total/8), ...) is covered by the launch
     plan.maxTiles = (maxMTiles * plan.tilesN + kXcds - 1) / kXcds * kXcds;
@@ -519,6 +532,7 @@ hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStrea
     sa.groupListIsInt64 = p.groupListIsInt64 ? 1 : 0;
     sa.isCount = static_cast<int32_t>(p.groupListKind);
     sa.tileM = plan.tileM;
+    sa.mayLower = plan.lowTileM > 0 ? 1 : 0;
     sa.maxMTiles = plan.maxMTiles;
     sa.M = p.M;
 

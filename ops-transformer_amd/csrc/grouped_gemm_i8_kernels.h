@@ -103,7 +103,7 @@ constexpr int kLdsBudget = 160 * 1024;
 // ---------------------------------------------------------------------------------------------- scheduling table
 // int32 layout, all written by the scheduling kernel:
 //   header, 32 ints: [0] big m-tiles, [1] small m-tiles, [2] cost of the small ones, [3] cost of the big ones (see below),
-//                    [4] / [5] band width of the big / small run, [6] total rows covered by the groups;
+//                    [4] / [5] band width of the big / small run, [6] total rows covered by the groups, [7] rows per m-tile;
 //   16 tile counters in one 128-byte line (32 ints): counter [2 * xcd + list], zeroed;
 //   the m-tile table, 4 ints per m-tile {group, first row, rows, 0} (at most maxMTiles of them): the big m-tiles in group
 //   order, then the small ones.  A GEMM kernel finds everything about a tile with one 16-byte load.
@@ -119,6 +119,9 @@ constexpr int kSmallCost = 3;
 constexpr int kQueueHeaderInts = 32;
 constexpr int kQueueCounterInts = 32;
 constexpr int kHdrCoveredRows = 6;
+constexpr int kHdrTileM = 7;
+// A height that the scheduling kernel may choose instead of 192 rows (Plan::lowTileM).
+constexpr int kLowTileM = 160;
 __host__ __device__ inline int SchedTotalInts(int maxMTiles) { return kQueueHeaderInts + kQueueCounterInts + 4 * maxMTiles; }
 
 
@@ -1234,6 +1237,11 @@ __global__ __launch_bounds__(64 * kWn * (kSub1 > 0 ? 2 : 1)) void StreamGemmKern
 // walk and the non-temporal weight loads of the decode shapes.  A workgroup serves the run it prefers (the small run gets the share
 // of each XCD's workgroups that its cost is of the whole) until that run's counters are used up on every XCD, lets its
 // ring drain, and serves the other; a launch without small m-tiles costs the workgroups that looked for them one draw.
+//
+// kHasLow: the scheduling kernel may have cut the groups into m-tiles of kLowTileM rows instead; these run in one geometry.
+template <int kSub0, int kSub1, Epilogue kEpi>
+constexpr bool kHasLow = kSub0 == 3 && kSub1 == 3 && kEpi != Epilogue::kSwiglu;
+
 template <int kSub0, int kSub1, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
 __global__ __launch_bounds__(512) void MixedGemmKernel(KernelArgs a, const int32_t* __restrict__ sched) {
     static_assert(StreamCfg<1, 1, 128>::kTileM == kSmallRows, "the small run's geometry is that of the 64-row tiles");
@@ -1241,6 +1249,13 @@ __global__ __launch_bounds__(512) void MixedGemmKernel(KernelArgs a, const int32
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const uint64_t spanStart = a.wgSpans != nullptr ? __builtin_amdgcn_s_memrealtime() : 0;
     uint64_t spanTiles = 0;
+    if constexpr (kHasLow<kSub0, kSub1, kEpi>) {
+        if (sched[kHdrTileM] == kLowTileM) {
+            StreamGemmBody<3, 2, 128, kEpi, kNz, kNMajor, kWavesN, kBothRuns, kTail>(a, sched, lds, spanTiles);
+            WriteSpan(a, spanStart, spanTiles);
+            return;
+        }
+    }
     const int64_t costSmall = sched[2], costAll = costSmall + sched[3];
     const int32_t slots = gridDim.x / kXcds, slot = blockIdx.x / kXcds;
     int64_t forSmall = costAll > 0 ? (slots * costSmall + costAll / 2) / costAll : 0;
@@ -1380,7 +1395,9 @@ template <int kSub0, int kSub1, Epilogue kEpi, bool kNz, bool kNMajor, bool kTai
 hipError_t LaunchMixed(const KernelArgs& args, const int32_t* sched, int64_t maxTiles, hipStream_t stream) {
     using Big = StreamCfg<kSub0, kSub1, 128>;
     using Small = StreamCfg<1, 1, 128>;
-    constexpr int kLdsBytes = Big::kLdsBytes > Small::kLdsBytes ? Big::kLdsBytes : Small::kLdsBytes;
+    using Low = StreamCfg<3, 2, 128>;
+    static_assert(Low::kTileM == kLowTileM && Low::kThreads == 512, "one workgroup size for all");
+    constexpr int kLdsBytes = std::max({Big::kLdsBytes, Small::kLdsBytes, kHasLow<kSub0, kSub1, kEpi> ? Low::kLdsBytes : 0});
     auto kernel = MixedGemmKernel<kSub0, kSub1, kEpi, kNz, kNMajor, kTail>;
     static std::atomic<uint64_t> optedIn{0};
     const hipError_t attr = opapi::EnsureDynamicLds(reinterpret_cast<const void*>(kernel), kLdsBytes, optedIn);

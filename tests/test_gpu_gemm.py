@@ -509,3 +509,49 @@ def test_swiglu_workspace_cap_runs_in_row_bands(aclnn, oracle, dev, monkeypatch,
     diff = np.abs(q2[:int(cumsum[-1])].astype(np.int32) - q_ref.astype(np.int32))
     assert diff.max() <= 1 and (diff != 0).mean() < 1e-3
     np.testing.assert_allclose(qs2[:int(cumsum[-1])], qs_ref, rtol=1e-5)
+
+
+@pytest.mark.parametrize("layout", ["kmajor", "nz", "nd"])
+@pytest.mark.parametrize("K", [1152, 1168])
+@pytest.mark.parametrize("head,height", [
+    ([160, 161, 0, 97], 160),                # two of 40 groups with a small last m-tile: the lower height
+    ([160, 161, 193, 46, 170, 1], 160),      # an eighth of them
+    ([160, 161, 193, 46, 170, 1, 2], 192),   # and one more
+    ([900, 64, 1, 320, 0, 30, 10, 65, 4, 3, 2, 1], 192)])
+def test_tile_height_chosen_from_the_groups(aclnn, oracle, dev, K, layout, head, height):
+    """Means of 107 to 130 rows without the SwiGLU epilogue: the scheduling kernel takes 160-row m-tiles where at most an eighth
+    of the groups ends in a small one, 192-row m-tiles otherwise.  int32 and bf16 outputs bit-exact in both."""
+    rng = np.random.default_rng(K + len(layout))
+    E, N = 40, 256 * 26
+    groups = head + [120] * (E - len(head))
+    M = 120 * E
+    groups[-1] += M - sum(groups) if sum(groups) < M else 0
+    M = max(M, sum(groups))
+    cumsum = np.cumsum(groups).astype(np.int64)
+    small = sum(0 < r % 160 <= 64 for r in groups)
+    assert (8 * small <= E) == (height == 160)
+    x = rng.integers(-127, 128, (M, K)).astype(np.int8)
+    wt = rng.integers(-127, 128, (E, N, K)).astype(np.int8)
+    scale = rng.uniform(1e-3, 1e-2, (E, N)).astype(np.float32)
+    pt = rng.uniform(0.01, 0.1, M).astype(np.float32)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    w_dev = t(wt)
+    if layout == "nz":
+        w_nz = w_dev.view(E, N // 32, 32, K // 16, 16).permute(0, 1, 3, 4, 2).contiguous()
+        wkw, wv = dict(weight_nz=(w_nz, "nz5d")), None
+    else:
+        wkw, wv = {}, [w_dev.transpose(1, 2) if layout == "kmajor" else w_dev.transpose(1, 2).contiguous()]
+    ws = aclnn.Workspace()
+    acc = aclnn.grouped_matmul_v4([t(x)], wv, group_list=t(cumsum), split_item=3, group_type=0, workspace=ws, **wkw)[0]
+    torch.cuda.synchronize()
+    assert ws.tensor.view(torch.int32)[7].item() == height
+    y = aclnn.grouped_matmul_v4([t(x)], wv, scale=[t(scale)], per_token_scale=[t(pt)], group_list=t(cumsum), split_item=3,
+                                group_type=0, output_dtype=torch.bfloat16, workspace=ws, **wkw)[0]
+    torch.cuda.synchronize()
+    rows = rng.choice(M, 400, replace=False)                     # of the rows of every group, the oracle checks these
+    keep = np.sort(np.concatenate([rows, cumsum[:-1][cumsum[:-1] < M], cumsum[cumsum > 0] - 1]))
+    keep = np.unique(keep)
+    kept = np.searchsorted(keep, cumsum, side="left").astype(np.int64)   # groups of the kept rows
+    assert np.array_equal(acc.cpu().numpy()[keep], oracle.grouped_matmul_i32(x[keep], wt, kept, w_trans=True))
+    ref = oracle.grouped_matmul_dequant(x[keep], wt, scale, pt[keep], kept, w_trans=True, out_dtype=oracle.DT_BF16)
+    assert np.array_equal(y.view(torch.int16).cpu().numpy().view(np.uint16)[keep], ref)
