@@ -649,13 +649,14 @@ __global__ __launch_bounds__(kGatherThreads) void QuantGatherRowsKernel(QuantGat
 // through LDS, the writes); the general kernel's second read of the row, and its index load in front of every four-byte
 // store, bounded that one.
 // Measured before and now: 2047 tokens of 4096 bf16, top-8: 39.6 -> 22.8 us (3.7 TB/s of rows read and copies written); 23
-// tokens: 14.3 -> 5.2 us.
+// tokens: 14.3 -> 5.2 us.  A narrow row has a workgroup of its own width: with 512 threads for any row, 16384 rows of 256
+// bf16, top-2, took 30.4 us, longer than the general kernel's 27.7, and take 15.4; of 1024, top-8, 41.7 -> 31.2 (general: 65).
 constexpr int kQuantRowThreads = 512;
 constexpr int kQuantRowMaxPackets = 4;
 
-template <int kDtype, int kPackets>
-__global__ __launch_bounds__(kQuantRowThreads) void QuantGatherPacketsKernel(QuantGatherArgs a) {
-    __shared__ float waveMax[kQuantRowThreads / kWaveSize];
+template <int kDtype, int kThreads, int kPackets>
+__global__ __launch_bounds__(kThreads) void QuantGatherPacketsKernel(QuantGatherArgs a) {
+    __shared__ float waveMax[kThreads / kWaveSize];
     __shared__ int32_t dsts[kMaxCachedK];
     const int64_t n = blockIdx.x;
     const int cols = static_cast<int>(a.cols);
@@ -663,7 +664,7 @@ __global__ __launch_bounds__(kQuantRowThreads) void QuantGatherPacketsKernel(Qua
     float v[kPackets][8];
 #pragma unroll
     for (int p = 0; p < kPackets; ++p) {
-        const int c = (p * kQuantRowThreads + static_cast<int>(threadIdx.x)) * 8;
+        const int c = (p * kThreads + static_cast<int>(threadIdx.x)) * 8;
         const int64_t at = n * a.cols + c;
         uint32_t word[8] = {};
         if (c < cols) {
@@ -696,7 +697,7 @@ __global__ __launch_bounds__(kQuantRowThreads) void QuantGatherPacketsKernel(Qua
     __syncthreads();
     mx = waveMax[0];
 #pragma unroll
-    for (int w = 1; w < kQuantRowThreads / kWaveSize; ++w) mx = fmaxf(mx, waveMax[w]);
+    for (int w = 1; w < kThreads / kWaveSize; ++w) mx = fmaxf(mx, waveMax[w]);
     const float scale = mx / 127.0f;
     if (threadIdx.x < a.topK) {
         const int32_t dst = dsts[threadIdx.x];
@@ -704,7 +705,7 @@ __global__ __launch_bounds__(kQuantRowThreads) void QuantGatherPacketsKernel(Qua
     }
 #pragma unroll
     for (int p = 0; p < kPackets; ++p) {
-        const int c = (p * kQuantRowThreads + static_cast<int>(threadIdx.x)) * 8;
+        const int c = (p * kThreads + static_cast<int>(threadIdx.x)) * 8;
         if (c >= cols) continue;
         uint32_t q[2] = {0, 0};
 #pragma unroll
@@ -720,13 +721,22 @@ __global__ __launch_bounds__(kQuantRowThreads) void QuantGatherPacketsKernel(Qua
     }
 }
 
+template <int kDtype, int kThreads, int kPackets>
+void LaunchQuantGather(const QuantGatherArgs& q, int64_t tokens, hipStream_t stream) {
+    static_assert(kMaxCachedK <= kThreads, "a thread per copy");
+    hipLaunchKernelGGL((QuantGatherPacketsKernel<kDtype, kThreads, kPackets>), dim3(static_cast<unsigned>(tokens)), dim3(kThreads), 0,
+                       stream, q);
+}
+
 template <int kDtype>
 void LaunchQuantGatherPackets(const QuantGatherArgs& q, int64_t tokens, hipStream_t stream) {
-    const dim3 grid(static_cast<unsigned>(tokens)), block(kQuantRowThreads);
-    const int64_t packets = (q.cols + 8 * kQuantRowThreads - 1) / (8 * kQuantRowThreads);
-    if (packets <= 1) hipLaunchKernelGGL((QuantGatherPacketsKernel<kDtype, 1>), grid, block, 0, stream, q);
-    else if (packets <= 2) hipLaunchKernelGGL((QuantGatherPacketsKernel<kDtype, 2>), grid, block, 0, stream, q);
-    else hipLaunchKernelGGL((QuantGatherPacketsKernel<kDtype, kQuantRowMaxPackets>), grid, block, 0, stream, q);
+    const int64_t lanes = (q.cols + 7) / 8;
+    if (lanes <= 64) LaunchQuantGather<kDtype, 64, 1>(q, tokens, stream);
+    else if (lanes <= 128) LaunchQuantGather<kDtype, 128, 1>(q, tokens, stream);
+    else if (lanes <= 256) LaunchQuantGather<kDtype, 256, 1>(q, tokens, stream);
+    else if (lanes <= kQuantRowThreads) LaunchQuantGather<kDtype, kQuantRowThreads, 1>(q, tokens, stream);
+    else if (lanes <= 2 * kQuantRowThreads) LaunchQuantGather<kDtype, kQuantRowThreads, 2>(q, tokens, stream);
+    else LaunchQuantGather<kDtype, kQuantRowThreads, kQuantRowMaxPackets>(q, tokens, stream);
 }
 
 // Drop/pad mode with dynamic quantisation: capacity rows beyond an expert's (capped) count get scale 0.

@@ -436,11 +436,13 @@ def test_decode_sized_calls_sort_and_gather_in_one_launch(aclnn, oracle, dev, T,
 
 @pytest.mark.parametrize("T,K,H,dtype_name", [
     (3, 2, 8, "bf16"), (5, 4, 4096, "f32"), (5, 4, 4104, "f16"), (4, 8, 8192, "bf16"), (4, 3, 8200, "bf16"),
+    (5, 4, 8, "bf16"), (3, 64, 512, "f16"), (5, 4, 520, "f32"), (5, 4, 1024, "bf16"), (3, 64, 1032, "bf16"), (5, 4, 2048, "f32"),
+    (5, 4, 2056, "f16"),         # workgroups of 64, 128, 256 and 512 threads
     (2, 64, 16384, "f16"),       # the widest row and the most experts per token of the packet kernel
     (2, 65, 64, "bf16"), (2, 4, 16392, "bf16"), (3, 4, 4100, "bf16")])  # one past either, and no whole packets
 def test_dynamic_quant_row_widths(aclnn, oracle, dev, T, K, H, dtype_name):
-    """Dynamic quantisation without a smooth scale at the widths where its kernels change hands (4096 elements per packet
-    of a workgroup, up to four packets), through both operators, on outputs that do not start at zero."""
+    """Dynamic quantisation without a smooth scale at the widths where its kernels change hands (workgroups as wide as the row
+    up to 4096 elements, then two or up to four packets per thread), through both operators, on outputs that do not start at zero."""
     rng = np.random.default_rng(T * 3 + H)
     E = 70
     xt, bits, idx, code = _quant_v2_inputs(rng, T, K, E, H, dtype_name, oracle)
@@ -483,3 +485,23 @@ def test_dynamic_quant_of_a_row_without_columns(aclnn, dev, dirty_memory, drop_p
     if not drop_pad:
         _, _, counts, scale = aclnn.moe_init_routing_v3(x, idx, expert_num=4, expert_tokens_num_type=1, quant_mode=1)
         assert scale.tolist() == [0.0] and counts.tolist() == [1, 0, 0, 0]
+
+
+def test_dynamic_quant_of_narrow_rows_beats_the_general_kernel(aclnn, dev):
+    """Rows of 256 elements: the packet kernel takes 15.4 us for 16384 of them, the general one (any smooth scale takes the call
+    there) twice that; with workgroups wider than the row the packet kernel took 30.4."""
+    x = torch.randn((16384, 256), device=dev).bfloat16()
+    idx = torch.randint(0, 64, (16384, 2), dtype=torch.int32, device=dev)
+    ones = torch.ones((1, 256), device=dev)
+
+    def gather_ms(scale):
+        call = lambda: aclnn.moe_init_routing_quant_v2(x, idx, 1, scale, None, expert_num=64, expert_tokens_count_or_cumsum_flag=2)
+        call()
+        aclnn.kernel_timer_enable(True)
+        for _ in range(10):
+            call()
+        torch.cuda.synchronize()
+        report = aclnn.kernel_timer_report()
+        aclnn.kernel_timer_enable(False)
+        return report["routing_quant_gather"][1]
+    assert np.median([gather_ms(None) / gather_ms(ones) for _ in range(5)]) < 0.8
