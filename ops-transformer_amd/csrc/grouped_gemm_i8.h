@@ -54,10 +54,12 @@ struct Problem {
 };
 
 // Limits of the kernels for a handful of rows per group (grouped_gemm_i8_slim.h): channels per tile (kSwiglu: half of them
-// activated), groups, and rows (the prefix table in LDS holds 16-bit entries).
+// activated), groups, rows (the prefix table in LDS holds 16-bit entries) and tiles side by side (a tile's number has 32 bits,
+// and groups that overlap in a malformed list can fill the prefix table).
 constexpr int kSlimTileN = 128;
 constexpr int kSlimMaxGroups = 512;
 constexpr int64_t kSlimMaxRows = 65535;
+constexpr int64_t kSlimMaxTilesN = 16384;
 
 // Tile shape chosen from the static shape (M, groups); fixed for the lifetime of a plan.
 struct Plan {

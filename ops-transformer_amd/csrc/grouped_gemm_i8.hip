@@ -397,11 +397,12 @@ int SlimTileRows(const Problem& p, double meanRows) {
         return 0;
     }
     if (p.epilogue == Epilogue::kSwiglu && static_cast<uint64_t>(p.M) * static_cast<uint64_t>(p.N / 2) * 4 > SwigluWorkspaceCap()) return 0;
+    const int64_t cols = p.epilogue == Epilogue::kSwiglu ? p.N / 2 : p.N;
+    const int64_t wide = p.epilogue == Epilogue::kSwiglu ? kTileN / 2 : kTileN, slim = wide * kSlimTileN / kTileN;
+    if (cols > kSlimMaxTilesN * slim) return 0;
     const double want = RowsOfNearlyEveryGroup(meanRows);
     if (want <= 16.0) return 16;
     if (want <= 32.0) return 32;
-    const int64_t cols = p.epilogue == Epilogue::kSwiglu ? p.N / 2 : p.N;
-    const int64_t wide = p.epilogue == Epilogue::kSwiglu ? kTileN / 2 : kTileN, slim = wide * kSlimTileN / kTileN;
     if (p.groups * static_cast<int64_t>(std::ceil(want / 64.0)) * ((cols + slim - 1) / slim) <= DeviceCuCount()) return 64;
     if (want > 64.0) return 0;
     return RoundEfficiency(p.groups * ((cols + slim - 1) / slim)) > 1.06 * RoundEfficiency(p.groups * ((cols + wide - 1) / wide)) ? 64 : 0;

@@ -731,3 +731,13 @@ def test_tile_height_leaves_room_for_uneven_groups(aclnn, monkeypatch):
         monkeypatch.setenv("OPAPI_GEMM_TILE_M", str(rows))
         of_height[rows] = workspace()
     assert chosen == of_height[96] != of_height[64]
+
+
+def test_slim_tiles_are_numbered_in_32_bits(aclnn):
+    """Two million channels are the widest that the kernels for a handful of rows take (their workspace is a header alone); beyond,
+    65535 m-tiles of a malformed list times the tiles side by side would not fit a tile number, and the ring kernels run."""
+    for N, ws in ((16384 * 128, 256), (16384 * 128 + 128, 512)):
+        w = T(aclnn, (2, 128, N), I8, strides=[128 * N, 1, 128], storage=(2, N, 128))
+        args = _gmm_args(aclnn, M=8, K=128, N=N, E=2)
+        args[1] = _tl(aclnn, [w])
+        assert _status(aclnn, "aclnnGroupedMatmulV4", args) == (0, ws)
