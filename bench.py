@@ -2,7 +2,7 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--config c1] [--no-cpu-baseline] [--no-other-configs]
                     [--calibration-copy] [--fused-combine] [--graph] [--routing v2|v3]
-                    [--weight-nz | --weight-row-major]
+                    [--weight-nz | --weight-row-major] [--record FILE]
 
 A step is one pass of the path (routing -> gate/up GEMM + SwiGLU + requant -> down GEMM -> finalize) over one batch of
 synthetic tokens whose inputs and expert weights are already resident in HBM.  Prints ONE JSON line: tokens/s for the
@@ -21,7 +21,9 @@ measurement of the other halves of the metric: the decode shape c3 (eager and as
 Mixtral prefill shape c2 (the MFMA-bound one), the skewed shape c4, and c1 again as a graph replay and behind the other
 routing operator -- each with its ms per pass, per-kernel durations and both kernels' rooflines from the same timer
 (min(K, 20) passes each; ten times as many for the 0.4 ms decode pass, so that a block between two synchronisations is
-long against them -- with --config c3 give --steps 200 or more for the same reason).
+long against them -- with --config c3 give --steps 200 or more for the same reason).  The printed line is kept short enough
+for a log's tail (about 5 KB): of `other_configs` it has the times and the rooflines' fractions, and the numbers are rounded to
+six digits.  --record FILE writes everything, the blocks of passes, workspace bytes and tile balance among it.
 
 --calibration-copy appends, after the timed region, a few launches of the library's plain 1 GiB copy kernel: under
 `rocprofv3 --pmc FETCH_SIZE` / `--pmc WRITE_SIZE` its counter readings give the factor that converts the counters to
@@ -149,13 +151,21 @@ def _kernel_roofline(name, kernel, timer_name, nbytes, ops, kernels, passes, tra
     return roofline
 
 
+def _gemm_kernel_name(kernels, passes, epilogue):
+    """Which grouped GEMM kernels ran: those for a handful of rows per expert have no scheduling launch in front of them."""
+    scheduled = kernels.get("gmm_schedule", (0, 0.0))[0] / float(max(passes, 1))
+    kind = ("SlimGemmKernel" if scheduled == 0 else "StreamGemmKernel or MixedGemmKernel" if scheduled >= 2
+            else "SlimGemmKernel, StreamGemmKernel or MixedGemmKernel")
+    return "%s (%s)" % (kind, epilogue)
+
+
 def _gate_up_roofline(cfg, touched, kernels, passes):
     """Gate/up grouped GEMM.  Algorithmic bytes of one launch: the touched experts' gate/up weights and channel scales,
     the expanded int8 rows and their scales in, the int8 activations and their scales out.  Ops: 4 * M * H * I."""
     M, H, I = cfg.tokens * cfg.top_k, cfg.hidden, cfg.inter
     nbytes = touched * 2 * H * I + touched * 2 * I * 4 + M * H + M * 4 + M * I + M * 4
     traffic, traffic_source = _recorded_traffic(cfg.name)
-    return _kernel_roofline("gate_up", "StreamGemmKernel<..., kSwiglu> (gate/up GEMM + SwiGLU; timer name gmm_swiglu)",
+    return _kernel_roofline("gate_up", _gemm_kernel_name(kernels, passes, "gate/up GEMM + SwiGLU; timer name gmm_swiglu"),
                             "gmm_swiglu", nbytes, 4 * M * H * I, kernels, passes, traffic, traffic_source)
 
 
@@ -164,7 +174,7 @@ def _down_roofline(cfg, touched, kernels, passes):
     scales, the int8 activations and their scales in, the bf16 rows out.  Ops: 2 * M * H * I."""
     M, H, I = cfg.tokens * cfg.top_k, cfg.hidden, cfg.inter
     nbytes = touched * H * I + touched * H * 4 + M * I + M * 4 + M * H * 2
-    return _kernel_roofline("down", "StreamGemmKernel<..., kDequant> (down GEMM + dequant; timer name gmm_dequant)",
+    return _kernel_roofline("down", _gemm_kernel_name(kernels, passes, "down GEMM + dequant; timer name gmm_dequant"),
                             "gmm_dequant", nbytes, 2 * M * H * I, kernels, passes)
 
 
@@ -324,6 +334,28 @@ def _other_configs(pkg, dev, headline, steps, warmup):
     return out
 
 
+def _rounded(value):
+    if isinstance(value, float):
+        return float("%.6g" % value)
+    if isinstance(value, dict):
+        return {k: _rounded(v) for k, v in value.items()}
+    return [_rounded(v) for v in value] if isinstance(value, (list, tuple)) else value
+
+
+def brief_line(result):
+    """The record as one line that a log's tail holds whole."""
+    line = {k: v for k, v in result.items() if k not in ("gemm_tile_balance", "workspace_bytes", "other_configs", "ms_per_step_repeats")}
+    if "ms_per_step_repeats" in result:
+        line["ms_per_step_min"], line["ms_per_step_max"] = (result["ms_per_step_repeats"][k] for k in ("min", "max"))
+    if "other_configs" in result:
+        line["other_configs"] = {
+            name: {"workload": s["workload"], "ms_per_step": s["ms_per_step"], "tokens_per_s": s["tokens_per_s"],
+                   "kernels_ms": s["kernels_ms"], "gate_up": {k: s["roofline"][k] for k in ("bound", "frac")},
+                   "down": {k: s["roofline_down_gemm"][k] for k in ("bound", "frac")}}
+            for name, s in result["other_configs"].items()}
+    return json.dumps(_rounded(line), separators=(",", ":"))
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -347,6 +379,7 @@ def main():
                     help="give the GEMM operators contiguous row-major [E, K, N] weights (the reference's plain ND layout)")
     ap.add_argument("--fused-combine", action="store_true",
                     help="end the chain with aclnnGroupedMatmulFinalizeRoutingV3 instead of GroupedMatmulV4 + MoeFinalizeRoutingV2")
+    ap.add_argument("--record", metavar="FILE", help="write the whole record there (the printed line is a part of it)")
     args = ap.parse_args()
     if args.gpus != 1:
         print("bench.py measures one GPU: this build has no multi-GPU path (expert parallelism is a design note only); "
@@ -420,7 +453,10 @@ def main():
                                   "sample": desc}
     if not args.no_other_configs:
         result["other_configs"] = _other_configs(pkg, dev, head, steps=min(args.steps, 20), warmup=min(args.warmup, 2))
-    print(json.dumps(result))
+    if args.record:
+        with open(args.record, "w") as f:
+            json.dump(result, f, indent=1)
+    print(brief_line(result))
 
 
 if __name__ == "__main__":
