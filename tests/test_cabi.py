@@ -719,6 +719,23 @@ def test_packed_descriptors(aclnn, dims):
         aclnn.tensor_of(torch.zeros((1,) * 9))
 
 
+@pytest.mark.parametrize("shape,stride,dtype", [
+    ((16, 256), (256, 1), torch.int8), ((16, 256), (512, 1), torch.int8), ((16, 256), (1, 16), torch.int8),
+    ((256, 16), (16, 1), torch.int8), ((16, 256), (256, 1), torch.float16)])
+def test_packed_descriptor_is_the_one_of_acl_create_tensor(aclnn, shape, stride, dtype):
+    """Extents, strides and type arrive where aclCreateTensor puts them: the first phase says the same to both, and to each of
+    these but the first something else than to a contiguous int8 [16, 256] (a copy in the workspace, an error)."""
+    x = torch.empty(1 << 14, dtype=dtype).as_strided(shape, stride)
+    seen = []
+    for handle in (aclnn.tensor_of(x), aclnn.create_tensor(list(shape), aclnn._DTYPE_CODE[dtype], x.data_ptr(), list(stride))):
+        args = _swiglu_args(aclnn, M=16, K=256, N=512, E=4)
+        args[0] = handle
+        seen.append(_status(aclnn, "aclnnGroupedMatmulSwigluQuant", args))
+    assert seen[0] == seen[1]
+    plain = _status(aclnn, "aclnnGroupedMatmulSwigluQuant", _swiglu_args(aclnn, M=16, K=256, N=512, E=4))
+    assert plain[0] == 0 and (seen[0] == plain) == ((shape, stride, dtype) == ((16, 256), (256, 1), torch.int8))
+
+
 def test_tile_height_leaves_room_for_uneven_groups(aclnn, monkeypatch):
     """45 rows each on average: 96-row tiles, since a router's groups are less even than their mean.  The workspace holds a
     table entry for every m-tile that the height allows."""

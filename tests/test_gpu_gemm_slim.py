@@ -6,9 +6,10 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# rows of each group, K, N (even; SwiGLU halves it).  The mean picks the tile (16, 32 or 64 rows); few tiles pick the deep ring.
+# rows of each group, K, N (even; SwiGLU halves it).  The mean picks the tile (16, 32 or 64 rows); each height has a ring depth of
+# its own.
 CASES = {
-    "one_token_two_experts": ([0, 1, 0, 0, 1, 0], 1024, 512),                       # deep, 16-row tile, idle groups
+    "one_token_two_experts": ([0, 1, 0, 0, 1, 0], 1024, 512),                       # 16-row tile, idle groups
     "one_row_k_one_step": ([1], 128, 256),                                            # a tile of one k-step
     "tile16_edges": ([16, 0, 15, 1, 17, 3, 2, 0, 1, 5] * 2, 256, 704),                # either side of 16 rows, partial n-tile
     "tile16_many_groups": ([(i * 7) % 5 for i in range(512)], 144, 192),              # the widest group list, K off the grid
@@ -25,6 +26,9 @@ CASES = {
     "tile16_as_64": ([0, 0, 0, 0, 0, 0, 0, 0, 65, 0, 0, 0, 0, 0, 0, 0, 0, 63] * 16, 144, 2048),
     "tile32_as_64": ([0, 130, 0, 0, 0, 1, 0, 64, 0, 0] * 12, 272, 2112),
 }
+
+
+PLANNED = {"one_token_two_experts": 16, "one_row_k_one_step": 16, "skewed": 32}  # the others have theirs in their name
 
 
 def _to_nz(w_dev):
@@ -54,6 +58,14 @@ def test_against_oracle(aclnn, oracle, dev, name, layout):
         wkw, wv = {}, [w]
     xd, ptd = t(x), t(pt)
     acc_ref = oracle.grouped_matmul_i32(x, wt, cumsum, w_trans=True)
+    if layout != "nd":  # row-major weights stay with the ring kernels
+        ws = aclnn.Workspace()
+        aclnn.gemm_workgroup_spans_enable(True)
+        aclnn.grouped_matmul_v4([xd], wv, group_list=t(cumsum), split_item=3, group_type=0, workspace=ws, **wkw)
+        span = next(iter(aclnn.gemm_workgroup_spans_report().values()))
+        aclnn.gemm_workgroup_spans_enable(False)
+        assert list(ws.requested.values()) == [256]          # no tile table in the workspace: the kernels under test
+        assert span["tile_rows"] == (PLANNED.get(name) or int(name[4:6]))
     for values, kind, dtype in ((cumsum, 0, torch.int64), (sizes, 1, torch.int32)):
         acc = torch.full((M + tail, N), -7, dtype=torch.int32, device=dev)
         aclnn.grouped_matmul_v4([xd], wv, group_list=t(values).to(dtype), split_item=3, group_type=0, group_list_type=kind,
@@ -98,6 +110,12 @@ def test_malformed_lists_stay_in_bounds(aclnn, dev, kind, values):
                             split_item=3, group_type=0, group_list_type=kind, out=[guard[:M]])
     torch.cuda.synchronize()
     assert bool((guard[M:] == -7).all())
+    q, q_scale = torch.full((M + 64, N // 2), 77, dtype=torch.int8, device=dev), torch.full((M + 64,), -7.0, device=dev)
+    if kind == 0:  # the SwiGLU operator takes cumulative sums only
+        aclnn.grouped_matmul_swiglu_quant(x, w.transpose(1, 2), torch.tensor(values, dtype=torch.int64, device=dev),
+                                          torch.rand((5, N), device=dev), torch.rand(M, device=dev), out=(q[:M], q_scale[:M]))
+        torch.cuda.synchronize()
+        assert bool((q[M:] == 77).all()) and bool((q_scale[M:] == -7).all())
 
 
 @pytest.mark.parametrize("rows,planned", [(128, 16), (512, 32)])

@@ -10,9 +10,11 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("layout", ["kmajor", "nd", "nz"])
 @pytest.mark.parametrize("tile_m,K", [(32, 144), (64, 240), (64, 1040), (96, 160), (128, 208), (128, 1136), (160, 1120),
-                                      (192, 144), (192, 1072), (256, 176), (256, 1088)])
+                                      (192, 144), (192, 1072), (256, 176), (256, 1088),
+                                      (96, 1008), (192, 912), (256, 960)])
 def test_k_off_the_step_grid(aclnn, oracle, dev, monkeypatch, tile_m, K, layout):
-    """Overlaps of 16 to 112 bytes in every tile height and layout; K of nine steps is pulled where the height allows it.
+    """Overlaps of 16 to 112 bytes in every tile height and layout; K of eight
+    steps (the fewest) and of nine is pulled where the height allows it.
     Several tiles per workgroup, an empty group, groups past a tile, and the tensors' last rows in the last tile."""
     monkeypatch.setenv("OPAPI_GEMM_TILE_M", str(tile_m))
     rng = np.random.default_rng(tile_m + K)

@@ -434,13 +434,24 @@ def test_decode_sized_calls_sort_and_gather_in_one_launch(aclnn, oracle, dev, T,
             assert np.array_equal(ex.view(np.uint8), ex_r.view(np.uint8))
 
 
+@pytest.fixture
+def dirty_memory(monkeypatch):
+    """torch.empty hands out 77s and NaNs: an output element that nothing writes shows."""
+    empty = torch.empty
+
+    def dirty(*args, **kw):
+        t = empty(*args, **kw)
+        return t.fill_(float("nan") if t.is_floating_point() else 77)
+    monkeypatch.setattr(torch, "empty", dirty)
+
+
 @pytest.mark.parametrize("T,K,H,dtype_name", [
     (3, 2, 8, "bf16"), (5, 4, 4096, "f32"), (5, 4, 4104, "f16"), (4, 8, 8192, "bf16"), (4, 3, 8200, "bf16"),
     (5, 4, 8, "bf16"), (3, 64, 512, "f16"), (5, 4, 520, "f32"), (5, 4, 1024, "bf16"), (3, 64, 1032, "bf16"), (5, 4, 2048, "f32"),
     (5, 4, 2056, "f16"),         # workgroups of 64, 128, 256 and 512 threads
     (2, 64, 16384, "f16"),       # the widest row and the most experts per token of the packet kernel
     (2, 65, 64, "bf16"), (2, 4, 16392, "bf16"), (3, 4, 4100, "bf16")])  # one past either, and no whole packets
-def test_dynamic_quant_row_widths(aclnn, oracle, dev, T, K, H, dtype_name):
+def test_dynamic_quant_row_widths(aclnn, oracle, dev, dirty_memory, T, K, H, dtype_name):
     """Dynamic quantisation without a smooth scale at the widths where its kernels change hands (workgroups as wide as the row
     up to 4096 elements, then two or up to four packets per thread), through both operators, on outputs that do not start at zero."""
     rng = np.random.default_rng(T * 3 + H)
@@ -449,7 +460,6 @@ def test_dynamic_quant_row_widths(aclnn, oracle, dev, T, K, H, dtype_name):
     x, i = xt.to(dev), torch.from_numpy(idx).to(dev)
     for kw in (dict(expert_tokens_count_or_cumsum_flag=2), dict(expert_tokens_count_or_cumsum_flag=1, active_num=T),
                dict(drop_pad_mode=1, expert_capacity=max(1, T // 2), expert_tokens_before_capacity_flag=True)):
-        torch.full((64 << 20,), 77, dtype=torch.int8, device=dev)  # what the allocator hands out next is not zero
         got = aclnn.moe_init_routing_quant_v2(x, i, 1, None, None, expert_num=E, **kw)
         want = oracle.moe_init_routing_quant_v2(
             bits, idx, 1, None, None, active_num=kw.get("active_num", 0), expert_capacity=kw.get("expert_capacity", 0),
@@ -462,17 +472,6 @@ def test_dynamic_quant_row_widths(aclnn, oracle, dev, T, K, H, dtype_name):
         want = oracle.moe_init_routing_v3_quant(bits, idx, None, E, rng_, mode, 1, dtype=code)
         for g, w in zip(got, want):
             assert np.array_equal(g.cpu().numpy(), w)
-
-
-@pytest.fixture
-def dirty_memory(monkeypatch):
-    """torch.empty hands out 77s and NaNs: an output element that nothing writes shows."""
-    empty = torch.empty
-
-    def dirty(*args, **kw):
-        t = empty(*args, **kw)
-        return t.fill_(float("nan") if t.is_floating_point() else 77)
-    monkeypatch.setattr(torch, "empty", dirty)
 
 
 @pytest.mark.parametrize("drop_pad", [0, 1])
@@ -505,3 +504,31 @@ def test_dynamic_quant_of_narrow_rows_beats_the_general_kernel(aclnn, dev):
         aclnn.kernel_timer_enable(False)
         return report["routing_quant_gather"][1]
     assert np.median([gather_ms(None) / gather_ms(ones) for _ in range(5)]) < 0.8
+
+
+@pytest.mark.parametrize("T,K,H", [(3, 2, 8), (40, 8, 256), (2000, 8, 24), (5, 4, 1)])
+def test_copied_rows_leave_no_output_unwritten(aclnn, oracle, dev, dirty_memory, T, K, H):
+    """Rows copied unchanged (quant_mode -1), with and without a per-token scale, over all experts and over a range of them, and
+    static quantisation: every element of every output is written or starts at zero."""
+    rng = np.random.default_rng(T + H)
+    E = 70
+    x, idx = rng.standard_normal((T, H)).astype(np.float32), rng.integers(0, E, (T, K)).astype(np.int32)
+    scale = rng.uniform(0.1, 1.0, T).astype(np.float32)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    for with_scale in (False, True):
+        for mode, rng_ in ((0, None), (1, None), (2, None), (1, (10, 40))):
+            got = aclnn.moe_init_routing_v3(t(x), t(idx), scale=t(scale) if with_scale else None, expert_num=E,
+                                            expert_tokens_num_type=mode, active_expert_range=rng_)
+            want = oracle.moe_init_routing_v3(x, idx, scale if with_scale else None, E, rng_, mode, 1)
+            for g, w in zip(got, want):
+                assert (g is None and w is None) or np.array_equal(g.cpu().numpy(), w), (with_scale, mode, rng_)
+    one, off = np.array([3.0], np.float32), np.array([0.5], np.float32)
+    for kw in (dict(expert_tokens_count_or_cumsum_flag=2), dict(expert_tokens_count_or_cumsum_flag=1, active_num=T),
+               dict(drop_pad_mode=1, expert_capacity=max(1, T // 2), expert_tokens_before_capacity_flag=True)):
+        got = aclnn.moe_init_routing_quant_v2(t(x), t(idx), 0, t(one), t(off), expert_num=E, **kw)
+        want = oracle.moe_init_routing_quant_v2(
+            x, idx, 0, one, off, active_num=kw.get("active_num", 0), expert_capacity=kw.get("expert_capacity", 0), expert_num=E,
+            drop_pad_mode=kw.get("drop_pad_mode", 0), count_flag=kw.get("expert_tokens_count_or_cumsum_flag", 0),
+            before_capacity_flag=kw.get("expert_tokens_before_capacity_flag", False))
+        for g, w, name in zip(got, want, ("expandedX", "expandedRowIdx", "countOrCumsum", "beforeCapacity", "dynScale")):
+            assert _same(g, w), (kw, name)
