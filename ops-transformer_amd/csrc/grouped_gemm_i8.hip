@@ -93,7 +93,7 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
         for (int i = 0; i < wave; ++i) base += waveTotal64[i];
         return v + base;
     };
-    // group boundaries, clamped into [0, M] and made monotonic so that a malformed list cannot push rows out of range
+    // group boundaries, clamped into [0, M], no end before its begin, so that a malformed list cannot push rows out of range
     int64_t begin = 0, end = 0;
     if (a.isCount == 2) {
         // Sparse list [groups, 2]: pair p = (expert id, rows); pairs take consecutive row ranges in list order and the
