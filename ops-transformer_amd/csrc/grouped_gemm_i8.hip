@@ -1,7 +1,7 @@
 // Expert-grouped int8 x int8 -> int32 GEMM for gfx950 (CDNA4) with fused epilogues.
 //
 // Computes, for every group e and every row r of that group, acc[r, c] = sum_k x[r, k] * w[e, k, c] on
-// v_mfma_i32_32x32x32_i8 and applies one of three epilogues in registers:
+// v_mfma_i32_16x16x64_i8 and applies one of three epilogues in registers:
 //   kInt32   raw accumulators                                   (aclnnGroupedMatmulV4, int32 output)
 //   kDequant (float(acc) * scale[e, c]) * rowScale[r] -> bf16 / fp16 / fp32
 //            (reference order: gmm/grouped_matmul/op_kernel/grouped_matmul_quant_mixcore.h:248-291,293-310)
@@ -19,9 +19,9 @@
 // This file: the scheduling kernel, the requantisation kernel, planning and the launch sequence.  The GEMM kernels
 // themselves are in grouped_gemm_i8_kernels.h and are instantiated by one translation unit per epilogue:
 //   StreamGemmKernel  the fast path (K a multiple of 16; K-contiguous, blocked or row-major [K, N] weights).  Persistent
-//                     workgroups; operands go global -> LDS with global_load_lds_dwordx4 into a ring of 2..4 stages of
+//                     workgroups; operands go global -> LDS with global_load_lds_dwordx4 into rings of 2..4 stages of
 //                     128 k-bytes (192-row tiles: two activation and three weight stages), so several stages of weights
-//                     are in flight per CU with no staging registers, and the ring already holds the next tile's first
+//                     are in flight per CU with no staging registers, and the rings already hold the next tile's first
 //                     steps while the current tile's epilogue runs.
 //   MixedGemmKernel   the same body twice, once per run of the table with a stage geometry of its own (pulled tiles of
 //                     192 and 256 rows).
@@ -253,7 +253,6 @@ __device__ __forceinline__ int8_t QuantOne(float s, float inv) {
 __global__ __launch_bounds__(256) void RequantKernel(RequantArgs a) {
     const int64_t row = a.rowBegin + blockIdx.x;
     if (row >= a.sched[kHdrCoveredRows]) return;
-    typedef float Float4 __attribute__((ext_vector_type(4)));
     const float* src = a.s + static_cast<int64_t>(blockIdx.x) * a.halfN;
     int8_t* dst = a.y + row * a.halfN;
     const bool packets = (a.halfN & 3) == 0;
@@ -486,8 +485,6 @@ Plan MakePlan(const Problem& p) {
         plan.pullTiles = StreamOk(p) && kSteps >= 8 && plan.maxTiles < (1ll << 31) && std::atoi(env) != 0;
     }
     if (lowHolds && plan.tileM == 192 && plan.pullTiles && std::getenv("OPAPI_GEMM_TILE_M") == nullptr) plan.lowTileM = kLowTileM;
-    plan.wavesM = plan.tileM >= 64 && StreamOk(p) ? 2 : 1;
-    plan.subTilesM = (plan.tileM / 32 + plan.wavesM - 1) / plan.wavesM;
     const int64_t maxMTiles = p.M / (plan.lowTileM > 0 ? plan.lowTileM : plan.tileM) + groups;
     plan.maxMTiles = static_cast<int32_t>(maxMTiles);
     // round up so that every XCD's share [xcd * ceil(total/8), ...) is covered by the launch

@@ -88,8 +88,10 @@ namespace {
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) v2i* LdsV2iPtr;
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(3))) const v4i* LdsV4iPtr;
 typedef float Float2 __attribute__((ext_vector_type(2)));
+typedef float Float4 __attribute__((ext_vector_type(4)));
+typedef uint32_t Uint2 __attribute__((ext_vector_type(2)));
 typedef __bf16 Bf16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kTileN = 256;
@@ -137,20 +139,21 @@ struct TileInfo {
 
 // Tile `logical` of one run of the m-tile table (`count` m-tiles from entry `first` on).  Bands of bandWidth m-tiles walk
 // the n-tiles together: consecutive tiles are the band's m-tiles at one n-tile, then the next n-tile.
-template <int kTileM, bool kSwiglu>
+template <bool kSwiglu>
 __device__ __forceinline__ TileInfo DecodeListTile(const KernelArgs& a, const int4* __restrict__ table, int32_t first,
-                                                   int32_t count, int32_t bandWidth, int64_t logical) {
+                                                   int32_t count, int32_t bandWidth, int32_t logical) {
     TileInfo t{};
     const int32_t perBand = bandWidth * a.tilesN;
-    const int32_t band = static_cast<int32_t>(logical / perBand);
-    const int32_t rem = static_cast<int32_t>(logical % perBand);
+    const int32_t band = logical / perBand;
+    const int32_t rem = logical - band * perBand;
     const int32_t bandTiles = min(bandWidth, count - bandWidth * band);
-    const int4 e = table[first + bandWidth * band + rem % bandTiles];
+    const int32_t tileN = rem / bandTiles;
+    const int4 e = table[first + bandWidth * band + rem - tileN * bandTiles];
     t.valid = 1;
     t.group = e.x;
     t.rowBase = e.y;
-    t.rows = e.z;  // 1..kTileM
-    t.tileN = rem / bandTiles;
+    t.rows = e.z;
+    t.tileN = tileN;
     t.colBase = kSwiglu ? t.tileN * (kTileN / 2) : t.tileN * kTileN;
     return t;
 }
@@ -163,10 +166,10 @@ __device__ __forceinline__ TileInfo DecodeListTile(const KernelArgs& a, const in
 // while tiles are left anywhere.  The counters are only ever added to (values past a share's size mean "used up").
 // (The lists' sizes travel as plain values: a structure handed round by reference, or an array indexed at run time,
 // ends up in scratch memory.)
-__device__ __forceinline__ void QueueShare(int64_t tilesBig, int64_t tilesSmall, int counter, int64_t* first, int64_t* size) {
-    const int64_t total = (counter & 1) ? tilesSmall : tilesBig;
-    const int64_t per = (total + kXcds - 1) / kXcds;
-    const int64_t begin = (counter >> 1) * per;
+__device__ __forceinline__ void QueueShare(int32_t tilesBig, int32_t tilesSmall, int counter, int32_t* first, int32_t* size) {
+    const int32_t total = (counter & 1) ? tilesSmall : tilesBig;
+    const int32_t per = (total + kXcds - 1) / kXcds;
+    const int32_t begin = (counter >> 1) * per;
     *first = begin;
     *size = total - begin < 0 ? 0 : (total - begin < per ? total - begin : per);
 }
@@ -194,12 +197,12 @@ struct QueueDraw {
     int32_t logical;  // tile inside that list's run
     uint32_t usedUp;  // the caller's mask of used-up counters, updated
 };
-__device__ __forceinline__ QueueDraw QueueResolve(int64_t tilesBig, int64_t tilesSmall, int32_t* counters, int home, int prefer,
+__device__ __forceinline__ QueueDraw QueueResolve(int32_t tilesBig, int32_t tilesSmall, int32_t* counters, int home, int prefer,
                                                   uint32_t usedUp, int c, int32_t v, bool onlyPreferred = false) {
     while (c >= 0) {
-        int64_t first, size;
+        int32_t first, size;
         QueueShare(tilesBig, tilesSmall, c, &first, &size);
-        if (v < size) return QueueDraw{c & 1, static_cast<int32_t>(first + v), usedUp};
+        if (v < size) return QueueDraw{c & 1, first + v, usedUp};
         usedUp |= 1u << c;
         // a look at all sixteen counters at once (one round trip) spares a failed draw, i.e. a round trip, per used-up share
         int32_t now[2 * kXcds];  // fully unrolled below: stays in registers
@@ -216,13 +219,44 @@ __device__ __forceinline__ QueueDraw QueueResolve(int64_t tilesBig, int64_t tile
     return QueueDraw{-1, 0, usedUp};
 }
 
-// Output channel held in row r of the weight tile (clamped: channels past N are loaded but never stored).
+// ---------------------------------------------------------------------------------------------- tiles and their waves
+// A tile is up to kRows rows x 256 channels, computed by eight waves: two wave rows x four wave columns.  The matrix
+// instruction is v_mfma_i32_16x16x64_i8: per operation it costs the power of 0.85 of a 32x32x32 one -- eight waves per CU on
+// register operands sustain 4.10 POP/s with it against 3.48, uniform random bytes, both at the power limit (4.84 / 4.92
+// with zeros) -- and it splits a tile's rows in sixteens.
+//   Rows: 16-row block b of the tile belongs to wave row b & 1, and there to its first half (b & 2 == 0) or its second, as
+//   number b >> 2: whatever the tile's row count, the four (wave row, half) pairs hold the same number of blocks but for one.
+//   Channels: the 256 channels are two halves of 128 rows in LDS, 32 of each belonging to each wave column, as two blocks
+//   of sixteen.  kSwiglu: the first half is activated, the second linear.
+constexpr int kWaves = 8;
+constexpr int kThreads = 64 * kWaves;
+
+// Which channel a row of a weight half is.  Weights by channel (K-contiguous) may lie in LDS in any order, and they lie so
+// that the accumulators of a lane are neighbouring channels: four (kSwiglu: two of S), one store.  The two layouts with the
+// channels side by side in memory hand sixteen neighbours to sixteen lanes.
+constexpr int kOrderLane = 0;   // K-contiguous: wave column w, block j, lane l: channel 64 w + 4 l + 2 half + j
+constexpr int kOrderBlock = 1;  // blocked: 64 w + 32 half + 16 j + l
+constexpr int kOrderFar = 2;    // row-major: 128 half + 32 w + 16 j + l
+template <bool kNz, bool kNMajor>
+constexpr int kOrderOf = kNz ? kOrderBlock : kNMajor ? kOrderFar : kOrderLane;
+
+// Scatter-add of the rows wants neighbouring lanes on neighbouring channels: the order of the blocked layout.
+__device__ __forceinline__ bool LanesHoldNeighbours(const KernelArgs& a) { return a.combineIndex == nullptr; }
+
+// Channel of column block n = 2 * half + j (j = 0, 1) and lane l of wave column w, from the tile's first on
+// (kSwiglu: column of S, the same for both halves).
+template <int kOrder, bool kSwiglu>
+__device__ __forceinline__ int ColumnInTile(int w, int n, int l, bool neighbours) {
+    if (kSwiglu) return 32 * w + (kOrder == kOrderLane ? 2 * l + (n & 1) : 16 * (n & 1) + l);
+    if (kOrder == kOrderFar) return 128 * (n >> 1) + 32 * w + 16 * (n & 1) + l;
+    return 64 * w + (kOrder == kOrderLane && neighbours ? 4 * l + n : 16 * n + l);
+}
+
+// Channel held in row r of weight half `half`, K-contiguous weights (clamped: channels past N are loaded but never stored).
 template <bool kSwiglu>
-__device__ __forceinline__ int32_t ChannelOfRow(const KernelArgs& a, const TileInfo& t, int r) {
-    int32_t n;
-    if (kSwiglu) n = r < kTileN / 2 ? t.colBase + r : a.halfN + t.colBase + (r - kTileN / 2);
-    else n = t.colBase + r;
-    return n < a.N ? n : a.N - 1;
+__device__ __forceinline__ int32_t ChannelOfRow(const KernelArgs& a, const TileInfo& t, int half, int r) {
+    const int32_t col = t.colBase + ColumnInTile<kOrderLane, kSwiglu>(r >> 5, 2 * half + ((r >> 4) & 1), r & 15, LanesHoldNeighbours(a));
+    return min(kSwiglu && half ? a.halfN + col : col, a.N - 1);
 }
 
 __device__ __forceinline__ float LoadScale(const void* p, int64_t i, int dtype) {
@@ -241,314 +275,318 @@ __device__ __forceinline__ uint16_t HalfBitsOfRounded(float f) {
     return __half_as_ushort(__float2half_rn(f));
 }
 
+// Two values to bf16 (else fp16), the first in the low half.
+template <bool kToBf16>
+__device__ __forceinline__ uint32_t PackHalves(float lo, float hi) {
+    if constexpr (kToBf16) {
+        const Float2 f = {lo, hi};
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, Bf16x2));  // v_cvt_pk_bf16_f32
+    } else {
+        return static_cast<uint32_t>(HalfBitsOfRounded(lo)) | (static_cast<uint32_t>(HalfBitsOfRounded(hi)) << 16);
+    }
+}
+
+// The value of another lane of the row of sixteen (kCtl: a DPP control).
+template <int kCtl>
+__device__ __forceinline__ float RowLane(float v) {
+    return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(__float_as_uint(v)), kCtl, 0xF, 0xF, true)));
+}
+
+// Maximum over the 16 lanes of a row group, in every lane (rotations inside the row: no LDS).
+__device__ __forceinline__ float MaxOver16(float v) {
+    v = fmaxf(v, RowLane<0x128>(v));  // row_ror:8
+    v = fmaxf(v, RowLane<0x124>(v));
+    v = fmaxf(v, RowLane<0x122>(v));
+    return fmaxf(v, RowLane<0x121>(v));
+}
+
+// Maxima of four values over the 16 lanes of a row group: lane l gets that of value l >> 2.  A halving butterfly: a lane
+// gives its partner the values that it drops.
+__device__ __forceinline__ float FourMaxOver16(const float (&m)[4], int l16) {
+    const bool b3 = (l16 & 8) != 0, b2 = (l16 & 4) != 0;
+    const float k0 = fmaxf(b3 ? m[2] : m[0], RowLane<0x140>(b3 ? m[0] : m[2]));  // row_mirror: lane 15 - l
+    const float k1 = fmaxf(b3 ? m[3] : m[1], RowLane<0x140>(b3 ? m[1] : m[3]));
+    float k = fmaxf(b2 ? k1 : k0, RowLane<0x141>(b2 ? k0 : k1));                 // row_half_mirror: 7 - l in each eight
+    k = fmaxf(k, RowLane<0x4E>(k));                                              // quad_perm [2,3,0,1], [1,0,3,2]
+    return fmaxf(k, RowLane<0xB1>(k));
+}
+
 // Byte offset of (channel n, k = 0) inside one expert's weights; consecutive k are a.wStrideK bytes apart (32 in the
 // blocked layout: a 32-channel block holds its K rows of 32 channel bytes back to back).
 __device__ __forceinline__ int64_t WeightRowBase(const KernelArgs& a, int32_t n) {
     return a.wNz ? static_cast<int64_t>(n >> 5) * a.K * 32 + (n & 31) : static_cast<int64_t>(n) * a.wStrideN;
 }
 
-// Epilogue of one tile.  acc[mi][ni][v] is C[row, col] with row = waveRow0 + 32*mi + 8*(v/4) + 4*lhi + (v%4); the wave
-// owns column blocks ni = 0, 1, lane l32 inside each (plain: 64*waveN + 32*ni; kSwiglu: S column 32*waveN and its partner).
-// Only the first mySub accumulator tiles of the wave are real.  ldsRowScale holds the tile's per-row scales.
+// Blocks of a wave in the first and in the second half of its rows, tile of kRows rows.
+template <int kRows>
+struct RowBlocks {
+    static_assert(kRows % 32 == 0, "both wave rows hold the same number of 16-row blocks");
+    static constexpr int kFirst = (kRows + 63) / 64, kSecond = kRows / 64, kAll = kFirst + kSecond;
+    // first tile row of block m (first half, then second half) of wave row `waveM`
+    __device__ static __forceinline__ int RowOf(int m, int waveM) {
+        return 16 * (m < kFirst ? 4 * m + waveM : 4 * (m - kFirst) + 2 + waveM);
+    }
+};
+
+// Epilogue of one tile.  acc[m][n][v] is C[row, col] with row = RowOf(m) + 4 * quad + v and col = ColumnInTile(n) of lane l16.
+// ldsRowScale holds the tile's per-row scales.
 // afterScaleLoads() is called once the channel scales of the tile have been requested and before anything is stored: a
 // memory request made there queues behind loads whose answers the epilogue needs first, not in front of them.
+// Row checks are made per 16-row block, wave-uniformly: a block wholly inside the expert's rows takes a copy of the code
+// without checks, a block wholly outside is skipped, and only the one that straddles the last row tests every lane.  (A
+// per-lane test makes every element a predicated basic block of its own, and their independent chains no longer interleave.)
 struct NoHook {
     __device__ __forceinline__ void operator()() const {}
 };
-//
-// A wave that holds kNi = 4 column blocks (four waves per tile, 128 x 128 each) calls the per-wave part once per pair
-// of blocks: kPair picks acc[mi][2 * kPair] and acc[mi][2 * kPair + 1], and waveN is then the column position
-// 0..3 that this pair has in the tile (what the wave index is when eight waves hold one pair each).
-template <int kSubM, int kNi, int kPair, int kTileM, Epilogue kEpi, typename Hook = NoHook>
-__device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const TileInfo& t, v16i (&accAll)[kSubM][kNi], int mySub,
-                                                 int waveRow0, int waveN, int l32, int lhi,
-                                                 const float* ldsRowScale, float* ldsRowMax, Hook afterScaleLoads = NoHook{}) {
-    // the pair's two accumulator columns under the name the code below uses: acc(mi, 0 / 1)
-    auto acc = [&](int mi, int j) __attribute__((always_inline)) -> v16i& { return accAll[mi][2 * kPair + j]; };
+template <int kRows, Epilogue kEpi, int kOrder, typename Hook = NoHook>
+__device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const TileInfo& t, v4i (&acc)[RowBlocks<kRows>::kAll][4], int waveM,
+                                                 int waveN, int l16, int quad, const float* ldsRowScale, float* ldsRowMax,
+                                                 Hook afterScaleLoads = NoHook{}) {
+    using Blocks = RowBlocks<kRows>;
+    constexpr bool kSwiglu = kEpi == Epilogue::kSwiglu;
     const int32_t rows = t.rows, rowBase = t.rowBase, group = t.group;
     // The row / address arithmetic below depends only on the lane; hoisted out of the persistent tile loop it would
     // stay alive across the whole kernel and spill, and a reload in here waits for every store issued so far.  An
     // opaque per-call zero folded into the lane index keeps the arithmetic inside the epilogue.
     int opaqueZero;
     asm volatile("v_mov_b32 %0, 0" : "=v"(opaqueZero));
-    lhi += opaqueZero;
-    l32 += opaqueZero;
-    if (kEpi == Epilogue::kInt32 || kEpi == Epilogue::kDequant) {
+    quad += opaqueZero;
+    l16 += opaqueZero;
+    const bool neighbours = kOrder == kOrderLane && LanesHoldNeighbours(a);
+    if constexpr (!kSwiglu) {
         const bool hasRowScale = a.rowScale != nullptr;
-        const int32_t n0 = t.colBase + 64 * waveN + l32;  // column block 0; block 1 is 32 columns further
-        const bool valid0 = n0 < a.N, valid1 = n0 + 32 < a.N;
-        float sc0 = 0.0f, sc1 = 0.0f;
-        if (kEpi == Epilogue::kDequant) {
-            if (valid0) sc0 = LoadScale(a.scale, static_cast<int64_t>(group) * a.N + n0, a.scaleDtype);
-            if (valid1) sc1 = LoadScale(a.scale, static_cast<int64_t>(group) * a.N + n0 + 32, a.scaleDtype);
-        }
-        float bias0 = 0.0f, bias1 = 0.0f;
-        if (kEpi == Epilogue::kDequant && a.bias != nullptr) {
-            if (valid0) bias0 = LoadScale(a.bias, static_cast<int64_t>(group) * a.N + n0, a.biasDtype);
-            if (valid1) bias1 = LoadScale(a.bias, static_cast<int64_t>(group) * a.N + n0 + 32, a.biasDtype);
+        int32_t col[4];
+        bool valid[4];
+        float sc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            col[n] = t.colBase + ColumnInTile<kOrder, false>(waveN, n, l16, neighbours);
+            valid[n] = col[n] < a.N;
+            if (kEpi == Epilogue::kDequant && valid[n]) sc[n] = LoadScale(a.scale, static_cast<int64_t>(group) * a.N + col[n], a.scaleDtype);
         }
         afterScaleLoads();
-        // 16-bit outputs: a lane holds one column of each block, i.e. 2-byte pieces 64 bytes apart.  Neighbouring lanes
-        // swap one value so that an even lane owns columns (c, c+1) of block 0 and the odd lane next to it the same pair
-        // of block 1; every lane then stores one aligned 32-bit word and a half-wave covers a whole 128-byte row segment.
-        const bool pairStores = kEpi == Epilogue::kDequant && a.outDtype != 0 && (a.N & 1) == 0 &&
-                                t.colBase + 64 * waveN + 64 <= a.N;  // wave-uniform
-        const bool oddLane = (l32 & 1) != 0;
-        if (kEpi == Epilogue::kDequant && (a.outDtype == 27 || a.outDtype == 1) && pairStores) {
+        // wave-uniform: every channel of the wave exists
+        const bool whole = t.colBase + ColumnInTile<kOrder, false>(waveN, 3, 15, neighbours) < a.N;
+        const bool vectors = (a.N & 3) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;  // rows start on a lane's vector
+        const bool oddLane = (l16 & 1) != 0;
+        if (kEpi == Epilogue::kDequant && (a.outDtype == 27 || a.outDtype == 1) && whole &&
+            (kOrder == kOrderLane ? vectors : (a.N & 1) == 0)) {
+            // 16-bit results of whole column blocks, without per-element dtype dispatch; stores through a (uniform row pointer
+            // + 32-bit lane offset) address.  Past the caches: nothing reads them back before they have left these.
             const bool toBf16 = a.outDtype == 27;  // wave-uniform: bf16, else fp16
-            // The common case (16-bit output, whole column pairs) without per-element dtype dispatch: row scales come
-            // from LDS four at a time, every lane stores one 32-bit word per accumulator pair through a
-            // (uniform row pointer + 32-bit lane offset) address.
-            uint16_t* const outTile = static_cast<uint16_t*>(a.out) + static_cast<int64_t>(rowBase + waveRow0) * a.N;
-            const int32_t laneOff = 4 * lhi * a.N + (oddLane ? n0 + 31 : n0);
+            uint16_t* const outTile = static_cast<uint16_t*>(a.out) + static_cast<int64_t>(rowBase) * a.N;
+            // lanes of channels side by side swap one value with their neighbour, and an even lane stores columns (c, c + 1) of
+            // the first of two blocks, the odd lane next to it the same pair of the second
+            const int32_t laneOff = 4 * quad * a.N + (kOrder == kOrderLane ? col[0] : oddLane ? col[0] + 15 : col[0]);
+            constexpr int kPairStride = kOrder == kOrderFar ? 128 : 32;  // columns from the first two blocks to the other two
+            auto block = [&](int m, auto fullTag, auto bf16Tag) __attribute__((always_inline)) {
+                constexpr bool kFull = decltype(fullTag)::value;
+                constexpr bool kToBf16 = decltype(bf16Tag)::value;  // compile-time: a run-time choice per element splits the block
+                const int rTop = Blocks::RowOf(m, waveM);
+                float4 rs = make_float4(1.0f, 1.0f, 1.0f, 1.0f);  // multiplying by 1 is exact
+                if (hasRowScale) rs = *reinterpret_cast<const float4*>(ldsRowScale + rTop + 4 * quad);
+                const float rsv[4] = {rs.x, rs.y, rs.z, rs.w};
 #pragma unroll
-            for (int mi = 0; mi < kSubM; ++mi) {
-                const int rTop = waveRow0 + 32 * mi;
-                if (mi >= mySub || rTop >= rows) continue;
-                // The row checks are made per group of eight rows (accumulator entries 4q .. 4q + 3 of the two lane
-                // halves), wave-uniformly: a group wholly inside the expert's rows takes a copy of the code without
-                // checks, a group wholly outside is skipped, and only the one group that straddles the last row tests
-                // every lane.  A per-lane test makes every element a predicated basic block of its own, and the
-                // independent chains of a tile no longer interleave.
-                // the tile's 32 row scales, read in one go (one wave-uniform test instead of one per row group)
-                float4 rsTile[4];
+                for (int v = 0; v < 4; ++v) {
+                    float y[4];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) rsTile[q] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);  // multiplying by 1 is exact
-                if (hasRowScale) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) rsTile[q] = *reinterpret_cast<const float4*>(ldsRowScale + rTop + 8 * q + 4 * lhi);
-                }
-                auto rowGroup = [&](int q, auto fullTag, auto bf16Tag) __attribute__((always_inline)) {
-                    constexpr bool kFull = decltype(fullTag)::value;
-                    constexpr bool kToBf16 = decltype(bf16Tag)::value;  // compile-time: a run-time choice per element splits the block
-                    const float4 rs = rsTile[q];
-                    const float rsv[4] = {rs.x, rs.y, rs.z, rs.w};
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int v = 4 * q + i;
-                        const Float2 f = {__fmul_rn(__fmul_rn(static_cast<float>(acc(mi, 0)[v]), sc0), rsv[i]),
-                                          __fmul_rn(__fmul_rn(static_cast<float>(acc(mi, 1)[v]), sc1), rsv[i])};
-                        uint32_t pk;
-                        if constexpr (kToBf16) {
-                            pk = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, Bf16x2));
-                        } else {
-                            pk = static_cast<uint32_t>(HalfBitsOfRounded(f[0])) | (static_cast<uint32_t>(HalfBitsOfRounded(f[1])) << 16);
-                        }
-                        const uint32_t got = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(pk), 0xB1, 0xF, 0xF, true));
-                        const uint32_t word = __builtin_amdgcn_perm(got, pk, oddLane ? 0x03020706u : 0x05040100u);
-                        uint16_t* const rowPtr = outTile + static_cast<int64_t>(32 * mi + 8 * q + i) * a.N;
-                        if (kFull || rTop + 8 * q + 4 * lhi + i < rows) __builtin_nontemporal_store(word, reinterpret_cast<uint32_t*>(rowPtr + laneOff));
-                    }
-                };
-                auto rowsOfTile = [&](auto bf16Tag) __attribute__((always_inline)) {
-                    if (rTop + 32 <= rows) {
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) rowGroup(q, std::true_type{}, bf16Tag);
+                    for (int n = 0; n < 4; ++n) y[n] = __fmul_rn(__fmul_rn(static_cast<float>(acc[m][n][v]), sc[n]), rsv[v]);
+                    uint32_t word[2] = {PackHalves<kToBf16>(y[0], y[1]), PackHalves<kToBf16>(y[2], y[3])};
+                    uint16_t* const rowPtr = outTile + static_cast<int64_t>(rTop + v) * a.N;
+                    const bool ok = kFull || rTop + 4 * quad + v < rows;
+                    if constexpr (kOrder == kOrderLane) {
+                        if (ok) __builtin_nontemporal_store(Uint2{word[0], word[1]}, reinterpret_cast<Uint2*>(rowPtr + laneOff));
                     } else {
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            if (rTop + 8 * q >= rows) break;
-                            if (rTop + 8 * q + 8 <= rows) rowGroup(q, std::true_type{}, bf16Tag);
-                            else rowGroup(q, std::false_type{}, bf16Tag);
+                        for (int p = 0; p < 2; ++p) {
+                            const uint32_t got = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(word[p]), 0xB1, 0xF, 0xF, true));
+                            word[p] = __builtin_amdgcn_perm(got, word[p], oddLane ? 0x03020706u : 0x05040100u);
+                            if (ok) __builtin_nontemporal_store(word[p], reinterpret_cast<uint32_t*>(rowPtr + laneOff + kPairStride * p));
                         }
                     }
-                };
-                if (toBf16) rowsOfTile(std::true_type{});
-                else rowsOfTile(std::false_type{});
+                }
+            };
+#pragma unroll
+            for (int m = 0; m < Blocks::kAll; ++m) {
+                const int rTop = Blocks::RowOf(m, waveM);
+                if (rTop >= rows) continue;
+                if (rTop + 16 <= rows) {
+                    if (toBf16) block(m, std::true_type{}, std::true_type{});
+                    else block(m, std::true_type{}, std::false_type{});
+                } else {
+                    if (toBf16) block(m, std::false_type{}, std::true_type{});
+                    else block(m, std::false_type{}, std::false_type{});
+                }
             }
             return;
         }
+        const bool vectorStores = neighbours && whole && vectors;
+        float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (kEpi == Epilogue::kDequant && a.bias != nullptr) {
 #pragma unroll
-        for (int mi = 0; mi < kSubM; ++mi) {
-            if (mi >= mySub || waveRow0 + 32 * mi >= rows) continue;
+            for (int n = 0; n < 4; ++n) {
+                if (valid[n]) bias[n] = LoadScale(a.bias, static_cast<int64_t>(group) * a.N + col[n], a.biasDtype);
+            }
+        }
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int r = waveRow0 + 32 * mi + 8 * (v / 4) + 4 * lhi + (v % 4);
+        for (int m = 0; m < Blocks::kAll; ++m) {
+            const int rTop = Blocks::RowOf(m, waveM);
+            if (rTop >= rows) continue;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int r = rTop + 4 * quad + v;
+                if (r >= rows) continue;
                 const int64_t rowOff = static_cast<int64_t>(rowBase + r) * a.N;
-                if (kEpi == Epilogue::kInt32) {
-                    if (r < rows && valid0) static_cast<int32_t*>(a.out)[rowOff + n0] = acc(mi, 0)[v];
-                    if (r < rows && valid1) static_cast<int32_t*>(a.out)[rowOff + n0 + 32] = acc(mi, 1)[v];
+                if constexpr (kEpi == Epilogue::kInt32) {
+                    int32_t* const out = static_cast<int32_t*>(a.out) + rowOff;
+                    if (vectorStores) {
+                        *reinterpret_cast<v4i*>(out + col[0]) = v4i{acc[m][0][v], acc[m][1][v], acc[m][2][v], acc[m][3][v]};
+                    } else {
+#pragma unroll
+                        for (int n = 0; n < 4; ++n) {
+                            if (valid[n]) out[col[n]] = acc[m][n][v];
+                        }
+                    }
                     continue;
                 }
-                float y0 = __fmul_rn(static_cast<float>(acc(mi, 0)[v]), sc0);
-                float y1 = __fmul_rn(static_cast<float>(acc(mi, 1)[v]), sc1);
-                if (hasRowScale) {
-                    const float rs = ldsRowScale[r < rows ? r : 0];
-                    y0 = __fmul_rn(y0, rs);
-                    y1 = __fmul_rn(y1, rs);
+                const float rs = hasRowScale ? ldsRowScale[r] : 1.0f;
+                float y[4];
+#pragma unroll
+                for (int n = 0; n < 4; ++n) {
+                    y[n] = __fmul_rn(static_cast<float>(acc[m][n][v]), sc[n]);
+                    if (hasRowScale) y[n] = __fmul_rn(y[n], rs);
                 }
                 if (a.outDtype == 0) {
                     if (a.combineIndex != nullptr) {
-                        if (r >= rows) continue;
                         const int64_t src = rowBase + r;
                         const int64_t dst = a.combineIndexIsInt64 ? static_cast<const int64_t*>(a.combineIndex)[src]
                                                                   : static_cast<const int32_t*>(a.combineIndex)[src];
                         if (dst < 0 || dst >= a.combineRows) continue;
                         if (a.bias != nullptr) {
                             const float wgt = a.combineWeight != nullptr ? a.combineWeight[src] : 1.0f;
-                            y0 = __fadd_rn(y0, __fmul_rn(wgt, bias0));
-                            y1 = __fadd_rn(y1, __fmul_rn(wgt, bias1));
+#pragma unroll
+                            for (int n = 0; n < 4; ++n) y[n] = __fadd_rn(y[n], __fmul_rn(wgt, bias[n]));
                         }
                         float* const dstRow = static_cast<float*>(a.out) + dst * a.N;
-                        if (valid0) unsafeAtomicAdd(dstRow + n0, y0);
-                        if (valid1) unsafeAtomicAdd(dstRow + n0 + 32, y1);
+#pragma unroll
+                        for (int n = 0; n < 4; ++n) {
+                            if (valid[n]) unsafeAtomicAdd(dstRow + col[n], y[n]);
+                        }
                         continue;
                     }
-                    if (r < rows && valid0) static_cast<float*>(a.out)[rowOff + n0] = y0;
-                    if (r < rows && valid1) static_cast<float*>(a.out)[rowOff + n0 + 32] = y1;
+                    float* const out = static_cast<float*>(a.out) + rowOff;
+                    if (vectorStores) {
+                        *reinterpret_cast<Float4*>(out + col[0]) = Float4{y[0], y[1], y[2], y[3]};
+                    } else {
+#pragma unroll
+                        for (int n = 0; n < 4; ++n) {
+                            if (valid[n]) out[col[n]] = y[n];
+                        }
+                    }
                     continue;
                 }
-                // both values rounded to nearest even and packed (low half = block 0)
-                uint32_t pk;
-                if (a.outDtype == 27) {
-                    const Float2 f = {y0, y1};
-                    pk = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, Bf16x2));  // v_cvt_pk_bf16_f32
-                } else {
-                    pk = static_cast<uint32_t>(HalfBitsOfRounded(y0)) | (static_cast<uint32_t>(HalfBitsOfRounded(y1)) << 16);
-                }
-                if (pairStores) {
-                    // quad_perm [1,0,3,2]: exchange with the lane whose index differs in bit 0, then keep
-                    // (own block-0 value, neighbour's block-0 value) on even lanes and
-                    // (neighbour's block-1 value, own block-1 value) on odd lanes
-                    const uint32_t got = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(pk), 0xB1, 0xF, 0xF, true));
-                    const uint32_t word = __builtin_amdgcn_perm(got, pk, oddLane ? 0x03020706u : 0x05040100u);
-                    const int32_t col = oddLane ? n0 + 31 : n0;  // odd lane l: block 1, columns 32 + (l - 1), 32 + l
-                    if (r < rows) *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(a.out) + rowOff + col) = word;
-                } else {
-                    if (r < rows && valid0) static_cast<uint16_t*>(a.out)[rowOff + n0] = static_cast<uint16_t>(pk & 0xffffu);
-                    if (r < rows && valid1) static_cast<uint16_t*>(a.out)[rowOff + n0 + 32] = static_cast<uint16_t>(pk >> 16);
+                uint16_t* const out = static_cast<uint16_t*>(a.out) + rowOff;
+#pragma unroll
+                for (int n = 0; n < 4; ++n) {
+                    const uint32_t bits = a.outDtype == 27 ? PackHalves<true>(y[n], 0.0f) : PackHalves<false>(y[n], 0.0f);
+                    if (valid[n]) out[col[n]] = static_cast<uint16_t>(bits & 0xffffu);
                 }
             }
         }
     } else {
-        const int32_t j = t.colBase + 32 * waveN + l32;  // column of S
-        const bool jValid = j < a.halfN;
-        float scA = 0.0f, scB = 0.0f;
-        if (jValid) {
-            scA = LoadScale(a.scale, static_cast<int64_t>(group) * a.N + j, a.scaleDtype);
-            scB = LoadScale(a.scale, static_cast<int64_t>(group) * a.N + a.halfN + j, a.scaleDtype);
+        float scA[2], scB[2];
+        int32_t col[2];  // columns of S
+        bool valid[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            col[j] = t.colBase + ColumnInTile<kOrder, true>(waveN, j, l16, true);
+            valid[j] = col[j] < a.halfN;
+            scA[j] = scB[j] = 0.0f;
+            if (valid[j]) {
+                scA[j] = LoadScale(a.scale, static_cast<int64_t>(group) * a.N + col[j], a.scaleDtype);
+                scB[j] = LoadScale(a.scale, static_cast<int64_t>(group) * a.N + a.halfN + col[j], a.scaleDtype);
+            }
         }
         afterScaleLoads();
-        const bool wholeColumns = t.colBase + 32 * waveN + 32 <= a.halfN;  // wave-uniform
+        // swish(ca) * cb with the hardware exp2 / reciprocal: a few ulp from the correctly rounded value, far inside the
+        // +-1 LSB the int8 requantisation is held to
+        auto activated = [&](int m, int j, int v, float xs) __attribute__((always_inline)) {
+            const float ca = __fmul_rn(__fmul_rn(static_cast<float>(acc[m][j][v]), xs), scA[j]);
+            const float cb = __fmul_rn(__fmul_rn(static_cast<float>(acc[m][2 + j][v]), xs), scB[j]);
+            return __fmul_rn(__fmul_rn(ca, __builtin_amdgcn_rcpf(__fadd_rn(1.0f, __expf(-ca)))), cb);
+        };
+        // wave-uniform: every column of the wave exists, and S rows start on a lane's pair
+        const bool whole = t.colBase + 32 * waveN + 32 <= a.halfN && (kOrder != kOrderLane || (a.halfN & 1) == 0);
+        if (whole) {
+            float* const sTile = a.sOut + static_cast<int64_t>(rowBase) * a.halfN;
+            const int32_t laneOff = 4 * quad * a.halfN + col[0];
+            auto block = [&](int m, auto fullTag) __attribute__((always_inline)) {
+                constexpr bool kFull = decltype(fullTag)::value;
+                const int rTop = Blocks::RowOf(m, waveM);
+                const float4 xs4 = *reinterpret_cast<const float4*>(ldsRowScale + rTop + 4 * quad);
+                const float xs[4] = {xs4.x, xs4.y, xs4.z, xs4.w};
+                float top[4];
 #pragma unroll
-        for (int mi = 0; mi < kSubM; ++mi) {
-            if (mi >= mySub) continue;  // wave-uniform
-            const int rTop = waveRow0 + 32 * mi;
-            if (wholeColumns && rTop < rows) {
-                // Fast form for whole column blocks: row scales four at a time, no column checks, and the 16 row
-                // maxima of the MFMA tile reduced across the 32 lanes by a halving butterfly (16 exchanges, not 80).
-                float* const sTile = a.sOut + static_cast<int64_t>(rowBase + rTop) * a.halfN;
-                const int32_t laneOff = 4 * lhi * a.halfN + j;
-                float m[16];
-                // Row checks per group of eight rows, wave-uniformly, as in the 16-bit stores above.
-                auto rowGroup = [&](int q, auto fullTag) __attribute__((always_inline)) {
-                    constexpr bool kFull = decltype(fullTag)::value;
-                    const float4 xs4 = *reinterpret_cast<const float4*>(ldsRowScale + rTop + 8 * q + 4 * lhi);
-                    const float xsv[4] = {xs4.x, xs4.y, xs4.z, xs4.w};
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int v = 4 * q + i;
-                        const float ca = __fmul_rn(__fmul_rn(static_cast<float>(acc(mi, 0)[v]), xsv[i]), scA);
-                        const float cb = __fmul_rn(__fmul_rn(static_cast<float>(acc(mi, 1)[v]), xsv[i]), scB);
-                        float sv = __fmul_rn(__fmul_rn(ca, __builtin_amdgcn_rcpf(__fadd_rn(1.0f, __expf(-ca)))), cb);
-                        const bool ok = kFull || rTop + 8 * q + 4 * lhi + i < rows;
-                        if (ok) __builtin_nontemporal_store(sv, &sTile[static_cast<int64_t>(8 * q + i) * a.halfN + laneOff]);
-                        m[v] = ok ? fabsf(sv) : 0.0f;
+                for (int v = 0; v < 4; ++v) {
+                    const float s0 = activated(m, 0, v, xs[v]), s1 = activated(m, 1, v, xs[v]);
+                    float* const sRow = sTile + static_cast<int64_t>(rTop + v) * a.halfN;
+                    const bool ok = kFull || rTop + 4 * quad + v < rows;
+                    if constexpr (kOrder == kOrderLane) {
+                        if (ok) __builtin_nontemporal_store(Float2{s0, s1}, reinterpret_cast<Float2*>(sRow + laneOff));
+                    } else {
+                        if (ok) __builtin_nontemporal_store(s0, sRow + laneOff);
+                        if (ok) __builtin_nontemporal_store(s1, sRow + laneOff + 16);
                     }
-                };
-                if (rTop + 32 <= rows) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) rowGroup(q, std::true_type{});
-                } else {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        if (rTop + 8 * q >= rows) {
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) m[4 * q + i] = 0.0f;
-                        } else if (rTop + 8 * q + 8 <= rows) {
-                            rowGroup(q, std::true_type{});
-                        } else {
-                            rowGroup(q, std::false_type{});
-                        }
-                    }
+                    top[v] = ok ? fmaxf(fabsf(s0), fabsf(s1)) : 0.0f;
                 }
-                // lanes l and l ^ 16: one instruction trades the upper-row half of m[i] for the lower-row half of
-                // m[i + 8]; afterwards lanes 0..15 of each half-wave own v = i and lanes 16..31 own v = i + 8
-                typedef unsigned int Uint2 __attribute__((ext_vector_type(2)));
-                float k8[8];
+                const float m16 = FourMaxOver16(top, l16);
+                if ((l16 & 3) == 0) ldsRowMax[waveN * kRows + rTop + 4 * quad + (l16 >> 2)] = m16;
+            };
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const Uint2 sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(m[i]), __float_as_uint(m[i + 8]), false, false);
-                    k8[i] = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-                }
-                const bool b3 = (l32 & 8) != 0, b2 = (l32 & 4) != 0, b1 = (l32 & 2) != 0;
-                float k4[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {  // partner l ^ 8: lanes with bit 3 clear keep i, the others i + 4
-                    const float send = b3 ? k8[i] : k8[i + 4];
-                    k4[i] = fmaxf(b3 ? k8[i + 4] : k8[i], __shfl_xor(send, 8, 64));
-                }
-                float k2[2];
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const float send = b2 ? k4[i] : k4[i + 2];
-                    k2[i] = fmaxf(b2 ? k4[i + 2] : k4[i], __shfl_xor(send, 4, 64));
-                }
-                const float send1 = b1 ? k2[0] : k2[1];
-                float k1 = fmaxf(b1 ? k2[1] : k2[0], __shfl_xor(send1, 2, 64));
-                k1 = fmaxf(k1, __shfl_xor(k1, 1, 64));
-                // the lane pair (2p, 2p + 1) of a half-wave now holds the maximum of accumulator index v = p:
-                // bit 4 of the lane chose bit 3 of v, bit 3 -> bit 2, bit 2 -> bit 1, bit 1 -> bit 0
-                const int v = l32 >> 1;
-                if ((l32 & 1) == 0) ldsRowMax[waveN * kTileM + rTop + 8 * (v / 4) + 4 * lhi + (v % 4)] = k1;
-                continue;
+            for (int m = 0; m < Blocks::kAll; ++m) {
+                const int rTop = Blocks::RowOf(m, waveM);
+                if (rTop >= rows) continue;
+                if (rTop + 16 <= rows) block(m, std::true_type{});
+                else block(m, std::false_type{});
             }
+            return;
+        }
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int r = waveRow0 + 32 * mi + 8 * (v / 4) + 4 * lhi + (v % 4);
-                const bool valid = r < rows && jValid;
-                float s = 0.0f;
-                if (valid) {
-                    const float xs = ldsRowScale[r];
-                    const float ca = __fmul_rn(__fmul_rn(static_cast<float>(acc(mi, 0)[v]), xs), scA);
-                    const float cb = __fmul_rn(__fmul_rn(static_cast<float>(acc(mi, 1)[v]), xs), scB);
-                    // swish(ca) * cb with the hardware exp2 / reciprocal: a few ulp from the correctly rounded value,
-                    // far inside the +-1 LSB the int8 requantisation is held to
-                    s = __fmul_rn(__fmul_rn(ca, __builtin_amdgcn_rcpf(__fadd_rn(1.0f, __expf(-ca)))), cb);
-                    a.sOut[static_cast<int64_t>(rowBase + r) * a.halfN + j] = s;
+        for (int m = 0; m < Blocks::kAll; ++m) {
+            const int rTop = Blocks::RowOf(m, waveM);
+            if (rTop >= rows) continue;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int r = rTop + 4 * quad + v;
+                float top = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    if (r < rows && valid[j]) {
+                        const float s = activated(m, j, v, ldsRowScale[r]);
+                        a.sOut[static_cast<int64_t>(rowBase + r) * a.halfN + col[j]] = s;
+                        top = fmaxf(top, fabsf(s));
+                    }
                 }
-                // max |S| of this row over the wave's 32 columns, kept by the first lane of each half-wave
-                float m = fabsf(s);
-#pragma unroll
-                for (int d = 1; d < 32; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
-                if (l32 == 0) ldsRowMax[waveN * kTileM + r] = m;
+                top = MaxOver16(top);
+                if (l16 == 0) ldsRowMax[waveN * kRows + r] = top;
             }
         }
     }
 }
 
-// The part of the kSwiglu epilogue that follows the waves' own work: folds the four column positions' partial row maxima
+// The part of the kSwiglu epilogue that follows the waves' own work: folds the four wave columns' partial row maxima
 // into one per (n-tile, row).  Contains a workgroup barrier: every wave must call it (the workgroup has at least
-// kTileM threads).
-template <int kTileM>
+// kRows threads).
+template <int kRows>
 __device__ __forceinline__ void TileEpilogueFoldMax(const KernelArgs& a, const TileInfo& t, int tid, const float* ldsRowMax) {
     __syncthreads();
     // one partial maximum per (n-tile, row): no atomics and nothing to pre-zero; the requantisation folds them
     if (tid < t.rows) {
         float m = ldsRowMax[tid];
 #pragma unroll
-        for (int w = 1; w < kWavesN; ++w) m = fmaxf(m, ldsRowMax[w * kTileM + tid]);
+        for (int w = 1; w < kWavesN; ++w) m = fmaxf(m, ldsRowMax[w * kRows + tid]);
         a.rowMax[static_cast<int64_t>(t.tileN) * a.M + t.rowBase + tid] = m;
     }
-}
-
-// Eight-wave form (one pair of column blocks per wave): the per-wave part, then the fold.
-template <int kSubM, int kTileM, Epilogue kEpi, typename Hook = NoHook>
-__device__ __forceinline__ void TileEpilogue(const KernelArgs& a, const TileInfo& t, v16i (&acc)[kSubM][2], int mySub,
-                                             int waveRow0, int waveN, int l32, int lhi, int tid,
-                                             const float* ldsRowScale, float* ldsRowMax, Hook afterScaleLoads = NoHook{}) {
-    TileEpilogueWave<kSubM, 2, 0, kTileM, kEpi>(a, t, acc, mySub, waveRow0, waveN, l32, lhi, ldsRowScale, ldsRowMax, afterScaleLoads);
-    if (kEpi == Epilogue::kSwiglu) TileEpilogueFoldMax<kTileM>(a, t, tid, ldsRowMax);
 }
 
 // Calls f(std::integral_constant<int, n>) for n = count clamped into 0..kMax.
@@ -563,74 +601,69 @@ __device__ __forceinline__ void ForCount(int count, F& f) {
 }
 
 // ---------------------------------------------------------------------------------------------- fast path: LDS-DMA ring
-// kStep = k-bytes per ring stage: 128 streams weights in whole 128-byte lines (best HBM efficiency).
-// The tile's rows are split over one or two wave rows: wave row 0 owns kSub0 MFMA tiles (32 rows each), wave row 1 the
-// next kSub1 (kSub1 <= kSub0; kSub1 == 0 means four waves only).
+// k-bytes per ring stage: 128 streams weights in whole lines (best HBM efficiency).
+constexpr int kStep = 128;
+
+// A stage is kRows activation rows and 256 weight channels of 128 k-bytes each; the two kinds have rings of their own depth in
+// LDS.  A k-step multiplies a stage in four products, two halves of the wave's rows times two slices of 64 k, and the fragments
+// of a product are read from LDS while the one before it is multiplied (fragment double buffers).  The buffers that a step reads
+// are refilled in two goes, each behind a barrier:
+//     product    first half x 0    first half x 1     second half x 0    second half x 1
+//     reads      weights, 1        second half, 0     second half, 1     of the next step: weights and first half, 0
+//                first half, 1
+//     requests                                        even slots         odd slots
+// The barrier in the middle says that every wave has read the weights and the first half of the rows, the one in front of the
+// last product that it has read the second half, and that the next stage has landed.  The requests go out one at a time between
+// the matrix instructions.
+// What bounds it: with few experts of thousands of rows the matrix unit's power; with about a hundred rows each, the HBM and the
+// latency under it.  Gate/up and down in us, as 32x32x32 instructions on whole stages refilled in one burst behind a step's
+// barrier, and now: 16384 tokens top-2 of 8 experts, hidden 4096, intermediate 14336: 3922 / 1761 -> 3367 / 1515 (2.29 and 2.54
+// POP/s); 4096 top-8 of 256, 7168, 2048: 1526 / 876 -> 1461 / 836; 8192 of these at popularity rank^-1.2: 2278 / 1305 -> 2031 /
+// 1152; 2047 top-8 of 128, 4096, 1536: 360 / 230 -> 352 / 223.
+// (With the first barrier a quarter of a step earlier, so that every part had as long to land, its wait for the fragments just
+// requested showed: 16384 tokens, 8 experts, hidden 4096, intermediate 14336, 3716 against 3418 us gate/up and 1685 / 1578 down.
+// Eight barriers a step, the two wave rows half a phase apart: 3400 / 1480 there, but 254 against 219 us where a tile has 128 rows
+// and twelve steps.)
 //
-// A stage is kTileM activation rows and kTileN weight channels of kStep k-bytes each.  Every wave fetches, per stage,
-// instructions wave, wave + kWaves, ... of the stage's list (activation part first, then weight part).
+// Wave row 0 requests the weights, wave row 1 the activation rows.  A wave's loads return in issue order, so a wave that had
+// to wait for activation rows, which come out of L2 and need one or two stages in flight, would wait for all weights
+// requested before them, which come out of HBM and want to be three stages ahead.
 //
-// Common depth (every height but 192 rows): a ring of whole stages.
-//
-// Staggered depths (192 rows).  Whole stages fit twice there, but three weight stages and two activation stages fit as
-// well -- and the depth matters for the weights, which come out of HBM, not for the activation rows, which the n-tiles
-// of an expert re-read from L2.  So the two parts live in rings of their own depth (the activation ring first), and
-// each has its own issue cursor: at k-step s a wave issues its activation share of step s + 2 and then its weight share
-// of step s + 3.  A wave's loads return in issue order; with the activation share going out first, "at most one weight
-// share outstanding" certifies both the activation stage issued one step ago and the weight stage issued two steps ago.
-//
-// kWn = waves side by side along the channels: four (a wave owns 64 channels, two MFMA column blocks) or two (128
-// channels, four column blocks: with two wave rows that is four waves per workgroup, one per SIMD, each holding a
-// 128 x 128 block of the tile -- a third fewer fragment bytes out of LDS per MFMA, the accumulators in AccVGPRs).
-// Only kWn = 4 is launched.  The four-wave form of the 256-row tile gives the same bits and measured 16 % slower on the
-// matrix-bound shape (4.14 against 3.58 ms): with one wave per SIMD nothing runs under a wave's sixteen operand
-// requests per k-step or under its epilogue, and what it saves in LDS reads is not what bounds the step.
-template <int kSub0, int kSub1, int kStep, int kWn = kWavesN>
+// One DMA instruction moves 64 lanes x 16 bytes = 8 rows of 128 k-bytes.  Slot q of wave column w is instruction w + 4 q of
+// its kind, i.e. 32 rows per slot: even slots of the activation rows are the first half of the wave rows' blocks.
+template <int kRows>
 struct StreamCfg {
-    static_assert(kSub1 <= kSub0, "wave row 0 is the taller one");
-    static_assert(kWn == 4 || kWn == 2, "a wave owns two or four column blocks");
-    static constexpr int kWavesM = kSub1 > 0 ? 2 : 1;
-    static constexpr int kWaves = kWn * kWavesM;
-    static constexpr int kNi = kTileN / 32 / kWn;  // MFMA column blocks per wave
-    static constexpr int kThreads = 64 * kWaves;
-    static constexpr int kTileM = 32 * (kSub0 + kSub1);
-    static constexpr int kStageBytesA = kTileM * kStep;
+    using Blocks = RowBlocks<kRows>;
+    static constexpr int kStageBytesA = kRows * kStep;
     static constexpr int kStageBytesB = kTileN * kStep;
-    static constexpr int kQueueLdsInts = 16;  // the workgroup's tile sequence (four {list, tile} pairs) and its draw state
-    static constexpr int kScratchBytes = (1 + kWavesN) * kTileM * 4 + kQueueLdsInts * 4;
-    static constexpr bool kStaggered = kTileM == 192;
-    static constexpr int kFitWhole = (kLdsBudget - kScratchBytes) / (kStageBytesA + kStageBytesB);
-    static constexpr int kStagesB = kStaggered ? (kLdsBudget - kScratchBytes - 2 * kStageBytesA) / kStageBytesB
-                                               : (kFitWhole > 8 ? 8 : kFitWhole);
-    static constexpr int kStagesA = kStaggered ? 2 : kStagesB;
-    static constexpr int kLdsBytes = kStagesA * kStageBytesA + kStagesB * kStageBytesB + kScratchBytes;
-    // one DMA instruction moves 64 lanes x 16 bytes = kRowsPerInstr tile rows of kStep k-bytes
-    static constexpr int kChunksPerRow = kStep / kChunk;
-    static constexpr int kRowsPerInstr = 64 / kChunksPerRow;
-    static constexpr int kInstrA = kTileM / kRowsPerInstr;
-    static constexpr int kInstrB = kTileN / kRowsPerInstr;
-    static constexpr int kInstr = kInstrA + kInstrB;
-    static_assert(kTileM % kRowsPerInstr == 0, "tile rows must fill whole DMA instructions");
-    static_assert(kThreads >= kTileM, "one thread per tile row stages the row scales and folds the row maxima");
-    // Every wave issues exactly kMaxPerWave DMA instructions per stage: slots past the last instruction repeat it (same
-    // bytes to the same place), which keeps the issue code free of branches and the vmcnt arithmetic uniform.
-    static constexpr int kMaxPerWave = (kInstr + kWaves - 1) / kWaves;
-    // staggered depths: the first kSlotsA slots of every wave are activation instructions, the others weight instructions
-    static constexpr int kSlotsA = kInstrA / kWaves;
-    static constexpr int kSlotsB = kMaxPerWave - kSlotsA;
-    static_assert(!kStaggered || (kInstrA % kWaves == 0 && kInstrB % kWaves == 0), "the same split of slots in every wave");
-    static_assert(kStagesA >= 2 && kStagesB >= kStagesA, "each ring needs at least two stages");
-    static_assert(kStagesB * kMaxPerWave <= 63, "vmcnt is a 6-bit counter");
+    static constexpr int kHalfBytesB = kStageBytesB / 2;
+    static constexpr int kQueueLdsInts = 36;  // the workgroup's next eight tiles and its draw state
+    static constexpr int kScratchBytes = (1 + kWavesN) * kRows * 4 + kQueueLdsInts * 4;
+    static constexpr int kRingBytes = kLdsBudget - kScratchBytes;
+    // as many weight stages as leave room for two of activation rows, then as many of those as fit
+    static constexpr int kFitB = (kRingBytes - 2 * kStageBytesA) / kStageBytesB;
+    static constexpr int kStagesB = kFitB > 4 ? 4 : kFitB;
+    static constexpr int kFitA = (kRingBytes - kStagesB * kStageBytesB) / kStageBytesA;
+    static constexpr int kStagesA = kFitA > kStagesB ? kStagesB : kFitA;
+    static constexpr int kFirstB = kStagesA * kStageBytesA;  // the ring of weight stages, behind that of the activation rows
+    static constexpr int kLdsBytes = kFirstB + kStagesB * kStageBytesB + kScratchBytes;
+    static constexpr int kSlotsA = kRows / 32, kSlotsB = kTileN / 32;  // a wave's DMA instructions per stage
+    static_assert(kSlotsA <= kSlotsB && kStagesA >= 2 && kStagesB >= 2 && kThreads >= kRows, "");
+    // a wave's DMA instructions younger than the next stage's last one, in front of the last product of a step
+    static constexpr int kYoungerA = (kStagesA - 2) * kSlotsA + (kSlotsA + 1) / 2;
+    static constexpr int kYoungerB = (kStagesB - 2) * kSlotsB + (kSlotsB + 1) / 2;
+    static_assert(kStagesB * kSlotsB <= 63, "vmcnt is a 6-bit counter");
 };
 
-// Byte offset of 16-byte chunk `chunk` of row `row` in a stage whose rows are kStep bytes.  The LDS serves 16 lanes per
+// Byte offset of 16-byte chunk `chunk` of row `row` in a stage whose rows are 128 bytes.  The LDS serves 16 lanes per
 // clock out of 64 banks (256 bytes): the chunk index is XOR-ed with row bits such that 16 consecutive rows reading the
 // same logical chunk land in 16 different 16-byte bank groups.
-template <int kStep>
-__device__ __forceinline__ int LdsOffset(int row, int chunk) {
-    if (kStep == 64) return row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4);
-    return row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4);
-}
+__device__ __forceinline__ int LdsOffset(int row, int chunk) { return row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4); }
+
+// What the 16-byte chunk index of k-row k of a row-major weight half (rows of 128 channel bytes) is XOR-ed with: the 32
+// lanes that the LDS serves together read one chunk of eight consecutive k-rows and of those sixteen further on, and these
+// sixteen pieces land in different bank groups.
+__device__ __forceinline__ int RowMajorSwizzle(int k) { return ((k >> 1) & 3) | (((k >> 4) & 1) << 2); }
 
 // A wave-uniform pointer, forced into scalar registers.
 __device__ __forceinline__ const char* UniformPtr(const char* p) {
@@ -645,6 +678,20 @@ __device__ __forceinline__ uint32_t LdsAddress(const char* p) {
     typedef __attribute__((address_space(3))) const char* LdsPtr;
     return static_cast<uint32_t>(
         __builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<uint32_t>(reinterpret_cast<size_t>((LdsPtr)p)))));
+}
+
+// 16 bytes of LDS at a 32-bit address and a constant (in the instruction's offset field).
+__device__ __forceinline__ v4i LdsRead16(uint32_t addr, int offset) {
+    typedef __attribute__((address_space(3))) const char* LdsPtr;
+    return *(LdsV4iPtr)(reinterpret_cast<LdsPtr>(addr) + offset);
+}
+
+// Sixteen consecutive k of one channel, from two transposing loads of eight k-rows each.
+__device__ __forceinline__ v4i LdsReadTransposed(uint32_t addr, int offset, int eightK) {
+    typedef __attribute__((address_space(3))) char* LdsPtr;
+    const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((LdsV2iPtr)(reinterpret_cast<LdsPtr>(addr) + offset));
+    const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((LdsV2iPtr)(reinterpret_cast<LdsPtr>(addr) + offset + eightK));
+    return v4i{lo[0], lo[1], hi[0], hi[1]};
 }
 
 // 16 bytes per lane from (uniform base + 32-bit lane offset) straight into LDS at ldsAddr + lane * 16 (ldsAddr is the
@@ -675,9 +722,32 @@ __device__ __forceinline__ int Opaque(int v) {
     return v;
 }
 
+// The kernel's arguments (its first parameter), read again from memory.  What only the epilogue wants of them would otherwise stay
+// in scalar registers across the k loop, and those of the tallest tiles, once spilled, cost vector registers that are not there.
+__device__ __forceinline__ KernelArgs ReloadArgs() {
+    auto p = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    KernelArgs a;
+    __builtin_memcpy(&a, (const void*)p, sizeof(a));
+    return a;
+}
+
 template <int kCount>
 __device__ __forceinline__ void WaitVmcnt() {  // s_waitcnt vmcnt(kCount), leaving expcnt / lgkmcnt untouched
     __builtin_amdgcn_s_waitcnt(0x0f70 | (kCount & 15) | ((kCount >> 4) << 14));
+}
+
+// This wave's LDS reads and writes have been carried out (s_waitcnt lgkmcnt(0) alone).
+__device__ __forceinline__ void WaitLds() { __builtin_amdgcn_s_waitcnt(0xc07f); }
+
+// The workgroup's barrier, and nothing crosses it in the compiler's order.  Unlike __syncthreads() it waits for no memory
+// request: what has to have landed in front of it is waited for by count.
+__device__ __forceinline__ void PhaseBarrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
 }
 
 // Persistent: the grid is one workgroup per CU (a multiple of 8); workgroup b serves XCD b % 8 and walks that XCD's
@@ -687,14 +757,14 @@ __device__ __forceinline__ void WaitVmcnt() {  // s_waitcnt vmcnt(kCount), leavi
 // K x 32 bytes, so a stage's weight part is eight 4 KB pieces that land in LDS as [block][k][32 channels]; the MFMA
 // operand (16 consecutive k of one channel per lane) is read back with the transposing LDS load ds_read_b64_tr_b8:
 // per 16 lanes, lanes 2r and 2r + 1 supply the two 8-byte halves of row r (r = 0..7) and lane i receives column i,
-// i.e. with rows = 8 consecutive k and columns = 16 channels each lane gets 8 consecutive k of its channel.
+// i.e. with rows = 8 consecutive k and columns = 16 channels each lane gets 8 consecutive k of its channel.  (The two
+// sixteen-channel halves of a k-row lie swapped where bit 4 of k is set: the 32 lanes served together read k-rows sixteen
+// apart.)
 //
 // kNMajor: the weights are row-major [K, N] per expert (N contiguous), the reference's plain ND layout of the grouped
-// matmul.  A stage's weight part is then 128 k-rows of the tile's 256 channel bytes (one 256-byte run per k-row, two of
-// 128 bytes for the gate and up halves of a SwiGLU tile); it lies in LDS as [k][256] with the 16-byte chunk index of row
-// k XOR-ed by 2 * (k & 7), and the operands come out through the same transposing load as for the blocked layout: the
-// 32 lanes the LDS serves together read one pair of neighbouring chunks from each of 8 consecutive k-rows, and the
-// swizzle puts those 8 pairs into 8 different bank groups (a row of 256 bytes spans all 64 banks once).
+// matmul.  A stage's weight half is then 128 k-rows of 128 channel bytes (kSwiglu: of the gate or of the up half); it lies
+// in LDS as [k][128] with the chunks of row k swizzled (RowMajorSwizzle), and the operands come out through the same
+// transposing load as for the blocked layout.
 //
 // kRun: which runs of the m-tile table the body serves.  kBothRuns: all of it (pulled or in fixed shares).  kBigRun /
 // kSmallRun: that run only, pulled, until its counters are used up on every XCD -- the form in which MixedGemmKernel
@@ -702,47 +772,33 @@ __device__ __forceinline__ void WaitVmcnt() {  // s_waitcnt vmcnt(kCount), leavi
 //
 // kTail: K is a multiple of 16 and at least one k-step, but no multiple of a k-step.  The last k-step then starts kStep
 // bytes before the end of K instead of behind the step before it: every DMA stays inside its row and is as wide as any
-// other, and the k that the step before has already covered are multiplied by zero (the activation fragments of that one
-// step are masked; it is a copy of the k-step's code behind the loop, so the loop itself is that of the other K).
+// other, and the k that the step before has already covered are multiplied by zero (the weight fragments of that one
+// step are masked).
 // Before, such K went through the byte-wise kernel: a 301-token pass over 32 experts with hidden 2880 and intermediate
 // 1440 took 1.396 ms and takes 0.162 ms (its 398 MB of weights alone are 0.06 ms at the HBM's streaming rate).
 constexpr int kBigRun = 0, kSmallRun = 1, kBothRuns = 2;
-template <int kSub0, int kSub1, int kStep, Epilogue kEpi, bool kNz, bool kNMajor, int kWn, int kRun, bool kTail>
+template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, int kRun, bool kTail>
 __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_t* __restrict__ sched, char* const lds,
                                                uint64_t& spanTiles) {
-    static_assert(!(kNz || kNMajor) || kStep == 128, "the blocked and row-major weight layouts are built for 128-byte k-steps");
     static_assert(!(kNz && kNMajor), "one weight layout at a time");
-    using Cfg = StreamCfg<kSub0, kSub1, kStep, kWn>;
-    constexpr int kSubM = kSub0;  // accumulator tiles per wave (wave row 1 uses the first kSub1 of them)
-    constexpr int kNi = Cfg::kNi;
-    constexpr int kTileM = Cfg::kTileM;
-    constexpr int kStagesA = Cfg::kStagesA, kStagesB = Cfg::kStagesB;
-    constexpr int kStageBytesA = Cfg::kStageBytesA, kStageBytesB = Cfg::kStageBytesB;
-    // LDS layout.  Common depth: stage after stage, each its activation part followed by its weight part.  Staggered
-    // depths: the ring of activation stages, behind it the ring of weight stages.
-    constexpr bool kStaggered = Cfg::kStaggered;
-    constexpr int kStrideA = kStaggered ? kStageBytesA : kStageBytesA + kStageBytesB;  // from one activation stage to the next
-    constexpr int kStrideB = kStaggered ? kStageBytesB : kStageBytesA + kStageBytesB;
-    constexpr int kFirstB = kStaggered ? kStagesA * kStageBytesA : kStageBytesA;       // weight part of stage 0
+    using Cfg = StreamCfg<kRows>;
+    using Blocks = RowBlocks<kRows>;
     constexpr bool kSwiglu = kEpi == Epilogue::kSwiglu;
-    float* const ldsRowScale = reinterpret_cast<float*>(lds + kStagesA * kStageBytesA + kStagesB * kStageBytesB);  // [kTileM]
-    float* const ldsRowMax = ldsRowScale + kTileM;                                      // [kWavesN][kTileM]
+    float* const ldsRowScale = reinterpret_cast<float*>(lds + Cfg::kFirstB + Cfg::kStagesB * Cfg::kStageBytesB);  // [kRows]
+    float* const ldsRowMax = ldsRowScale + kRows;                                            // [kWavesN][kRows]
 
     const int tid = threadIdx.x;
-    const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int waveN = wave % kWn;
-    const int waveM = wave / kWn;
-    const int l32 = lane & 31;
-    const int lhi = lane >> 5;
+    const int waveN = wave % kWavesN;
+    const int waveM = wave / kWavesN;
 
     // ---- this workgroup's sequence of tiles ----
-    // Workgroup b serves XCD b % 8 as its slot b / 8.  With a.pullTiles the sequence comes out of the tile counters (see
-    // QueueShare): thread 0 draws, the result reaches the other waves through a four-entry ring in LDS, and tile n + 2
-    // is drawn while tile n's epilogue runs (the draw goes out at its head, the answer is looked at behind it),
-    // because the issue side already reads tile n + 1's operands during tile n.  Otherwise the two runs of
-    // the m-tile table are one list cut into eight fixed shares, which the workgroups of an XCD walk with stride
-    // gridDim / 8.
+    // Workgroup b serves XCD b % 8 as its slot b / 8.  Thread 0 finds the tiles and leaves them, decoded, in an eight-entry ring
+    // in LDS.  With a.pullTiles they come out of the tile counters (see QueueShare), and tile n + 2 is drawn while tile n's
+    // epilogue runs (the draw goes out at its head, the answer is looked at behind it), because the issue side already reads
+    // tile n + 1's operands during tile n.  Otherwise the two runs of the m-tile table are one list cut into eight fixed
+    // shares, which the workgroups of an XCD walk with stride gridDim / 8, and the ring holds six tiles (tiles of one k-step
+    // have the issue side five tiles ahead).
     const int32_t* const queueHdr = sched;
     const int32_t countBig = queueHdr[0], countSmall = queueHdr[1];  // m-tiles per list
     const int32_t bandBig = queueHdr[4], bandSmall = queueHdr[5];
@@ -752,12 +808,13 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     const int32_t slot = blockIdx.x / kXcds;
     constexpr bool kOneRun = kRun != kBothRuns;
     const bool pull = kOneRun || a.pullTiles != 0;
-    const int64_t bigTiles = static_cast<int64_t>(countBig) * a.tilesN;
-    const int64_t totalTiles = bigTiles + static_cast<int64_t>(countSmall) * a.tilesN;
-    const int64_t perXcd = (totalTiles + kXcds - 1) / kXcds;
-    const int64_t xcdFirst = static_cast<int64_t>(xcd) * perXcd;
-    int32_t* const ldsSeq = reinterpret_cast<int32_t*>(ldsRowMax + kWavesN * kTileM);
-    constexpr int kSeqUsedUp = 8, kSeqDrawCounter = 9;  // thread 0's draw state, behind the ring
+    const int32_t bigTiles = countBig * a.tilesN;
+    const int32_t totalTiles = bigTiles + countSmall * a.tilesN;
+    const int32_t perXcd = (totalTiles + kXcds - 1) / kXcds;
+    const int32_t xcdFirst = xcd * perXcd;
+    int32_t* const ldsSeq = reinterpret_cast<int32_t*>(ldsRowMax + kWavesN * kRows);
+    constexpr int kSeqUsedUp = 32, kSeqDrawCounter = 33;  // thread 0's draw state, behind the ring
+    constexpr int kTilesAhead = 6;
     // Which list this workgroup draws from first: the small m-tiles get the share of each XCD's workgroups that their
     // cost is of the whole, so that both lists run dry at about the same time; until then a part of the machine
     // streams weights for a handful of rows each while the rest multiplies.
@@ -769,413 +826,333 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         if (countBig == 0) forSmall = slots;
         prefer = kOneRun ? kRun : (slot < forSmall ? 1 : 0);
     }
-    auto listTile = [&](int32_t list, int64_t logical) __attribute__((always_inline)) {
-        return DecodeListTile<kTileM, kSwiglu>(a, mTileTable, list ? countBig : 0, list ? countSmall : countBig,
-                                               list ? bandSmall : bandBig, logical);
+    // thread 0: tile `logical` of a run (list < 0: none) as this workgroup's n-th
+    auto leaveTile = [&](int32_t n, int32_t list, int32_t logical) __attribute__((always_inline)) {
+        int4 e = make_int4(0, 0, 0, 0);
+        if (list >= 0) {
+            const TileInfo t = DecodeListTile<kSwiglu>(a, mTileTable, list ? countBig : 0, list ? countSmall : countBig,
+                                                       list ? bandSmall : bandBig, logical);
+            e = make_int4(t.group, t.rowBase, t.rows, t.tileN);
+        }
+        *reinterpret_cast<int4*>(ldsSeq + 4 * (n & 7)) = e;
     };
-    // the n-th tile of this workgroup (n at most two ahead of the tile being computed)
+    auto leaveShareTile = [&](int32_t n) __attribute__((always_inline)) {
+        const int32_t local = slot + n * slots;
+        const int32_t logical = xcdFirst + local;
+        const bool none = local >= perXcd || logical >= totalTiles;
+        leaveTile(n, none ? -1 : logical < bigTiles ? 0 : 1, logical < bigTiles ? logical : logical - bigTiles);
+    };
+    // the n-th tile of this workgroup, out of the ring
     auto tileAt = [&](int32_t n) __attribute__((always_inline)) -> TileInfo {
-        if (pull) {
-            const int32_t list = __builtin_amdgcn_readfirstlane(ldsSeq[2 * (n & 3)]);
-            const int32_t logical = __builtin_amdgcn_readfirstlane(ldsSeq[2 * (n & 3) + 1]);
-            if (list < 0) return TileInfo{};
-            return listTile(list, logical);
-        }
-        const int64_t local = slot + static_cast<int64_t>(n) * slots;
-        const int64_t logical = xcdFirst + local;
-        if (local >= perXcd || logical >= totalTiles) return TileInfo{};
-        return logical < bigTiles ? listTile(0, logical) : listTile(1, logical - bigTiles);
+        const int4 e = *reinterpret_cast<const int4*>(ldsSeq + 4 * (n & 7));
+        TileInfo t;
+        t.group = __builtin_amdgcn_readfirstlane(e.x);
+        t.rowBase = __builtin_amdgcn_readfirstlane(e.y);
+        t.rows = __builtin_amdgcn_readfirstlane(e.z);
+        t.tileN = __builtin_amdgcn_readfirstlane(e.w);
+        t.valid = t.rows > 0;
+        t.colBase = kSwiglu ? t.tileN * (kTileN / 2) : t.tileN * kTileN;
+        return t;
     };
-    if (pull) {
-        if (tid == 0) {
+    if (tid == 0) {
+        if (pull) {
+            // With no more tiles than workgroups everybody's first draw finds all of them; a second tile drawn along with it
+            // would be missing where another workgroup is idle (128 tiles of K 14336: 200 us, or 400 where one had two).
+            const bool oneRound = (kRun == kBigRun ? bigTiles : kRun == kSmallRun ? totalTiles - bigTiles : totalTiles) <= static_cast<int32_t>(gridDim.x);
             // the first two tiles: both draws go out together
-            uint32_t usedUp = 0;
-            const int c = QueueFirstOpen(usedUp, xcd, prefer, kOneRun);
-            const int32_t v0 = QueueTake(a.queueCounters, c);
-            const int32_t v1 = QueueTake(a.queueCounters, c);
-            QueueDraw d = QueueResolve(bigTiles, totalTiles - bigTiles, a.queueCounters, xcd, prefer, usedUp, c, v0, kOneRun);
-            ldsSeq[0] = d.list;
-            ldsSeq[1] = d.logical;
-            if (d.list >= 0) d = QueueResolve(bigTiles, totalTiles - bigTiles, a.queueCounters, xcd, prefer, d.usedUp, c, v1, kOneRun);
-            ldsSeq[2] = d.list;
-            ldsSeq[3] = d.logical;
+            const int c = QueueFirstOpen(0, xcd, prefer, kOneRun);
+            int32_t v[2];
+            v[0] = QueueTake(a.queueCounters, c);
+            v[1] = oneRound ? 0 : QueueTake(a.queueCounters, c);
+            QueueDraw d{0, 0, 0};
+#pragma unroll 1
+            for (int n = 0; n < 2; ++n) {
+                if (n == 1 && oneRound) d.list = -1;
+                if (d.list >= 0) {
+                    d = QueueResolve(bigTiles, totalTiles - bigTiles, a.queueCounters, xcd, prefer, d.usedUp, c, n == 0 ? v[0] : v[1], kOneRun);
+                }
+                leaveTile(n, d.list, d.logical);
+            }
             ldsSeq[kSeqUsedUp] = static_cast<int32_t>(d.usedUp);
+        } else {
+#pragma unroll 1
+            for (int n = 0; n < kTilesAhead; ++n) leaveShareTile(n);
         }
-        __syncthreads();
     }
+    __syncthreads();
 
     int32_t curNo = 0;  // position of the tile being computed in this workgroup's sequence
     TileInfo cur = tileAt(0);
     if (!cur.valid) return;
     const int kSteps = kTail ? (a.K + kStep - 1) / kStep : a.K / kStep;
     // Small tiles are the decode shapes: a handful of rows per expert, every weight byte used once, pure streaming.
-    constexpr bool kSmallTile = kTileM <= 64;
+    constexpr bool kSmallTile = kRows <= 64;
+    // On small tiles the k-steps of a tile are walked from a start that differs between workgroups (integer
+    // accumulation does not care about the order).  When rows lie a power-of-two stride apart (K = 4096 with
+    // K-contiguous weights), the low address bits of every row of every expert depend on the k offset alone:
+    // workgroups that all sit at the same k-step all queue on the same memory channels.  Only for small tiles, where
+    // every weight byte is used once: on the large-tile shapes neighbouring workgroups share operands through L2,
+    // and walking k in step is what makes those hits.
     const int kRotate = kSmallTile && !kTail ? static_cast<int>((blockIdx.x * 7u + blockIdx.x / kXcds) % static_cast<unsigned>(kSteps)) : 0;
 
-    // ---- issue side: runs ahead of the compute side by the depth of the ring(s), across tile boundaries ----
-    // A cursor walks this workgroup's tiles k-step by k-step.  Cursor B drives the weight part -- and the activation
-    // part too where the depths are the same; with staggered depths the activation part has cursor A, one k-step behind.
-    // (Plain variables, picked by if constexpr: a cursor struct handed round by reference ends up in vector registers.)
+    // ---- issue side: runs ahead of the compute side by the depth of the ring, across tile boundaries ----
+    // The cursor walks this workgroup's tiles k-step by k-step, for the kind of operand that this wave requests.
+    const bool forWeights = waveM == 0;
     const uint32_t ldsBase = LdsAddress(lds);
-    TileInfo issTileA = cur, issTileB = cur;
-    int32_t issNoA = 0, issNoB = 0;            // position of each cursor's tile in the sequence
-    int issStepA = 0, issStepB = 0;            // k-step of the tile that goes out next
-    int issSlotA = 0, issSlotB = 0;            // ring buffer it goes into
-    bool issDrainedA = false, issDrainedB = false;  // no further tile: the issue slots re-read one hot kilobyte (see advance)
-    const char* issBaseA = nullptr;  // the tile's activation rows
-    const char* issBaseB = nullptr;  // its expert's weights
-    uint32_t laneOff[Cfg::kMaxPerWave];
-    constexpr int kPartA = 1, kPartB = 2, kBothParts = 3;
-    using PartATag = std::integral_constant<int, kPartA>;
-    using PartBTag = std::integral_constant<int, kPartB>;
-    using BothPartsTag = std::integral_constant<int, kBothParts>;
-    // instruction of slot q in the stage's list (activation part, then weight part)
-    auto slotInstr = [&](int q) __attribute__((always_inline)) { return min(wave + q * Cfg::kWaves, Cfg::kInstr - 1); };
-
-    // 256-row tiles (the matrix-bound shapes): the tile's two base pointers are moved into scalar registers once per tile,
-    // and every slot of a stage is of the same part (activation / weight) in every wave.  A DMA then costs three
-    // instructions (LDS address, m0, the load) instead of nine (a select, a 64-bit vector add and two v_readfirstlane
-    // on top): the burst of refill requests behind a step's barrier, under which the matrix pipe has little to run, is a
-    // third as long.  Same-box A/B: Mixtral prefill gate/up 3.66 -> 3.56 ms, down 1.70 -> 1.67; the 192-row tiles of
-    // the HBM-bound shape measured 1.2 % slower with it and keep the vector form.
-    constexpr bool kScalarIssue = kTileM >= 256;
-    auto scalarBase = [&](const char* p) __attribute__((always_inline)) { return kScalarIssue ? UniformPtr(p) : p; };
+    TileInfo issTile = cur;
+    int32_t issNo = 0;        // position of the cursor's tile in the sequence
+    int issStep = 0;          // k-step of the tile that goes out next
+    bool issDrained = false;  // no further tile: the issue slots re-read one hot kilobyte (see advance)
+    const uint32_t issFirst = ldsBase + (forWeights ? Cfg::kFirstB : 0) + 1024 * waveN;  // where slot 0 goes, first buffer of the ring
+    const uint32_t issStride = forWeights ? Cfg::kStageBytesB : Cfg::kStageBytesA;
+    const uint32_t issEnd = issFirst + (forWeights ? Cfg::kStagesB * Cfg::kStageBytesB : Cfg::kStagesA * Cfg::kStageBytesA);
+    uint32_t issAddr = issFirst;
+    const char* issBase = nullptr;  // the tile's activation rows, or its expert's weights
+    uint32_t laneOff[Cfg::kSlotsB];
 
     // The lambdas below are forced inline: left to the inliner's size heuristics, one of them staying a real call puts
     // the whole issue state (captured by reference) into scratch memory and the kernel runs three times slower.
-    // Bases and lane offsets of the given part(s) for tile t.
-    auto setupIssue = [&](const TileInfo& t, auto partsTag) __attribute__((always_inline)) {
-        constexpr int kParts = decltype(partsTag)::value;
-        if (kParts & kPartA) issBaseA = scalarBase(reinterpret_cast<const char*>(a.x) + static_cast<int64_t>(t.rowBase) * a.K);
-        if (kParts & kPartB) issBaseB = scalarBase(reinterpret_cast<const char*>(a.w) + static_cast<int64_t>(t.group) * a.wGroupStride);
-        // lane -> (row inside the instruction, LDS chunk slot); the global chunk it fetches is the one LdsOffset puts there
-        const int lane = Opaque(tid & 63);
-        const int rowIn = lane / Cfg::kChunksPerRow;
-        const int slot = lane % Cfg::kChunksPerRow;
+    // Base (in scalar registers: a DMA is then three instructions, LDS address, m0 and the load) and lane offsets for tile t.
+    auto setupIssue = [&](const TileInfo& t) __attribute__((always_inline)) {
+        const int lane = Opaque(tid) & 63;
+        const int rowIn = lane >> 3, slot = lane & 7;  // row inside the instruction, LDS chunk slot
+        if (!forWeights) {
+            issBase = UniformPtr(reinterpret_cast<const char*>(a.x) + static_cast<int64_t>(t.rowBase) * a.K);
 #pragma unroll
-        for (int q = 0; q < Cfg::kMaxPerWave; ++q) {
-            if (kParts != kBothParts && (q < Cfg::kSlotsA) != (kParts == kPartA)) continue;
-            const int g = slotInstr(q);
-            const int j = g < Cfg::kInstrA ? g : g - Cfg::kInstrA;  // instruction of its part
-            if (g < Cfg::kInstrA) {
+            for (int q = 0; q < Cfg::kSlotsA; ++q) {
                 // rows past the tile's last row are never used: such lanes re-read the last real row (same cache
                 // lines as its own lanes), and an instruction wholly past it reads one chunk, so the number of DMAs
                 // per stage stays constant while the activation traffic follows the real row count
-                const int r = Cfg::kRowsPerInstr * j + rowIn;
-                const int c = (LdsOffset<kStep>(r, slot) >> 4) % Cfg::kChunksPerRow;
-                const bool wholeInstrPast = Cfg::kRowsPerInstr * j >= t.rows;
-                laneOff[q] = wholeInstrPast ? 0u : static_cast<uint32_t>(min(r, t.rows - 1) * a.K + c * kChunk);
-            } else if (kNMajor) {
-                // weight instruction j moves k-rows 4 * j .. + 3 of the stage, 256 channel bytes each; lane ->
-                // (k-row lane / 16, LDS chunk slot lane % 16), fetching the logical chunk that the swizzle puts there.
-                // Chunks past the last channel are never stored: such lanes re-read the last real chunk.
-                const int k = 4 * j + lane / 16;
-                const int c = (lane % 16) ^ ((k & 7) << 1);
-                int32_t col;
-                if (kSwiglu) {
-                    col = c < 8 ? min(t.colBase + 16 * c, a.halfN - 16) : min(a.halfN + t.colBase + 16 * (c - 8), a.N - 16);
-                } else {
-                    col = min(t.colBase + 16 * c, a.N - 16);
-                }
+                const int firstRow = 8 * (waveN + kWavesN * q), r = firstRow + rowIn;
+                laneOff[q] = firstRow >= t.rows ? 0u : static_cast<uint32_t>(min(r, t.rows - 1) * a.K + (slot ^ ((r >> 1) & 7)) * kChunk);
+            }
+            return;
+        }
+        issBase = UniformPtr(reinterpret_cast<const char*>(a.w) + static_cast<int64_t>(t.group) * a.wGroupStride);
+#pragma unroll
+        for (int q = 0; q < Cfg::kSlotsB; ++q) {
+            constexpr int kPerHalf = Cfg::kSlotsB / 2;
+            const int half = q / kPerHalf, j = waveN + kWavesN * (q % kPerHalf);  // instruction j of its half of the channels
+            if (kNMajor) {
+                // instruction j moves k-rows 8 * j .. + 7 of the stage, 128 channel bytes each; chunks past the last
+                // channel are never stored: such lanes re-read the last real chunk
+                const int k = 8 * j + rowIn;
+                const int c = slot ^ RowMajorSwizzle(k);
+                const int32_t col = kSwiglu ? (half ? min(a.halfN + t.colBase + 16 * c, a.N - 16) : min(t.colBase + 16 * c, a.halfN - 16))
+                                            : min(t.colBase + 128 * half + 16 * c, a.N - 16);
                 laneOff[q] = static_cast<uint32_t>(k * a.N + col);
             } else if (kNz) {
-                // weight instruction j moves 32 k-rows (x 32 channel bytes) of channel block j / 4: 1 KB, contiguous
-                // in memory and in LDS; lane -> (k-row lane / 2, 16-byte half lane % 2)
-                const int32_t block = ChannelOfRow<kSwiglu>(a, t, 32 * (j / 4)) >> 5;
-                laneOff[q] = static_cast<uint32_t>(block * a.K * 32 + ((j % 4) * 32 + lane / 2) * 32 + (lane % 2) * kChunk);
+                // instruction j moves 32 k-rows (x 32 channel bytes) of channel block j / 4: 1 KB, contiguous in memory and
+                // in LDS; lane -> (k-row lane / 2, 16-byte half, swapped with bit 4 of k)
+                const int k = (j % 4) * 32 + lane / 2;
+                const int32_t col = t.colBase + (kSwiglu ? (half ? a.halfN : 0) + 32 * (j / 4) : 64 * (j / 4) + 32 * half);
+                const int32_t block = min(col, a.N - 1) >> 5;
+                laneOff[q] = static_cast<uint32_t>(block * a.K * 32 + k * 32 + ((lane ^ (k >> 4)) & 1) * kChunk);
             } else {
-                const int r = Cfg::kRowsPerInstr * j + rowIn;
-                const int c = (LdsOffset<kStep>(r, slot) >> 4) % Cfg::kChunksPerRow;
-                laneOff[q] = static_cast<uint32_t>(ChannelOfRow<kSwiglu>(a, t, r) * a.K + c * kChunk);
+                const int r = 8 * j + rowIn;
+                laneOff[q] = static_cast<uint32_t>(ChannelOfRow<kSwiglu>(a, t, half, r) * a.K + (slot ^ ((r >> 1) & 7)) * kChunk);
             }
         }
     };
-    // Moves the cursor of the given part(s) to the next k-step (after the last instruction of a stage has gone out).
-    auto advance = [&](auto partsTag) __attribute__((always_inline)) {
-        constexpr int kParts = decltype(partsTag)::value;
-        constexpr bool kCursorA = kParts == kPartA;
-        TileInfo& tile = kCursorA ? issTileA : issTileB;
-        int32_t& tileNo = kCursorA ? issNoA : issNoB;
-        int& step = kCursorA ? issStepA : issStepB;
-        int& slot = kCursorA ? issSlotA : issSlotB;
-        bool& drained = kCursorA ? issDrainedA : issDrainedB;
-        constexpr int kDepth = kCursorA ? kStagesA : kStagesB;
-        slot = slot + 1 == kDepth ? 0 : slot + 1;
-        if (++step == kSteps) {
+    // Moves the cursor to the next k-step.
+    auto advance = [&]() __attribute__((always_inline)) {
+        issAddr = issAddr + issStride == issEnd ? issFirst : issAddr + issStride;
+        if (__builtin_expect(++issStep == kSteps, 0)) {
             // move to this workgroup's next tile.  Past the last one the issue slots still go out (that keeps the number
-            // of outstanding DMAs per stage, hence the vmcnt arithmetic, constant) into ring slots nobody reads -- but
+            // of outstanding DMAs per stage, hence the vmcnt arithmetic, constant) into ring buffers nobody reads -- but
             // every one of them then re-reads the same first kilobyte of the last tile's weights, which stays in L2,
             // instead of pulling more stages of weights from HBM per workgroup.
-            step = 0;
-            const TileInfo next = tileAt(tileNo + 1);
+            issStep = 0;
+            const TileInfo next = tileAt(issNo + 1);
             if (next.valid) {
-                tile = next;
-                ++tileNo;
-                setupIssue(tile, partsTag);
-            } else if (!drained) {
-                drained = true;
+                issTile = next;
+                ++issNo;
+                setupIssue(issTile);
+            } else if (!issDrained) {
+                issDrained = true;
                 // any mapped, 16-byte aligned kilobyte will do: the start of the last tile's expert's weights
-                const char* const hot = scalarBase(reinterpret_cast<const char*>(a.w) + static_cast<int64_t>(tile.group) * a.wGroupStride);
-                if (kParts & kPartA) issBaseA = hot;
-                if (kParts & kPartB) issBaseB = hot;
+                issBase = UniformPtr(reinterpret_cast<const char*>(a.w) + static_cast<int64_t>(issTile.group) * a.wGroupStride);
 #pragma unroll
-                for (int q = 0; q < Cfg::kMaxPerWave; ++q) {
-                    if (kParts != kBothParts && (q < Cfg::kSlotsA) != (kParts == kPartA)) continue;
-                    laneOff[q] = static_cast<uint32_t>(lane) * kChunk;
-                }
+                for (int q = 0; q < Cfg::kSlotsB; ++q) laneOff[q] = static_cast<uint32_t>(Opaque(tid) & 63) * kChunk;
             }
         }
     };
-    // This wave's DMA instructions of the given part(s) of the stage at the part's cursor.
-    auto emitParts = [&](auto partsTag) __attribute__((always_inline)) {
-        constexpr int kParts = decltype(partsTag)::value;
-        constexpr bool kOwnA = kParts == kPartA;  // else the activation part, if any, follows cursor B
-        // On small tiles the k-steps of a tile are walked from a start that differs between workgroups (integer
-        // accumulation does not care about the order).  When rows lie a power-of-two stride apart (K = 4096 with
-        // K-contiguous weights), the low address bits of every row of every expert depend on the k offset alone:
-        // workgroups that all sit at the same k-step all queue on the same memory channels.  Only for small tiles, where
-        // every weight byte is used once: on the large-tile shapes neighbouring workgroups share operands through L2,
-        // and walking k in step is what makes those hits.
-        auto kOffset = [&](int step, bool drained) __attribute__((always_inline)) {
-            const int kIdx = step + kRotate;
-            if (kTail) return drained ? 0 : min(kIdx * kStep, a.K - kStep);
-            return drained ? 0 : (kIdx >= kSteps ? kIdx - kSteps : kIdx) * kStep;
-        };
-        const int kOffB = kOffset(issStepB, issDrainedB);
-        const int kOffA = kOwnA ? kOffset(issStepA, issDrainedA) : kOffB;
+    // This wave's DMA instruction of slot q of the stage at the cursor.  Activation rows always stay cacheable (the
+    // n-tiles of a group re-read them from L2); on small tiles (every weight byte is used exactly once) the weights stream
+    // past the caches.  On large tiles the m-tiles of a group share their weight columns through L2 and must not.
+    auto request = [&](int q) __attribute__((always_inline)) {
+        const int kIdx = issStep + kRotate;
+        const int kOff = issDrained ? 0 : kTail ? min(kIdx * kStep, a.K - kStep) : (kIdx >= kSteps ? kIdx - kSteps : kIdx) * kStep;
         // weights -- blocked layout: one k is 32 bytes further; row-major: N bytes
-        const int kOffW = kNz ? kOffB * 32 : (kNMajor ? kOffB * a.N : kOffB);
-        // instruction g lands g KB behind dstA (activation part) or dstB (weight part, whose first instruction is kInstrA)
-        const uint32_t dstA = ldsBase + (kOwnA ? issSlotA : issSlotB) * kStrideA;
-        const uint32_t dstB = ldsBase + kFirstB + issSlotB * kStrideB - Cfg::kInstrA * 1024;
-#pragma unroll
-        for (int q = 0; q < Cfg::kMaxPerWave; ++q) {
-            if (kParts != kBothParts && (q < Cfg::kSlotsA) != (kParts == kPartA)) continue;
-            const int g = slotInstr(q);
-            // where the activation instructions divide evenly among the waves, slot q is of the same part in every wave
-            constexpr bool kStaticSplit = kScalarIssue && Cfg::kInstrA % Cfg::kWaves == 0;
-            const bool isA = kStaticSplit ? q < Cfg::kInstrA / Cfg::kWaves : g < Cfg::kInstrA;
-            // wave-uniform choice: activation rows always stay cacheable (the n-tiles of a group re-read them from L2);
-            // on small tiles (every weight byte is used exactly once) the weights stream past the caches.  On large
-            // tiles the m-tiles of a group share their weight columns through L2 and must not.
-            if constexpr (kSmallTile) {
-                if (isA) DmaToLdsAddr16<false>(issBaseA + kOffA, laneOff[q], dstA + g * 1024);
-                else DmaToLdsAddr16<true>(issBaseB + kOffW, laneOff[q], dstB + g * 1024);
-            } else {  // selects, no branch: the k-step stays one basic block
-                DmaToLdsAddr16<false>(isA ? issBaseA + kOffA : issBaseB + kOffW, laneOff[q], (isA ? dstA : dstB) + g * 1024);
-            }
-        }
-    };
-    // One k-step's worth of issue: a whole stage, or (staggered depths) the activation share and then the weight share,
-    // each of the stage its own cursor has reached.
-    // The cursors move when all of it has gone out, so that the DMAs of a k-step stay in one basic block.
-    auto issueStage = [&]() __attribute__((always_inline)) {
-        if constexpr (kStaggered) {
-            emitParts(PartATag{});
-            emitParts(PartBTag{});
-            advance(PartATag{});
-            advance(PartBTag{});
+        const char* const base = issBase + ((kNz || kNMajor) && forWeights ? static_cast<int64_t>(kOff) * (kNz ? 32 : a.N) : kOff);
+        const uint32_t dst = issAddr + 1024 * kWavesN * q;
+        if constexpr (kSmallTile) {
+            if (forWeights) DmaToLdsAddr16<true>(base, laneOff[q], dst);
+            else if (q < Cfg::kSlotsA) DmaToLdsAddr16<false>(base, laneOff[q], dst);
         } else {
-            emitParts(BothPartsTag{});
-            advance(BothPartsTag{});
+            if (q < Cfg::kSlotsA || forWeights) DmaToLdsAddr16<false>(base, laneOff[q], dst);
         }
     };
-    // vmcnt that certifies the stage the compute side needs next with `younger` whole k-steps' worth of issue behind it
-    // (staggered depths: and that stage's own weight share, which went out after its activation share)
-    auto waitStage = [&](auto tag) __attribute__((always_inline)) {
-        constexpr int kYounger = decltype(tag)::value;
-        WaitVmcnt<kYounger * Cfg::kMaxPerWave + (kStaggered ? Cfg::kSlotsB : 0)>();
-    };
+    using FirstHalf = std::integral_constant<int, 0>;
+    using SecondHalf = std::integral_constant<int, 1>;
 
-    // Shifted barrier (tall tiles).  The plain k-step opens with its barrier -- the stage has landed, the previous one is
-    // no longer read -- after which every wave waits for its first fragments before it has any MFMA to issue.  Here the
-    // step's one barrier sits in front of its LAST block of MFMAs instead: by then every k-slice of the stage has been
-    // read, so the buffers take their refill a quarter of a step earlier, the same barrier certifies the next stage as
-    // landed, and the next step's first fragments are read while the matrix pipe still has a block of MFMAs to run.  All
-    // buffers of both rings are in use.
-    constexpr bool kEarly = kTileM >= 96;
-    static_assert(!kStaggered || kEarly, "staggered depths are built on the shifted barrier");
-    setupIssue(cur, BothPartsTag{});
-    if constexpr (kStaggered) {
-        // the order the steady state would have left behind: weight stages 0 .. kStagesB - kStagesA - 1 alone, then
-        // (activation stage i, weight stage kStagesB - kStagesA + i) for i = 0 .. kStagesA - 1
+    setupIssue(cur);
 #pragma unroll 1
-        for (int s = 0; s < kStagesB - kStagesA; ++s) {
-            emitParts(PartBTag{});
-            advance(PartBTag{});
-        }
-#pragma unroll 1
-        for (int s = 0; s < kStagesA; ++s) issueStage();
-    } else {
-#pragma unroll 1
-        for (int s = 0; s < (kEarly ? kStagesB : kStagesB - 1); ++s) issueStage();
+    for (int s = 0; s < (forWeights ? Cfg::kStagesB : Cfg::kStagesA); ++s) {
+#pragma unroll
+        for (int q = 0; q < Cfg::kSlotsB; ++q) request(q);
+        advance();
     }
-    int ringA = 0, ringB = 0;  // buffers the compute side reads next (one index where the depths are the same)
-    if constexpr (kEarly) {
-        waitStage(std::integral_constant<int, kStagesA - 1>{});
-        __syncthreads();  // stage 0 has landed for every wave
-    }
-
-    if (kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kTileM) {
+    if (kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kRows) {
         ldsRowScale[tid] = a.rowScale[cur.rowBase + (tid < cur.rows ? tid : cur.rows - 1)];
     }
+    // the first stage has landed (the row scales' load makes that only stricter)
+    if (forWeights) WaitVmcnt<(Cfg::kStagesB - 1) * Cfg::kSlotsB>();
+    else WaitVmcnt<(Cfg::kStagesA - 1) * Cfg::kSlotsA>();
+    __syncthreads();
 
-    // The tile's real rows (rounded up to whole 32-row MFMA tiles) are split between the two wave rows tile by tile:
-    // wave row 0 takes the first half (rounded up), wave row 1 the rest, and MFMA tiles that hold no real row are never
-    // computed -- on the memory-bound shapes the matrix pipe's power is what is worth saving.  The k loop is
-    // instantiated once per MFMA-tile count (0..kSub0) so that its body stays straight-line code.
-    int waveRow0 = 0;  // first tile row of this wave
-    int mySub = 0;     // MFMA tiles of this wave in the current tile
-    // Row of the weight tile where the wave's column block ni begins.  Blocks come in pairs (2p, 2p + 1) that sit at
-    // column position kNi / 2 * waveN + p of the tile: plain epilogues, the two halves of 64 neighbouring channels;
-    // kSwiglu, 32 activated channels (rows 0..127 of the tile) and their 32 linear partners (rows 128..255).
-    auto bRow = [&](int ni) __attribute__((always_inline)) {
-        const int position = kNi / 2 * waveN + ni / 2;
-        return kSwiglu ? 32 * position + (ni & 1) * (kTileN / 2) : 64 * position + 32 * (ni & 1);
+    uint32_t ringA = ldsBase, ringB = ldsBase + Cfg::kFirstB;  // buffers that the compute side reads
+    // Lane part of the fragment addresses.  Rows sixteen apart swizzle alike.
+    const int l16 = Opaque(tid) & 15, quad = (Opaque(tid) >> 4) & 3;
+    const uint32_t rowChunk = l16 * 128 + ((quad ^ ((l16 >> 1) & 7)) << 4);
+    const uint32_t laneA = rowChunk + waveM * 16 * 128;  // slice 1 of a k-step is 64 bytes on, or back: buffers and rows begin on 128
+    // Weights of the wave's column.  K-contiguous: as the rows (the second block is sixteen rows on).  Otherwise: the two blocks
+    // (slice 1 is 64 k-rows on and swizzles alike; with the transposing loads this lane supplies half a chunk of k-row k).
+    uint32_t laneB[kNz || kNMajor ? 2 : 1];
+    {
+        const int k = 16 * quad + (l16 >> 1);
+#pragma unroll
+        for (int i = 0; i < (kNz || kNMajor ? 2 : 1); ++i) {
+            if (kNMajor) laneB[i] = k * 128 + (((2 * waveN + i) ^ RowMajorSwizzle(k)) << 4) + 8 * (l16 & 1);
+            else if (kNz) laneB[i] = waveN * 4096 + k * 32 + 16 * (i ^ (quad & 1)) + 8 * (l16 & 1);
+            else laneB[i] = rowChunk + 32 * waveN * 128;
+        }
+    }
+    // the wave's four blocks of weights, slice ks
+    auto readB = [&](v4i (&b)[4], uint32_t buffer, int ks) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const uint32_t base = buffer;
+            const int half = (n >> 1) * Cfg::kHalfBytesB, j = n & 1;
+            if constexpr (kNz || kNMajor) {
+                constexpr int kEightK = kNz ? 8 * 32 : 8 * 128;  // the swizzles of k and k + 8 are the same
+                b[n] = LdsReadTransposed(base + laneB[j], half + ks * 8 * kEightK, kEightK);
+            } else {
+                b[n] = LdsRead16((base + laneB[0]) ^ (64 * ks), half + j * 16 * 128);
+            }
+        }
     };
-    v16i acc[kSubM][kNi];
 
+    v4i acc[Blocks::kAll][4];
     while (true) {
         const TileInfo following = tileAt(curNo + 1);
-        // the next tile's per-row scale travels in a register until this tile's epilogue has read the LDS copy
-        float followingRowScale = 0.0f;
-        if (following.valid && kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kTileM) {
-            followingRowScale = a.rowScale[following.rowBase + (tid < following.rows ? tid : following.rows - 1)];
+#pragma unroll
+        for (int m = 0; m < Blocks::kAll; ++m) {
+#pragma unroll
+            for (int n = 0; n < 4; ++n) acc[m][n] = v4i{0, 0, 0, 0};
         }
-#pragma unroll
-        for (int mi = 0; mi < kSubM; ++mi)
-#pragma unroll
-            for (int ni = 0; ni < kNi; ++ni)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0;
 
-        // The k loop of a wave with kMy MFMA tiles.  A k-step is straight-line code: the operands of k-slice ks + 1 are
-        // read from LDS before the MFMAs of k-slice ks are issued (fragment double buffer af / bf).
-        // Plain form: one barrier at the start of a step (the stage has landed, the previous one is no longer read),
-        // and the refill of the buffer it frees goes out behind the first block of MFMAs.
-        // kEarly form: see above; the fragments of a step's first k-slice are read at the end of the step before.
+        // The k loop of a wave with kMy row blocks (the loop is instantiated once per count, so that its body stays
+        // straight-line code: blocks that hold no real row are never multiplied -- on the memory-bound shapes the matrix
+        // pipe's power is what is worth saving).
         auto runTile = [&](auto myTag) __attribute__((always_inline)) {
             constexpr int kMy = decltype(myTag)::value;
-            constexpr int kSlices = kStep / 32;
-            static_assert(kSlices % 2 == 0, "the fragment double buffer is handed over between steps at slot 0");
-            v4i bf[2][kNi];
-            v4i af[2][kMy > 0 ? kMy : 1];
-            auto loadSlice = [&](int stageA, int stageB, int ks, int buf) __attribute__((always_inline)) {
-                if (kMy == 0) return;
-                const char* const A = lds + (kStaggered ? stageA : stageB) * kStrideA;  // common depth: one ring index
-                const char* const B = lds + kFirstB + stageB * kStrideB;
-                const int chunk = 2 * ks + lhi;
-                if constexpr (kNMajor) {
-                    // 16-lane group g: channels 16 * (g % 2) .. + 15 of the 32-channel block, k-half g / 2 (= lhi) of the
-                    // slice; lane j of the group supplies bytes (k = kBase + j / 2, channels 8 * (j % 2) .. + 7)
-                    const int j = lane & 15;
-                    const int k = 32 * ks + 16 * lhi + (j >> 1);
-                    const uint32_t bBase = ldsBase + kFirstB + stageB * kStrideB + 8 * (j & 1);
+            constexpr int kMy0 = (kMy + 1) / 2, kMy1 = kMy / 2;
+            v4i af[2][kMy0 > 0 ? kMy0 : 1];  // [slice][block]
+            v4i bf[2][4];                    // [slice][block]
+            auto readA = [&](v4i (&f)[kMy0 > 0 ? kMy0 : 1], uint32_t buffer, auto halfTag, int ks) __attribute__((always_inline)) {
+                constexpr int kHalf = decltype(halfTag)::value;
 #pragma unroll
-                    for (int ni = 0; ni < kNi; ++ni) {
-                        const int c = (bRow(ni) + 16 * ((lane >> 4) & 1)) >> 4;  // logical 16-byte chunk of the row
-                        // k and k + 8 share their low three bits, hence their swizzle
-                        const uint32_t lo = bBase + k * 256 + ((c ^ ((k & 7) << 1)) << 4);
-                        const uint32_t hi = lo + 8 * 256;
-                        const v2i vlo = __builtin_amdgcn_ds_read_tr8_b64_v2i32(reinterpret_cast<LdsV2iPtr>(lo));
-                        const v2i vhi = __builtin_amdgcn_ds_read_tr8_b64_v2i32(reinterpret_cast<LdsV2iPtr>(hi));
-                        bf[buf][ni] = v4i{vlo[0], vlo[1], vhi[0], vhi[1]};
+                for (int i = 0; i < (kHalf ? kMy1 : kMy0); ++i) f[i] = LdsRead16((buffer + laneA) ^ (64 * ks), (4 * i + 2 * kHalf) * 16 * 128);
+            };
+            // The product of one half of the rows with one slice, and between its instructions, if asked for, the requests of the even
+            // or the odd slots.  From one row block to the next the weight blocks are walked back and forth: consecutive instructions
+            // share an operand, which costs the matrix unit 2 % less power (4.02 / 4.14 POP/s on register operands).
+            auto multiply = [&](auto halfTag, int ks, bool requests, int odd = 0) __attribute__((always_inline)) {
+                constexpr int kHalf = decltype(halfTag)::value;
+                constexpr int kCount = kHalf ? kMy1 : kMy0, kOnes = kCount > 0 ? kCount : 1;
+#pragma unroll
+                for (int i = 0; i < kOnes; ++i) {
+                    if constexpr (kCount > 0) {
+#pragma unroll
+                        for (int step = 0; step < 4; ++step) {
+                            const int n = i & 1 ? 3 - step : step;
+                            v4i& c = acc[kHalf * Blocks::kFirst + i][n];
+                            c = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[ks][i], bf[ks][n], c, 0, 0, 0);
+                        }
                     }
-                } else if constexpr (kNz) {
-                    // 16-lane group g: channels 16 * (g % 2) .. + 15 of the block, k-half g / 2 (= lhi) of the slice;
-                    // lane j of the group supplies bytes (k = kBase + j / 2, channels 8 * (j % 2) .. + 7)
-                    const int j = lane & 15;
-                    const int inBlock = (32 * ks + 16 * lhi + (j >> 1)) * 32 + 16 * ((lane >> 4) & 1) + 8 * (j & 1);
+                    if (requests) {
+                        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int ni = 0; ni < kNi; ++ni) {
-                        // addressed through the 32-bit LDS address: no generic-to-LDS pointer conversion in the loop
-                        const uint32_t blk = ldsBase + kFirstB + stageB * kStrideB + (bRow(ni) >> 5) * 4096 + inBlock;
-                        const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32(reinterpret_cast<LdsV2iPtr>(blk));
-                        const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32(reinterpret_cast<LdsV2iPtr>(blk + 8 * 32));
-                        bf[buf][ni] = v4i{lo[0], lo[1], hi[0], hi[1]};
+                        for (int r = 4 * i / kOnes; r < 4 * (i + 1) / kOnes; ++r) request(2 * r + odd);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
-                } else {
-#pragma unroll
-                    for (int ni = 0; ni < kNi; ++ni) {
-                        bf[buf][ni] = *reinterpret_cast<const v4i*>(B + LdsOffset<kStep>(bRow(ni) + l32, chunk));
-                    }
-                }
-#pragma unroll
-                for (int mi = 0; mi < kMy; ++mi) {
-                    af[buf][mi] = *reinterpret_cast<const v4i*>(A + LdsOffset<kStep>(waveRow0 + mi * 32 + l32, chunk));
                 }
             };
-            if constexpr (kEarly) loadSlice(ringA, ringB, 0, 0);  // the tile's first stage was certified at the end of the tile before
-            auto kStepOf = [&](int step, auto tailTag) __attribute__((always_inline)) {
-                constexpr bool kTailStep = decltype(tailTag)::value;
-                if constexpr (!kEarly) {
-                    // the oldest stage in flight has landed once at most (stages - 2) stages' worth of this wave's DMAs remain
-                    waitStage(std::integral_constant<int, kStagesA - 2>{});
-                    __syncthreads();  // every wave's share of the stage is in LDS, and the previous stage is no longer read
-                    loadSlice(ringA, ringB, 0, 0);
+            // last step of kTail: the weights of the k that the step before has covered count zero (a lane's fragments hold
+            // k 64 * ks + 16 * quad .. + 15 of the stage)
+            auto maskB = [&](int ks, bool last) __attribute__((always_inline)) {
+                if (kTail && last) {
+                    if (64 * ks + 16 * ((Opaque(tid) >> 4) & 3) < kSteps * kStep - a.K) {
+#pragma unroll
+                        for (int n = 0; n < 4; ++n) bf[ks][n] = v4i{0, 0, 0, 0};
+                    }
                 }
-                const int nextA = !kStaggered ? 0 : ringA + 1 == kStagesA ? 0 : ringA + 1;  // unused with a common depth
-                const int nextB = ringB + 1 == kStagesB ? 0 : ringB + 1;
-#pragma unroll
-                for (int ks = 0; ks < kSlices; ++ks) {
-                    if (!kEarly || ks + 1 < kSlices) {
-                        if (ks + 1 < kSlices) loadSlice(ringA, ringB, ks + 1, (ks + 1) & 1);
-                    } else {
-                        // Before the step's last block of MFMAs: every k-slice of this stage has been read (the reads
-                        // of the last one returned in the shadow of the block before), and the next stage, issued one
-                        // step ago, should have landed.  One barrier certifies both; inside a tile, the next step's
-                        // first fragments are read behind the MFMAs.
-                        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS reads have returned
-                        waitStage(std::integral_constant<int, kStagesA - 2>{});
-                        __syncthreads();
-                        issueStage();  // into the buffer(s) that this step read
-                        if (step + 1 < kSteps) loadSlice(nextA, nextB, 0, 0);
-                    }
-#pragma unroll
-                    for (int mi = 0; mi < kMy; ++mi) {
-                        v4i av = af[ks & 1][mi];
-                        if constexpr (kTailStep) {
-                            // k of this fragment: 32 * ks + 16 * lhi .. + 15 of the stage; those the step before covered count zero
-                            if (32 * ks + 16 * lhi < kSteps * kStep - a.K) av = v4i{0, 0, 0, 0};
-                        }
-#pragma unroll
-                        for (int ni = 0; ni < kNi; ++ni) {
-                            acc[mi][ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bf[ks & 1][ni], acc[mi][ni], 0, 0, 0);
-                        }
-                    }
-                    if constexpr (kEarly && kMy > 0) {
-                        if (ks + 1 < kSlices) {
-                            // The k-slice's pipeline, pinned: the reads of the next slice go out behind the first MFMA
-                            // and return under the others.  Left alone, the scheduler makes this order on some builds
-                            // and, at the register limit of the tallest tiles, on others a late-read order that stalls
-                            // the matrix pipe.  (Reading each fragment only when the one before it has retired saves
-                            // registers and measures slower.)
-                            constexpr int kReads = kMy + ((kNz || kNMajor) ? 2 * kNi : kNi);
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);              // one MFMA
-                            __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);         // the LDS reads
-                            __builtin_amdgcn_sched_group_barrier(0x008, kNi * kMy - 1, 0);  // the other MFMAs
-                        }
-                    }
-                    if (!kEarly && ks == 0) issueStage();  // into the buffer that the step before read
+            };
+            auto kStepOf = [&](bool last) __attribute__((always_inline)) {
+                const uint32_t nextA = ringA + Cfg::kStageBytesA == ldsBase + Cfg::kFirstB ? ldsBase : ringA + Cfg::kStageBytesA;
+                const uint32_t nextB = ringB + Cfg::kStageBytesB == ldsBase + Cfg::kFirstB + Cfg::kStagesB * Cfg::kStageBytesB
+                                           ? ldsBase + Cfg::kFirstB : ringB + Cfg::kStageBytesB;
+                if (kMy > 0) readB(bf[1], ringB, 1);
+                readA(af[1], ringA, FirstHalf{}, 1);
+                __builtin_amdgcn_sched_barrier(0);
+                maskB(0, last);
+                multiply(FirstHalf{}, 0, false);
+                __builtin_amdgcn_sched_barrier(0);
+                readA(af[0], ringA, SecondHalf{}, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                maskB(1, last);
+                multiply(FirstHalf{}, 1, false);
+                PhaseBarrier();  // this wave's reads of weights and first half have returned: the products above used them
+                readA(af[1], ringA, SecondHalf{}, 1);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(SecondHalf{}, 0, true, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                WaitLds();
+                if (forWeights) WaitVmcnt<Cfg::kYoungerB>();
+                else WaitVmcnt<Cfg::kYoungerA>();
+                PhaseBarrier();
+                if (kMy > 0 && !last) {
+                    readB(bf[0], nextB, 0);
+                    readA(af[0], nextA, FirstHalf{}, 0);
                 }
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(SecondHalf{}, 1, true, 1);
+                __builtin_amdgcn_sched_barrier(0);
+                advance();
                 ringA = nextA;
                 ringB = nextB;
             };
+            // the tile's first stage was certified in front of the loop
+            if (kMy > 0) readB(bf[0], ringB, 0);
+            readA(af[0], ringA, FirstHalf{}, 0);
 #pragma unroll 1
-            for (int step = 0; step < (kTail ? kSteps - 1 : kSteps); ++step) kStepOf(step, std::false_type{});
-            if constexpr (kTail) kStepOf(kSteps - 1, std::true_type{});
+            for (int step = 0; step < kSteps; ++step) kStepOf(step + 1 == kSteps);
         };
-        {
-            const int active = (cur.rows + 31) >> 5;                       // MFMA tiles with real rows, 1..kSub0+kSub1
-            const int share0 = Cfg::kWavesM == 2 ? (active + 1) >> 1 : active;  // wave row 0's share
-            waveRow0 = waveM == 0 ? 0 : 32 * share0;
-            mySub = waveM == 0 ? share0 : active - share0;
+        const int active = (cur.rows + 15) >> 4;  // blocks with real rows
+        auto runOne = [&](auto myTag) __attribute__((always_inline)) { runTile(myTag); };
+        ForCount<Blocks::kAll>((active + 1 - waveM) >> 1, runOne);
+
+        // The next tile's per-row scale travels in a register until this tile's epilogue has read the LDS copy.  (Not across the k
+        // loop: the tallest tiles have no register left there.)
+        float followingRowScale = 0.0f;
+        if (following.valid && kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kRows) {
+            followingRowScale = a.rowScale[following.rowBase + (tid < following.rows ? tid : following.rows - 1)];
         }
-        ForCount<kSub0>(mySub, runTile);
 
         // The draw for the tile after the next goes out inside the epilogue and is looked at behind it.  A wave's memory
         // requests are counted back in issue order and the draw, an atomic that is settled at the memory side, takes
-        // microseconds on a loaded machine: in front of the k loop it would hold up the count of every operand stage
+        // microseconds on a loaded machine: in front of the k loop it would hold up the count of every operand part
         // issued after it.  During the epilogue the ring is full and nothing is issued.
         int32_t drawValue = 0;
         auto draw = [&]() __attribute__((always_inline)) {
@@ -1185,13 +1162,10 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                 if (c >= 0) drawValue = QueueTake(a.queueCounters, c);
             }
         };
-        TileEpilogueWave<kSubM, kNi, 0, kTileM, kEpi>(a, cur, acc, mySub, waveRow0, kNi / 2 * waveN, Opaque(l32), Opaque(lhi),
-                                                      ldsRowScale, ldsRowMax, draw);
-        if constexpr (kNi == 4) {
-            TileEpilogueWave<kSubM, kNi, 1, kTileM, kEpi>(a, cur, acc, mySub, waveRow0, kNi / 2 * waveN + 1, Opaque(l32), Opaque(lhi),
-                                                          ldsRowScale, ldsRowMax);
-        }
-        if constexpr (kSwiglu) TileEpilogueFoldMax<kTileM>(a, cur, Opaque(tid), ldsRowMax);
+        const KernelArgs epilogueArgs = ReloadArgs();
+        TileEpilogueWave<kRows, kEpi, kOrderOf<kNz, kNMajor>>(epilogueArgs, cur, acc, waveM, waveN, Opaque(tid) & 15, (Opaque(tid) >> 4) & 3, ldsRowScale,
+                                                              ldsRowMax, draw);
+        if constexpr (kSwiglu) TileEpilogueFoldMax<kRows>(epilogueArgs, cur, Opaque(tid), ldsRowMax);
         // Loads and stores may retire out of order with respect to each other, so drain everything (the epilogue's
         // stores and the DMAs in flight, which had the whole epilogue to land) before counting DMAs again.
         WaitVmcnt<0>();
@@ -1200,12 +1174,13 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         if (pull && tid == 0) {
             const QueueDraw d = QueueResolve(bigTiles, totalTiles - bigTiles, a.queueCounters, xcd, prefer,
                                              static_cast<uint32_t>(ldsSeq[kSeqUsedUp]), ldsSeq[kSeqDrawCounter], drawValue, kOneRun);
-            ldsSeq[2 * ((curNo + 2) & 3)] = d.list;
-            ldsSeq[2 * ((curNo + 2) & 3) + 1] = d.logical;
+            leaveTile(curNo + 2, d.list, d.logical);
             ldsSeq[kSeqUsedUp] = static_cast<int32_t>(d.usedUp);
         }
+        if (!pull && tid == 0) leaveShareTile(curNo + kTilesAhead);
         __syncthreads();  // the epilogue's reads of ldsRowScale / ldsRowMax are done; the drawn tile is in the ring
-        if (kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kTileM) ldsRowScale[tid] = followingRowScale;
+        if (kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kRows) ldsRowScale[Opaque(tid)] = followingRowScale;
+        WaitLds();
         cur = following;
         ++curNo;
     }
@@ -1220,13 +1195,12 @@ __device__ __forceinline__ void WriteSpan(const KernelArgs& a, uint64_t start, u
     }
 }
 
-template <int kSub0, int kSub1, int kStep, Epilogue kEpi, bool kNz, bool kNMajor, int kWn, bool kTail>
-__global__ __launch_bounds__(64 * kWn * (kSub1 > 0 ? 2 : 1)) void StreamGemmKernel(
-    KernelArgs a, const int32_t* __restrict__ sched) {
-    extern __shared__ __attribute__((aligned(16))) char lds[];
+template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
+__global__ __launch_bounds__(kThreads) void StreamGemmKernel(KernelArgs a, const int32_t* __restrict__ sched) {
+    extern __shared__ __attribute__((aligned(128))) char lds[];
     const uint64_t spanStart = a.wgSpans != nullptr ? __builtin_amdgcn_s_memrealtime() : 0;
     uint64_t spanTiles = 0;
-    StreamGemmBody<kSub0, kSub1, kStep, kEpi, kNz, kNMajor, kWn, kBothRuns, kTail>(a, sched, lds, spanTiles);
+    StreamGemmBody<kRows, kEpi, kNz, kNMajor, kBothRuns, kTail>(a, sched, lds, spanTiles);
     WriteSpan(a, spanStart, spanTiles);
 }
 
@@ -1239,19 +1213,17 @@ __global__ __launch_bounds__(64 * kWn * (kSub1 > 0 ? 2 : 1)) void StreamGemmKern
 // ring drain, and serves the other; a launch without small m-tiles costs the workgroups that looked for them one draw.
 //
 // kHasLow: the scheduling kernel may have cut the groups into m-tiles of kLowTileM rows instead; these run in one geometry.
-template <int kSub0, int kSub1, Epilogue kEpi>
-constexpr bool kHasLow = kSub0 == 3 && kSub1 == 3 && kEpi != Epilogue::kSwiglu;
+template <int kRows, Epilogue kEpi>
+constexpr bool kHasLow = kRows == 192 && kEpi != Epilogue::kSwiglu;
 
-template <int kSub0, int kSub1, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
-__global__ __launch_bounds__(512) void MixedGemmKernel(KernelArgs a, const int32_t* __restrict__ sched) {
-    static_assert(StreamCfg<1, 1, 128>::kTileM == kSmallRows, "the small run's geometry is that of the 64-row tiles");
-    static_assert(StreamCfg<1, 1, 128>::kThreads == 512 && StreamCfg<kSub0, kSub1, 128>::kThreads == 512, "one workgroup size for both");
-    extern __shared__ __attribute__((aligned(16))) char lds[];
+template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
+__global__ __launch_bounds__(kThreads) void MixedGemmKernel(KernelArgs a, const int32_t* __restrict__ sched) {
+    extern __shared__ __attribute__((aligned(128))) char lds[];
     const uint64_t spanStart = a.wgSpans != nullptr ? __builtin_amdgcn_s_memrealtime() : 0;
     uint64_t spanTiles = 0;
-    if constexpr (kHasLow<kSub0, kSub1, kEpi>) {
+    if constexpr (kHasLow<kRows, kEpi>) {
         if (sched[kHdrTileM] == kLowTileM) {
-            StreamGemmBody<3, 2, 128, kEpi, kNz, kNMajor, kWavesN, kBothRuns, kTail>(a, sched, lds, spanTiles);
+            StreamGemmBody<kLowTileM, kEpi, kNz, kNMajor, kBothRuns, kTail>(a, sched, lds, spanTiles);
             WriteSpan(a, spanStart, spanTiles);
             return;
         }
@@ -1261,122 +1233,115 @@ __global__ __launch_bounds__(512) void MixedGemmKernel(KernelArgs a, const int32
     int64_t forSmall = costAll > 0 ? (slots * costSmall + costAll / 2) / costAll : 0;
     if (forSmall == 0 && sched[1] > 0 && slots > 1) forSmall = 1;
     if (slot < forSmall) {
-        StreamGemmBody<1, 1, 128, kEpi, kNz, kNMajor, kWavesN, kSmallRun, kTail>(a, sched, lds, spanTiles);
+        StreamGemmBody<kSmallRows, kEpi, kNz, kNMajor, kSmallRun, kTail>(a, sched, lds, spanTiles);
         __syncthreads();  // the other geometry lays LDS out anew
-        StreamGemmBody<kSub0, kSub1, 128, kEpi, kNz, kNMajor, kWavesN, kBigRun, kTail>(a, sched, lds, spanTiles);
+        StreamGemmBody<kRows, kEpi, kNz, kNMajor, kBigRun, kTail>(a, sched, lds, spanTiles);
     } else {
-        StreamGemmBody<kSub0, kSub1, 128, kEpi, kNz, kNMajor, kWavesN, kBigRun, kTail>(a, sched, lds, spanTiles);
+        StreamGemmBody<kRows, kEpi, kNz, kNMajor, kBigRun, kTail>(a, sched, lds, spanTiles);
         __syncthreads();
-        StreamGemmBody<1, 1, 128, kEpi, kNz, kNMajor, kWavesN, kSmallRun, kTail>(a, sched, lds, spanTiles);
+        StreamGemmBody<kSmallRows, kEpi, kNz, kNMajor, kSmallRun, kTail>(a, sched, lds, spanTiles);
     }
     WriteSpan(a, spanStart, spanTiles);
 }
 
 // ---------------------------------------------------------------------------------------------- generic path
-constexpr int kGenStep = 128;  // k-bytes per step
-
-__device__ __forceinline__ int Lds128Offset(int row, int chunk) { return row * kGenStep + ((chunk ^ ((row >> 1) & 7)) << 4); }
-
-// One tile per workgroup (grid = static upper bound of tiles), 4 waves, operands gathered byte by byte through
-// registers into a single LDS buffer.  Handles any K and both weight layouts.
-template <int kSubM, Epilogue kEpi>
-__global__ __launch_bounds__(256) void GenericGemmKernel(KernelArgs a, const int32_t* __restrict__ sched) {
-    constexpr int kThreads = 256;
-    constexpr int kTileM = 32 * kSubM;
-    constexpr int kChunksPerRow = kGenStep / kChunk;
-    constexpr int kALoads = kTileM * kChunksPerRow / kThreads;
+// One tile per workgroup (grid = static upper bound of tiles), operands gathered byte by byte through
+// registers into a single LDS buffer.  Handles any K and every weight layout.
+template <int kRows, Epilogue kEpi>
+__global__ __launch_bounds__(kThreads) void GenericGemmKernel(KernelArgs a, const int32_t* __restrict__ sched) {
+    using Blocks = RowBlocks<kRows>;
+    constexpr int kChunksPerRow = kStep / kChunk;
     constexpr int kBLoads = kTileN * kChunksPerRow / kThreads;
     constexpr bool kSwiglu = kEpi == Epilogue::kSwiglu;
-    __shared__ __attribute__((aligned(16))) char ldsA[kTileM * kGenStep];
-    __shared__ __attribute__((aligned(16))) char ldsB[kTileN * kGenStep];
-    __shared__ __attribute__((aligned(16))) float ldsRowScale[kTileM];
-    __shared__ float ldsRowMax[kWavesN * kTileM];
+    __shared__ __attribute__((aligned(16))) char ldsA[kRows * kStep];
+    __shared__ __attribute__((aligned(16))) char ldsB[kTileN * kStep];
+    __shared__ __attribute__((aligned(16))) float ldsRowScale[kRows];
+    __shared__ float ldsRowMax[kWavesN * kRows];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int waveN = tid >> 6;
-    const int l32 = lane & 31;
-    const int lhi = lane >> 5;
+    const int waveN = (tid >> 6) % kWavesN, waveM = __builtin_amdgcn_readfirstlane((tid >> 6) / kWavesN);
+    const int l16 = lane & 15;
+    const int quad = lane >> 4;
 
     // one tile per workgroup: the two runs of the m-tile table as one list, cut into eight contiguous shares
     const int32_t* const queueHdr = sched;
     const int4* const mTileTable = reinterpret_cast<const int4*>(queueHdr + kQueueHeaderInts + kQueueCounterInts);
     const int32_t countBig = queueHdr[0], countSmall = queueHdr[1];
-    const int64_t bigTiles = static_cast<int64_t>(countBig) * a.tilesN;
-    const int64_t totalTiles = bigTiles + static_cast<int64_t>(countSmall) * a.tilesN;
-    const int64_t perXcd = (totalTiles + kXcds - 1) / kXcds;
-    const int64_t local = blockIdx.x / kXcds;
-    const int64_t logical = static_cast<int64_t>(blockIdx.x % kXcds) * perXcd + local;
+    const int32_t bigTiles = countBig * a.tilesN;
+    const int32_t totalTiles = bigTiles + countSmall * a.tilesN;
+    const int32_t perXcd = (totalTiles + kXcds - 1) / kXcds;
+    const int32_t local = blockIdx.x / kXcds;
+    const int32_t logical = static_cast<int32_t>(blockIdx.x % kXcds) * perXcd + local;
     if (local >= perXcd || logical >= totalTiles) return;
     const TileInfo t = logical < bigTiles
-        ? DecodeListTile<kTileM, kSwiglu>(a, mTileTable, 0, countBig, queueHdr[4], logical)
-        : DecodeListTile<kTileM, kSwiglu>(a, mTileTable, countBig, countSmall, queueHdr[5], logical - bigTiles);
-    if (kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kTileM) {
+        ? DecodeListTile<kSwiglu>(a, mTileTable, 0, countBig, queueHdr[4], logical)
+        : DecodeListTile<kSwiglu>(a, mTileTable, countBig, countSmall, queueHdr[5], logical - bigTiles);
+    if (kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kRows) {
         ldsRowScale[tid] = a.rowScale[t.rowBase + (tid < t.rows ? tid : t.rows - 1)];
     }
     const int8_t* const wGroup = a.w + static_cast<int64_t>(t.group) * a.wGroupStride;
-    const int bRow0 = kSwiglu ? 32 * waveN : 64 * waveN;
-    const int bRowStep = kSwiglu ? kTileN / 2 : 32;
 
-    v16i acc[kSubM][2];
+    v4i acc[Blocks::kAll][4];
 #pragma unroll
-    for (int mi = 0; mi < kSubM; ++mi)
+    for (int m = 0; m < Blocks::kAll; ++m) {
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0;
+        for (int n = 0; n < 4; ++n) acc[m][n] = v4i{0, 0, 0, 0};
+    }
 
-    for (int k0 = 0; k0 < a.K; k0 += kGenStep) {
+    for (int k0 = 0; k0 < a.K; k0 += kStep) {
         // consecutive threads take consecutive tile rows so that N-contiguous weights still coalesce
-#pragma unroll
-        for (int i = 0; i < kALoads; ++i) {
-            const int p = i * kThreads + tid;
-            const int r = p % kTileM;
-            const int chunk = p / kTileM;
+        for (int p = tid; p < kRows * kChunksPerRow; p += kThreads) {
+            const int r = p % kRows;
+            const int chunk = p / kRows;
             const int8_t* src = a.x + static_cast<int64_t>(t.rowBase + (r < t.rows ? r : t.rows - 1)) * a.K;
             union { v4i v; int8_t b[16]; } u;
             for (int j = 0; j < kChunk; ++j) {
                 const int k = k0 + chunk * kChunk + j;
                 u.b[j] = k < a.K ? src[k] : static_cast<int8_t>(0);
             }
-            *reinterpret_cast<v4i*>(ldsA + Lds128Offset(r, chunk)) = u.v;
+            *reinterpret_cast<v4i*>(ldsA + LdsOffset(r, chunk)) = u.v;
         }
 #pragma unroll
         for (int i = 0; i < kBLoads; ++i) {
             const int p = i * kThreads + tid;
             const int r = p % kTileN;
             const int chunk = p / kTileN;
-            const int8_t* src = wGroup + WeightRowBase(a, ChannelOfRow<kSwiglu>(a, t, r));
+            const int8_t* src = wGroup + WeightRowBase(a, ChannelOfRow<kSwiglu>(a, t, r / 128, r % 128));
             union { v4i v; int8_t b[16]; } u;
             for (int j = 0; j < kChunk; ++j) {
                 const int k = k0 + chunk * kChunk + j;
                 u.b[j] = k < a.K ? src[static_cast<int64_t>(k) * a.wStrideK] : static_cast<int8_t>(0);
             }
-            *reinterpret_cast<v4i*>(ldsB + Lds128Offset(r, chunk)) = u.v;
+            *reinterpret_cast<v4i*>(ldsB + LdsOffset(r, chunk)) = u.v;
         }
         __syncthreads();
 #pragma unroll
-        for (int ks = 0; ks < kGenStep / 32; ++ks) {
-            const int chunk = 2 * ks + lhi;
-            const v4i b0 = *reinterpret_cast<const v4i*>(ldsB + Lds128Offset(bRow0 + l32, chunk));
-            const v4i b1 = *reinterpret_cast<const v4i*>(ldsB + Lds128Offset(bRow0 + bRowStep + l32, chunk));
+        for (int ks = 0; ks < 2; ++ks) {
+            const int chunk = 4 * ks + quad;
+            v4i b[4];
 #pragma unroll
-            for (int mi = 0; mi < kSubM; ++mi) {
-                const v4i av = *reinterpret_cast<const v4i*>(ldsA + Lds128Offset(mi * 32 + l32, chunk));
-                acc[mi][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, b0, acc[mi][0], 0, 0, 0);
-                acc[mi][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, b1, acc[mi][1], 0, 0, 0);
+            for (int n = 0; n < 4; ++n) {
+                b[n] = *reinterpret_cast<const v4i*>(ldsB + LdsOffset(128 * (n >> 1) + 32 * waveN + 16 * (n & 1) + l16, chunk));
+            }
+#pragma unroll
+            for (int m = 0; m < Blocks::kAll; ++m) {
+                const v4i av = *reinterpret_cast<const v4i*>(ldsA + LdsOffset(Blocks::RowOf(m, waveM) + l16, chunk));
+#pragma unroll
+                for (int n = 0; n < 4; ++n) acc[m][n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, b[n], acc[m][n], 0, 0, 0);
             }
         }
         __syncthreads();
     }
-    TileEpilogue<kSubM, kTileM, kEpi>(a, t, acc, kSubM, 0, waveN, l32, lhi, tid, ldsRowScale, ldsRowMax);
+    TileEpilogueWave<kRows, kEpi, kOrderLane>(a, t, acc, waveM, waveN, l16, quad, ldsRowScale, ldsRowMax);
+    if constexpr (kSwiglu) TileEpilogueFoldMax<kRows>(a, t, tid, ldsRowMax);
 }
 
 // ---------------------------------------------------------------------------------------------- launchers
-template <int kSub0, int kSub1, int kStep, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail, int kWn = kWavesN>
+template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
 hipError_t LaunchStream(const KernelArgs& args, const int32_t* sched, int64_t maxTiles, hipStream_t stream) {
-    using Cfg = StreamCfg<kSub0, kSub1, kStep, kWn>;
-    auto kernel = StreamGemmKernel<kSub0, kSub1, kStep, kEpi, kNz, kNMajor, kWn, kTail>;
+    using Cfg = StreamCfg<kRows>;
+    auto kernel = StreamGemmKernel<kRows, kEpi, kNz, kNMajor, kTail>;
     static std::atomic<uint64_t> optedIn{0};
     const hipError_t attr = opapi::EnsureDynamicLds(reinterpret_cast<const void*>(kernel), Cfg::kLdsBytes, optedIn);
     if (attr != hipSuccess) return attr;
@@ -1386,19 +1351,16 @@ hipError_t LaunchStream(const KernelArgs& args, const int32_t* sched, int64_t ma
     grid = grid / kXcds * kXcds;
     if (grid < kXcds) grid = kXcds;
     KernelArgs launchArgs = args;
-    launchArgs.wgSpans = SpanBufferFor(kEpi, static_cast<int>(grid), Cfg::kTileM);
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(Cfg::kThreads), Cfg::kLdsBytes, stream, launchArgs, sched);
+    launchArgs.wgSpans = SpanBufferFor(kEpi, static_cast<int>(grid), kRows);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), Cfg::kLdsBytes, stream, launchArgs, sched);
     return hipGetLastError();
 }
 
-template <int kSub0, int kSub1, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
+template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
 hipError_t LaunchMixed(const KernelArgs& args, const int32_t* sched, int64_t maxTiles, hipStream_t stream) {
-    using Big = StreamCfg<kSub0, kSub1, 128>;
-    using Small = StreamCfg<1, 1, 128>;
-    using Low = StreamCfg<3, 2, 128>;
-    static_assert(Low::kTileM == kLowTileM && Low::kThreads == 512, "one workgroup size for all");
-    constexpr int kLdsBytes = std::max({Big::kLdsBytes, Small::kLdsBytes, kHasLow<kSub0, kSub1, kEpi> ? Low::kLdsBytes : 0});
-    auto kernel = MixedGemmKernel<kSub0, kSub1, kEpi, kNz, kNMajor, kTail>;
+    constexpr int kLdsBytes = std::max({StreamCfg<kRows>::kLdsBytes, StreamCfg<kSmallRows>::kLdsBytes,
+                                        kHasLow<kRows, kEpi> ? StreamCfg<kLowTileM>::kLdsBytes : 0});
+    auto kernel = MixedGemmKernel<kRows, kEpi, kNz, kNMajor, kTail>;
     static std::atomic<uint64_t> optedIn{0};
     const hipError_t attr = opapi::EnsureDynamicLds(reinterpret_cast<const void*>(kernel), kLdsBytes, optedIn);
     if (attr != hipSuccess) return attr;
@@ -1407,31 +1369,29 @@ hipError_t LaunchMixed(const KernelArgs& args, const int32_t* sched, int64_t max
     grid = grid / kXcds * kXcds;
     if (grid < kXcds) grid = kXcds;
     KernelArgs launchArgs = args;
-    launchArgs.wgSpans = SpanBufferFor(kEpi, static_cast<int>(grid), Big::kTileM);
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(512), kLdsBytes, stream, launchArgs, sched);
+    launchArgs.wgSpans = SpanBufferFor(kEpi, static_cast<int>(grid), kRows);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), kLdsBytes, stream, launchArgs, sched);
     return hipGetLastError();
 }
 
-// Tile heights and their (wave row 0, wave row 1, k-step) shapes.  Up to 192 rows the weight ring holds three or more
-// 128-byte stages; from 192 rows on the activation ring holds two.
 template <Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
 hipError_t LaunchStreamShapeOf(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream) {
     switch (plan.tileM) {
-        case 32: return LaunchStream<1, 0, 128, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
-        case 64: return LaunchStream<1, 1, 128, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
-        case 96: return LaunchStream<2, 1, 128, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
-        case 128: return LaunchStream<2, 2, 128, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
+        case 32: return LaunchStream<32, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
+        case 64: return LaunchStream<64, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
+        case 96: return LaunchStream<96, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
+        case 128: return LaunchStream<128, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
         // (160-row tiles were measured in the two-geometry form as well: the down projection of the DeepSeek-V3 prefill
         // shape, whose few overflowing experts leave small second m-tiles, 0.834 against 0.820 ms -- sixteen k-steps
         // per tile do not repay a change of geometry)
-        case 160: return LaunchStream<3, 2, 128, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
+        case 160: return LaunchStream<160, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
         // pulled tiles of 192 and 256 rows: the two runs of the table with a stage geometry each
         case 192:
-            if (plan.pullTiles) return LaunchMixed<3, 3, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
-            return LaunchStream<3, 3, 128, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
+            if (plan.pullTiles) return LaunchMixed<192, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
+            return LaunchStream<192, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
         default:
-            if (plan.pullTiles) return LaunchMixed<4, 4, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
-            return LaunchStream<4, 4, 128, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
+            if (plan.pullTiles) return LaunchMixed<256, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
+            return LaunchStream<256, kEpi, kNz, kNMajor, kTail>(args, sched, plan.maxTiles, stream);
     }
 }
 
@@ -1445,8 +1405,8 @@ hipError_t LaunchStreamShape(const Plan& plan, const KernelArgs& args, const int
 template <Epilogue kEpi>
 hipError_t LaunchGenericShape(const Plan& plan, const KernelArgs& args, const int32_t* sched, hipStream_t stream) {
     const dim3 grid(static_cast<unsigned>(plan.maxTiles));
-    if (plan.tileM <= 32) hipLaunchKernelGGL((GenericGemmKernel<1, kEpi>), grid, dim3(256), 0, stream, args, sched);
-    else hipLaunchKernelGGL((GenericGemmKernel<4, kEpi>), grid, dim3(256), 0, stream, args, sched);
+    if (plan.tileM <= 32) hipLaunchKernelGGL((GenericGemmKernel<32, kEpi>), grid, dim3(kThreads), 0, stream, args, sched);
+    else hipLaunchKernelGGL((GenericGemmKernel<128, kEpi>), grid, dim3(kThreads), 0, stream, args, sched);
     return hipGetLastError();
 }
 

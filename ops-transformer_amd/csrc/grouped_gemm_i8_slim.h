@@ -62,18 +62,6 @@ __device__ __forceinline__ void DmaToLdsAddr4(const char* base, uint32_t laneOff
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(m0), "v"(laneOffset), "s"(sbase) : "memory");
 }
 
-// Maximum over the 16 lanes of a row group, in every lane (rotations inside the row: no LDS).
-__device__ __forceinline__ float MaxOver16(float v) {
-    auto ror = [](float f, auto ctl) __attribute__((always_inline)) {
-        return __uint_as_float(static_cast<uint32_t>(
-            __builtin_amdgcn_mov_dpp(static_cast<int>(__float_as_uint(f)), decltype(ctl)::value, 0xF, 0xF, true)));
-    };
-    v = fmaxf(v, ror(v, std::integral_constant<int, 0x128>{}));  // row_ror:8
-    v = fmaxf(v, ror(v, std::integral_constant<int, 0x124>{}));
-    v = fmaxf(v, ror(v, std::integral_constant<int, 0x122>{}));
-    return fmaxf(v, ror(v, std::integral_constant<int, 0x121>{}));
-}
-
 // Relative cost of a tile of 16, 32 or 64 rows: its weights are the same, but a taller one leaves the ring fewer stages (64
 // tokens evenly over 128 experts, hidden 4096, intermediate 1536: 247 / 251 / 262 us gate/up).  A launch costs its rounds of
 // tiles times that.  What speaks for a taller tile is groups that need several of the lower ones; how many there are is known
@@ -417,8 +405,8 @@ __device__ __forceinline__ void SlimGemmBody(const KernelArgs& a, const SlimGrou
             for (int ks = 0; ks < 2; ++ks) {
                 const int chunk = 4 * ks + quad;
                 if constexpr (!kNz) {
-                    bf[ks][0] = *reinterpret_cast<const v4i*>(B + LdsOffset<128>(bRow0 + l16, chunk));
-                    bf[ks][1] = *reinterpret_cast<const v4i*>(B + LdsOffset<128>(bRow1 + l16, chunk));
+                    bf[ks][0] = *reinterpret_cast<const v4i*>(B + LdsOffset(bRow0 + l16, chunk));
+                    bf[ks][1] = *reinterpret_cast<const v4i*>(B + LdsOffset(bRow1 + l16, chunk));
                 } else {
                     // lane j of a 16-lane group supplies bytes (k = kBase + j / 2, channels 8 * (j % 2) .. + 7) and receives
                     // eight consecutive k of channel j
@@ -434,7 +422,7 @@ __device__ __forceinline__ void SlimGemmBody(const KernelArgs& a, const SlimGrou
                     }
                 }
 #pragma unroll
-                for (int mi = 0; mi < kMi; ++mi) af[ks][mi] = *reinterpret_cast<const v4i*>(A + LdsOffset<128>(16 * mi + l16, chunk));
+                for (int mi = 0; mi < kMi; ++mi) af[ks][mi] = *reinterpret_cast<const v4i*>(A + LdsOffset(16 * mi + l16, chunk));
             }
             // The refill goes out while the fragments are on their way (in front of them, the wave would wait for the address
             // unit first, which takes sixteen clocks per DMA), into the buffer that the step before read.

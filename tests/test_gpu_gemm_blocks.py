@@ -1,0 +1,71 @@
+"""The ring GEMM kernels where their tiles end: row counts around the 16-row blocks and the 256-row tile, channel counts around
+a lane's vector of four and a tile's 256, launches of at most one tile per workgroup and of one more, in the three weight
+layouts and with every output type, against exact integer products (float64) and the epilogue's own fp32 arithmetic."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(w_enk, layout):
+    """(weight view, weight_nz) of K-contiguous int8 storage [E, N, K]."""
+    if layout == "nz":
+        E, N, K = w_enk.shape
+        return None, (w_enk.view(E, N // 32, 32, K // 16, 16).permute(0, 1, 3, 4, 2).contiguous(), "nz5d")
+    view = w_enk.transpose(1, 2)
+    return (view.contiguous() if layout == "nd" else view), None
+
+
+def _run(aclnn, sizes, N, K, layout, out_dtype, seed):
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(seed)
+    E, M = len(sizes), sum(sizes)
+    x = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8)
+    w = torch.randint(-127, 128, (E, N, K), generator=g, dtype=torch.int8)
+    scale = torch.rand((E, N), generator=g) * 0.01 + 1e-3
+    row_scale = torch.rand((M,), generator=g) * 0.05 + 1e-2
+    cumsum = torch.cumsum(torch.tensor(sizes), 0)
+    acc = torch.empty((M, N), dtype=torch.float64)
+    begin = 0
+    for e, n in enumerate(sizes):
+        acc[begin:begin + n] = x[begin:begin + n].double() @ w[e].double().t()
+        begin += n
+    out = torch.full((M, N), 7, dtype=out_dtype, device=dev)
+    view, nz = _weights(w.to(dev), layout)
+    scales = {} if out_dtype == torch.int32 else {"scale": [scale.to(dev)], "per_token_scale": [row_scale.to(dev)]}
+    aclnn.grouped_matmul_v4([x.to(dev)], None if view is None else [view], weight_nz=nz, group_list=cumsum.to(dev), split_item=3,
+                            group_type=0, group_list_type=0, out=[out], **scales)
+    if out_dtype == torch.int32:
+        return out.cpu(), acc.to(torch.int32)
+    group = torch.repeat_interleave(torch.arange(E), torch.tensor(sizes))
+    return out.cpu(), ((acc.float() * scale[group]) * row_scale[:, None]).to(out_dtype)
+
+
+# rows of the groups: around a 16-row block, the 32 rows of a wave-row pair, and the tallest tile
+ROWS = {"blocks": [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65], "tile": [255, 0, 256, 257, 271, 272, 273]}
+
+
+@pytest.mark.parametrize("out_dtype", [torch.int32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", sorted(ROWS))
+@pytest.mark.parametrize("height", [32, 96, 160, 192, 256])
+def test_row_remainders(aclnn, monkeypatch, height, rows, out_dtype):
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", str(height))
+    got, want = _run(aclnn, ROWS[rows], 512, 256, "k", out_dtype, height)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("out_dtype", [torch.int32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout,N", [("k", 4), ("k", 30), ("k", 62), ("k", 66), ("k", 257), ("k", 258), ("k", 260), ("nd", 16),
+                                      ("nd", 144), ("nd", 272), ("nz", 32), ("nz", 96), ("nz", 288)])
+def test_channel_remainders(aclnn, monkeypatch, layout, N, out_dtype):
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", "128")
+    got, want = _run(aclnn, [100, 0, 37, 130], N, 384, layout, out_dtype, N)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("groups,height", [(128, 256), (129, 256), (192, 192)])
+def test_one_round_of_pulled_tiles_and_one_more(aclnn, monkeypatch, groups, height):
+    """Two n-tiles per group: 256 and 258 tiles of 256 rows (256 workgroups), and 384 of 192."""
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", str(height))
+    got, want = _run(aclnn, [80] * groups, 512, 1024, "k", torch.int32, groups)
+    assert torch.equal(got, want)
