@@ -119,6 +119,9 @@ def lib():
         l.opapiCreateTensorPacked.restype = _VP
         l.opapiDestroyTensors.argtypes = [ctypes.c_char_p, ctypes.c_uint64]
         l.opapiDestroyTensors.restype = None
+        l.opapiMoeFfnForward.argtypes = [ctypes.c_char_p, ctypes.c_uint64, _VP, ctypes.c_uint64, _VP, _U64P,
+                                         ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_char_p)]
+        l.opapiMoeFfnForward.restype = ctypes.c_int32
         l.aclCreateTensorList.argtypes = [ctypes.POINTER(_VP), ctypes.c_uint64]
         l.aclCreateTensorList.restype = _VP
         l.aclDestroyTensorList.argtypes = [_VP]
@@ -562,6 +565,37 @@ def moe_finalize_routing_v2(expanded_x, expanded_row_idx, x1=None, x2=None, bias
     finally:
         h.close()
     return out
+
+
+def _packed(t):
+    shape = t.shape
+    n = len(shape)
+    return _PACK[n](n, _DTYPE_CODE[t.dtype], t.data_ptr(), *shape, *t.stride())
+
+
+_FFN_OPERATORS = (("aclnnMoeInitRoutingV2", "aclnnGroupedMatmulSwigluQuant", "aclnnGroupedMatmulV4"),
+                  ("aclnnMoeInitRoutingV3", "aclnnGroupedMatmulSwigluQuant", "aclnnGroupedMatmulV4"))
+
+
+def moe_ffn_forward(routing, tensors, workspace, device):
+    """The operators of one expert FFN pass in one foreign call (include/opapi_moe_ffn.h): routing 2 or 3, then the sixteen
+    tensors in that header's order."""
+    l = lib()
+    packed = struct.pack("q", routing) + b"".join(map(_packed, tensors))
+    sizes = (ctypes.c_uint64 * 5)()
+    enqueued = ctypes.c_int32(0)
+    failed = ctypes.c_char_p(None)
+    for _ in range(2):
+        ws = workspace.tensor
+        st = l.opapiMoeFfnForward(packed, len(packed) // 8, None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+                                  _stream_ptr(), sizes, ctypes.byref(enqueued), ctypes.byref(failed))
+        if st != ACLNN_SUCCESS:
+            raise AclnnError(failed.value.decode(), st, last_error())
+        if enqueued.value:
+            break
+        workspace.reserve(sizes[4], device)
+    for api, nbytes in zip(_FFN_OPERATORS[routing - 2], sizes):
+        workspace.requested[api] = max(workspace.requested.get(api, 0), nbytes)
 
 
 # ------------------------------------------------------------------------------------------------ kernel timing

@@ -36,6 +36,7 @@ SOURCES = [
     "grouped_matmul_v4.hip",
     "grouped_matmul_finalize_routing.hip",
     "moe_finalize_routing_v2.hip",
+    "moe_ffn_forward.hip",
     "calibration_copy.hip",
 ]
 

@@ -29,6 +29,7 @@
 #include "aclnnop/aclnn_moe_init_routing_quant_v2.h"
 #include "aclnnop/aclnn_moe_init_routing_v2.h"
 #include "aclnnop/aclnn_moe_init_routing_v3.h"
+#include "moe_init_routing.h"
 
 namespace {
 
@@ -1032,7 +1033,8 @@ class InitRoutingExecutor : public aclOpExecutor {
     }
 };
 
-// Shared first phase of aclnnMoeInitRoutingV2 (quantMode -1: rows are copied) and aclnnMoeInitRoutingQuantV2
+// Shared first phase of aclnnMoeInitRoutingV2 (quantMode -1: rows are copied, and with them a per-token scale where
+// PlanScaledRoutingV2 passes one as scaleOptional, into dynamicQuantScaleOut) and aclnnMoeInitRoutingQuantV2
 // (quantMode 0: static, 1: dynamic quantisation to INT8; rules of
 // moe/moe_init_routing_quant_v2/op_host/moe_init_routing_quant_v2_tiling.cpp:132-219).
 aclnnStatus PlanRoutingV2(const aclTensor* x, const aclTensor* expertIdx, const aclTensor* scaleOptional,
@@ -1163,6 +1165,15 @@ aclnnStatus PlanRoutingV2(const aclTensor* x, const aclTensor* expertIdx, const 
                     (long long)want);
         OPAPI_CHECK(IsContiguous(dynamicQuantScaleOut) && (total == 0 || dynamicQuantScaleOut->data != nullptr), kInvalid,
                     "dynamicQuantScale must be contiguous device memory");
+    } else if (scaleOptional != nullptr) {
+        OPAPI_CHECK(scaleOptional->dtype == ACL_FLOAT && scaleOptional->dims.size() == 1 && scaleOptional->dims[0] == tokens, kInvalid,
+                    "the per-token scale must be FLOAT [%lld]", (long long)tokens);
+        OPAPI_CHECK(dynamicQuantScaleOut != nullptr, ACLNN_ERR_PARAM_NULLPTR, "the routed scale is nullptr");
+        OPAPI_CHECK(dynamicQuantScaleOut->dtype == ACL_FLOAT && dynamicQuantScaleOut->dims.size() == 1 &&
+                        dynamicQuantScaleOut->dims[0] == activeRows && IsContiguous(dynamicQuantScaleOut),
+                    kInvalid, "the routed scale must be contiguous FLOAT [%lld]", (long long)activeRows);
+        OPAPI_CHECK(total == 0 || (cols > 0 && scaleOptional->data != nullptr && dynamicQuantScaleOut->data != nullptr), kInvalid,
+                    "the per-token scale and the routed scale must be device memory beside rows that have columns");
     }
 
     auto* ex = new (std::nothrow) InitRoutingExecutor();
@@ -1175,6 +1186,9 @@ aclnnStatus PlanRoutingV2(const aclTensor* x, const aclTensor* expertIdx, const 
         OPAPI_BIND(ex, scaleOptional, &ex->scale);
         ex->smoothPerExpert = smoothPerExpert;
         ex->smoothRows = scaleOptional != nullptr ? scaleOptional->dims[0] : 0;
+        ex->expandedScale = reinterpret_cast<float*>(DataPtr(dynamicQuantScaleOut));
+    } else if (scaleOptional != nullptr) {
+        OPAPI_BIND(ex, scaleOptional, &ex->scale);
         ex->expandedScale = reinterpret_cast<float*>(DataPtr(dynamicQuantScaleOut));
     }
     ex->xDtype = x->dtype;
@@ -1202,6 +1216,13 @@ aclnnStatus PlanRoutingV2(const aclTensor* x, const aclTensor* expertIdx, const 
 }
 
 }  // namespace
+
+aclnnStatus opapi::PlanScaledRoutingV2(const aclTensor* x, const aclTensor* expertIdx, const aclTensor* xScale, int64_t expertNum,
+                                       const aclTensor* expandedX, const aclTensor* expandedRowIdx, const aclTensor* cumsum,
+                                       const aclTensor* expandedScale, uint64_t* workspaceSize, aclOpExecutor** executor) {
+    return PlanRoutingV2(x, expertIdx, xScale, nullptr, 0, 0, expertNum, 0, 1, false, /*quantMode=*/-1, expandedX, expandedRowIdx, cumsum,
+                         nullptr, expandedScale, workspaceSize, executor);
+}
 
 extern "C" aclnnStatus aclnnMoeInitRoutingV2GetWorkspaceSize(
     const aclTensor* x, const aclTensor* expertIdx, int64_t activeNum, int64_t expertCapacity, int64_t expertNum,

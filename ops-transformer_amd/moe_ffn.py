@@ -5,8 +5,8 @@
 The reference has no in-repo code that chains them; real callers (torch_npu, vLLM-Ascend) do what ``forward`` does.
 Glue between the operators:
   * activations arrive already quantized per token (int8 rows + fp32 scale); MoeInitRoutingV2 routes the int8 rows
-    (INT8 x is this build's extension: a row gather commutes with per-row quantization bit-exactly) and a second
-    MoeInitRoutingV2 call routes the [T, 1] column of per-token scales the same way;
+    (INT8 x is this build's extension: a row gather commutes with per-row quantization bit-exactly) and copies the
+    per-token scales along with them;
   * routing emits the int32 cumsum (expertTokensCountOrCumsumFlag 1), which both GEMM operators take as groupList (the
     reference wants int64 there; int32 is accepted as an extension, so no cast kernel sits between the operators);
   * MoeFinalizeRoutingV2 is called with dropPadMode 2 because V2's index is the row arrangement
@@ -77,7 +77,6 @@ class MoeFfnW8A8:
         self.expanded_row_idx = torch.empty((M,), dtype=torch.int32, device=dev)
         self.cumsum = torch.empty((E,), dtype=torch.int64 if self.routing == "v3" else torch.int32, device=dev)
         self.expanded_scale = torch.empty((M,), dtype=torch.float32, device=dev)
-        self.row_idx_scratch = torch.empty((M,), dtype=torch.int32, device=dev)
         self.h = torch.empty((M, I), dtype=torch.int8, device=dev)
         self.h_scale = torch.empty((M,), dtype=torch.float32, device=dev)
         self.y = torch.empty((M, H), dtype=self.out_dtype, device=dev)
@@ -90,36 +89,24 @@ class MoeFfnW8A8:
         """xq int8 [T, H]; x_scale fp32 [T]; topk_idx int32 [T, K]; topk_weight fp32/bf16 [T, K] -> out [T, H]."""
         T, K = topk_idx.shape
         self._buffers(T, K)
-        E = self.num_experts
-        if self.routing == "v3":
-            aclnn.moe_init_routing_v3(xq, topk_idx, x_scale, expert_num=E, expert_tokens_num_type=0, quant_mode=-1,
-                                      row_idx_type=0 if self.fused_combine else 1,
-                                      out=(self.expanded_x, self.expanded_row_idx, self.cumsum, self.expanded_scale),
-                                      workspace=self.workspace)
-        else:
-            aclnn.moe_init_routing_v2(xq, topk_idx, 0, 0, E, 0, 1, False,
-                                      out=(self.expanded_x, self.expanded_row_idx, self.cumsum, None),
-                                      workspace=self.workspace)
-            aclnn.moe_init_routing_v2(x_scale.view(T, 1), topk_idx, 0, 0, E, 0, 0, False,
-                                      out=(self.expanded_scale.view(T * K, 1), self.row_idx_scratch, None, None),
-                                      workspace=self.workspace)
-        aclnn.grouped_matmul_swiglu_quant(self.expanded_x, None if self.w13_nz is not None else self.w13_view, self.cumsum,
-                                          self.w13_scale, self.expanded_scale, out=(self.h, self.h_scale),
-                                          weight_nz=None if self.w13_nz is None else (self.w13_nz, "nz5d"),
-                                          workspace=self.workspace)
-        if self.fused_combine:
-            source = self.expanded_row_idx.long()                       # expanded row -> flat (token, k) position
-            logit = topk_weight.reshape(-1).float()[source]
-            aclnn.grouped_matmul_finalize_routing(self.h, self.w2_view, self.w2_scale, source // K, T, self.cumsum,
-                                                  group_list_type=0, per_token_scale=self.h_scale, logit=logit,
-                                                  out=self.out, workspace=self.workspace)
+        if not self.fused_combine:
+            aclnn.moe_ffn_forward(3 if self.routing == "v3" else 2,
+                                  (xq, x_scale if self.routing == "v3" else x_scale.view(T), topk_idx, topk_weight,
+                                   self.w13_view if self.w13_nz is None else self.w13_nz, self.w13_scale,
+                                   self.w2_view if self.w2_nz is None else self.w2_nz, self.w2_scale,
+                                   self.expanded_x, self.expanded_row_idx, self.cumsum, self.expanded_scale,
+                                   self.h, self.h_scale, self.y, self.out), self.workspace, self.device)
             return self.out
-        aclnn.grouped_matmul_v4([self.h], None if self.w2_nz is not None else [self.w2_view],
-                                weight_nz=None if self.w2_nz is None else (self.w2_nz, "nz5d"),
-                                scale=[self.w2_scale], per_token_scale=[self.h_scale],
-                                group_list=self.cumsum, split_item=3, group_type=0, group_list_type=0, act_type=0,
-                                out=[self.y], workspace=self.workspace)
-        aclnn.moe_finalize_routing_v2(self.y, self.expanded_row_idx, scales=topk_weight, drop_pad_mode=2, out=self.out)
+        aclnn.moe_init_routing_v3(xq, topk_idx, x_scale, expert_num=self.num_experts, expert_tokens_num_type=0, quant_mode=-1,
+                                  row_idx_type=0, out=(self.expanded_x, self.expanded_row_idx, self.cumsum, self.expanded_scale),
+                                  workspace=self.workspace)
+        aclnn.grouped_matmul_swiglu_quant(self.expanded_x, self.w13_view, self.cumsum, self.w13_scale, self.expanded_scale,
+                                          out=(self.h, self.h_scale), workspace=self.workspace)
+        source = self.expanded_row_idx.long()                       # expanded row -> flat (token, k) position
+        logit = topk_weight.reshape(-1).float()[source]
+        aclnn.grouped_matmul_finalize_routing(self.h, self.w2_view, self.w2_scale, source // K, T, self.cumsum,
+                                              group_list_type=0, per_token_scale=self.h_scale, logit=logit,
+                                              out=self.out, workspace=self.workspace)
         return self.out
 
     def capture(self, xq, x_scale, topk_idx, topk_weight):

@@ -1,0 +1,84 @@
+"""The one-call expert FFN (opapiMoeFfnForward, what MoeFfnW8A8.forward runs): what it refuses, on the CPU, and on the GPU that
+its results are those of the four operators called one by one."""
+import ctypes
+import struct
+
+import pytest
+import torch
+
+
+def _call(aclnn, data, workspace=None, nbytes=0):
+    sizes = (ctypes.c_uint64 * 5)()
+    enqueued, failed = ctypes.c_int32(-1), ctypes.c_char_p(None)
+    st = aclnn.lib().opapiMoeFfnForward(data, len(data) // 8, workspace, nbytes, None, sizes, ctypes.byref(enqueued), ctypes.byref(failed))
+    return st, list(sizes), enqueued.value, (failed.value or b"").decode()
+
+
+def _tensors(T, H, I, E, K, v3=False, dev="cpu"):
+    M = T * K
+    i8 = lambda *s: torch.zeros(s, dtype=torch.int8, device=dev)
+    f = lambda *s: torch.zeros(s, device=dev)
+    return [i8(T, H), f(T), torch.zeros((T, K), dtype=torch.int32, device=dev), f(T, K), i8(E, 2 * I, H).transpose(1, 2), f(E, 2 * I),
+            i8(E, H, I).transpose(1, 2), f(E, H), i8(M, H), torch.zeros(M, dtype=torch.int32, device=dev),
+            torch.zeros(E, dtype=torch.int64 if v3 else torch.int32, device=dev), f(M), i8(M, I), f(M),
+            torch.zeros((M, H), dtype=torch.bfloat16, device=dev), torch.zeros((T, H), dtype=torch.bfloat16, device=dev)]
+
+
+def _pack(aclnn, routing, tensors):
+    return struct.pack("q", routing) + b"".join(aclnn._packed(t) for t in tensors)
+
+
+@pytest.mark.parametrize("routing", [2, 3])
+def test_too_small_a_workspace_enqueues_nothing(aclnn, routing):
+    st, sizes, enqueued, _ = _call(aclnn, _pack(aclnn, routing, _tensors(4, 128, 64, 4, 2, routing == 3)))
+    assert st == 0 and enqueued == 0
+    assert sizes[0] > 0 and sizes[1] > 0 and sizes[4] == max(sizes[:4])
+
+
+def test_malformed_arrays_are_refused(aclnn):
+    good = _pack(aclnn, 2, _tensors(4, 128, 64, 4, 2))
+    bad_rank = bytearray(good)
+    bad_rank[8:16] = struct.pack("q", 9)
+    negative_rank = bytearray(good)
+    negative_rank[8:16] = struct.pack("q", -1)
+    for data in (b"", struct.pack("q", 2), good[:-8], good + b"\0" * 8, struct.pack("q", 1) + good[8:], bytes(bad_rank), bytes(negative_rank)):
+        st, _, enqueued, name = _call(aclnn, data)
+        assert st == aclnn.ACLNN_ERR_PARAM_INVALID and enqueued == 0 and name == "opapiMoeFfnForward"
+    assert _call(aclnn, good)[0] == 0
+
+
+@pytest.mark.parametrize("which,replacement,operator", [
+    (0, torch.zeros((5, 128), dtype=torch.int8), "aclnnMoeInitRoutingV2GetWorkspaceSize"),
+    (1, torch.zeros(4, dtype=torch.float16), "aclnnMoeInitRoutingV2GetWorkspaceSize"),
+    (1, torch.zeros(5), "aclnnMoeInitRoutingV2GetWorkspaceSize"),
+    (11, torch.zeros(7), "aclnnMoeInitRoutingV2GetWorkspaceSize"),
+    (5, torch.zeros((4, 64)), "aclnnGroupedMatmulSwigluQuantGetWorkspaceSize"),
+    (14, torch.zeros((8, 64), dtype=torch.bfloat16), "aclnnGroupedMatmulV4GetWorkspaceSize"),
+    (15, torch.zeros((4, 64), dtype=torch.bfloat16), "aclnnMoeFinalizeRoutingV2GetWorkspaceSize")])
+def test_each_operator_still_checks_its_tensors(aclnn, which, replacement, operator):
+    tensors = _tensors(4, 128, 64, 4, 2)
+    tensors[which] = replacement
+    st, _, enqueued, name = _call(aclnn, _pack(aclnn, 2, tensors))
+    assert st != 0 and enqueued == 0 and name == operator and aclnn.last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("routing", ["v2", "v3"])
+@pytest.mark.parametrize("tokens", [1, 3, 257, 1300])
+def test_equals_the_operators_one_by_one(pkg, aclnn, dev, tokens, routing):
+    H, I, E, K = 256, 128, 8, 3
+    g = torch.Generator(device=dev).manual_seed(tokens)
+    i8 = lambda *s: torch.empty(s, dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    f = lambda *s: torch.rand(s, device=dev, generator=g) * 0.01 + 1e-3
+    w13, w2, w13s, w2s, xq = i8(E, 2 * I, H), i8(E, H, I), f(E, 2 * I), f(E, H), i8(tokens, H)
+    xs = f(tokens, 2)[:, 1] if routing == "v2" else f(tokens)  # a strided column of scales
+    idx = torch.rand((tokens, E), device=dev, generator=g).topk(K, dim=1)[1].int()
+    wgt = f(tokens, K)
+    got = pkg.MoeFfnW8A8(w13, w13s, w2, w2s, routing=routing).forward(xq, xs, idx, wgt)
+    ex, row_idx, cumsum, _ = aclnn.moe_init_routing_v2(xq, idx, 0, 0, E, 0, 1, False)
+    es, _, _, _ = aclnn.moe_init_routing_v2(xs.contiguous().view(tokens, 1), idx, 0, 0, E, 0, 0, False)
+    h, hs = aclnn.grouped_matmul_swiglu_quant(ex, w13.transpose(1, 2), cumsum, w13s, es.view(-1))
+    y = aclnn.grouped_matmul_v4([h], [w2.transpose(1, 2)], scale=[w2s], per_token_scale=[hs], group_list=cumsum, split_item=3,
+                                group_type=0, group_list_type=0, output_dtype=torch.bfloat16)[0]
+    want = aclnn.moe_finalize_routing_v2(y, row_idx, scales=wgt, drop_pad_mode=2)
+    assert torch.equal(got, want)
