@@ -65,6 +65,7 @@ constexpr int64_t kSlimMaxTilesN = 16384;
 struct Plan {
     int tileM = 0;          // rows per workgroup tile (multiple of 32; slim: 16, 32 or 64, the lowest that the kernel may take)
     int lowTileM = 0;       // a lower height that the scheduling kernel may choose instead (0: none)
+    bool lowForRounds = false;  // it chooses by rounds of the machine, else by the rows that groups leave over
     int64_t maxTiles = 0;   // launch bound on workgroups
     int32_t maxMTiles = 0;  // upper bound on m-tiles over all groups (M / tileM + groups)
     int32_t tilesN = 0;

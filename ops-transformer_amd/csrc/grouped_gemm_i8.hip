@@ -48,7 +48,9 @@ struct SchedArgs {
     int32_t groupListIsInt64;
     int32_t isCount;  // 0 cumsum, 1 counts, 2 sparse (expert id, count) pairs
     int32_t tileM;
-    int32_t mayLower;  // 1: m-tiles of kLowTileM rows instead where they leave at most an eighth of the groups a small last one
+    int32_t mayLower;  // 1: m-tiles of kLowTileM rows instead where they leave at most an eighth of the groups a small last one;
+                       // 2: where they fill at most two rounds of the machine, and no more of them than the tall ones
+    int32_t cus, tilesN;
     int32_t maxMTiles;
     int64_t M;
     int64_t rowBegin, rowEnd;  // only rows in [rowBegin, rowEnd) get tiles (one band of a launch that runs in row bands)
@@ -61,7 +63,9 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
         return a.groupListIsInt64 ? static_cast<const int64_t*>(a.groupList)[i]
                                   : static_cast<int64_t>(static_cast<const int32_t*>(a.groupList)[i]);
     };
-    // inclusive prefix sum over the 1024 threads: shuffles inside each wave, then the sixteen wave totals through LDS
+    // Inclusive prefix sums over the 1024 threads: shuffles inside each wave, then the sixteen wave totals through LDS, all of
+    // which every thread reads (one round trip; a loop over the waves before it was fifteen).  Each is called once at most, so that
+    // nobody waits for earlier totals to have been read.
     __shared__ int32_t waveTotal[16];
     auto inclusiveScan = [&](int32_t v) -> int32_t {
         const int lane = t & 63, wave = t >> 6;
@@ -70,28 +74,34 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
             const int32_t below = __shfl_up(v, d, 64);
             if (lane >= d) v += below;
         }
-        __syncthreads();  // the totals of an earlier call have been read
         if (lane == 63) waveTotal[wave] = v;
         __syncthreads();
-        int32_t base = 0;
-        for (int i = 0; i < wave; ++i) base += waveTotal[i];
-        return v + base;
+#pragma unroll
+        for (int i = 0; i < 15; ++i) v += i < wave ? waveTotal[i] : 0;
+        return v;
     };
-    // the same over two 32-bit counts packed into one 64-bit value (neither half may overflow into the other)
-    __shared__ uint64_t waveTotal64[16];
-    auto inclusiveScan64 = [&](uint64_t v) -> uint64_t {
+    // the same over two values of two 32-bit counts each, packed into 64 bits (neither half may overflow into the other)
+    __shared__ uint64_t waveTotal64[2][16];
+    auto inclusiveScan64 = [&](uint64_t& v, uint64_t& w) {
         const int lane = t & 63, wave = t >> 6;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
-            const uint64_t below = __shfl_up(v, d, 64);
-            if (lane >= d) v += below;
+            const uint64_t belowV = __shfl_up(v, d, 64), belowW = __shfl_up(w, d, 64);
+            if (lane >= d) {
+                v += belowV;
+                w += belowW;
+            }
+        }
+        if (lane == 63) {
+            waveTotal64[0][wave] = v;
+            waveTotal64[1][wave] = w;
         }
         __syncthreads();
-        if (lane == 63) waveTotal64[wave] = v;
-        __syncthreads();
-        uint64_t base = 0;
-        for (int i = 0; i < wave; ++i) base += waveTotal64[i];
-        return v + base;
+#pragma unroll
+        for (int i = 0; i < 15; ++i) {
+            v += i < wave ? waveTotal64[0][i] : 0;
+            w += i < wave ? waveTotal64[1][i] : 0;
+        }
     };
     // group boundaries, clamped into [0, M], no end before its begin, so that a malformed list cannot push rows out of range
     int64_t begin = 0, end = 0;
@@ -146,27 +156,59 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
     begin = begin < a.rowBegin ? a.rowBegin : (begin > a.rowEnd ? a.rowEnd : begin);
     end = end < a.rowBegin ? a.rowBegin : (end > a.rowEnd ? a.rowEnd : end);
     const int32_t rows = t < a.groups ? static_cast<int32_t>(end - begin) : 0;
-    int32_t tileM = a.tileM;
-    if (a.mayLower) {
+    int32_t tileM = a.tileM, cut = tileM;  // cut: rows per m-tile of this group
+    if (a.mayLower == 2) {
+        // Whole rounds of the machine, one of low tiles costing 0.7 to 0.85 of one of tall ones: their ring is a stage deeper, and
+        // the launch ends with its tallest tile.  Low tiles where they are one round; where they are two, only if the tall ones
+        // are two as well, not counting what runs as small tiles.  us, planned height -> this, K-contiguous / row-major:
+        //   8 experts, K 14336 x N 4096: 180 rows each 157 -> 134 / 164 -> 141, 250 rows 176 -> 143 / 176 -> 154, 600 rows 326 -> 274 / 330 -> 293
+        //   8 experts, 1024 x 1024 and gate/up 1024 x 2 x 1024: 250 rows 31 -> 27 and 34 -> 30
+        //   two rounds for one and a few small tiles, left alone: 16 experts, K 8192 x N 1024, 1000 rows 149 (154 low)
+        const uint32_t low = (rows + kLowTileM - 1) / kLowTileM, tall = (rows + tileM - 1 - kSmallRows) / tileM;
+        __shared__ uint32_t sLow, sTall;
+        if (t == 0) sLow = sTall = 0;
+        __syncthreads();
+        if ((t & ~63) < a.groups) {  // the sums of a wave by shuffles: atomics of 64 lanes are a loop of 64 trips each
+            uint32_t lowSum = low, tallSum = tall;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                lowSum += __shfl_xor(lowSum, d, 64);
+                tallSum += __shfl_xor(tallSum, d, 64);
+            }
+            if ((t & 63) == 0) {
+                atomicAdd(&sLow, lowSum);
+                atomicAdd(&sTall, tallSum);
+            }
+        }
+        __syncthreads();
+        // (neither product overflows: a launch with this choice has at most two rounds of M / kLowTileM rows)
+        const uint32_t cus = a.cus, lowTiles = sLow * a.tilesN;
+        if (lowTiles <= cus || (lowTiles <= 2 * cus && sTall * a.tilesN > cus)) {
+            tileM = kLowTileM;
+            // the group's m-tiles are alike: 160 + 20 rows would read the weights twice, at two paces
+            cut = low > 0 ? static_cast<int32_t>(((rows + low - 1) / low + 15) & ~15u) : kLowTileM;
+        }
+    } else if (a.mayLower) {
         const int32_t last = rows % kLowTileM;
-        if (__syncthreads_count(last > 0 && last <= kSmallRows) * 8 <= a.groups) tileM = kLowTileM;
+        if (__syncthreads_count(last > 0 && last <= kSmallRows) * 8 <= a.groups) tileM = cut = kLowTileM;
     }
-    const int32_t tiles = (rows + tileM - 1) / tileM;
+    const int32_t tiles = (rows + cut - 1) / cut;
     // big and small m-tiles of this group (with tiles of at most kSmallRows rows every m-tile is small; otherwise only
     // a group's last, partly filled m-tile can be) and the cost of the big ones; two packed prefix sums give every
     // group the positions of its m-tiles in the two runs of the table, and the launch the totals
     const bool allSmall = tileM <= kSmallRows;
-    const int32_t lastRows = tiles > 0 ? rows - (tiles - 1) * tileM : 0;
+    const int32_t lastRows = tiles > 0 ? rows - (tiles - 1) * cut : 0;
     const int32_t smallCount = allSmall ? tiles : (tiles > 0 && lastRows <= kSmallRows ? 1 : 0);
     const int32_t bigCount = tiles - smallCount;
     int32_t bigCost = 0;
     if (bigCount > 0) {
         const bool lastIsBig = smallCount == 0;
         const int32_t lastSub = (lastRows + 31) >> 5;
-        bigCost = (bigCount - (lastIsBig ? 1 : 0)) * max(tileM >> 5, kSmallCost) + (lastIsBig ? max(lastSub, kSmallCost) : 0);
+        bigCost = (bigCount - (lastIsBig ? 1 : 0)) * max(cut >> 5, kSmallCost) + (lastIsBig ? max(lastSub, kSmallCost) : 0);
     }
-    const uint64_t countsInc = inclusiveScan64(static_cast<uint64_t>(tiles) | (static_cast<uint64_t>(bigCount) << 32));
-    const uint64_t costInc = inclusiveScan64(static_cast<uint64_t>(bigCost) | (static_cast<uint64_t>(tiles > 0 ? 1 : 0) << 32));
+    uint64_t countsInc = static_cast<uint64_t>(tiles) | (static_cast<uint64_t>(bigCount) << 32);
+    uint64_t costInc = static_cast<uint64_t>(bigCost) | (static_cast<uint64_t>(tiles > 0 ? 1 : 0) << 32);
+    inclusiveScan64(countsInc, costInc);
     const int32_t tileInc = static_cast<int32_t>(countsInc & 0xffffffffu), bigInc = static_cast<int32_t>(countsInc >> 32);
     // rows covered by the list: the end of the last group, or with a sparse list the furthest end of any expert
     int32_t covered = static_cast<int32_t>(end);
@@ -180,10 +222,11 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
         covered = scan[0];
         __syncthreads();
     }
-    __shared__ int32_t sRowStart[kMaxGroups], sRows[kMaxGroups], sBigBefore[kMaxGroups], sSmallBefore[kMaxGroups];
+    __shared__ int32_t sRowStart[kMaxGroups], sRows[kMaxGroups], sCut[kMaxGroups], sBigBefore[kMaxGroups], sSmallBefore[kMaxGroups];
     __shared__ int32_t totals[4];
     sRowStart[t] = static_cast<int32_t>(begin);
     sRows[t] = rows;
+    sCut[t] = cut;
     sBigBefore[t] = bigInc - bigCount;
     sSmallBefore[t] = (tileInc - bigInc) - smallCount;
     __shared__ int32_t sCovered;
@@ -221,11 +264,11 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
             if (scan[mid] > m) hi = mid; else lo = mid;
         }
         const int32_t inGroup = m - (hi > 0 ? scan[hi - 1] : 0);
-        const int32_t tileRows = min(tileM, sRows[hi] - inGroup * tileM);
+        const int32_t tileRows = min(sCut[hi], sRows[hi] - inGroup * sCut[hi]);
         const bool small = allSmall || tileRows <= kSmallRows;
         const int32_t pos = small ? nBig + sSmallBefore[hi] + (allSmall ? inGroup : 0) : sBigBefore[hi] + inGroup;
         const int32_t limit = small ? nBig + nSmall : nBig;
-        if (pos < limit) mTileTable[pos] = make_int4(hi, sRowStart[hi] + inGroup * tileM, tileRows, 0);
+        if (pos < limit) mTileTable[pos] = make_int4(hi, sRowStart[hi] + inGroup * sCut[hi], tileRows, 0);
     }
 }
 
@@ -485,6 +528,13 @@ Plan MakePlan(const Problem& p) {
         plan.pullTiles = StreamOk(p) && kSteps >= 8 && plan.maxTiles < (1ll << 31) && std::atoi(env) != 0;
     }
     if (lowHolds && plan.tileM == 192 && plan.pullTiles && std::getenv("OPAPI_GEMM_TILE_M") == nullptr) plan.lowTileM = kLowTileM;
+    // Launches of at most two rounds of low tiles: the scheduling kernel decides, where it knows the groups (its figures are
+    // there).  Asked and answered with the tall ones, it takes 0.5 us longer.
+    if (plan.pullTiles && plan.tileM > kLowTileM && plan.lowTileM == 0 && std::getenv("OPAPI_GEMM_TILE_M") == nullptr &&
+        (p.M + kLowTileM - 1) / kLowTileM * plan.tilesN <= 2ll * DeviceCuCount()) {
+        plan.lowTileM = kLowTileM;
+        plan.lowForRounds = true;
+    }
     const int64_t maxMTiles = p.M / (plan.lowTileM > 0 ? plan.lowTileM : plan.tileM) + groups;
     plan.maxMTiles = static_cast<int32_t>(maxMTiles);
     // round up so that every XCD's share [xcd * ceil(total/8), ...) is covered by the launch
@@ -530,7 +580,9 @@ hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStrea
     sa.groupListIsInt64 = p.groupListIsInt64 ? 1 : 0;
     sa.isCount = static_cast<int32_t>(p.groupListKind);
     sa.tileM = plan.tileM;
-    sa.mayLower = plan.lowTileM > 0 ? 1 : 0;
+    sa.mayLower = plan.lowForRounds ? 2 : plan.lowTileM > 0 ? 1 : 0;
+    sa.cus = DeviceCuCount();
+    sa.tilesN = plan.tilesN;
     sa.maxMTiles = plan.maxMTiles;
     sa.M = p.M;
 

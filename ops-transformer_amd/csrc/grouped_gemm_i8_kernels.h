@@ -122,7 +122,7 @@ constexpr int kQueueHeaderInts = 32;
 constexpr int kQueueCounterInts = 32;
 constexpr int kHdrCoveredRows = 6;
 constexpr int kHdrTileM = 7;
-// A height that the scheduling kernel may choose instead of 192 rows (Plan::lowTileM).
+// A height that the scheduling kernel may choose instead of 192 or 256 rows (Plan::lowTileM).
 constexpr int kLowTileM = 160;
 __host__ __device__ inline int SchedTotalInts(int maxMTiles) { return kQueueHeaderInts + kQueueCounterInts + 4 * maxMTiles; }
 
@@ -1223,21 +1223,17 @@ __global__ __launch_bounds__(kThreads) void StreamGemmKernel(KernelArgs a, const
 // of each XCD's workgroups that its cost is of the whole) until that run's counters are used up on every XCD, lets its
 // ring drain, and serves the other; a launch without small m-tiles costs the workgroups that looked for them one draw.
 //
-// kHasLow: the scheduling kernel may have cut the groups into m-tiles of kLowTileM rows instead; these run in one geometry.
-template <int kRows, Epilogue kEpi>
-constexpr bool kHasLow = kRows == 192 && kEpi != Epilogue::kSwiglu;
+// The scheduling kernel may have cut the groups into m-tiles of at most kLowTileM rows instead; these run in one geometry.
 
 template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
 __global__ __launch_bounds__(kThreads) void MixedGemmKernel(KernelArgs a, const int32_t* __restrict__ sched) {
     extern __shared__ __attribute__((aligned(128))) char lds[];
     const uint64_t spanStart = a.wgSpans != nullptr ? __builtin_amdgcn_s_memrealtime() : 0;
     uint64_t spanTiles = 0;
-    if constexpr (kHasLow<kRows, kEpi>) {
-        if (sched[kHdrTileM] == kLowTileM) {
-            StreamGemmBody<kLowTileM, kEpi, kNz, kNMajor, kBothRuns, kTail>(a, sched, lds, spanTiles);
-            WriteSpan(a, spanStart, spanTiles);
-            return;
-        }
+    if (sched[kHdrTileM] == kLowTileM) {
+        StreamGemmBody<kLowTileM, kEpi, kNz, kNMajor, kBothRuns, kTail>(a, sched, lds, spanTiles);
+        WriteSpan(a, spanStart, spanTiles);
+        return;
     }
     const int64_t costSmall = sched[2], costAll = costSmall + sched[3];
     const int32_t slots = gridDim.x / kXcds, slot = blockIdx.x / kXcds;
@@ -1369,8 +1365,7 @@ hipError_t LaunchStream(const KernelArgs& args, const int32_t* sched, int64_t ma
 
 template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
 hipError_t LaunchMixed(const KernelArgs& args, const int32_t* sched, int64_t maxTiles, hipStream_t stream) {
-    constexpr int kLdsBytes = std::max({StreamCfg<kRows>::kLdsBytes, StreamCfg<kSmallRows>::kLdsBytes,
-                                        kHasLow<kRows, kEpi> ? StreamCfg<kLowTileM>::kLdsBytes : 0});
+    constexpr int kLdsBytes = std::max({StreamCfg<kRows>::kLdsBytes, StreamCfg<kSmallRows>::kLdsBytes, StreamCfg<kLowTileM>::kLdsBytes});
     auto kernel = MixedGemmKernel<kRows, kEpi, kNz, kNMajor, kTail>;
     static std::atomic<uint64_t> optedIn{0};
     const hipError_t attr = opapi::EnsureDynamicLds(reinterpret_cast<const void*>(kernel), kLdsBytes, optedIn);

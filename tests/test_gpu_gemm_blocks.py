@@ -69,3 +69,40 @@ def test_one_round_of_pulled_tiles_and_one_more(aclnn, monkeypatch, groups, heig
     monkeypatch.setenv("OPAPI_GEMM_TILE_M", str(height))
     got, want = _run(aclnn, [80] * groups, 512, 1024, "k", torch.int32, groups)
     assert torch.equal(got, want)
+
+
+# Launches of few tiles, which the scheduling kernel may cut lower than planned, and each group evenly: groups around one and two low
+# tiles, around a short even tile and one of ten (ten even tiles of 1441 rows are nine rows short of the tenth), idle groups, and
+# (four of 250 rows beside 64 n-tiles: two rounds instead of one) a launch that stays as it is
+FEW = {"even": ([250] * 8, 1024), "uneven": ([161, 0, 320, 321, 64, 65, 160, 1], 1024), "many": ([1441, 1760, 7], 512), "tall": ([250] * 4, 16384)}
+
+
+@pytest.mark.parametrize("layout,K", [("k", 1024), ("k", 1040), ("nd", 1024), ("nz", 1040)])
+@pytest.mark.parametrize("name", sorted(FEW))
+def test_few_tiles(aclnn, monkeypatch, name, layout, K):
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    sizes, N = FEW[name]
+    got, want = _run(aclnn, sizes, N, K, layout, torch.bfloat16, K)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("layout", ["k", "nd"])
+@pytest.mark.parametrize("name", sorted(FEW))
+def test_few_tiles_swiglu_equals_a_forced_height(aclnn, dev, monkeypatch, name, layout):
+    """S and its row maximum do not depend on how the rows are cut into tiles."""
+    sizes, N = FEW[name]
+    K, E, M = 1024, len(sizes), sum(sizes)
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.empty((M, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    w = torch.empty((E, N, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g).transpose(1, 2)
+    w = w.contiguous() if layout == "nd" else w
+    scale, x_scale = torch.rand((E, N), device=dev, generator=g) * 1e-3, torch.rand((M,), device=dev, generator=g) * 1e-2
+    cumsum = torch.cumsum(torch.tensor(sizes), 0).to(dev)
+    results = []
+    for height in (None, "256"):
+        monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+        if height is not None:
+            monkeypatch.setenv("OPAPI_GEMM_TILE_M", height)
+        results.append(aclnn.grouped_matmul_swiglu_quant(x, w, cumsum, scale, x_scale))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    assert results[0][0].any()
