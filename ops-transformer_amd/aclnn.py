@@ -594,6 +594,8 @@ def moe_ffn_forward(routing, tensors, workspace, device):
         if enqueued.value:
             break
         workspace.reserve(sizes[4], device)
+    else:  # the outputs still hold whatever an earlier pass left in them
+        raise AclnnError("opapiMoeFfnForward", ACLNN_ERR_RUNTIME_ERROR, "nothing was enqueued: %d bytes of workspace are needed" % sizes[4])
     for api, nbytes in zip(_FFN_OPERATORS[routing - 2], sizes):
         workspace.requested[api] = max(workspace.requested.get(api, 0), nbytes)
 

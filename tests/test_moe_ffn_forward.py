@@ -35,6 +35,17 @@ def test_too_small_a_workspace_enqueues_nothing(aclnn, routing):
     assert sizes[0] > 0 and sizes[1] > 0 and sizes[4] == max(sizes[:4])
 
 
+@pytest.mark.parametrize("routing", [2, 3])
+def test_a_pass_that_was_not_enqueued_is_an_error(aclnn, monkeypatch, routing):
+    """The outputs are reused from pass to pass: returning without having enqueued one would hand out the last one's."""
+    class NeverGrows(aclnn.Workspace):
+        def reserve(self, nbytes, device, api=None):
+            return None
+    monkeypatch.setattr(aclnn, "_stream_ptr", lambda: None)
+    with pytest.raises(aclnn.AclnnError, match="workspace"):
+        aclnn.moe_ffn_forward(routing, _tensors(4, 128, 64, 4, 2, routing == 3), NeverGrows(), "cpu")
+
+
 def test_malformed_arrays_are_refused(aclnn):
     good = _pack(aclnn, 2, _tensors(4, 128, 64, 4, 2))
     bad_rank = bytearray(good)
