@@ -142,6 +142,39 @@ def check_ring_kernel_codegen(asm_path):
     return checked
 
 
+def check_ring_barrier_waits(asm_path):
+    """Third build-time guard: a barrier among a ring kernel's matrix instructions frees LDS buffers for DMAs that the compiler does
+    not see, so the wave's reads of them have to have been waited for.  In the device assembly of StreamGemmKernel and
+    MixedGemmKernel, going back from every s_barrier inside a basic block that multiplies, a wait for LDS (lgkmcnt of at most four:
+    the reads of the rows' second half, which the barrier does not free) has to come before any LDS read.
+    Returns the number of barriers checked."""
+    checked = 0
+    for body in open(asm_path).read().split("; -- Begin function ")[1:]:
+        name = body.split()[0]
+        if not any(ring in name for ring in ("StreamGemmKernel", "MixedGemmKernel")):
+            continue
+        block = []
+        for l in body.split("; -- End function")[0].splitlines() + ["end:"]:
+            l = l.split(";")[0].strip()
+            if l.endswith(":") or l.startswith("s_cbranch"):  # a basic block ends
+                multiplies = any(i.startswith("v_mfma") for i in block)
+                for at in [i for i, ins in enumerate(block) if multiplies and ins.startswith("s_barrier")]:
+                    settled = False
+                    for ins in reversed(block[:at]):
+                        if ins.startswith("s_waitcnt") and "lgkmcnt(" in ins and int(ins.split("lgkmcnt(")[1].split(")")[0]) <= 4:
+                            settled = True
+                            break
+                        if ins.startswith("ds_read"):
+                            break
+                    if not settled:
+                        raise RuntimeError("%s: %s: a barrier frees LDS buffers whose reads have not been waited for" % (asm_path, name))
+                    checked += 1
+                block = []
+            elif l and not l.startswith("."):
+                block.append(l)
+    return checked
+
+
 def _headers():
     out = []
     for base in (CSRC, os.path.join(ROOT, "include")):
@@ -181,6 +214,8 @@ def _compile(src, force):
         try:
             check_lds_dma_assembly(stem + "-hip-amdgcn-amd-amdhsa-gfx950.s")
             check_ring_kernel_codegen(stem + "-hip-amdgcn-amd-amdhsa-gfx950.s")
+            if "slim" not in src and check_ring_barrier_waits(stem + "-hip-amdgcn-amd-amdhsa-gfx950.s") == 0:
+                raise RuntimeError("%s: no barrier found among the matrix instructions" % src)
         except Exception:
             os.remove(obj)  # never leave an object behind that the guard refused
             raise

@@ -737,8 +737,13 @@ __device__ __forceinline__ void WaitVmcnt() {  // s_waitcnt vmcnt(kCount), leavi
     __builtin_amdgcn_s_waitcnt(0x0f70 | (kCount & 15) | ((kCount >> 4) << 14));
 }
 
-// This wave's LDS reads and writes have been carried out (s_waitcnt lgkmcnt(0) alone).
-__device__ __forceinline__ void WaitLds() { __builtin_amdgcn_s_waitcnt(0xc07f); }
+// This wave's LDS reads and writes have been carried out, all but the youngest kPending (they are carried out in order;
+// s_waitcnt lgkmcnt(kPending) alone).
+template <int kPending = 0>
+__device__ __forceinline__ void WaitLds() {
+    static_assert(kPending < 16, "lgkmcnt is a 4-bit counter");
+    __builtin_amdgcn_s_waitcnt(0xc07f | (kPending << 8));
+}
 
 // The workgroup's barrier, and nothing crosses it in the compiler's order.  Unlike __syncthreads() it waits for no memory
 // request: what has to have landed in front of it is waited for by count.
@@ -1124,7 +1129,12 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                 __builtin_amdgcn_sched_barrier(0);
                 maskB(1, last);
                 multiply(FirstHalf{}, 1, false);
-                PhaseBarrier();  // this wave's reads of weights and first half have returned: the products above used them
+                // This wave's reads of weights and first half have returned: the products above used them, so the compiler has
+                // waited for them already.  But nothing orders those register instructions against the barrier, behind which DMAs
+                // that the compiler does not see overwrite what was read.  The kMy1 reads of the second half may be outstanding.
+                __builtin_amdgcn_sched_barrier(0);
+                WaitLds<kMy1>();
+                PhaseBarrier();
                 readA(af[1], ringA, SecondHalf{}, 1);
                 __builtin_amdgcn_sched_barrier(0);
                 multiply(SecondHalf{}, 0, true, 0);

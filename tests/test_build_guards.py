@@ -1,6 +1,7 @@
 """The build-time guards of ops-transformer_amd/build.py around the LDS-DMA kernels: the compiler pin, the check that, in
 the device assembly, m0 is written only as the first half of an (s_mov_b32 m0, global_load_lds_dwordx4) pair, and the
-check of the generated code for scratch use, generic memory instructions and merged multiply-convert instructions."""
+check of the generated code for scratch use, generic memory instructions and merged multiply-convert instructions, and the
+check that a barrier among matrix instructions comes behind a wait for the LDS reads of what it frees."""
 import importlib.util
 import os
 
@@ -93,3 +94,41 @@ def test_codegen_guard_refuses(build, tmp_path, bad):
     assert bad != CODEGEN_GOOD
     with pytest.raises(RuntimeError):
         build.check_ring_kernel_codegen(_write(tmp_path, bad))
+
+
+BARRIER_GOOD = """
+; -- Begin function _ZN4gemm16StreamGemmKernelILi96EEEvv
+_ZN4gemm16StreamGemmKernelILi96EEEvv:
+	s_barrier
+.LBB0_1:
+	ds_read_b128 v[0:3], v9
+	s_waitcnt lgkmcnt(0)
+	v_mfma_i32_16x16x64_i8 a[0:3], v[0:3], v[4:7], a[0:3]
+	ds_read_b128 v[0:3], v9 offset:64
+	s_waitcnt vmcnt(3) lgkmcnt(1)
+	v_mfma_i32_16x16x64_i8 a[0:3], v[0:3], v[4:7], a[0:3]
+	s_barrier
+	s_cbranch_scc1 .LBB0_1
+	s_endpgm
+; -- End function
+"""
+
+
+def test_barrier_guard_accepts_waited_reads(build, tmp_path):
+    assert build.check_ring_barrier_waits(_write(tmp_path, BARRIER_GOOD)) == 1
+
+
+@pytest.mark.parametrize("bad", [
+    BARRIER_GOOD.replace("\ts_waitcnt vmcnt(3) lgkmcnt(1)\n", ""),                       # no wait between the last read and the barrier
+    BARRIER_GOOD.replace("vmcnt(3) lgkmcnt(1)", "vmcnt(3)"),                             # a wait for something else
+    BARRIER_GOOD.replace("lgkmcnt(1)", "lgkmcnt(5)"),                                    # more reads in flight than a half has blocks
+    BARRIER_GOOD.replace("\ts_barrier\n\ts_cb", "\tds_read_b128 v[0:3], v9\n\ts_barrier\n\ts_cb"),  # a read behind the wait
+])
+def test_barrier_guard_refuses(build, tmp_path, bad):
+    assert bad != BARRIER_GOOD
+    with pytest.raises(RuntimeError, match="barrier"):
+        build.check_ring_barrier_waits(_write(tmp_path, bad))
+
+
+def test_barrier_guard_checks_ring_kernels_only(build, tmp_path):
+    assert build.check_ring_barrier_waits(_write(tmp_path, BARRIER_GOOD.replace("StreamGemm", "GenericGemm"))) == 0
