@@ -67,11 +67,11 @@ struct Plan {
     int lowTileM = 0;       // a lower height that the scheduling kernel may choose instead (0: none)
     bool lowForRounds = false;  // it chooses by rounds of the machine, else by the rows that groups leave over
     int64_t maxTiles = 0;   // launch bound on workgroups
-    int32_t maxMTiles = 0;  // upper bound on m-tiles over all groups (M / tileM + groups)
+    int32_t maxMTiles = 0;  // upper bound on m-tiles of a launch over all groups (its rows / tileM + groups)
     int32_t tilesN = 0;
     bool pullTiles = false; // LDS-ring kernels: workgroups draw their tiles from counters instead of walking fixed shares
     bool slim = false;      // a handful of rows per group: the kernels of grouped_gemm_i8_slim.h, without a scheduling kernel
-    int64_t bandRows = 0;   // kSwiglu: rows of S held in the workspace at a time (M when the launch runs as one band)
+    int64_t bandRows = 0;   // rows of one launch sequence, and of S held in the workspace at a time (M, or 0: all rows in one)
     uint64_t offSched = 0, offRowMax = 0, offS = 0;
     uint64_t workspaceBytes = 0;
 };

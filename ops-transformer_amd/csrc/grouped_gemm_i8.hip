@@ -399,6 +399,10 @@ bool StreamOk(const Problem& p) {
            reinterpret_cast<uintptr_t>(p.w) % kChunk == 0 && p.N * p.K < (1ll << 31) && p.N * p.K >= 64 * kChunk;
 }
 
+// Tiles of one launch of the LDS-ring kernels: their numbers, and what the workgroups add to the tile counters past the last
+// one, stay below 2^31.
+constexpr int64_t kMaxTiles = 1ll << 30;
+
 uint64_t Align256(uint64_t v) { return (v + 255) / 256 * 256; }
 
 // S, the fp32 SwiGLU result that the requantisation reads back, is held for a band of rows at a time: at most 512 MiB of it
@@ -523,9 +527,9 @@ Plan MakePlan(const Problem& p) {
     // (the issue side then never runs more than one tile ahead, which is what the two-tile look-ahead of the draw
     // covers) and more than 64 rows; the handful-of-rows tiles of a decode step keep their fixed shares.
     // OPAPI_GEMM_PULL=0 / 1 switches it off / on for every shape with eight k-steps.
-    plan.pullTiles = StreamOk(p) && kSteps >= 8 && plan.tileM > 64 && plan.maxTiles < (1ll << 31);
+    plan.pullTiles = StreamOk(p) && kSteps >= 8 && plan.tileM > 64;
     if (const char* env = std::getenv("OPAPI_GEMM_PULL")) {
-        plan.pullTiles = StreamOk(p) && kSteps >= 8 && plan.maxTiles < (1ll << 31) && std::atoi(env) != 0;
+        plan.pullTiles = StreamOk(p) && kSteps >= 8 && std::atoi(env) != 0;
     }
     if (lowHolds && plan.tileM == 192 && plan.pullTiles && std::getenv("OPAPI_GEMM_TILE_M") == nullptr) plan.lowTileM = kLowTileM;
     // Launches of at most two rounds of low tiles: the scheduling kernel decides, where it knows the groups (its figures are
@@ -535,7 +539,15 @@ Plan MakePlan(const Problem& p) {
         plan.lowTileM = kLowTileM;
         plan.lowForRounds = true;
     }
-    const int64_t maxMTiles = p.M / (plan.lowTileM > 0 ? plan.lowTileM : plan.tileM) + groups;
+    const int64_t lowest = plan.lowTileM > 0 ? plan.lowTileM : plan.tileM;
+    // The LDS-ring kernels number the tiles of a launch in 32 bits.  More than kMaxTiles of them (the scatter-add alone can ask for so
+    // many: its output has few rows) run as several launches, each over a band of rows.  One expert's weights stay below 2 GB
+    // (StreamOk), so that every group's last m-tile is a small part of the limit: 1024 groups x 65536 n-tiles.
+    int64_t bandRows = p.M;
+    if (StreamOk(p) && (p.M / lowest + groups) * plan.tilesN > kMaxTiles) {
+        bandRows = (kMaxTiles / plan.tilesN - groups) * lowest / plan.tileM * plan.tileM;
+    }
+    const int64_t maxMTiles = bandRows / lowest + groups;
     plan.maxMTiles = static_cast<int32_t>(maxMTiles);
     // round up so that every XCD's share [xcd * ceil(total/8), ...) is covered by the launch
     plan.maxTiles = (maxMTiles * plan.tilesN + kXcds - 1) / kXcds * kXcds;
@@ -551,12 +563,13 @@ Plan MakePlan(const Problem& p) {
         // costs nothing (halving the limit twice costs 2 % and 7 % of the pass).
         const uint64_t capBytes = SwigluWorkspaceCap();
         const uint64_t rowBytes = static_cast<uint64_t>(p.N / 2) * 4;
-        int64_t bandRows = rowBytes > 0 ? static_cast<int64_t>(capBytes / rowBytes) / plan.tileM * plan.tileM : p.M;
-        if (bandRows < plan.tileM) bandRows = plan.tileM;
-        plan.bandRows = bandRows < p.M ? bandRows : p.M;
+        int64_t capRows = rowBytes > 0 ? static_cast<int64_t>(capBytes / rowBytes) / plan.tileM * plan.tileM : p.M;
+        if (capRows < plan.tileM) capRows = plan.tileM;
+        if (capRows < bandRows) bandRows = capRows;
         plan.offS = off;
-        off += Align256(static_cast<uint64_t>(plan.bandRows) * rowBytes);
+        off += Align256(static_cast<uint64_t>(bandRows) * rowBytes);
     }
+    plan.bandRows = bandRows;
     plan.workspaceBytes = off;
     return plan;
 }
@@ -617,10 +630,11 @@ hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStrea
     ka.pullTiles = plan.pullTiles ? 1 : 0;
 
     hipError_t e = hipSuccess;
-    // One band covers every row unless S is held for a band of rows at a time (kSwiglu with a capped workspace): then
-    // schedule, GEMM and requantisation run once per band, the schedule handing out only the band's rows, and S is
-    // addressed as if the band's first row were at sBuf (the kernels index S by the row of the problem).
-    const int64_t bandRows = swiglu && plan.bandRows > 0 ? plan.bandRows : p.M;
+    // One band covers every row unless S is held for a band of rows at a time (kSwiglu with a capped workspace) or the rows
+    // have more tiles than a launch can number: then schedule, GEMM and requantisation run once per band, the schedule
+    // handing out only the band's rows, and S is addressed as if the band's first row were at sBuf (the kernels index S by the
+    // row of the problem).
+    const int64_t bandRows = plan.bandRows > 0 ? plan.bandRows : p.M;
     for (int64_t rowBegin = 0; rowBegin < p.M; rowBegin += bandRows) {
         const int64_t rowEnd = rowBegin + bandRows < p.M ? rowBegin + bandRows : p.M;
         sa.rowBegin = rowBegin;

@@ -758,3 +758,17 @@ def test_slim_tiles_are_numbered_in_32_bits(aclnn):
         args = _gmm_args(aclnn, M=8, K=128, N=N, E=2)
         args[1] = _tl(aclnn, [w])
         assert _status(aclnn, "aclnnGroupedMatmulV4", args) == (0, ws)
+
+
+@pytest.mark.parametrize("M,N,E", [(1 << 30, 1 << 23, 1), (1 << 28, 1 << 23, 1024), (300_000_000, 5_000_000, 8)])
+def test_ring_tiles_are_numbered_in_32_bits(aclnn, monkeypatch, M, N, E):
+    """A combine may have rows enough for more tiles than 32 bits can number; its launches then cover a band of rows each.  The
+    workspace is one launch's table, sixteen bytes for each m-tile behind 256 bytes of header and counters, and the row factors."""
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    N = N // 32 * 32
+    code, ws = _status(aclnn, *_combine_args(aclnn, M=M, K=128, N=N, E=E, batch=16))
+    assert code == 0
+    m_tiles = (ws - 4 * M) // 16 - 16
+    assert E <= m_tiles and m_tiles * ((N + 255) // 256) < 1 << 31
+    code, ws = _status(aclnn, *_combine_args(aclnn, M=65536, K=128, N=N, E=E, batch=16))
+    assert code == 0 and (ws - 4 * 65536) // 16 - 16 >= 256  # one launch: every row has its place in the table
