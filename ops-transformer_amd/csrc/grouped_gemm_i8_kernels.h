@@ -91,7 +91,10 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const v4i* LdsV4iPtr;
 typedef float Float2 __attribute__((ext_vector_type(2)));
 typedef float Float4 __attribute__((ext_vector_type(4)));
-typedef uint32_t Uint2 __attribute__((ext_vector_type(2)));
+// Vectors that begin on any four bytes, which is all that a global store of several dwords asks for.
+typedef uint32_t Uint2Dword __attribute__((ext_vector_type(2), aligned(4)));
+typedef int Int4Dword __attribute__((ext_vector_type(4), aligned(4)));
+typedef float Float4Dword __attribute__((ext_vector_type(4), aligned(4)));
 typedef __bf16 Bf16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kTileN = 256;
@@ -367,10 +370,11 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
         afterScaleLoads();
         // wave-uniform: every channel of the wave exists
         const bool whole = t.colBase + ColumnInTile<kOrder, false>(waveN, 3, 15, neighbours) < a.N;
-        const bool vectors = (a.N & 3) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;  // rows start on a lane's vector
+        // Pairs of 16-bit results start on whole dwords; 32-bit results always do.  us, K 2048 x N 4098, with vectors only where rows
+        // start on 16 bytes -> on any dword: 16 groups of 128 rows bf16 71 -> 63, int32 74 -> 61; of 1000 rows 210 -> 195, 231 -> 180.
+        const bool pairs = (a.N & 1) == 0 && (kOrder != kOrderLane || (reinterpret_cast<uintptr_t>(a.out) & 3) == 0);
         const bool oddLane = (l16 & 1) != 0;
-        if (kEpi == Epilogue::kDequant && (a.outDtype == 27 || a.outDtype == 1) && whole &&
-            (kOrder == kOrderLane ? vectors : (a.N & 1) == 0)) {
+        if (kEpi == Epilogue::kDequant && (a.outDtype == 27 || a.outDtype == 1) && whole && pairs) {
             // 16-bit results of whole column blocks, without per-element dtype dispatch; stores through a (uniform row pointer
             // + 32-bit lane offset) address.  Past the caches: nothing reads them back before they have left these.
             const bool toBf16 = a.outDtype == 27;  // wave-uniform: bf16, else fp16
@@ -395,7 +399,7 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
                     uint16_t* const rowPtr = outTile + static_cast<int64_t>(rTop + v) * a.N;
                     const bool ok = kFull || rTop + 4 * quad + v < rows;
                     if constexpr (kOrder == kOrderLane) {
-                        if (ok) __builtin_nontemporal_store(Uint2{word[0], word[1]}, reinterpret_cast<Uint2*>(rowPtr + laneOff));
+                        if (ok) __builtin_nontemporal_store(Uint2Dword{word[0], word[1]}, reinterpret_cast<Uint2Dword*>(rowPtr + laneOff));
                     } else {
 #pragma unroll
                         for (int p = 0; p < 2; ++p) {
@@ -420,7 +424,7 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
             }
             return;
         }
-        const bool vectorStores = neighbours && whole && vectors;
+        const bool vectorStores = neighbours && whole;
         float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         if (kEpi == Epilogue::kDequant && a.bias != nullptr) {
 #pragma unroll
@@ -440,7 +444,7 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
                 if constexpr (kEpi == Epilogue::kInt32) {
                     int32_t* const out = static_cast<int32_t*>(a.out) + rowOff;
                     if (vectorStores) {
-                        *reinterpret_cast<v4i*>(out + col[0]) = v4i{acc[m][0][v], acc[m][1][v], acc[m][2][v], acc[m][3][v]};
+                        *reinterpret_cast<Int4Dword*>(out + col[0]) = Int4Dword{acc[m][0][v], acc[m][1][v], acc[m][2][v], acc[m][3][v]};
                     } else {
 #pragma unroll
                         for (int n = 0; n < 4; ++n) {
@@ -476,7 +480,7 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
                     }
                     float* const out = static_cast<float*>(a.out) + rowOff;
                     if (vectorStores) {
-                        *reinterpret_cast<Float4*>(out + col[0]) = Float4{y[0], y[1], y[2], y[3]};
+                        *reinterpret_cast<Float4Dword*>(out + col[0]) = Float4Dword{y[0], y[1], y[2], y[3]};
                     } else {
 #pragma unroll
                         for (int n = 0; n < 4; ++n) {

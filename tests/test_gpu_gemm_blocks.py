@@ -16,7 +16,8 @@ def _weights(w_enk, layout):
     return (view.contiguous() if layout == "nd" else view), None
 
 
-def _run(aclnn, sizes, N, K, layout, out_dtype, seed):
+def _run(aclnn, sizes, N, K, layout, out_dtype, seed, offset=0):
+    """offset: values in front of the output in its buffer (and sixteen behind it), which no store may touch."""
     dev = torch.device("cuda")
     g = torch.Generator().manual_seed(seed)
     E, M = len(sizes), sum(sizes)
@@ -30,11 +31,13 @@ def _run(aclnn, sizes, N, K, layout, out_dtype, seed):
     for e, n in enumerate(sizes):
         acc[begin:begin + n] = x[begin:begin + n].double() @ w[e].double().t()
         begin += n
-    out = torch.full((M, N), 7, dtype=out_dtype, device=dev)
+    buffer = torch.full((offset + M * N + 16,), 7, dtype=out_dtype, device=dev)
+    out = buffer[offset:offset + M * N].view(M, N)
     view, nz = _weights(w.to(dev), layout)
     scales = {} if out_dtype == torch.int32 else {"scale": [scale.to(dev)], "per_token_scale": [row_scale.to(dev)]}
     aclnn.grouped_matmul_v4([x.to(dev)], None if view is None else [view], weight_nz=nz, group_list=cumsum.to(dev), split_item=3,
                             group_type=0, group_list_type=0, out=[out], **scales)
+    assert (buffer[:offset] == 7).all() and (buffer[offset + M * N:] == 7).all()
     if out_dtype == torch.int32:
         return out.cpu(), acc.to(torch.int32)
     group = torch.repeat_interleave(torch.arange(E), torch.tensor(sizes))
@@ -60,6 +63,17 @@ def test_row_remainders(aclnn, monkeypatch, height, rows, out_dtype):
 def test_channel_remainders(aclnn, monkeypatch, layout, N, out_dtype):
     monkeypatch.setenv("OPAPI_GEMM_TILE_M", "128")
     got, want = _run(aclnn, [100, 0, 37, 130], N, 384, layout, out_dtype, N)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("layout", ["k", "nd", "nz"])
+@pytest.mark.parametrize("out_dtype,offset", [(torch.bfloat16, 1), (torch.bfloat16, 2), (torch.float16, 4), (torch.int32, 1), (torch.int32, 2)])
+@pytest.mark.parametrize("N", [512, 514, 516])
+def test_outputs_off_the_vector_grid(aclnn, monkeypatch, N, out_dtype, offset, layout):
+    """Vectors of two and four dwords that begin on a dword: views into a buffer, and rows of 4k + 2 channels."""
+    N = {"k": N, "nd": 512, "nz": 512}[layout]
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", "128")
+    got, want = _run(aclnn, [100, 0, 37, 130], N, 256, layout, out_dtype, N, offset)
     assert torch.equal(got, want)
 
 
