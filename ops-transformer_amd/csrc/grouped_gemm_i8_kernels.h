@@ -255,10 +255,10 @@ __device__ __forceinline__ int ColumnInTile(int w, int n, int l, bool neighbours
     return 64 * w + (kOrder == kOrderLane && neighbours ? 4 * l + n : 16 * n + l);
 }
 
-// Channel held in row r of weight half `half`, K-contiguous weights (clamped: channels past N are loaded but never stored).
-template <bool kSwiglu>
+// Channel held in row r of weight half `half`, rows by channel (clamped: channels past N are loaded but never stored).
+template <int kOrder, bool kSwiglu>
 __device__ __forceinline__ int32_t ChannelOfRow(const KernelArgs& a, const TileInfo& t, int half, int r) {
-    const int32_t col = t.colBase + ColumnInTile<kOrderLane, kSwiglu>(r >> 5, 2 * half + ((r >> 4) & 1), r & 15, LanesHoldNeighbours(a));
+    const int32_t col = t.colBase + ColumnInTile<kOrder, kSwiglu>(r >> 5, 2 * half + ((r >> 4) & 1), r & 15, LanesHoldNeighbours(a));
     return min(kSwiglu && half ? a.halfN + col : col, a.N - 1);
 }
 
@@ -969,7 +969,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                 laneOff[q] = static_cast<uint32_t>(block * a.K * 32 + k * 32 + ((lane ^ (k >> 4)) & 1) * kChunk);
             } else {
                 const int r = 8 * j + rowIn;
-                laneOff[q] = static_cast<uint32_t>(ChannelOfRow<kSwiglu>(a, t, half, r) * a.K + (slot ^ ((r >> 1) & 7)) * kChunk);
+                laneOff[q] = static_cast<uint32_t>(ChannelOfRow<kOrderLane, kSwiglu>(a, t, half, r) * a.K + (slot ^ ((r >> 1) & 7)) * kChunk);
             }
         }
     };
@@ -1311,7 +1311,8 @@ __global__ __launch_bounds__(kThreads) void GenericGemmKernel(KernelArgs a, cons
     }
 
     for (int k0 = 0; k0 < a.K; k0 += kStep) {
-        // consecutive threads take consecutive tile rows so that N-contiguous weights still coalesce
+        // consecutive threads take consecutive tile rows, and those of the weights consecutive channels (kOrderBlock), so that
+        // N-contiguous weights still coalesce
         for (int p = tid; p < kRows * kChunksPerRow; p += kThreads) {
             const int r = p % kRows;
             const int chunk = p / kRows;
@@ -1328,7 +1329,7 @@ __global__ __launch_bounds__(kThreads) void GenericGemmKernel(KernelArgs a, cons
             const int p = i * kThreads + tid;
             const int r = p % kTileN;
             const int chunk = p / kTileN;
-            const int8_t* src = wGroup + WeightRowBase(a, ChannelOfRow<kSwiglu>(a, t, r / 128, r % 128));
+            const int8_t* src = wGroup + WeightRowBase(a, ChannelOfRow<kOrderBlock, kSwiglu>(a, t, r / 128, r % 128));
             union { v4i v; int8_t b[16]; } u;
             for (int j = 0; j < kChunk; ++j) {
                 const int k = k0 + chunk * kChunk + j;
@@ -1354,7 +1355,7 @@ __global__ __launch_bounds__(kThreads) void GenericGemmKernel(KernelArgs a, cons
         }
         __syncthreads();
     }
-    TileEpilogueWave<kRows, kEpi, kOrderLane>(a, t, acc, waveM, waveN, l16, quad, ldsRowScale, ldsRowMax);
+    TileEpilogueWave<kRows, kEpi, kOrderBlock>(a, t, acc, waveM, waveN, l16, quad, ldsRowScale, ldsRowMax);
     if constexpr (kSwiglu) TileEpilogueFoldMax<kRows>(a, t, tid, ldsRowMax);
 }
 

@@ -66,6 +66,15 @@ def test_channel_remainders(aclnn, monkeypatch, layout, N, out_dtype):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("out_dtype", [torch.int32, torch.bfloat16])
+@pytest.mark.parametrize("sizes", [[20, 0, 17], [100, 0, 37, 130]])  # the byte-wise kernel's tiles of 32 and of 128 rows
+@pytest.mark.parametrize("layout,N,K", [("k", 30, 100), ("k", 257, 1001), ("k", 258, 100), ("nd", 33, 100), ("nd", 258, 333), ("nz", 288, 64)])
+def test_bytewise_channel_remainders(aclnn, monkeypatch, layout, N, K, sizes, out_dtype):
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    got, want = _run(aclnn, sizes, N, K, layout, out_dtype, N)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("layout", ["k", "nd", "nz"])
 @pytest.mark.parametrize("out_dtype,offset", [(torch.bfloat16, 1), (torch.bfloat16, 2), (torch.float16, 4), (torch.int32, 1), (torch.int32, 2)])
 @pytest.mark.parametrize("N", [512, 514, 516])
