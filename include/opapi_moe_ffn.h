@@ -18,7 +18,7 @@ extern "C" {
 
 // packed: routing (2 or 3), then sixteen tensors, each as opapiCreateTensorPacked takes it (number of dimensions, data type,
 // address, extents, strides), in the order
-//   x int8 [T, H], xScale fp32 [T], expertIdx int32 [T, K], weights of the combine [T, K],
+//   x int8 [T, H], xScale fp32 [T], expertIdx int32 [T, K], weights of the combine [T, K] (no dimensions at address 0: none, K 1),
 //   w13 [E, H, 2I], w13Scale [E, 2I], w2 [E, I, H], w2Scale [E, H]  (a five-dimensional weight is FRACTAL_NZ),
 //   expandedX, expandedRowIdx, cumsum, expandedScale, h, hScale, y, out.
 // count: values in the array.  workspaceSizes[5]: what each operator asks for, and the largest of them.  When that is more

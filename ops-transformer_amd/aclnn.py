@@ -568,6 +568,8 @@ def moe_finalize_routing_v2(expanded_x, expanded_row_idx, x1=None, x2=None, bias
 
 
 def _packed(t):
+    if t is None:
+        return _PACK[0](0, 0, 0)
     shape = t.shape
     n = len(shape)
     return _PACK[n](n, _DTYPE_CODE[t.dtype], t.data_ptr(), *shape, *t.stride())
@@ -579,7 +581,7 @@ _FFN_OPERATORS = (("aclnnMoeInitRoutingV2", "aclnnGroupedMatmulSwigluQuant", "ac
 
 def moe_ffn_forward(routing, tensors, workspace, device):
     """The operators of one expert FFN pass in one foreign call (include/opapi_moe_ffn.h): routing 2 or 3, then the sixteen
-    tensors in that header's order."""
+    tensors in that header's order (the weights of the combine may be None)."""
     l = lib()
     packed = struct.pack("q", routing) + b"".join(map(_packed, tensors))
     sizes = (ctypes.c_uint64 * 5)()

@@ -88,7 +88,9 @@ extern "C" aclnnStatus opapiMoeFfnForward(const int64_t* packed, uint64_t count,
                                               nullptr, nullptr, 3, 0, 0, 0, &out, nullptr, nullptr, &workspaceSizes[2], &ex.of[2]);
     if (st != ACLNN_SUCCESS) return st;
     *failedOperator = "aclnnMoeFinalizeRoutingV2GetWorkspaceSize";
-    st = aclnnMoeFinalizeRoutingV2GetWorkspaceSize(&t[kY], &t[kExpandedRowIdx], nullptr, nullptr, nullptr, &t[kTopKWeight], nullptr, 2,
+    const bool weighted = !t[kTopKWeight].dims.empty() || t[kTopKWeight].data != nullptr;
+    st = aclnnMoeFinalizeRoutingV2GetWorkspaceSize(&t[kY], &t[kExpandedRowIdx], nullptr, nullptr, nullptr,
+                                                   weighted ? &t[kTopKWeight] : nullptr, nullptr, 2,
                                                    &t[kOut], &workspaceSizes[3], &ex.of[3]);
     if (st != ACLNN_SUCCESS) return st;
     workspaceSizes[4] = *std::max_element(workspaceSizes, workspaceSizes + 4);

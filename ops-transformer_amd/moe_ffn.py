@@ -86,7 +86,8 @@ class MoeFfnW8A8:
         self._buf_key = (T, K)
 
     def forward(self, xq, x_scale, topk_idx, topk_weight):
-        """xq int8 [T, H]; x_scale fp32 [T]; topk_idx int32 [T, K]; topk_weight fp32/bf16 [T, K] -> out [T, H]."""
+        """xq int8 [T, H]; x_scale fp32 [T]; topk_idx int32 [T, K]; topk_weight fp32/bf16 [T, K] (top-1: or
+        None, unweighted) -> out [T, H]."""
         T, K = topk_idx.shape
         self._buffers(T, K)
         if not self.fused_combine:

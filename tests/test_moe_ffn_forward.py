@@ -73,6 +73,26 @@ def test_each_operator_still_checks_its_tensors(aclnn, which, replacement, opera
     assert st != 0 and enqueued == 0 and name == operator and aclnn.last_error()
 
 
+def test_weights_of_the_combine_may_be_absent(aclnn):
+    """As with the operator itself: one expert per token, unweighted.  Without them a row of more experts has nowhere to go."""
+    for K, ok in ((1, True), (2, False)):
+        tensors = _tensors(4, 128, 64, 4, K)
+        tensors[3] = None
+        st, sizes, enqueued, name = _call(aclnn, _pack(aclnn, 2, tensors))
+        assert (st == 0) == ok and enqueued == 0 and name == "aclnnMoeFinalizeRoutingV2GetWorkspaceSize"
+
+
+@pytest.mark.gpu
+def test_top_1_without_weights(pkg, dev):
+    g = torch.Generator(device=dev).manual_seed(1)
+    i8 = lambda *s: torch.empty(s, dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    f = lambda *s: torch.rand(s, device=dev, generator=g) * 0.01 + 1e-3
+    ffn = pkg.MoeFfnW8A8(i8(4, 256, 256), f(4, 256), i8(4, 256, 128), f(4, 256))
+    xq, xs, idx = i8(9, 256), f(9), torch.randint(0, 4, (9, 1), device=dev, generator=g, dtype=torch.int32)
+    want = ffn.forward(xq, xs, idx, torch.ones((9, 1), device=dev)).clone()
+    assert torch.equal(ffn.forward(xq, xs, idx, None), want) and want.any()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("routing", ["v2", "v3"])
 @pytest.mark.parametrize("tokens", [1, 3, 257, 1300])
