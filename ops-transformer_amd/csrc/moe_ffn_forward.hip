@@ -44,7 +44,7 @@ struct Executors {
 
 extern "C" aclnnStatus opapiMoeFfnForward(const int64_t* packed, uint64_t count, void* workspace, uint64_t workspaceSize,
                                           aclrtStream stream, uint64_t* workspaceSizes, int32_t* enqueued,
-                                          const char** failedOperator) {
+                                          const char** failedOperator) try {
     using namespace opapi;
     ClearError();
     OPAPI_CHECK_NOTNULL(packed, "packed");
@@ -108,4 +108,7 @@ extern "C" aclnnStatus opapiMoeFfnForward(const int64_t* packed, uint64_t count,
     }
     *enqueued = 1;
     return ACLNN_SUCCESS;
+} catch (...) {  // no exception may cross the C boundary
+    opapi::SetError("out of host memory");
+    return ACLNN_ERR_INNER;
 }

@@ -1,7 +1,10 @@
 """The one-call expert FFN (opapiMoeFfnForward, what MoeFfnW8A8.forward runs): what it refuses, on the CPU, and on the GPU that
 its results are those of the four operators called one by one."""
 import ctypes
+import os
 import struct
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -71,6 +74,55 @@ def test_each_operator_still_checks_its_tensors(aclnn, which, replacement, opera
     tensors[which] = replacement
     st, _, enqueued, name = _call(aclnn, _pack(aclnn, 2, tensors))
     assert st != 0 and enqueued == 0 and name == operator and aclnn.last_error()
+
+
+FAILING_NEW = """
+#include <cstdlib>
+#include <new>
+static thread_local long left = -1;  // allocations until the one that fails; negative: none does
+extern "C" void fail_new_after(long n) { left = n; }
+void* operator new(std::size_t n) {
+    if (left >= 0 && left-- == 0) throw std::bad_alloc();
+    if (void* p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
+"""
+
+CHILD = """
+import ctypes, sys
+sys.path[:0] = [{root!r}, {tests!r}]
+from __graft_entry__ import load_package
+import test_moe_ffn_forward as t
+aclnn = load_package().aclnn
+arm = ctypes.CDLL({lib!r}).fail_new_after
+arm.argtypes = [ctypes.c_long]
+for routing in (2, 3):
+    data = t._pack(aclnn, routing, t._tensors(4, 128, 64, 4, 2, routing == 3))
+    aclnn.lib()
+    for n in range(10000):
+        arm(n)
+        st, _, enqueued, _ = t._call(aclnn, data)
+        arm(-1)
+        assert enqueued == 0
+        if st == 0:
+            break
+    print("survived", routing, n)
+    assert n > 16
+"""
+
+
+def test_running_out_of_host_memory_is_a_status(tmp_path):
+    """Every allocation of the call in turn fails: no exception leaves the C entry (it would end the process)."""
+    src, lib = tmp_path / "failing_new.cpp", tmp_path / "libfailing_new.so"
+    src.write_text(FAILING_NEW)
+    subprocess.check_call(["g++", "-O1", "-shared", "-fPIC", str(src), "-o", str(lib)])
+    tests = os.path.dirname(os.path.abspath(__file__))
+    env = dict(os.environ, LD_PRELOAD=":".join([str(lib)] + [p for p in [os.environ.get("LD_PRELOAD")] if p]))
+    res = subprocess.run([sys.executable, "-c", CHILD.format(root=os.path.dirname(tests), tests=tests, lib=str(lib))], env=env,
+                         stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert res.returncode == 0 and res.stdout.count("survived") == 2, res.stdout[-2000:]
 
 
 def test_weights_of_the_combine_may_be_absent(aclnn):
