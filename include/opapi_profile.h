@@ -61,7 +61,8 @@ __attribute__((visibility("default"))) void opapiGemmWorkgroupSpansEnable(int en
 
 /*
  * Synchronises the device, then writes one text line per recorded kind into buf (NUL-terminated):
- * "<name> workgroups <n> tile_rows <r> span_us <last end - first start>" followed, per XCD x = 0..7, by
+ * "<name> workgroups <n> tile_rows <r> span_us <last end - first start>" (r: rows of the tallest tiles, as planned or, where the
+ * scheduling kernel has chosen lower ones for the list it found, of those) followed, per XCD x = 0..7, by
  * " xcd<x> end_us <when its last workgroup ended> busy <mean (end - start) / span of its workgroups> tiles <min>-<max>".
  * Returns the number of lines, or -1 on an error.
  */

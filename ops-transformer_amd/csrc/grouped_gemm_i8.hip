@@ -725,12 +725,13 @@ extern "C" __attribute__((visibility("default"))) int opapiGemmWorkgroupSpansRep
         if (gSpanBuf[k] == nullptr || grid <= 0) continue;
         if (hipMemcpy(host.data(), gSpanBuf[k], static_cast<size_t>(grid) * 3 * sizeof(uint64_t), hipMemcpyDeviceToHost) != hipSuccess) return -1;
         uint64_t first = ~0ull, last = 0;
+        const int tileRows = host[2] >> 32 != 0 ? static_cast<int>(host[2] >> 32) : gSpanTileM[k];
         for (int b = 0; b < grid; ++b) {
             first = std::min(first, host[3 * b]);
             last = std::max(last, host[3 * b + 1]);
         }
         const double span = static_cast<double>(last - first) / 100.0;  // 100 MHz counter -> microseconds
-        int n = snprintf(buf + used, cap - used, "%s workgroups %d tile_rows %d span_us %.1f", kNames[k], grid, gSpanTileM[k], span);
+        int n = snprintf(buf + used, cap - used, "%s workgroups %d tile_rows %d span_us %.1f", kNames[k], grid, tileRows, span);
         if (n < 0 || static_cast<size_t>(n) >= cap - used) break;
         used += static_cast<size_t>(n);
         // per XCD (workgroup b runs on XCD b % 8): when its last workgroup ended, relative to the launch's first start,
@@ -742,8 +743,8 @@ extern "C" __attribute__((visibility("default"))) int opapiGemmWorkgroupSpansRep
             for (int b = x; b < grid; b += kXcds) {
                 xLast = std::max(xLast, host[3 * b + 1]);
                 busy += static_cast<double>(host[3 * b + 1] - host[3 * b]);
-                tMin = std::min(tMin, host[3 * b + 2]);
-                tMax = std::max(tMax, host[3 * b + 2]);
+                tMin = std::min(tMin, host[3 * b + 2] & 0xffffffffu);
+                tMax = std::max(tMax, host[3 * b + 2] & 0xffffffffu);
                 ++count;
             }
             n = snprintf(buf + used, cap - used, " xcd%d end_us %.1f busy %.3f tiles %llu-%llu", x,

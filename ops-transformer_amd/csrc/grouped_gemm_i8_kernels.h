@@ -45,8 +45,8 @@ struct KernelArgs {
     const float* combineWeight;
     const void* bias;
     int32_t biasDtype;
-    // workgroup spans (include/opapi_profile.h): per workgroup {start, end} of the 100 MHz real-time counter and the
-    // number of tiles it computed; null unless span recording is on
+    // workgroup spans (include/opapi_profile.h): per workgroup what WriteSpan leaves, times of the 100 MHz real-time counter;
+    // null unless span recording is on
     uint64_t* wgSpans;
     // LDS-ring kernels: the tile counters of the scheduling table as a pointer the kernel may write through (the table
     // itself is a read-only kernel parameter), and whether workgroups pull their tiles from the counters (1) or walk a
@@ -1211,12 +1211,13 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     }
 }
 
-// Workgroup span record (include/opapi_profile.h): start, end, tiles computed.
-__device__ __forceinline__ void WriteSpan(const KernelArgs& a, uint64_t start, uint64_t tiles) {
+// Workgroup span record (include/opapi_profile.h): start, end, tiles computed, and above those, in the upper half of the word,
+// the rows of a tile where the scheduling kernel has chosen other ones than planned (else 0).
+__device__ __forceinline__ void WriteSpan(const KernelArgs& a, uint64_t start, uint64_t tiles, uint32_t otherRows = 0) {
     if (a.wgSpans != nullptr && threadIdx.x == 0) {
         a.wgSpans[3 * blockIdx.x] = start;
         a.wgSpans[3 * blockIdx.x + 1] = __builtin_amdgcn_s_memrealtime();
-        a.wgSpans[3 * blockIdx.x + 2] = tiles;
+        a.wgSpans[3 * blockIdx.x + 2] = tiles | static_cast<uint64_t>(otherRows) << 32;
     }
 }
 
@@ -1246,7 +1247,7 @@ __global__ __launch_bounds__(kThreads) void MixedGemmKernel(KernelArgs a, const 
     uint64_t spanTiles = 0;
     if (sched[kHdrTileM] == kLowTileM) {
         StreamGemmBody<kLowTileM, kEpi, kNz, kNMajor, kBothRuns, kTail>(a, sched, lds, spanTiles);
-        WriteSpan(a, spanStart, spanTiles);
+        WriteSpan(a, spanStart, spanTiles, kLowTileM);
         return;
     }
     const int64_t costSmall = sched[2], costAll = costSmall + sched[3];

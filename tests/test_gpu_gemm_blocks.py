@@ -1,6 +1,7 @@
 """The ring GEMM kernels where their tiles end: row counts around the 16-row blocks and the 256-row tile, channel counts around
 a lane's vector of four and a tile's 256, launches of at most one tile per workgroup and of one more, in the three weight
 layouts and with every output type, against exact integer products (float64) and the epilogue's own fp32 arithmetic."""
+import numpy as np
 import pytest
 import torch
 
@@ -16,7 +17,7 @@ def _weights(w_enk, layout):
     return (view.contiguous() if layout == "nd" else view), None
 
 
-def _run(aclnn, sizes, N, K, layout, out_dtype, seed, offset=0):
+def _run(aclnn, sizes, N, K, layout, out_dtype, seed, offset=0, kind="cumsum"):
     """offset: values in front of the output in its buffer (and sixteen behind it), which no store may touch."""
     dev = torch.device("cuda")
     g = torch.Generator().manual_seed(seed)
@@ -25,22 +26,29 @@ def _run(aclnn, sizes, N, K, layout, out_dtype, seed, offset=0):
     w = torch.randint(-127, 128, (E, N, K), generator=g, dtype=torch.int8)
     scale = torch.rand((E, N), generator=g) * 0.01 + 1e-3
     row_scale = torch.rand((M,), generator=g) * 0.05 + 1e-2
-    cumsum = torch.cumsum(torch.tensor(sizes), 0)
+    if kind == "sparse":  # pairs in falling order of the experts, those without rows left out
+        order = [e for e in reversed(range(E)) if sizes[e] > 0]
+        listed = torch.tensor([[e, sizes[e]] for e in order] + [[0, 0]] * (E - len(order)))
+    else:
+        order = list(range(E))
+        listed = torch.cumsum(torch.tensor(sizes), 0) if kind == "cumsum" else torch.tensor(sizes)
+    listed = listed.int() if kind == "counts32" else listed
     acc = torch.empty((M, N), dtype=torch.float64)
     begin = 0
-    for e, n in enumerate(sizes):
+    for e in order:
+        n = sizes[e]
         acc[begin:begin + n] = x[begin:begin + n].double() @ w[e].double().t()
         begin += n
     buffer = torch.full((offset + M * N + 16,), 7, dtype=out_dtype, device=dev)
     out = buffer[offset:offset + M * N].view(M, N)
     view, nz = _weights(w.to(dev), layout)
     scales = {} if out_dtype == torch.int32 else {"scale": [scale.to(dev)], "per_token_scale": [row_scale.to(dev)]}
-    aclnn.grouped_matmul_v4([x.to(dev)], None if view is None else [view], weight_nz=nz, group_list=cumsum.to(dev), split_item=3,
-                            group_type=0, group_list_type=0, out=[out], **scales)
+    aclnn.grouped_matmul_v4([x.to(dev)], None if view is None else [view], weight_nz=nz, group_list=listed.to(dev), split_item=3,
+                            group_type=0, group_list_type={"cumsum": 0, "sparse": 2}.get(kind, 1), out=[out], **scales)
     assert (buffer[:offset] == 7).all() and (buffer[offset + M * N:] == 7).all()
     if out_dtype == torch.int32:
         return out.cpu(), acc.to(torch.int32)
-    group = torch.repeat_interleave(torch.arange(E), torch.tensor(sizes))
+    group = torch.repeat_interleave(torch.tensor(order), torch.tensor([sizes[e] for e in order]))
     return out.cpu(), ((acc.float() * scale[group]) * row_scale[:, None]).to(out_dtype)
 
 
@@ -96,8 +104,26 @@ def test_one_round_of_pulled_tiles_and_one_more(aclnn, monkeypatch, groups, heig
 
 # Launches of few tiles, which the scheduling kernel may cut lower than planned, and each group evenly: groups around one and two low
 # tiles, around a short even tile and one of ten (ten even tiles of 1441 rows are nine rows short of the tenth), idle groups, and
-# (four of 250 rows beside 64 n-tiles: two rounds instead of one) a launch that stays as it is
-FEW = {"even": ([250] * 8, 1024), "uneven": ([161, 0, 320, 321, 64, 65, 160, 1], 1024), "many": ([1441, 1760, 7], 512), "tall": ([250] * 4, 16384)}
+# (four of 250 rows beside 64 n-tiles: two rounds instead of one) a launch that stays as it is.  With half the channels ("narrow") only
+# row-major weights take this path: the other layouts' 64-row tiles of the kernels for a handful of rows are one round.
+FEW = {"even": ([250] * 8, 1024), "uneven": ([161, 0, 320, 321, 64, 65, 160, 1], 2048), "many": ([1441, 1760, 7], 1024), "tall": ([250] * 4, 16384),
+       "uneven_narrow": ([161, 0, 320, 321, 64, 65, 160, 1], 1024), "many_narrow": ([1441, 1760, 7], 512)}
+
+
+def _few_rows(name, layout):
+    return 256 if name == "tall" else 64 if name.endswith("narrow") and layout != "nd" else 160
+
+
+def _spanned(aclnn, call):
+    """(what call returns, rows of the ring kernels' tallest tiles in it)"""
+    aclnn.gemm_workgroup_spans_enable(True)
+    try:
+        result = call()
+        spans = aclnn.gemm_workgroup_spans_report()
+    finally:
+        aclnn.gemm_workgroup_spans_enable(False)
+    assert len(spans) == 1
+    return result, next(iter(spans.values()))["tile_rows"]
 
 
 @pytest.mark.parametrize("layout,K", [("k", 1024), ("k", 1040), ("nd", 1024), ("nz", 1040)])
@@ -105,27 +131,51 @@ FEW = {"even": ([250] * 8, 1024), "uneven": ([161, 0, 320, 321, 64, 65, 160, 1],
 def test_few_tiles(aclnn, monkeypatch, name, layout, K):
     monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
     sizes, N = FEW[name]
-    got, want = _run(aclnn, sizes, N, K, layout, torch.bfloat16, K)
+    (got, want), rows = _spanned(aclnn, lambda: _run(aclnn, sizes, N, K, layout, torch.bfloat16, K))
+    assert rows == _few_rows(name, layout)
     assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("layout", ["k", "nd"])
+@pytest.mark.parametrize("kind", ["counts", "counts32", "sparse"])
+def test_few_tiles_of_other_lists(aclnn, monkeypatch, kind, layout):
+    """The even cut on counts and on (expert, rows) pairs, whose groups lie in the order of the list."""
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    sizes, N = FEW["uneven"]
+    (got, want), rows = _spanned(aclnn, lambda: _run(aclnn, sizes, N, 1024, layout, torch.bfloat16, 3, kind=kind))
+    assert rows == 160
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("bands", [False, True])
+@pytest.mark.parametrize("layout", ["k", "nd"])
 @pytest.mark.parametrize("name", sorted(FEW))
-def test_few_tiles_swiglu_equals_a_forced_height(aclnn, dev, monkeypatch, name, layout):
-    """S and its row maximum do not depend on how the rows are cut into tiles."""
+def test_few_tiles_swiglu_equals_a_forced_height(aclnn, oracle, dev, monkeypatch, name, layout, bands):
+    """Every row against the same call at a forced height (S and its row maximum do not depend on how the rows are cut into tiles), rows
+    at the ends of groups and tiles against the oracle.  bands: S for one band of rows at a time, each cut by itself."""
     sizes, N = FEW[name]
     K, E, M = 1024, len(sizes), sum(sizes)
+    monkeypatch.delenv("OPAPI_SWIGLU_WORKSPACE_MB", raising=False)
+    if bands:
+        monkeypatch.setenv("OPAPI_SWIGLU_WORKSPACE_MB", str(max(1, 512 * N * 2 >> 20)))  # 512 rows
     g = torch.Generator(device=dev).manual_seed(M)
     x = torch.empty((M, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
-    w = torch.empty((E, N, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g).transpose(1, 2)
-    w = w.contiguous() if layout == "nd" else w
+    w_enk = torch.empty((E, N, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    w = w_enk.transpose(1, 2).contiguous() if layout == "nd" else w_enk.transpose(1, 2)
     scale, x_scale = torch.rand((E, N), device=dev, generator=g) * 1e-3, torch.rand((M,), device=dev, generator=g) * 1e-2
     cumsum = torch.cumsum(torch.tensor(sizes), 0).to(dev)
-    results = []
-    for height in (None, "256"):
-        monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
-        if height is not None:
-            monkeypatch.setenv("OPAPI_GEMM_TILE_M", height)
-        results.append(aclnn.grouped_matmul_swiglu_quant(x, w, cumsum, scale, x_scale))
-    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
-    assert results[0][0].any()
+    call = lambda: aclnn.grouped_matmul_swiglu_quant(x, w, cumsum, scale, x_scale)
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    (y, ys), rows = _spanned(aclnn, call)  # of the last band
+    # (a launch that runs in bands is none of a handful of rows, and the second band of the tall one is small)
+    assert rows == (160 if bands else _few_rows(name, layout))
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", "256")
+    (y256, ys256), rows = _spanned(aclnn, call)
+    assert rows == 256 and torch.equal(y, y256) and torch.equal(ys, ys256)
+    begins = [sum(sizes[:e]) for e in range(E)]
+    sample = sorted({b + r for b, n in zip(begins, sizes) for r in (0, 15, 16, 79, 80, 127, 128, 159, 160, 255, 256, n - 1) if r < n})[:60]
+    h, hs = oracle.grouped_matmul_swiglu_quant(x.cpu().numpy(), w_enk.cpu().numpy(), scale.cpu().numpy(), x_scale.cpu().numpy(),
+                                               cumsum.cpu().numpy(), w_trans=True, rows=np.array(sample))
+    diff = np.abs(y.cpu().numpy()[sample].astype(np.int32) - h.astype(np.int32))
+    assert diff.max() <= 1 and (diff != 0).mean() < 1e-3  # an LSB where exp and division round differently
+    np.testing.assert_allclose(ys.cpu().numpy()[sample], hs, rtol=1e-5)
