@@ -443,7 +443,7 @@ def main():
     result["int8_mfma_rate_probe"] = {
         "zero_operands_tops": aclnn.int8_mfma_rate_probe(False) / 1e12,
         "uniform_random_operands_tops": aclnn.int8_mfma_rate_probe(True) / 1e12,
-        "note": "back-to-back v_mfma_i32_32x32x32_i8 on register operands, 8 waves per CU, no memory traffic; "
+        "note": "back-to-back v_mfma_i32_16x16x64_i8 on register operands, 8 waves per CU, no memory traffic; "
                 "roofline.peak stays the published 5000 TOP/s"}
     if not args.no_cpu_baseline:
         oracle = graft.load_oracle()

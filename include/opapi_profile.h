@@ -37,8 +37,8 @@ __attribute__((visibility("default"))) int opapiKernelTimerReport(char* buf, siz
 __attribute__((visibility("default"))) int opapiCalibrationCopy(void* dst, const void* src, size_t bytes, void* stream);
 
 /*
- * Matrix-pipe rate probe: runs nothing but back-to-back v_mfma_i32_32x32x32_i8 on register operands (eight waves per CU,
- * one workgroup per CU, `iterations` x 16 MFMAs per wave, one warm-up launch and one timed launch on the null stream)
+ * Matrix-pipe rate probe: runs nothing but back-to-back v_mfma_i32_16x16x64_i8 on register operands (eight waves per CU,
+ * one workgroup per CU, `iterations` x 32 MFMAs per wave, one warm-up launch and one timed launch on the null stream)
  * and writes the achieved int8 operations per second (2 per multiply-add).  uniformRandomOperands = 0: all-zero operands;
  * non-zero: every operand byte uniform over [-127, 127], like the benchmark's weights.  The engine clock under matrix load
  * follows the switching activity of the operands, so the second figure is the ceiling for a GEMM on such data.  Allocates

@@ -4,7 +4,7 @@
 // the same counter is read for this kernel (whose traffic is exactly `bytes` in and `bytes` out) and for the kernel
 // under study, and the ratio of the two readings converts counter units to bytes.
 //
-// A matrix-pipe rate probe: nothing but back-to-back v_mfma_i32_32x32x32_i8 on operands held in registers, eight waves
+// A matrix-pipe rate probe: nothing but back-to-back v_mfma_i32_16x16x64_i8, the GEMM kernels' instruction, on operands held in registers, eight waves
 // per CU.  The engine clock this chip sustains under matrix load depends on how much the operand bits toggle: the probe
 // reports the int8 rate for operands of a chosen kind (zeros, or uniform random bytes like the benchmark's weights), i.e.
 // the ceiling that a GEMM on such data cannot pass however well it is fed.
@@ -30,32 +30,31 @@ __global__ __launch_bounds__(kCopyThreads) void CalibrationCopyKernel(uint4* __r
 }
 
 typedef int V4i __attribute__((ext_vector_type(4)));
-typedef int V16i __attribute__((ext_vector_type(16)));
 constexpr int kProbeThreads = 512;
 constexpr int kProbeOperands = 12;  // 8 A fragments + 4 B fragments per lane
 
-// 16 MFMAs per iteration on 8 independent accumulators (128 registers, the footprint of a 128 x 64 wave tile).
+// 32 MFMAs per iteration on as many independent accumulators (128 registers, the footprint of a 128 x 64 wave tile), walked back and
+// forth along the weights as the GEMM kernels do it, so that consecutive instructions share an operand.
 __global__ __launch_bounds__(kProbeThreads) void MfmaRateProbeKernel(const V4i* __restrict__ operands, int iterations, int* sink) {
     V4i a[8], b[4];
     for (int i = 0; i < 8; ++i) a[i] = operands[i * kProbeThreads + threadIdx.x];
     for (int i = 0; i < 4; ++i) b[i] = operands[(8 + i) * kProbeThreads + threadIdx.x];
-    V16i acc[4][2];
-    for (int m = 0; m < 4; ++m)
-        for (int n = 0; n < 2; ++n)
-            for (int v = 0; v < 16; ++v) acc[m][n][v] = 0;
+    V4i acc[8][4];
+    for (int m = 0; m < 8; ++m)
+        for (int n = 0; n < 4; ++n) acc[m][n] = V4i{0, 0, 0, 0};
     for (int it = 0; it < iterations; ++it) {
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+        for (int m = 0; m < 8; ++m)
 #pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                acc[m][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[4 * s + m], b[2 * s], acc[m][0], 0, 0, 0);
-                acc[m][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[4 * s + m], b[2 * s + 1], acc[m][1], 0, 0, 0);
+            for (int step = 0; step < 4; ++step) {
+                const int n = m & 1 ? 3 - step : step;
+                acc[m][n] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[m], b[n], acc[m][n], 0, 0, 0);
             }
     }
     int x = 0;
-    for (int m = 0; m < 4; ++m)
-        for (int n = 0; n < 2; ++n)
-            for (int v = 0; v < 16; ++v) x ^= acc[m][n][v];
+    for (int m = 0; m < 8; ++m)
+        for (int n = 0; n < 4; ++n)
+            for (int v = 0; v < 4; ++v) x ^= acc[m][n][v];
     if (x == 0x12345678) sink[0] = x;  // keeps the accumulators alive
 }
 
@@ -101,8 +100,8 @@ extern "C" __attribute__((visibility("default"))) int opapiInt8MfmaRateProbe(int
             hipLaunchKernelGGL(MfmaRateProbeKernel, dim3(cus), dim3(kProbeThreads), 0, nullptr, operands, iterations, sink);
             if (hipEventRecord(stop, nullptr) == hipSuccess && hipEventSynchronize(stop) == hipSuccess &&
                 hipEventElapsedTime(&ms, start, stop) == hipSuccess && ms > 0.0f) {
-                // 8 waves x 16 MFMAs per iteration per workgroup, 32 * 32 * 32 * 2 operations each
-                *opsPerSecond = static_cast<double>(cus) * 8.0 * 16.0 * iterations * 65536.0 / (ms * 1e-3);
+                // 8 waves x 32 MFMAs per iteration per workgroup, 16 * 16 * 64 * 2 operations each
+                *opsPerSecond = static_cast<double>(cus) * 8.0 * 32.0 * iterations * 32768.0 / (ms * 1e-3);
                 status = ACL_SUCCESS;
             }
         }
