@@ -185,7 +185,8 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
         const uint32_t cus = a.cus, lowTiles = sLow * a.tilesN;
         if (lowTiles <= cus || (lowTiles <= 2 * cus && sTall * a.tilesN > cus)) {
             tileM = kLowTileM;
-            // the group's m-tiles are alike: 160 + 20 rows would read the weights twice, at two paces
+            // Even tiles, in sixteens: 160 + 20 rows would read the weights twice, at two paces.  The last one is what is left, of many
+            // tiles sometimes next to nothing (1441 rows: nine of 160 and one of 1); blocks dealt out exactly measured the same.
             cut = low > 0 ? static_cast<int32_t>(((rows + low - 1) / low + 15) & ~15u) : kLowTileM;
         }
     } else if (a.mayLower) {

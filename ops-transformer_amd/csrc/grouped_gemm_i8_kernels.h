@@ -784,7 +784,7 @@ __device__ __forceinline__ void PhaseBarrier() {
 // other, and the k that the step before has already covered are multiplied by zero (the weight fragments of that one
 // step are masked).
 // Before, such K went through the byte-wise kernel: a 301-token pass over 32 experts with hidden 2880 and intermediate
-// 1440 took 1.396 ms and takes 0.162 ms (its 398 MB of weights alone are 0.06 ms at the HBM's streaming rate).
+// 1440 took 1.396 ms and takes 0.126 ms (its 398 MB of weights alone are 0.06 ms at the HBM's streaming rate).
 constexpr int kBigRun = 0, kSmallRun = 1, kBothRuns = 2;
 template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, int kRun, bool kTail>
 __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_t* __restrict__ sched, char* const lds,
@@ -825,8 +825,8 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     constexpr int kSeqUsedUp = 32, kSeqDrawCounter = 33;  // thread 0's draw state, behind the ring
     constexpr int kTilesAhead = 6;
     // Which list this workgroup draws from first: the small m-tiles get the share of each XCD's workgroups that their
-    // cost is of the whole, so that both lists run dry at about the same time; until then a part of the machine
-    // streams weights for a handful of rows each while the rest multiplies.
+    // cost is of the whole, so that lists of many rounds run dry at about the same time (short ones: see the first draws);
+    // until then a part of the machine streams weights for a handful of rows each while the rest multiplies.
     int prefer = 0;
     {
         const int64_t costSmall = queueHdr[2], costAll = costSmall + queueHdr[3];
@@ -865,8 +865,12 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     };
     if (tid == 0) {
         if (pull) {
-            // With no more tiles than workgroups everybody's first draw finds all of them; a second tile drawn along with it
-            // would be missing where another workgroup is idle (128 tiles of K 14336: 200 us, or 400 where one had two).
+            // A run of no more tiles than there are workgroups: one tile each.  A second one drawn along with it would be missing
+            // where another workgroup is idle (128 tiles of K 14336: 200 us, or 400 where one had two).  In the two-geometry
+            // form fewer workgroups than that begin with the run; they go on to the other run after their one tile, and the tiles
+            // left of this one fill the last round of that.  us, drawing on until the run is used up -> one each: 8 experts of 1000
+            // rows, gate/up 7168 x 2 x 2048 with 4 of 40 rows 303 -> 262, K 14336 x N 4096 with 4 of 60 514 -> 448; K 1408 x
+            // N 2048, 216 big and 104 small tiles 67 -> 52; the other way round 830 -> 858 at most (of sixty launches).
             const bool oneRound = (kRun == kBigRun ? bigTiles : kRun == kSmallRun ? totalTiles - bigTiles : totalTiles) <= static_cast<int32_t>(gridDim.x);
             // the first two tiles: both draws go out together
             const int c = QueueFirstOpen(0, xcd, prefer, kOneRun);

@@ -3,7 +3,7 @@
 The oracle cannot run 10^14 MACs in a test, so each configuration is checked three ways:
   * routing (integer / byte work) against the oracle in full, bit-exact;
   * the two GEMM stages against the oracle on a sample of expanded rows that touches every expert (first and last row of
-    every non-empty group plus rows either side of the kernel's 32-row sub-tile boundaries), finalize in full;
+    every non-empty group plus rows either side of the kernel's 16-row block boundaries), finalize in full;
   * size-independent properties over ALL rows: the routing index is a permutation and the counts sum to M; negating the
     linear half's weight scales and doubling the down-projection scales gives exactly -2 x the output (sign symmetry of
     every rounding, exactness of powers of two); permuting the tokens permutes the output rows bit for bit (no row's
@@ -30,10 +30,10 @@ def _tile_heights_in_use(pkg, forward):
 
 
 def _sample_rows(cumsum, per_group_extra, seed, tile_heights=(256,)):
-    """First and last row of every non-empty group, the rows either side of every 32-row MFMA sub-tile edge up to the
-    tallest tile, and, for each tile height in use, the rows either side of the tile's end, of the boundary between its
-    two wave rows (wave row 0 takes the first ceil(active / 2) sub-tiles of a tile with `active` occupied ones) in the
-    group's last, partly filled tile, and of every further whole tile; plus random rows."""
+    """First and last row of every non-empty group; the rows either side of every edge of a 16-row block (where the tile's rows
+    change from one wave row to the other, and every second time between the halves of a wave row's) up to the tallest tile; for each
+    tile height in use the rows either side of every tile's end, and of the last occupied block in the group's last, partly filled
+    tile; plus random rows."""
     rng = np.random.default_rng(seed)
     start = np.concatenate([[0], cumsum[:-1]]).astype(np.int64)
     rows = []
@@ -42,14 +42,13 @@ def _sample_rows(cumsum, per_group_extra, seed, tile_heights=(256,)):
             continue
         n = e - s
         offs = {0, n - 1}
-        for b in range(32, 257, 32):                   # sub-tile edges: 31/32, 63/64, ..., 255/256
+        for b in range(16, 257, 16):                   # block edges: 15/16, 31/32, ..., 255/256
             offs.update((b - 1, b))
         for th in tile_heights:
             for t0 in range(0, int(n), th):            # every m-tile of the group at this height
                 offs.update((t0 - 1, t0))
-                active = (min(th, n - t0) + 31) // 32
-                split = t0 + 32 * ((active + 1) // 2)  # first row of wave row 1
-                offs.update((split - 1, split))
+                last = t0 + 16 * ((min(th, n - t0) - 1) // 16)  # first row of the tile's last occupied block
+                offs.update((last - 1, last))
         rows += [s + o for o in offs if 0 <= o < n]
         if per_group_extra:
             rows += list(rng.integers(s, e, size=per_group_extra))
