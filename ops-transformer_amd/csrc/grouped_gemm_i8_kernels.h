@@ -237,11 +237,10 @@ constexpr int kThreads = 64 * kWaves;
 // Which channel a row of a weight half is.  Weights by channel (K-contiguous) may lie in LDS in any order, and they lie so
 // that the accumulators of a lane are neighbouring channels: four (kSwiglu: two of S), one store.  The two layouts with the
 // channels side by side in memory hand sixteen neighbours to sixteen lanes.
-constexpr int kOrderLane = 0;   // K-contiguous: wave column w, block j, lane l: channel 64 w + 4 l + 2 half + j
-constexpr int kOrderBlock = 1;  // blocked: 64 w + 32 half + 16 j + l
-constexpr int kOrderFar = 2;    // row-major: 128 half + 32 w + 16 j + l
+constexpr int kOrderLane = 0;   // K-contiguous: wave column w, block n, lane l: channel 64 w + 4 l + n
+constexpr int kOrderBlock = 1;  // blocked and row-major: 64 w + 16 n + l
 template <bool kNz, bool kNMajor>
-constexpr int kOrderOf = kNz ? kOrderBlock : kNMajor ? kOrderFar : kOrderLane;
+constexpr int kOrderOf = kNz || kNMajor ? kOrderBlock : kOrderLane;
 
 // Scatter-add of the rows wants neighbouring lanes on neighbouring channels: the order of the blocked layout.
 __device__ __forceinline__ bool LanesHoldNeighbours(const KernelArgs& a) { return a.combineIndex == nullptr; }
@@ -251,7 +250,6 @@ __device__ __forceinline__ bool LanesHoldNeighbours(const KernelArgs& a) { retur
 template <int kOrder, bool kSwiglu>
 __device__ __forceinline__ int ColumnInTile(int w, int n, int l, bool neighbours) {
     if (kSwiglu) return 32 * w + (kOrder == kOrderLane ? 2 * l + (n & 1) : 16 * (n & 1) + l);
-    if (kOrder == kOrderFar) return 128 * (n >> 1) + 32 * w + 16 * (n & 1) + l;
     return 64 * w + (kOrder == kOrderLane && neighbours ? 4 * l + n : 16 * n + l);
 }
 
@@ -382,7 +380,7 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
             // lanes of channels side by side swap one value with their neighbour, and an even lane stores columns (c, c + 1) of
             // the first of two blocks, the odd lane next to it the same pair of the second
             const int32_t laneOff = 4 * quad * a.N + (kOrder == kOrderLane ? col[0] : oddLane ? col[0] + 15 : col[0]);
-            constexpr int kPairStride = kOrder == kOrderFar ? 128 : 32;  // columns from the first two blocks to the other two
+            constexpr int kPairStride = 32;  // columns from the first two blocks to the other two
             auto block = [&](int m, auto fullTag, auto bf16Tag) __attribute__((always_inline)) {
                 constexpr bool kFull = decltype(fullTag)::value;
                 constexpr bool kToBf16 = decltype(bf16Tag)::value;  // compile-time: a run-time choice per element splits the block
@@ -668,6 +666,8 @@ __device__ __forceinline__ int LdsOffset(int row, int chunk) { return row * 128 
 // lanes that the LDS serves together read one chunk of eight consecutive k-rows and of those sixteen further on, and these
 // sixteen pieces land in different bank groups.
 __device__ __forceinline__ int RowMajorSwizzle(int k) { return ((k >> 1) & 3) | (((k >> 4) & 1) << 2); }
+// The same for rows of 256 channel bytes, which begin on the same bank each.
+__device__ __forceinline__ int RowMajorWideSwizzle(int k) { return (k & 7) | (((k >> 4) & 1) << 3); }
 
 // A wave-uniform pointer, forced into scalar registers.
 __device__ __forceinline__ const char* UniformPtr(const char* p) {
@@ -957,12 +957,14 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
             constexpr int kPerHalf = Cfg::kSlotsB / 2;
             const int half = q / kPerHalf, j = waveN + kWavesN * (q % kPerHalf);  // instruction j of its half of the channels
             if (kNMajor) {
-                // instruction j moves k-rows 8 * j .. + 7 of the stage, 128 channel bytes each; chunks past the last
-                // channel are never stored: such lanes re-read the last real chunk
-                const int k = 8 * j + rowIn;
-                const int c = slot ^ RowMajorSwizzle(k);
-                const int32_t col = kSwiglu ? (half ? min(a.halfN + t.colBase + 16 * c, a.N - 16) : min(t.colBase + 16 * c, a.halfN - 16))
-                                            : min(t.colBase + 128 * half + 16 * c, a.N - 16);
+                // Instruction j moves k-rows 4 * j .. + 3 of the stage, 256 channel bytes each (kSwiglu, whose halves lie apart: of its
+                // half k-rows 8 * j .. + 7, 128 bytes each); chunks past the last channel are never stored: such lanes re-read the
+                // last real chunk.  us, 128-byte pieces of each half in all epilogues -> this: 32 experts of 37 rows, K 1440 x N 2880 (rows
+                // that begin inside a line) 42.5 -> 38.8; 128 of 4, 1536 x 4096 141 -> 139; 256 of 4, 2048 x 7168 631 -> 626.
+                const int k = kSwiglu ? 8 * j + rowIn : 4 * (waveN + kWavesN * q) + (lane >> 4);
+                const int c = kSwiglu ? slot ^ RowMajorSwizzle(k) : (lane & 15) ^ RowMajorWideSwizzle(k);
+                const int32_t col = !kSwiglu ? min(t.colBase + 16 * c, a.N - 16)
+                                    : half ? min(a.halfN + t.colBase + 16 * c, a.N - 16) : min(t.colBase + 16 * c, a.halfN - 16);
                 laneOff[q] = static_cast<uint32_t>(k * a.N + col);
             } else if (kNz) {
                 // instruction j moves 32 k-rows (x 32 channel bytes) of channel block j / 4: 1 KB, contiguous in memory and
@@ -1040,29 +1042,28 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     const int l16 = Opaque(tid) & 15, quad = (Opaque(tid) >> 4) & 3;
     const uint32_t rowChunk = l16 * 128 + ((quad ^ ((l16 >> 1) & 7)) << 4);
     const uint32_t laneA = rowChunk + waveM * 16 * 128;  // slice 1 of a k-step is 64 bytes on, or back: buffers and rows begin on 128
-    // Weights of the wave's column.  K-contiguous: as the rows (the second block is sixteen rows on).  Otherwise: the two blocks
-    // (slice 1 is 64 k-rows on and swizzles alike; with the transposing loads this lane supplies half a chunk of k-row k).
-    uint32_t laneB[kNz || kNMajor ? 2 : 1];
+    // Weights of the wave's column.  K-contiguous: as the rows (the second block is sixteen rows on).  Otherwise: the first block,
+    // the others being chunks beside it (slice 1 is 64 k-rows on and swizzles alike; with the transposing loads this lane supplies
+    // half a chunk of k-row k).
+    constexpr bool kWide = kNMajor && !kSwiglu;  // a k-row of a stage is 256 channels side by side, not 128 of each half
+    uint32_t laneB;
     {
         const int k = 16 * quad + (l16 >> 1);
-#pragma unroll
-        for (int i = 0; i < (kNz || kNMajor ? 2 : 1); ++i) {
-            if (kNMajor) laneB[i] = k * 128 + (((2 * waveN + i) ^ RowMajorSwizzle(k)) << 4) + 8 * (l16 & 1);
-            else if (kNz) laneB[i] = waveN * 4096 + k * 32 + 16 * (i ^ (quad & 1)) + 8 * (l16 & 1);
-            else laneB[i] = rowChunk + 32 * waveN * 128;
-        }
+        if (kWide) laneB = k * 256 + (((4 * waveN) ^ RowMajorWideSwizzle(k)) << 4) + 8 * (l16 & 1);
+        else if (kNMajor) laneB = k * 128 + (((2 * waveN) ^ RowMajorSwizzle(k)) << 4) + 8 * (l16 & 1);
+        else if (kNz) laneB = waveN * 4096 + k * 32 + 16 * (quad & 1) + 8 * (l16 & 1);
+        else laneB = rowChunk + 32 * waveN * 128;
     }
     // the wave's four blocks of weights, slice ks
     auto readB = [&](v4i (&b)[4], uint32_t buffer, int ks) __attribute__((always_inline)) {
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
-            const uint32_t base = buffer;
-            const int half = (n >> 1) * Cfg::kHalfBytesB, j = n & 1;
+            const int half = kWide ? 0 : (n >> 1) * Cfg::kHalfBytesB, j = kWide ? n : n & 1;
             if constexpr (kNz || kNMajor) {
-                constexpr int kEightK = kNz ? 8 * 32 : 8 * 128;  // the swizzles of k and k + 8 are the same
-                b[n] = LdsReadTransposed(base + laneB[j], half + ks * 8 * kEightK, kEightK);
+                constexpr int kEightK = kNz ? 8 * 32 : kWide ? 8 * 256 : 8 * 128;  // the swizzles of k and k + 8 are the same
+                b[n] = LdsReadTransposed((buffer + laneB) ^ (16 * j), half + ks * 8 * kEightK, kEightK);
             } else {
-                b[n] = LdsRead16((base + laneB[0]) ^ (64 * ks), half + j * 16 * 128);
+                b[n] = LdsRead16((buffer + laneB) ^ (64 * ks), half + j * 16 * 128);
             }
         }
     };

@@ -94,6 +94,16 @@ def test_outputs_off_the_vector_grid(aclnn, monkeypatch, N, out_dtype, offset, l
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("out_dtype", [torch.int32, torch.bfloat16])
+@pytest.mark.parametrize("layout,N", [("nd", 272), ("nz", 288)])
+@pytest.mark.parametrize("height,K", [(32, 128), (32, 400), (64, 256), (64, 1040), (256, 144)])
+def test_channels_side_by_side_at_every_depth(aclnn, monkeypatch, height, K, layout, N, out_dtype):
+    """Weights whose channels are neighbours in memory: fewer k-steps than the ring has stages, more, and a masked last one."""
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", str(height))
+    got, want = _run(aclnn, [20, 0, 17, 64, 33], N, K, layout, out_dtype, K)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("groups,height", [(128, 256), (129, 256), (192, 192)])
 def test_one_round_of_pulled_tiles_and_one_more(aclnn, monkeypatch, groups, height):
     """Two n-tiles per group: 256 and 258 tiles of 256 rows (256 workgroups), and 384 of 192."""
