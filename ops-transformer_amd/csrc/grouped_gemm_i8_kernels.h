@@ -644,7 +644,9 @@ struct StreamCfg {
     static constexpr int kRingBytes = kLdsBudget - kScratchBytes;
     // as many weight stages as leave room for two of activation rows, then as many of those as fit
     static constexpr int kFitB = (kRingBytes - 2 * kStageBytesA) / kStageBytesB;
-    static constexpr int kStagesB = kFitB > 4 ? 4 : kFitB;
+    // (64 rows: a fourth only puts off the first one's requests in a launch of a tile or two.  us, 8 experts of 20 rows, K 1024 x N 2048,
+    // row-major 16.3 -> 15.8; 16 of 30, K 512 x N 1024 13.4 -> 12.8; 60 of 24, K 768 x N 2048 26.8 -> 26.0; long launches the same.)
+    static constexpr int kStagesB = kRows == 64 ? 3 : kFitB > 4 ? 4 : kFitB;
     static constexpr int kFitA = (kRingBytes - kStagesB * kStageBytesB) / kStageBytesA;
     static constexpr int kStagesA = kFitA > kStagesB ? kStagesB : kFitA;
     static constexpr int kFirstB = kStagesA * kStageBytesA;  // the ring of weight stages, behind that of the activation rows
@@ -835,21 +837,19 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         if (countBig == 0) forSmall = slots;
         prefer = kOneRun ? kRun : (slot < forSmall ? 1 : 0);
     }
-    // thread 0: tile `logical` of a run (list < 0: none) as this workgroup's n-th
-    auto leaveTile = [&](int32_t n, int32_t list, int32_t logical) __attribute__((always_inline)) {
-        int4 e = make_int4(0, 0, 0, 0);
-        if (list >= 0) {
-            const TileInfo t = DecodeListTile<kSwiglu>(a, mTileTable, list ? countBig : 0, list ? countSmall : countBig,
-                                                       list ? bandSmall : bandBig, logical);
-            e = make_int4(t.group, t.rowBase, t.rows, t.tileN);
-        }
-        *reinterpret_cast<int4*>(ldsSeq + 4 * (n & 7)) = e;
+    // one thread: tile `logical` of a run (list < 0: none), decoded, and as this workgroup's n-th
+    auto decodeTile = [&](int32_t list, int32_t logical) __attribute__((always_inline)) -> int4 {
+        if (list < 0) return make_int4(0, 0, 0, 0);
+        const TileInfo t = DecodeListTile<kSwiglu>(a, mTileTable, list ? countBig : 0, list ? countSmall : countBig,
+                                                   list ? bandSmall : bandBig, logical);
+        return make_int4(t.group, t.rowBase, t.rows, t.tileN);
     };
-    auto leaveShareTile = [&](int32_t n) __attribute__((always_inline)) {
+    auto leaveTile = [&](int32_t n, int4 e) __attribute__((always_inline)) { *reinterpret_cast<int4*>(ldsSeq + 4 * (n & 7)) = e; };
+    auto shareTile = [&](int32_t n) __attribute__((always_inline)) -> int4 {
         const int32_t local = slot + n * slots;
         const int32_t logical = xcdFirst + local;
         const bool none = local >= perXcd || logical >= totalTiles;
-        leaveTile(n, none ? -1 : logical < bigTiles ? 0 : 1, logical < bigTiles ? logical : logical - bigTiles);
+        return decodeTile(none ? -1 : logical < bigTiles ? 0 : 1, logical < bigTiles ? logical : logical - bigTiles);
     };
     // the n-th tile of this workgroup, out of the ring
     auto tileAt = [&](int32_t n) __attribute__((always_inline)) -> TileInfo {
@@ -863,6 +863,8 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         t.colBase = kSwiglu ? t.tileN * (kTileN / 2) : t.tileN * kTileN;
         return t;
     };
+    // Side by side: their table entries are one round trip (0.3 to 1.2 us of a launch of shares, as one thread's loop).
+    if (!pull && tid < kTilesAhead) leaveTile(tid, shareTile(tid));
     if (tid == 0) {
         if (pull) {
             // A run of no more tiles than there are workgroups: one tile each.  A second one drawn along with it would be missing
@@ -884,12 +886,9 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                 if (d.list >= 0) {
                     d = QueueResolve(bigTiles, totalTiles - bigTiles, a.queueCounters, xcd, prefer, d.usedUp, c, n == 0 ? v[0] : v[1], kOneRun);
                 }
-                leaveTile(n, d.list, d.logical);
+                leaveTile(n, decodeTile(d.list, d.logical));
             }
             ldsSeq[kSeqUsedUp] = static_cast<int32_t>(d.usedUp);
-        } else {
-#pragma unroll 1
-            for (int n = 0; n < kTilesAhead; ++n) leaveShareTile(n);
         }
     }
     __syncthreads();
@@ -1184,8 +1183,11 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         // requests are counted back in issue order and the draw, an atomic that is settled at the memory side, takes
         // microseconds on a loaded machine: in front of the k loop it would hold up the count of every operand part
         // issued after it.  During the epilogue the ring is full and nothing is issued.
+        // A share's next tile is asked for there as well, on small tiles, whose epilogue is short beside the table's round trip.
         int32_t drawValue = 0;
+        int4 sharesNext = make_int4(0, 0, 0, 0);
         auto draw = [&]() __attribute__((always_inline)) {
+            if (kSmallTile && !pull && tid == 0) sharesNext = shareTile(curNo + kTilesAhead);
             if (pull && following.valid && tid == 0) {
                 const int c = QueueFirstOpen(static_cast<uint32_t>(ldsSeq[kSeqUsedUp]), xcd, prefer, kOneRun);
                 ldsSeq[kSeqDrawCounter] = c;
@@ -1204,10 +1206,10 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         if (pull && tid == 0) {
             const QueueDraw d = QueueResolve(bigTiles, totalTiles - bigTiles, a.queueCounters, xcd, prefer,
                                              static_cast<uint32_t>(ldsSeq[kSeqUsedUp]), ldsSeq[kSeqDrawCounter], drawValue, kOneRun);
-            leaveTile(curNo + 2, d.list, d.logical);
+            leaveTile(curNo + 2, decodeTile(d.list, d.logical));
             ldsSeq[kSeqUsedUp] = static_cast<int32_t>(d.usedUp);
         }
-        if (!pull && tid == 0) leaveShareTile(curNo + kTilesAhead);
+        if (!pull && tid == 0) leaveTile(curNo + kTilesAhead, kSmallTile ? sharesNext : shareTile(curNo + kTilesAhead));
         __syncthreads();  // the epilogue's reads of ldsRowScale / ldsRowMax are done; the drawn tile is in the ring
         if (kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kRows) ldsRowScale[Opaque(tid)] = followingRowScale;
         WaitLds();

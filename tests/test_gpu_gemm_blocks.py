@@ -104,6 +104,14 @@ def test_channels_side_by_side_at_every_depth(aclnn, monkeypatch, height, K, lay
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("height,groups,N,K", [(32, 400, 1024, 128), (64, 200, 4096, 384)])
+def test_shares_of_more_tiles_than_the_ring_holds(aclnn, monkeypatch, height, groups, N, K):
+    """1600 and 3200 small tiles: seven and thirteen to a workgroup, of which six are decoded ahead."""
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", str(height))
+    got, want = _run(aclnn, [1, 3] * (groups // 2), N, K, "k", torch.bfloat16, K)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("groups,height", [(128, 256), (129, 256), (192, 192)])
 def test_one_round_of_pulled_tiles_and_one_more(aclnn, monkeypatch, groups, height):
     """Two n-tiles per group: 256 and 258 tiles of 256 rows (256 workgroups), and 384 of 192."""
