@@ -91,8 +91,8 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const v4i* LdsV4iPtr;
 typedef float Float2 __attribute__((ext_vector_type(2)));
 typedef float Float4 __attribute__((ext_vector_type(4)));
-// Vectors that begin on any four bytes, which is all that a global store of several dwords asks for.
-typedef uint32_t Uint2Dword __attribute__((ext_vector_type(2), aligned(4)));
+// Vectors that begin on any element: a global store of several dwords may begin on any byte.
+typedef uint32_t Uint2Half __attribute__((ext_vector_type(2), aligned(2)));
 typedef int Int4Dword __attribute__((ext_vector_type(4), aligned(4)));
 typedef float Float4Dword __attribute__((ext_vector_type(4), aligned(4)));
 typedef __bf16 Bf16x2 __attribute__((ext_vector_type(2)));
@@ -293,6 +293,24 @@ __device__ __forceinline__ float RowLane(float v) {
     return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(__float_as_uint(v)), kCtl, 0xF, 0xF, true)));
 }
 
+template <int kCtl>
+__device__ __forceinline__ uint32_t RowLane(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), kCtl, 0xF, 0xF, true));
+}
+
+// kOrderBlock, 16-bit values: a lane holds channel l of each of its four blocks, 0 and 1 in the first word, 2 and 3 in the second.
+// In every four lanes side by side, lane i (l & 3) gets the four lanes' channels of block i: one store of eight bytes, and sixteen
+// lanes fill a cache line.  (Of int32 results, where this is sixteen instructions for four values, it measured 1 to 3 % slower than
+// stores of a block each: 16 groups of 1000 rows, K 2048 x N 4096 163 against 159 us.)
+__device__ __forceinline__ void BlockOfLane(uint32_t (&word)[2], int l16) {
+    const bool odd = (l16 & 1) != 0, far = (l16 & 2) != 0;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) word[p] = __builtin_amdgcn_perm(RowLane<0xB1>(word[p]), word[p], odd ? 0x03020706u : 0x05040100u);
+    const uint32_t got = RowLane<0x4E>(far ? word[0] : word[1]);
+    word[0] = far ? got : word[0];
+    word[1] = far ? word[1] : got;
+}
+
 // Maximum over the 16 lanes of a row group, in every lane (rotations inside the row: no LDS).
 __device__ __forceinline__ float MaxOver16(float v) {
     v = fmaxf(v, RowLane<0x128>(v));  // row_ror:8
@@ -368,19 +386,19 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
         afterScaleLoads();
         // wave-uniform: every channel of the wave exists
         const bool whole = t.colBase + ColumnInTile<kOrder, false>(waveN, 3, 15, neighbours) < a.N;
-        // Pairs of 16-bit results start on whole dwords; 32-bit results always do.  us, K 2048 x N 4098, with vectors only where rows
+        // Where a lane's four 16-bit results begin, which it stores at once (kOrderBlock: behind BlockOfLane).  us, stores of a block's half
+        // lines -> this, bf16, row-major / blocked: 16 groups of 500 rows, K 128 x N 4096 29.3 -> 23.7 / 28.8 -> 23.7; 32 of 400,
+        // K 512 x N 2048 32.4 -> 28.3 / 32.5 -> 28.7; 16 of 1000, K 2048 x N 4096 141 -> 131 / 140 -> 133.
+        const int32_t vectorCol = kOrder == kOrderLane ? col[0] : t.colBase + 64 * waveN + 16 * (l16 & 3) + 4 * (l16 >> 2);
+        // Rows of 16-bit results start on whole dwords, if the output does; 32-bit results always do.  us, K 2048 x N 4098, with vectors only where rows
         // start on 16 bytes -> on any dword: 16 groups of 128 rows bf16 71 -> 63, int32 74 -> 61; of 1000 rows 210 -> 195, 231 -> 180.
-        const bool pairs = (a.N & 1) == 0 && (kOrder != kOrderLane || (reinterpret_cast<uintptr_t>(a.out) & 3) == 0);
-        const bool oddLane = (l16 & 1) != 0;
+        const bool pairs = (a.N & 1) == 0;
         if (kEpi == Epilogue::kDequant && (a.outDtype == 27 || a.outDtype == 1) && whole && pairs) {
             // 16-bit results of whole column blocks, without per-element dtype dispatch; stores through a (uniform row pointer
             // + 32-bit lane offset) address.  Past the caches: nothing reads them back before they have left these.
             const bool toBf16 = a.outDtype == 27;  // wave-uniform: bf16, else fp16
             uint16_t* const outTile = static_cast<uint16_t*>(a.out) + static_cast<int64_t>(rowBase) * a.N;
-            // lanes of channels side by side swap one value with their neighbour, and an even lane stores columns (c, c + 1) of
-            // the first of two blocks, the odd lane next to it the same pair of the second
-            const int32_t laneOff = 4 * quad * a.N + (kOrder == kOrderLane ? col[0] : oddLane ? col[0] + 15 : col[0]);
-            constexpr int kPairStride = 32;  // columns from the first two blocks to the other two
+            const int32_t laneOff = 4 * quad * a.N + vectorCol;
             auto block = [&](int m, auto fullTag, auto bf16Tag) __attribute__((always_inline)) {
                 constexpr bool kFull = decltype(fullTag)::value;
                 constexpr bool kToBf16 = decltype(bf16Tag)::value;  // compile-time: a run-time choice per element splits the block
@@ -396,16 +414,8 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
                     uint32_t word[2] = {PackHalves<kToBf16>(y[0], y[1]), PackHalves<kToBf16>(y[2], y[3])};
                     uint16_t* const rowPtr = outTile + static_cast<int64_t>(rTop + v) * a.N;
                     const bool ok = kFull || rTop + 4 * quad + v < rows;
-                    if constexpr (kOrder == kOrderLane) {
-                        if (ok) __builtin_nontemporal_store(Uint2Dword{word[0], word[1]}, reinterpret_cast<Uint2Dword*>(rowPtr + laneOff));
-                    } else {
-#pragma unroll
-                        for (int p = 0; p < 2; ++p) {
-                            const uint32_t got = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(word[p]), 0xB1, 0xF, 0xF, true));
-                            word[p] = __builtin_amdgcn_perm(got, word[p], oddLane ? 0x03020706u : 0x05040100u);
-                            if (ok) __builtin_nontemporal_store(word[p], reinterpret_cast<uint32_t*>(rowPtr + laneOff + kPairStride * p));
-                        }
-                    }
+                    if constexpr (kOrder == kOrderBlock) BlockOfLane(word, l16);
+                    if (ok) __builtin_nontemporal_store(Uint2Half{word[0], word[1]}, reinterpret_cast<Uint2Half*>(rowPtr + laneOff));
                 }
             };
 #pragma unroll
