@@ -224,9 +224,9 @@ __device__ __forceinline__ QueueDraw QueueResolve(int32_t tilesBig, int32_t tile
 
 // ---------------------------------------------------------------------------------------------- tiles and their waves
 // A tile is up to kRows rows x 256 channels, computed by eight waves: two wave rows x four wave columns.  The matrix
-// instruction is v_mfma_i32_16x16x64_i8: per operation it costs the power of 0.85 of a 32x32x32 one -- eight waves per CU on
-// register operands sustain 4.10 POP/s with it against 3.48, uniform random bytes, both at the power limit (4.84 / 4.92
-// with zeros) -- and it splits a tile's rows in sixteens.
+// instruction is v_mfma_i32_16x16x64_i8: per operation it costs the power of 0.89 of a 32x32x32 one -- eight waves per CU on
+// register operands sustain 3.74 to 3.82 POP/s with it against 3.36 to 3.43, uniform random bytes, both at the power limit (4.83 to
+// 4.87 and 4.80 to 4.86 with zeros; opapiInt8MfmaRateProbe) -- and it splits a tile's rows in sixteens.
 //   Rows: 16-row block b of the tile belongs to wave row b & 1, and there to its first half (b & 2 == 0) or its second, as
 //   number b >> 2: whatever the tile's row count, the four (wave row, half) pairs hold the same number of blocks but for one.
 //   Channels: the 256 channels are two halves of 128 rows in LDS, 32 of each belonging to each wave column, as two blocks
@@ -390,8 +390,9 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
         // lines -> this, bf16, row-major / blocked: 16 groups of 500 rows, K 128 x N 4096 29.3 -> 23.7 / 28.8 -> 23.7; 32 of 400,
         // K 512 x N 2048 32.4 -> 28.3 / 32.5 -> 28.7; 16 of 1000, K 2048 x N 4096 141 -> 131 / 140 -> 133.
         const int32_t vectorCol = kOrder == kOrderLane ? col[0] : t.colBase + 64 * waveN + 16 * (l16 & 3) + 4 * (l16 >> 2);
-        // Rows of 16-bit results start on whole dwords, if the output does; 32-bit results always do.  us, K 2048 x N 4098, with vectors only where rows
-        // start on 16 bytes -> on any dword: 16 groups of 128 rows bf16 71 -> 63, int32 74 -> 61; of 1000 rows 210 -> 195, 231 -> 180.
+        // Rows of 16-bit results start on whole dwords, if the output does; 32-bit results always do.  us, K 2048 x N 4098, with vectors
+        // only where rows start on 16 bytes -> on any dword: 16 groups of 128 rows bf16 71 -> 63, int32 74 -> 61; of 1000 rows
+        // 210 -> 195, 231 -> 180.
         const bool pairs = (a.N & 1) == 0;
         if (kEpi == Epilogue::kDequant && (a.outDtype == 27 || a.outDtype == 1) && whole && pairs) {
             // 16-bit results of whole column blocks, without per-element dtype dispatch; stores through a (uniform row pointer
@@ -1101,7 +1102,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
             };
             // The product of one half of the rows with one slice, and between its instructions, if asked for, the requests of the even
             // or the odd slots.  From one row block to the next the weight blocks are walked back and forth: consecutive instructions
-            // share an operand, which costs the matrix unit 2 % less power (4.02 / 4.14 POP/s on register operands).
+            // share an operand, which costs the matrix unit 2 to 3 % less power.
             auto multiply = [&](auto halfTag, int ks, bool requests, int odd = 0) __attribute__((always_inline)) {
                 constexpr int kHalf = decltype(halfTag)::value;
                 constexpr int kCount = kHalf ? kMy1 : kMy0, kOnes = kCount > 0 ? kCount : 1;

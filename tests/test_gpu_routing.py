@@ -388,7 +388,7 @@ def test_quant_v2_outputs_are_rewritten_and_empty_input(aclnn, oracle, dev):
                                           (3000, 4, 5000, 0), (3000, 4, 5000, 777)])
 @pytest.mark.parametrize("dtype,H", [(np.float32, 1), (np.int8, 4), (np.float16, 2)])
 def test_four_byte_rows_are_copied_by_the_sort(aclnn, oracle, dev, T, K, E, active, dtype, H):
-    """Rows of exactly four bytes (the column of per-token scales that the chain routes with a second call) are written by
+    """Rows of exactly four bytes (a column of per-token scales, routed with a call of its own) are written by
     the sort's last scatter, without a gather launch: one-workgroup sort, three-kernel sort and the two-pass sort of a wide
     expert range, with and without activeNum cutting the rows off."""
     rng = np.random.default_rng(T + K + E + active + H)
