@@ -224,9 +224,9 @@ __device__ __forceinline__ QueueDraw QueueResolve(int32_t tilesBig, int32_t tile
 
 // ---------------------------------------------------------------------------------------------- tiles and their waves
 // A tile is up to kRows rows x 256 channels, computed by eight waves: two wave rows x four wave columns.  The matrix
-// instruction is v_mfma_i32_16x16x64_i8: per operation it costs the power of 0.89 of a 32x32x32 one -- eight waves per CU on
-// register operands sustain 3.74 to 3.82 POP/s with it against 3.36 to 3.43, uniform random bytes, both at the power limit (4.83 to
-// 4.87 and 4.80 to 4.86 with zeros; opapiInt8MfmaRateProbe) -- and it splits a tile's rows in sixteens.
+// instruction is v_mfma_i32_16x16x64_i8: per operation it costs the power of 0.85 to 0.9 of a 32x32x32 one -- eight waves per CU
+// on register operands sustain 3.7 to 4.1 POP/s with it, depending on the card, and 3.4 to 3.5 with that, uniform random bytes,
+// both at the power limit (4.8 to 4.9 both with zeros; opapiInt8MfmaRateProbe) -- and it splits a tile's rows in sixteens.
 //   Rows: 16-row block b of the tile belongs to wave row b & 1, and there to its first half (b & 2 == 0) or its second, as
 //   number b >> 2: whatever the tile's row count, the four (wave row, half) pairs hold the same number of blocks but for one.
 //   Channels: the 256 channels are two halves of 128 rows in LDS, 32 of each belonging to each wave column, as two blocks
