@@ -146,7 +146,9 @@ def check_ring_barrier_waits(asm_path):
     """Third build-time guard: a barrier among a ring kernel's matrix instructions frees LDS buffers for DMAs that the compiler does
     not see, so the wave's reads of them have to have been waited for.  In the device assembly of StreamGemmKernel and
     MixedGemmKernel, going back from every s_barrier inside a basic block that multiplies, a wait for LDS (lgkmcnt of at most four:
-    the reads of the rows' second half, which the barrier does not free) has to come before any LDS read.
+    the reads of the rows' second half, which the barrier does not free) has to come before any LDS read.  Nor may such a block wait for
+    every memory request (vmcnt(0) or a counter past it): the compiler does so where it believes a register's load still pending, and
+    the DMAs in flight are then drained in every k-step.
     Returns the number of barriers checked."""
     checked = 0
     for body in open(asm_path).read().split("; -- Begin function ")[1:]:
@@ -158,6 +160,8 @@ def check_ring_barrier_waits(asm_path):
             l = l.split(";")[0].strip()
             if l.endswith(":") or l.startswith("s_cbranch"):  # a basic block ends
                 multiplies = any(i.startswith("v_mfma") for i in block)
+                if multiplies and any(i.startswith("s_waitcnt") and "vmcnt(0)" in i for i in block):
+                    raise RuntimeError("%s: %s drains its DMAs in the k loop" % (asm_path, name))
                 for at in [i for i, ins in enumerate(block) if multiplies and ins.startswith("s_barrier")]:
                     settled = False
                     for ins in reversed(block[:at]):

@@ -255,7 +255,8 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
     const int32_t wideBands = totalMTiles >= 2 * totals[3] ? kGroupM : 1;
     if (t < kQueueHeaderInts) {
         a.sched[t] = t == 0 ? nBig : t == 1 ? nSmall : t == 2 ? nSmall * kSmallCost : t == 3 ? totals[2] : t == 4 ? wideBands
-                   : t == 5 ? (allSmall ? wideBands : 1) : t == kHdrCoveredRows ? sCovered : t == kHdrTileM ? tileM : 0;
+                   : t == 5 ? (allSmall ? wideBands : 1) : t == kHdrCoveredRows ? sCovered : t == kHdrTileM ? tileM
+                   : t == kHdrEven ? (totalMTiles * 8 <= totals[3] * 9 && nSmall * 8 <= totals[3] ? 1 : 0) : 0;
     }
     int4* const mTileTable = reinterpret_cast<int4*>(a.sched + kQueueHeaderInts + kQueueCounterInts);
     for (int32_t m = t; m < totalMTiles; m += 1024) {

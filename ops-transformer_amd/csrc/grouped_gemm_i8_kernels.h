@@ -108,7 +108,7 @@ constexpr int kLdsBudget = 160 * 1024;
 // ---------------------------------------------------------------------------------------------- scheduling table
 // int32 layout, all written by the scheduling kernel:
 //   header, 32 ints: [0] big m-tiles, [1] small m-tiles, [2] cost of the small ones, [3] cost of the big ones (see below),
-//                    [4] / [5] band width of the big / small run, [6] total rows covered by the groups, [7] rows per m-tile;
+//                    [4] / [5] band width of the big / small run, [6] total rows covered by the groups, [7] rows per m-tile, [8] 1: nearly every group is one big m-tile;
 //   16 tile counters in one 128-byte line (32 ints): counter [2 * xcd + list], zeroed;
 //   the m-tile table, 4 ints per m-tile {group, first row, rows, 0} (at most maxMTiles of them): the big m-tiles in group
 //   order, then the small ones.  A GEMM kernel finds everything about a tile with one 16-byte load.
@@ -125,6 +125,7 @@ constexpr int kQueueHeaderInts = 32;
 constexpr int kQueueCounterInts = 32;
 constexpr int kHdrCoveredRows = 6;
 constexpr int kHdrTileM = 7;
+constexpr int kHdrEven = 8;
 // A height that the scheduling kernel may choose instead of 192 or 256 rows (Plan::lowTileM).
 constexpr int kLowTileM = 160;
 __host__ __device__ inline int SchedTotalInts(int maxMTiles) { return kQueueHeaderInts + kQueueCounterInts + 4 * maxMTiles; }
@@ -140,6 +141,28 @@ struct TileInfo {
     int32_t colBase;  // first output channel (kSwiglu: first column of S)
 };
 
+// An entry of the m-tile table, which nothing writes while a GEMM kernel runs: where the index is the wave's, through the scalar
+// cache, past the DMAs that a vector load would wait behind.
+__device__ __forceinline__ v4i ConstantEntry(const int4* table, int32_t i) {
+    typedef __attribute__((address_space(4))) const v4i* EntryPtr;
+    return ((EntryPtr)(reinterpret_cast<uintptr_t>(table)))[i];
+}
+
+// What the header says of the two runs.  Read again wherever it is wanted: held in scalar registers across the k loop it would push out
+// what that needs there.
+struct RunTable {
+    const int4* entries;
+    int32_t countBig, countSmall;  // m-tiles
+    int32_t bandBig, bandSmall;
+};
+__device__ __forceinline__ RunTable ReadRunTable(const int32_t* sched) {
+    typedef __attribute__((address_space(4))) const int32_t* HeaderPtr;
+    auto h = (HeaderPtr)(reinterpret_cast<uintptr_t>(sched));
+    asm volatile("" : "+s"(h));
+    return RunTable{reinterpret_cast<const int4*>(reinterpret_cast<uintptr_t>(h) + (kQueueHeaderInts + kQueueCounterInts) * sizeof(int32_t)),
+                    h[0], h[1], h[4], h[5]};
+}
+
 // Tile `logical` of one run of the m-tile table (`count` m-tiles from entry `first` on).  Bands of bandWidth m-tiles walk
 // the n-tiles together: consecutive tiles are the band's m-tiles at one n-tile, then the next n-tile.
 template <bool kSwiglu>
@@ -151,11 +174,11 @@ __device__ __forceinline__ TileInfo DecodeListTile(const KernelArgs& a, const in
     const int32_t rem = logical - band * perBand;
     const int32_t bandTiles = min(bandWidth, count - bandWidth * band);
     const int32_t tileN = rem / bandTiles;
-    const int4 e = table[first + bandWidth * band + rem - tileN * bandTiles];
+    const v4i e = ConstantEntry(table, first + bandWidth * band + rem - tileN * bandTiles);
     t.valid = 1;
-    t.group = e.x;
-    t.rowBase = e.y;
-    t.rows = e.z;
+    t.group = e[0];
+    t.rowBase = e[1];
+    t.rows = e[2];
     t.tileN = tileN;
     t.colBase = kSwiglu ? t.tileN * (kTileN / 2) : t.tileN * kTileN;
     return t;
@@ -167,14 +190,29 @@ __device__ __forceinline__ TileInfo DecodeListTile(const KernelArgs& a, const in
 // [2 * xcd + list] hands out the tiles of a share in order.  A workgroup draws from its own XCD first -- the list it
 // prefers, then the other -- and, when both are used up, from the other XCDs' shares in ring order, so nobody idles
 // while tiles are left anywhere.  The counters are only ever added to (values past a share's size mean "used up").
+// The first `seated` tiles of every share are not drawn but dealt out (see the seats).
 // (The lists' sizes travel as plain values: a structure handed round by reference, or an array indexed at run time,
 // ends up in scratch memory.)
-__device__ __forceinline__ void QueueShare(int32_t tilesBig, int32_t tilesSmall, int counter, int32_t* first, int32_t* size) {
-    const int32_t total = (counter & 1) ? tilesSmall : tilesBig;
+struct QueueLists {
+    int32_t tilesBig, tilesSmall;
+    int32_t seatedBig, seatedSmall;  // tiles of a share that workgroups begin with
+};
+__device__ __forceinline__ void QueueShare(const QueueLists q, int counter, int32_t* first, int32_t* size) {
+    const int32_t total = (counter & 1) ? q.tilesSmall : q.tilesBig;
     const int32_t per = (total + kXcds - 1) / kXcds;
     const int32_t begin = (counter >> 1) * per;
-    *first = begin;
-    *size = total - begin < 0 ? 0 : (total - begin < per ? total - begin : per);
+    const int32_t all = max(min(total - begin, per), 0), seated = min((counter & 1) ? q.seatedSmall : q.seatedBig, all);
+    *first = begin + seated;
+    *size = all - seated;
+}
+// Workgroups of an XCD's `slots` that begin with the small m-tiles: the share that their cost is of the whole, so that lists of many
+// rounds run dry at about the same time; until then a part of the machine streams weights for a handful of rows each while
+// the rest multiplies.
+__device__ __forceinline__ int32_t SlotsForSmall(const int32_t* __restrict__ hdr, int32_t slots) {
+    const int64_t costSmall = hdr[2], costAll = costSmall + hdr[3];
+    int64_t forSmall = costAll > 0 ? (slots * costSmall + costAll / 2) / costAll : 0;
+    if (forSmall == 0 && hdr[1] > 0 && slots > 1) forSmall = 1;
+    return static_cast<int32_t>(forSmall);
 }
 // Counter i-th in the preference order of a workgroup on XCD `home` that prefers list `prefer`.
 __device__ __forceinline__ int QueueCandidate(int i, int home, int prefer) {
@@ -190,8 +228,12 @@ __device__ __forceinline__ int QueueFirstOpen(uint32_t usedUp, int home, int pre
     }
     return -1;
 }
+// (One lane's.  The zero keeps the address out of the compiler's sight: seen to be the same in every lane, it adds the wave's lanes up
+// first and waits for the answer on the spot to deal it out, microseconds in which the caller has other work to do.)
 __device__ __forceinline__ int32_t QueueTake(int32_t* counters, int c) {
-    return __hip_atomic_fetch_add(counters + c, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    int32_t zero;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+    return __hip_atomic_fetch_add(counters + c + zero, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // Completes a draw that began with QueueTake on counter c (value v; c < 0: nothing was open): returns the list (0 big,
 // 1 small) and the tile inside that list's run, or list -1 when every share is used up.  One thread of the workgroup.
@@ -200,11 +242,11 @@ struct QueueDraw {
     int32_t logical;  // tile inside that list's run
     uint32_t usedUp;  // the caller's mask of used-up counters, updated
 };
-__device__ __forceinline__ QueueDraw QueueResolve(int32_t tilesBig, int32_t tilesSmall, int32_t* counters, int home, int prefer,
+__device__ __forceinline__ QueueDraw QueueResolve(const QueueLists q, int32_t* counters, int home, int prefer,
                                                   uint32_t usedUp, int c, int32_t v, bool onlyPreferred = false) {
     while (c >= 0) {
         int32_t first, size;
-        QueueShare(tilesBig, tilesSmall, c, &first, &size);
+        QueueShare(q, c, &first, &size);
         if (v < size) return QueueDraw{c & 1, first + v, usedUp};
         usedUp |= 1u << c;
         // a look at all sixteen counters at once (one round trip) spares a failed draw, i.e. a round trip, per used-up share
@@ -213,7 +255,7 @@ __device__ __forceinline__ QueueDraw QueueResolve(int32_t tilesBig, int32_t tile
         for (int i = 0; i < 2 * kXcds; ++i) now[i] = __hip_atomic_load(counters + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
         for (int i = 0; i < 2 * kXcds; ++i) {
-            QueueShare(tilesBig, tilesSmall, i, &first, &size);
+            QueueShare(q, i, &first, &size);
             if (now[i] >= size) usedUp |= 1u << i;
         }
         c = QueueFirstOpen(usedUp, home, prefer, onlyPreferred);
@@ -319,6 +361,9 @@ __device__ __forceinline__ float MaxOver16(float v) {
     return fmaxf(v, RowLane<0x121>(v));
 }
 
+// Raises a maximum in LDS, kept as the bits of a float that is not negative, to m (NaN counts as nothing, as it does with fmaxf).
+__device__ __forceinline__ void RaiseRowMax(uint32_t* ldsMax, float m) { atomicMax(ldsMax, __float_as_uint(fmaxf(m, 0.0f))); }
+
 // Maxima of four values over the 16 lanes of a row group: lane l gets that of value l >> 2.  A halving butterfly: a lane
 // gives its partner the values that it drops.
 __device__ __forceinline__ float FourMaxOver16(const float (&m)[4], int l16) {
@@ -348,19 +393,27 @@ struct RowBlocks {
 };
 
 // Epilogue of one tile.  acc[m][n][v] is C[row, col] with row = RowOf(m) + 4 * quad + v and col = ColumnInTile(n) of lane l16.
-// ldsRowScale holds the tile's per-row scales.
-// afterScaleLoads() is called once the channel scales of the tile have been requested and before anything is stored: a
-// memory request made there queues behind loads whose answers the epilogue needs first, not in front of them.
+// ldsRowScale holds the tile's per-row scales, ldsChannelScale those of its 256 channels by their place in the tile (null: they are
+// loaded here).  kSwiglu: ldsRowMax, zero before, takes the tile's row maxima of |S| as float bits (TileEpilogueStoreMax).
+// beforeStores() is called between the arithmetic and the stores of whole column blocks, in front of both elsewhere (256 rows: see there).
 // Row checks are made per 16-row block, wave-uniformly: a block wholly inside the expert's rows takes a copy of the code
 // without checks, a block wholly outside is skipped, and only the one that straddles the last row tests every lane.  (A
 // per-lane test makes every element a predicated basic block of its own, and their independent chains no longer interleave.)
+// Values that may have been loaded are waited for here: were they still pending on some path into the k loop, the compiler would
+// drain every DMA there.
+template <int kCount>
+__device__ __forceinline__ void SettleLoads(float (&v)[kCount]) {
+#pragma unroll
+    for (int i = 0; i < kCount; ++i) asm volatile("" : "+v"(v[i]));
+}
+
 struct NoHook {
     __device__ __forceinline__ void operator()() const {}
 };
 template <int kRows, Epilogue kEpi, int kOrder, typename Hook = NoHook>
 __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const TileInfo& t, v4i (&acc)[RowBlocks<kRows>::kAll][4], int waveM,
-                                                 int waveN, int l16, int quad, const float* ldsRowScale, float* ldsRowMax,
-                                                 Hook afterScaleLoads = NoHook{}) {
+                                                 int waveN, int l16, int quad, const float* ldsChannelScale, const float* ldsRowScale,
+                                                 uint32_t* ldsRowMax, Hook beforeStores = NoHook{}) {
     using Blocks = RowBlocks<kRows>;
     constexpr bool kSwiglu = kEpi == Epilogue::kSwiglu;
     const int32_t rows = t.rows, rowBase = t.rowBase, group = t.group;
@@ -381,9 +434,12 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
         for (int n = 0; n < 4; ++n) {
             col[n] = t.colBase + ColumnInTile<kOrder, false>(waveN, n, l16, neighbours);
             valid[n] = col[n] < a.N;
-            if (kEpi == Epilogue::kDequant && valid[n]) sc[n] = LoadScale(a.scale, static_cast<int64_t>(group) * a.N + col[n], a.scaleDtype);
+            if (kEpi == Epilogue::kDequant) {
+                if (ldsChannelScale != nullptr) sc[n] = ldsChannelScale[ColumnInTile<kOrder, false>(waveN, n, l16, neighbours)];
+                else if (valid[n]) sc[n] = LoadScale(a.scale, static_cast<int64_t>(group) * a.N + col[n], a.scaleDtype);
+            }
         }
-        afterScaleLoads();
+        SettleLoads(sc);
         // wave-uniform: every channel of the wave exists
         const bool whole = t.colBase + ColumnInTile<kOrder, false>(waveN, 3, 15, neighbours) < a.N;
         // Where a lane's four 16-bit results begin, which it stores at once (kOrderBlock: behind BlockOfLane).  us, stores of a block's half
@@ -394,45 +450,72 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
         // only where rows start on 16 bytes -> on any dword: 16 groups of 128 rows bf16 71 -> 63, int32 74 -> 61; of 1000 rows
         // 210 -> 195, 231 -> 180.
         const bool pairs = (a.N & 1) == 0;
-        if (kEpi == Epilogue::kDequant && (a.outDtype == 27 || a.outDtype == 1) && whole && pairs) {
-            // 16-bit results of whole column blocks, without per-element dtype dispatch; stores through a (uniform row pointer
-            // + 32-bit lane offset) address.  Past the caches: nothing reads them back before they have left these.
-            const bool toBf16 = a.outDtype == 27;  // wave-uniform: bf16, else fp16
-            uint16_t* const outTile = static_cast<uint16_t*>(a.out) + static_cast<int64_t>(rowBase) * a.N;
-            const int32_t laneOff = 4 * quad * a.N + vectorCol;
-            auto block = [&](int m, auto fullTag, auto bf16Tag) __attribute__((always_inline)) {
-                constexpr bool kFull = decltype(fullTag)::value;
-                constexpr bool kToBf16 = decltype(bf16Tag)::value;  // compile-time: a run-time choice per element splits the block
-                const int rTop = Blocks::RowOf(m, waveM);
-                float4 rs = make_float4(1.0f, 1.0f, 1.0f, 1.0f);  // multiplying by 1 is exact
-                if (hasRowScale) rs = *reinterpret_cast<const float4*>(ldsRowScale + rTop + 4 * quad);
-                const float rsv[4] = {rs.x, rs.y, rs.z, rs.w};
+        // 16-bit results of whole column blocks, without per-element dtype dispatch; stores through a (uniform row pointer
+        // + 32-bit lane offset) address.  Past the caches: nothing reads them back before they have left these.
+        const bool halves = kEpi == Epilogue::kDequant && (a.outDtype == 27 || a.outDtype == 1) && whole && pairs;
+        const bool toBf16 = a.outDtype == 27;  // wave-uniform: bf16, else fp16
+        // The tallest tiles have no registers for the results of all blocks beside the accumulators of those to come: a block's are stored
+        // before the next one's are worked out, and beforeStores() comes behind them all, where the DMAs have landed.
+        constexpr bool kAllAtOnce = kRows < 256;
+        uint32_t word[kAllAtOnce ? Blocks::kAll : 1][4][2];
+        auto results = [&](int m, uint32_t (&w)[4][2], auto bf16Tag) __attribute__((always_inline)) {
+            constexpr bool kToBf16 = decltype(bf16Tag)::value;  // compile-time: a run-time choice per element splits the block
+            const int rTop = Blocks::RowOf(m, waveM);
+            float4 rs = make_float4(1.0f, 1.0f, 1.0f, 1.0f);  // multiplying by 1 is exact
+            if (hasRowScale) rs = *reinterpret_cast<const float4*>(ldsRowScale + rTop + 4 * quad);
+            const float rsv[4] = {rs.x, rs.y, rs.z, rs.w};
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    float y[4];
+            for (int v = 0; v < 4; ++v) {
+                float y[4];
 #pragma unroll
-                    for (int n = 0; n < 4; ++n) y[n] = __fmul_rn(__fmul_rn(static_cast<float>(acc[m][n][v]), sc[n]), rsv[v]);
-                    uint32_t word[2] = {PackHalves<kToBf16>(y[0], y[1]), PackHalves<kToBf16>(y[2], y[3])};
-                    uint16_t* const rowPtr = outTile + static_cast<int64_t>(rTop + v) * a.N;
-                    const bool ok = kFull || rTop + 4 * quad + v < rows;
-                    if constexpr (kOrder == kOrderBlock) BlockOfLane(word, l16);
-                    if (ok) __builtin_nontemporal_store(Uint2Half{word[0], word[1]}, reinterpret_cast<Uint2Half*>(rowPtr + laneOff));
-                }
-            };
+                for (int n = 0; n < 4; ++n) y[n] = __fmul_rn(__fmul_rn(static_cast<float>(acc[m][n][v]), sc[n]), rsv[v]);
+                w[v][0] = PackHalves<kToBf16>(y[0], y[1]);
+                w[v][1] = PackHalves<kToBf16>(y[2], y[3]);
+            }
+        };
+        auto forBlocks = [&](auto f) __attribute__((always_inline)) {
 #pragma unroll
             for (int m = 0; m < Blocks::kAll; ++m) {
                 const int rTop = Blocks::RowOf(m, waveM);
                 if (rTop >= rows) continue;
-                if (rTop + 16 <= rows) {
-                    if (toBf16) block(m, std::true_type{}, std::true_type{});
-                    else block(m, std::true_type{}, std::false_type{});
-                } else {
-                    if (toBf16) block(m, std::false_type{}, std::true_type{});
-                    else block(m, std::false_type{}, std::false_type{});
+                if (rTop + 16 <= rows) f(m, std::true_type{});
+                else f(m, std::false_type{});
+            }
+        };
+        if constexpr (kAllAtOnce) {
+            if (halves) {
+                if (toBf16) forBlocks([&](int m, auto) __attribute__((always_inline)) { results(m, word[m], std::true_type{}); });
+                else forBlocks([&](int m, auto) __attribute__((always_inline)) { results(m, word[m], std::false_type{}); });
+            }
+        }
+        if constexpr (kAllAtOnce) beforeStores();
+        if (halves) {
+            uint16_t* const outTile = static_cast<uint16_t*>(a.out) + static_cast<int64_t>(rowBase) * a.N;
+            const int32_t laneOff = 4 * quad * a.N + vectorCol;
+            auto store = [&](int m, uint32_t (&w)[4][2], auto fullTag) __attribute__((always_inline)) {
+                constexpr bool kFull = decltype(fullTag)::value;
+                const int rTop = Blocks::RowOf(m, waveM);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    uint16_t* const rowPtr = outTile + static_cast<int64_t>(rTop + v) * a.N;
+                    const bool ok = kFull || rTop + 4 * quad + v < rows;
+                    if constexpr (kOrder == kOrderBlock) BlockOfLane(w[v], l16);
+                    if (ok) __builtin_nontemporal_store(Uint2Half{w[v][0], w[v][1]}, reinterpret_cast<Uint2Half*>(rowPtr + laneOff));
                 }
+            };
+            if constexpr (kAllAtOnce) {
+                forBlocks([&](int m, auto fullTag) __attribute__((always_inline)) { store(m, word[m], fullTag); });
+            } else {
+                forBlocks([&](int m, auto fullTag) __attribute__((always_inline)) {
+                    if (toBf16) results(m, word[0], std::true_type{});
+                    else results(m, word[0], std::false_type{});
+                    store(m, word[0], fullTag);
+                });
+                beforeStores();
             }
             return;
         }
+        if constexpr (!kAllAtOnce) beforeStores();
         const bool vectorStores = neighbours && whole;
         float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         if (kEpi == Epilogue::kDequant && a.bias != nullptr) {
@@ -440,6 +523,7 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
             for (int n = 0; n < 4; ++n) {
                 if (valid[n]) bias[n] = LoadScale(a.bias, static_cast<int64_t>(group) * a.N + col[n], a.biasDtype);
             }
+            SettleLoads(bias);
         }
 #pragma unroll
         for (int m = 0; m < Blocks::kAll; ++m) {
@@ -515,12 +599,17 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
             col[j] = t.colBase + ColumnInTile<kOrder, true>(waveN, j, l16, true);
             valid[j] = col[j] < a.halfN;
             scA[j] = scB[j] = 0.0f;
-            if (valid[j]) {
+            if (ldsChannelScale != nullptr) {
+                const int c = ColumnInTile<kOrder, true>(waveN, j, l16, true);
+                scA[j] = ldsChannelScale[c];
+                scB[j] = ldsChannelScale[kTileN / 2 + c];
+            } else if (valid[j]) {
                 scA[j] = LoadScale(a.scale, static_cast<int64_t>(group) * a.N + col[j], a.scaleDtype);
                 scB[j] = LoadScale(a.scale, static_cast<int64_t>(group) * a.N + a.halfN + col[j], a.scaleDtype);
             }
         }
-        afterScaleLoads();
+        SettleLoads(scA);
+        SettleLoads(scB);
         // swish(ca) * cb with the hardware exp2 / reciprocal: a few ulp from the correctly rounded value, far inside the
         // +-1 LSB the int8 requantisation is held to
         auto activated = [&](int m, int j, int v, float xs) __attribute__((always_inline)) {
@@ -530,10 +619,9 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
         };
         // wave-uniform: every column of the wave exists, and S rows start on a lane's pair
         const bool whole = t.colBase + 32 * waveN + 32 <= a.halfN && (kOrder != kOrderLane || (a.halfN & 1) == 0);
+        Float2 s[Blocks::kAll][4];
         if (whole) {
-            float* const sTile = a.sOut + static_cast<int64_t>(rowBase) * a.halfN;
-            const int32_t laneOff = 4 * quad * a.halfN + col[0];
-            auto block = [&](int m, auto fullTag) __attribute__((always_inline)) {
+            auto results = [&](int m, auto fullTag) __attribute__((always_inline)) {
                 constexpr bool kFull = decltype(fullTag)::value;
                 const int rTop = Blocks::RowOf(m, waveM);
                 const float4 xs4 = *reinterpret_cast<const float4*>(ldsRowScale + rTop + 4 * quad);
@@ -541,26 +629,46 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
                 float top[4];
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    const float s0 = activated(m, 0, v, xs[v]), s1 = activated(m, 1, v, xs[v]);
-                    float* const sRow = sTile + static_cast<int64_t>(rTop + v) * a.halfN;
+                    s[m][v] = Float2{activated(m, 0, v, xs[v]), activated(m, 1, v, xs[v])};
                     const bool ok = kFull || rTop + 4 * quad + v < rows;
-                    if constexpr (kOrder == kOrderLane) {
-                        if (ok) __builtin_nontemporal_store(Float2{s0, s1}, reinterpret_cast<Float2*>(sRow + laneOff));
-                    } else {
-                        if (ok) __builtin_nontemporal_store(s0, sRow + laneOff);
-                        if (ok) __builtin_nontemporal_store(s1, sRow + laneOff + 16);
-                    }
-                    top[v] = ok ? fmaxf(fabsf(s0), fabsf(s1)) : 0.0f;
+                    top[v] = ok ? fmaxf(fabsf(s[m][v][0]), fabsf(s[m][v][1])) : 0.0f;
                 }
                 const float m16 = FourMaxOver16(top, l16);
-                if ((l16 & 3) == 0) ldsRowMax[waveN * kRows + rTop + 4 * quad + (l16 >> 2)] = m16;
+                if ((l16 & 3) == 0) RaiseRowMax(ldsRowMax + rTop + 4 * quad + (l16 >> 2), m16);
             };
 #pragma unroll
             for (int m = 0; m < Blocks::kAll; ++m) {
                 const int rTop = Blocks::RowOf(m, waveM);
                 if (rTop >= rows) continue;
-                if (rTop + 16 <= rows) block(m, std::true_type{});
-                else block(m, std::false_type{});
+                if (rTop + 16 <= rows) results(m, std::true_type{});
+                else results(m, std::false_type{});
+            }
+        }
+        beforeStores();
+        if (whole) {
+            float* const sTile = a.sOut + static_cast<int64_t>(rowBase) * a.halfN;
+            const int32_t laneOff = 4 * quad * a.halfN + col[0];
+            auto store = [&](int m, auto fullTag) __attribute__((always_inline)) {
+                constexpr bool kFull = decltype(fullTag)::value;
+                const int rTop = Blocks::RowOf(m, waveM);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    float* const sRow = sTile + static_cast<int64_t>(rTop + v) * a.halfN;
+                    const bool ok = kFull || rTop + 4 * quad + v < rows;
+                    if constexpr (kOrder == kOrderLane) {
+                        if (ok) __builtin_nontemporal_store(s[m][v], reinterpret_cast<Float2*>(sRow + laneOff));
+                    } else {
+                        if (ok) __builtin_nontemporal_store(s[m][v][0], sRow + laneOff);
+                        if (ok) __builtin_nontemporal_store(s[m][v][1], sRow + laneOff + 16);
+                    }
+                }
+            };
+#pragma unroll
+            for (int m = 0; m < Blocks::kAll; ++m) {
+                const int rTop = Blocks::RowOf(m, waveM);
+                if (rTop >= rows) continue;
+                if (rTop + 16 <= rows) store(m, std::true_type{});
+                else store(m, std::false_type{});
             }
             return;
         }
@@ -581,24 +689,19 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
                     }
                 }
                 top = MaxOver16(top);
-                if (l16 == 0) ldsRowMax[waveN * kRows + r] = top;
+                if (l16 == 0) RaiseRowMax(ldsRowMax + r, top);
             }
         }
     }
 }
 
-// The part of the kSwiglu epilogue that follows the waves' own work: folds the four wave columns' partial row maxima
-// into one per (n-tile, row).  Contains a workgroup barrier: every wave must call it (the workgroup has at least
-// kRows threads).
+// The part of the kSwiglu epilogue behind a barrier: one partial maximum per (n-tile, row) goes to memory -- no atomics there and
+// nothing to pre-zero; the requantisation folds them -- and the LDS copies start at zero again.  (The workgroup has at least kRows threads.)
 template <int kRows>
-__device__ __forceinline__ void TileEpilogueFoldMax(const KernelArgs& a, const TileInfo& t, int tid, const float* ldsRowMax) {
-    __syncthreads();
-    // one partial maximum per (n-tile, row): no atomics and nothing to pre-zero; the requantisation folds them
+__device__ __forceinline__ void TileEpilogueStoreMax(const KernelArgs& a, const TileInfo& t, int tid, uint32_t* ldsRowMax) {
     if (tid < t.rows) {
-        float m = ldsRowMax[tid];
-#pragma unroll
-        for (int w = 1; w < kWavesN; ++w) m = fmaxf(m, ldsRowMax[w * kRows + tid]);
-        a.rowMax[static_cast<int64_t>(t.tileN) * a.M + t.rowBase + tid] = m;
+        a.rowMax[static_cast<int64_t>(t.tileN) * a.M + t.rowBase + tid] = __uint_as_float(ldsRowMax[tid]);
+        ldsRowMax[tid] = 0;
     }
 }
 
@@ -650,8 +753,9 @@ struct StreamCfg {
     static constexpr int kStageBytesA = kRows * kStep;
     static constexpr int kStageBytesB = kTileN * kStep;
     static constexpr int kHalfBytesB = kStageBytesB / 2;
-    static constexpr int kQueueLdsInts = 36;  // the workgroup's next eight tiles and its draw state
-    static constexpr int kScratchBytes = (1 + kWavesN) * kRows * 4 + kQueueLdsInts * 4;
+    static constexpr int kQueueLdsInts = 40;  // the workgroup's next eight tiles and how it comes by them
+    static constexpr int kRowScales = (kRows + 63) / 64 * 64;  // in whole DMA instructions
+    static constexpr int kScratchBytes = (kTileN + kRowScales + kRows + kQueueLdsInts) * 4;  // channel scales, row scales, row maxima, tiles
     static constexpr int kRingBytes = kLdsBudget - kScratchBytes;
     // as many weight stages as leave room for two of activation rows, then as many of those as fit
     static constexpr int kFitB = (kRingBytes - 2 * kStageBytesA) / kStageBytesB;
@@ -730,6 +834,13 @@ __device__ __forceinline__ void DmaToLdsAddr16(const char* base, uint32_t laneOf
     }
 }
 
+// 4 bytes per lane from (uniform base + lane offset) into LDS at ldsAddr + lane * 4 (see DmaToLdsAddr16).
+__device__ __forceinline__ void DmaToLdsAddr4(const char* base, uint32_t laneOffset, uint32_t ldsAddr) {
+    const uint32_t m0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(ldsAddr)));
+    const char* const sbase = UniformPtr(base);
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(m0), "v"(laneOffset), "s"(sbase) : "memory");
+}
+
 // The value itself, through a statement the optimiser cannot see through: what is computed from the copy stays where it
 // is written.  Used on lane indices at the head of per-tile code, so that the per-lane offsets and addresses of that code
 // are recomputed once per tile instead of being hoisted out of the tile loop and held in registers (or spilled) across the
@@ -741,11 +852,14 @@ __device__ __forceinline__ int Opaque(int v) {
 
 // The kernel's arguments (its first parameter), read again from memory.  What only the epilogue wants of them would otherwise stay
 // in scalar registers across the k loop, and those of the tallest tiles, once spilled, cost vector registers that are not there.
+// (Through the address space of constants, i.e. the scalar cache: vector loads, which is what a plain pointer gives here, would wait
+// behind every DMA in flight.)
 __device__ __forceinline__ KernelArgs ReloadArgs() {
-    auto p = __builtin_amdgcn_kernarg_segment_ptr();
+    typedef __attribute__((address_space(4))) const KernelArgs* ArgsPtr;
+    auto p = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(p));
     KernelArgs a;
-    __builtin_memcpy(&a, (const void*)p, sizeof(a));
+    __builtin_memcpy(&a, p, sizeof(a));
     return a;
 }
 
@@ -790,7 +904,7 @@ __device__ __forceinline__ void PhaseBarrier() {
 //
 // kRun: which runs of the m-tile table the body serves.  kBothRuns: all of it (pulled or in fixed shares).  kBigRun /
 // kSmallRun: that run only, pulled, until its counters are used up on every XCD -- the form in which MixedGemmKernel
-// calls the body twice, once per run with a stage geometry of that run's own.
+// calls the body twice, once per run with a stage geometry of that run's own; `begins` says for which of them.
 //
 // kTail: K is a multiple of 16 and at least one k-step, but no multiple of a k-step.  The last k-step then starts kStep
 // bytes before the end of K instead of behind the step before it: every DMA stays inside its row and is as wide as any
@@ -801,13 +915,14 @@ __device__ __forceinline__ void PhaseBarrier() {
 constexpr int kBigRun = 0, kSmallRun = 1, kBothRuns = 2;
 template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, int kRun, bool kTail>
 __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_t* __restrict__ sched, char* const lds,
-                                               uint64_t& spanTiles) {
+                                               uint64_t& spanTiles, bool begins = true) {
     static_assert(!(kNz && kNMajor), "one weight layout at a time");
     using Cfg = StreamCfg<kRows>;
     using Blocks = RowBlocks<kRows>;
     constexpr bool kSwiglu = kEpi == Epilogue::kSwiglu;
-    float* const ldsRowScale = reinterpret_cast<float*>(lds + Cfg::kFirstB + Cfg::kStagesB * Cfg::kStageBytesB);  // [kRows]
-    float* const ldsRowMax = ldsRowScale + kRows;                                            // [kWavesN][kRows]
+    float* const ldsChannelScale = reinterpret_cast<float*>(lds + Cfg::kFirstB + Cfg::kStagesB * Cfg::kStageBytesB);  // [kTileN]
+    float* const ldsRowScale = ldsChannelScale + kTileN;                                     // [kRowScales]
+    uint32_t* const ldsRowMax = reinterpret_cast<uint32_t*>(ldsRowScale + Cfg::kRowScales);  // [kRows]
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -815,53 +930,39 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     const int waveM = wave / kWavesN;
 
     // ---- this workgroup's sequence of tiles ----
-    // Workgroup b serves XCD b % 8 as its slot b / 8.  Thread 0 finds the tiles and leaves them, decoded, in an eight-entry ring
-    // in LDS.  With a.pullTiles they come out of the tile counters (see QueueShare), and tile n + 2 is drawn while tile n's
-    // epilogue runs (the draw goes out at its head, the answer is looked at behind it), because the issue side already reads
-    // tile n + 1's operands during tile n.  Otherwise the two runs of the m-tile table are one list cut into eight fixed
+    // Workgroup b serves XCD b % 8 as its slot b / 8.  Wave 0 finds the tiles and leaves them, decoded, in an eight-entry ring
+    // in LDS.  With a.pullTiles the first ones are its seat's and the others come out of the tile counters (see QueueShare): tile n + 2 is
+    // drawn while tile n's epilogue runs, because the issue side already reads tile n + 1's operands during tile n.  Otherwise the two runs of the m-tile table are one list cut into eight fixed
     // shares, which the workgroups of an XCD walk with stride gridDim / 8, and the ring holds six tiles (tiles of one k-step
     // have the issue side five tiles ahead).
-    const int32_t* const queueHdr = sched;
-    const int32_t countBig = queueHdr[0], countSmall = queueHdr[1];  // m-tiles per list
-    const int32_t bandBig = queueHdr[4], bandSmall = queueHdr[5];
-    const int4* const mTileTable = reinterpret_cast<const int4*>(queueHdr + kQueueHeaderInts + kQueueCounterInts);
     const int xcd = blockIdx.x % kXcds;
     const int32_t slots = gridDim.x / kXcds;
     const int32_t slot = blockIdx.x / kXcds;
     constexpr bool kOneRun = kRun != kBothRuns;
     const bool pull = kOneRun || a.pullTiles != 0;
-    const int32_t bigTiles = countBig * a.tilesN;
-    const int32_t totalTiles = bigTiles + countSmall * a.tilesN;
-    const int32_t perXcd = (totalTiles + kXcds - 1) / kXcds;
-    const int32_t xcdFirst = xcd * perXcd;
-    int32_t* const ldsSeq = reinterpret_cast<int32_t*>(ldsRowMax + kWavesN * kRows);
-    constexpr int kSeqUsedUp = 32, kSeqDrawCounter = 33;  // thread 0's draw state, behind the ring
+    int32_t* const ldsSeq = reinterpret_cast<int32_t*>(ldsRowMax + kRows);
+    // wave 0's state, behind the ring: used-up counters, tiles of a share that are dealt out (big, small), this workgroup's next tile of those,
+    // how many it has left, and how far apart they are
+    constexpr int kSeqUsedUp = 32, kSeqSeated = 33, kSeqSeatNext = 35, kSeqSeatLeft = 36, kSeqSeatStride = 37;
     constexpr int kTilesAhead = 6;
-    // Which list this workgroup draws from first: the small m-tiles get the share of each XCD's workgroups that their
-    // cost is of the whole, so that lists of many rounds run dry at about the same time (short ones: see the first draws);
-    // until then a part of the machine streams weights for a handful of rows each while the rest multiplies.
-    int prefer = 0;
-    {
-        const int64_t costSmall = queueHdr[2], costAll = costSmall + queueHdr[3];
-        int64_t forSmall = costAll > 0 ? (slots * costSmall + costAll / 2) / costAll : 0;
-        if (forSmall == 0 && countSmall > 0 && slots > 1) forSmall = 1;
-        if (countBig == 0) forSmall = slots;
-        prefer = kOneRun ? kRun : (slot < forSmall ? 1 : 0);
-    }
-    // one thread: tile `logical` of a run (list < 0: none), decoded, and as this workgroup's n-th
-    auto decodeTile = [&](int32_t list, int32_t logical) __attribute__((always_inline)) -> int4 {
-        if (list < 0) return make_int4(0, 0, 0, 0);
-        const TileInfo t = DecodeListTile<kSwiglu>(a, mTileTable, list ? countBig : 0, list ? countSmall : countBig,
-                                                   list ? bandSmall : bandBig, logical);
-        return make_int4(t.group, t.rowBase, t.rows, t.tileN);
+    // Which list this workgroup draws from first.
+    const int32_t forSmall = sched[0] == 0 ? slots : SlotsForSmall(sched, slots);
+    const int prefer = kOneRun ? kRun : (slot < forSmall ? 1 : 0);
+    // tile `logical` of a run (list < 0: none), decoded
+    auto decodeTile = [&](const KernelArgs& args, const RunTable& r, int32_t list, int32_t logical) __attribute__((always_inline)) -> v4i {
+        if (list < 0) return v4i{0, 0, 0, 0};
+        const TileInfo t = DecodeListTile<kSwiglu>(args, r.entries, list ? r.countBig : 0, list ? r.countSmall : r.countBig,
+                                                   list ? r.bandSmall : r.bandBig, logical);
+        return v4i{t.group, t.rowBase, t.rows, t.tileN};
     };
-    auto leaveTile = [&](int32_t n, int4 e) __attribute__((always_inline)) { *reinterpret_cast<int4*>(ldsSeq + 4 * (n & 7)) = e; };
-    auto shareTile = [&](int32_t n) __attribute__((always_inline)) -> int4 {
-        const int32_t local = slot + n * slots;
-        const int32_t logical = xcdFirst + local;
-        const bool none = local >= perXcd || logical >= totalTiles;
-        return decodeTile(none ? -1 : logical < bigTiles ? 0 : 1, logical < bigTiles ? logical : logical - bigTiles);
+    // the n-th tile of this workgroup in fixed shares
+    auto shareTile = [&](const KernelArgs& args, const RunTable& r, int32_t n) __attribute__((always_inline)) -> v4i {
+        const int32_t big = r.countBig * args.tilesN, total = big + r.countSmall * args.tilesN;
+        const int32_t perXcd = (total + kXcds - 1) / kXcds, local = slot + n * slots, logical = xcd * perXcd + local;
+        const bool none = local >= perXcd || logical >= total;
+        return decodeTile(args, r, none ? -1 : logical < big ? 0 : 1, logical < big ? logical : logical - big);
     };
+    auto leaveTile = [&](int32_t n, v4i e) __attribute__((always_inline)) { *reinterpret_cast<v4i*>(ldsSeq + 4 * (n & 7)) = e; };
     // the n-th tile of this workgroup, out of the ring
     auto tileAt = [&](int32_t n) __attribute__((always_inline)) -> TileInfo {
         const int4 e = *reinterpret_cast<const int4*>(ldsSeq + 4 * (n & 7));
@@ -875,29 +976,66 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         return t;
     };
     // Side by side: their table entries are one round trip (0.3 to 1.2 us of a launch of shares, as one thread's loop).
-    if (!pull && tid < kTilesAhead) leaveTile(tid, shareTile(tid));
-    if (tid == 0) {
-        if (pull) {
-            // A run of no more tiles than there are workgroups: one tile each.  A second one drawn along with it would be missing
-            // where another workgroup is idle (128 tiles of K 14336: 200 us, or 400 where one had two).  In the two-geometry
-            // form fewer workgroups than that begin with the run; they go on to the other run after their one tile, and the tiles
-            // left of this one fill the last round of that.  us, drawing on until the run is used up -> one each: 8 experts of 1000
-            // rows, gate/up 7168 x 2 x 2048 with 4 of 40 rows 303 -> 262, K 14336 x N 4096 with 4 of 60 514 -> 448; K 1408 x
-            // N 2048, 216 big and 104 small tiles 67 -> 52; the other way round 830 -> 858 at most (of sixty launches).
-            const bool oneRound = (kRun == kBigRun ? bigTiles : kRun == kSmallRun ? totalTiles - bigTiles : totalTiles) <= static_cast<int32_t>(gridDim.x);
-            // the first two tiles: both draws go out together
-            const int c = QueueFirstOpen(0, xcd, prefer, kOneRun);
-            int32_t v[2];
-            v[0] = QueueTake(a.queueCounters, c);
-            v[1] = oneRound ? 0 : QueueTake(a.queueCounters, c);
-            QueueDraw d{0, 0, 0};
+    if (!pull && tid < kTilesAhead) leaveTile(tid, shareTile(a, ReadRunTable(sched), tid));
+    if (kSwiglu && tid < kRows) ldsRowMax[tid] = 0;
+    // Seats: the first `each` tiles of a workgroup are not drawn but dealt out, those of seats side by side neighbours.  Two, so that no
+    // draw stands in front of the launch, and an XCD's workgroups walk neighbouring tiles from the start (two draws at once handed
+    // each of them two neighbours, its first round being every other tile of twice as many groups).  All whole rounds where the tiles are
+    // alike (kHdrEven): those launches are bound by memory, where a workgroup that lags gets the bandwidth that others leave, while one
+    // that is ahead and draws a tile more ends the launch alone.  us, 128 experts of 128 rows, gate/up 4096 x 2 x 1536 and down, six
+    // and eight rounds: drawn 344 / 207, two dealt out 334 / 204, all 327 / 194; 256 experts, 7168, 2048: 1441 / 800, 1425 / 772,
+    // 1427 / 762.  Not so where tiles differ: 65536 rows at popularity rank^-1.2, all dealt out, 2264 / 1220 against 1940 / 1080.
+    // A run of no more tiles than there are workgroups: one tile each.  A second one taken along with it would be missing
+    // where another workgroup is idle (128 tiles of K 14336: 200 us, or 400 where one had two).  In the two-geometry
+    // form fewer workgroups than that begin with the run; they go on to the other run after their one tile, and the tiles
+    // left of this one fill the last round of that.  us, drawing on until the run is used up -> one each: 8 experts of 1000
+    // rows, gate/up 7168 x 2 x 2048 with 4 of 40 rows 303 -> 262, K 14336 x N 4096 with 4 of 60 514 -> 448; K 1408 x
+    // N 2048, 216 big and 104 small tiles 67 -> 52; the other way round 830 -> 858 at most (of sixty launches).
+    if (wave == 0 && pull) {
+        const RunTable runs = ReadRunTable(sched);
+        const int32_t bigTiles = runs.countBig * a.tilesN, smallTiles = runs.countSmall * a.tilesN;
+        auto eachOf = [&](int32_t tiles, int32_t seats) __attribute__((always_inline)) {
+            return (kOneRun ? tiles : bigTiles + smallTiles) <= static_cast<int32_t>(gridDim.x) ? 1
+                   : max(2, sched[kHdrEven] != 0 && seats > 0 ? tiles / kXcds / seats : 0);
+        };
+        const int32_t eachBig = eachOf(bigTiles, slots - forSmall), eachSmall = eachOf(smallTiles, forSmall);
+        const QueueLists lists{bigTiles, smallTiles, eachBig * (slots - forSmall), eachSmall * forSmall};
+        const int32_t seats = prefer ? forSmall : slots - forSmall, seat = prefer ? slot : slot - forSmall;
+        const int32_t each = prefer ? eachSmall : eachBig;
+        int32_t first, size;
+        QueueShare(QueueLists{bigTiles, smallTiles, 0, 0}, 2 * xcd + prefer, &first, &size);
+        // tiles that this workgroup is dealt: seat, seat + seats, ... of the share
+        const int32_t dealt = begins && seat < size ? min(each, (size - seat + seats - 1) / seats) : 0;
+        int32_t drawnFirst, drawn;
+        QueueShare(lists, tid & (2 * kXcds - 1), &drawnFirst, &drawn);
+        const uint32_t allSeated = static_cast<uint32_t>(__ballot(tid < 2 * kXcds && drawn <= 0));  // shares without a tile to draw
+        if (tid == 0) {
+            ldsSeq[kSeqUsedUp] = static_cast<int32_t>(allSeated);
+            ldsSeq[kSeqSeated] = lists.seatedBig;
+            ldsSeq[kSeqSeated + 1] = lists.seatedSmall;
+            ldsSeq[kSeqSeatNext] = first + seat + 2 * seats;
+            ldsSeq[kSeqSeatLeft] = dealt - 2;
+            ldsSeq[kSeqSeatStride] = seats;
+        }
+        if (dealt >= min(each, 2)) {
+            const v4i tile0 = decodeTile(a, runs, prefer, first + seat), tile1 = decodeTile(a, runs, each == 1 ? -1 : prefer, first + seat + seats);
+            if (tid == 0) {
+                leaveTile(0, tile0);
+                leaveTile(1, tile1);
+            }
+        } else if (tid == 0) {  // both draws, if there are two, go out together
+            const int c = QueueFirstOpen(allSeated, xcd, prefer, kOneRun);
+            int32_t v[2] = {0, 0};
+            if (c >= 0) {
+                if (dealt < 1) v[0] = QueueTake(a.queueCounters, c);
+                if (each > 1) v[1] = QueueTake(a.queueCounters, c);
+            }
+            QueueDraw d{prefer, first + seat, allSeated};
 #pragma unroll 1
             for (int n = 0; n < 2; ++n) {
-                if (n == 1 && oneRound) d.list = -1;
-                if (d.list >= 0) {
-                    d = QueueResolve(bigTiles, totalTiles - bigTiles, a.queueCounters, xcd, prefer, d.usedUp, c, n == 0 ? v[0] : v[1], kOneRun);
-                }
-                leaveTile(n, decodeTile(d.list, d.logical));
+                if (n >= each) d.list = -1;
+                else if (n >= dealt && d.list >= 0) d = QueueResolve(lists, a.queueCounters, xcd, prefer, d.usedUp, c, n == 0 ? v[0] : v[1], kOneRun);
+                leaveTile(n, decodeTile(a, runs, d.list, d.logical));
             }
             ldsSeq[kSeqUsedUp] = static_cast<int32_t>(d.usedUp);
         }
@@ -1039,10 +1177,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         for (int q = 0; q < Cfg::kSlotsB; ++q) request(q);
         advance();
     }
-    if (kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kRows) {
-        ldsRowScale[tid] = a.rowScale[cur.rowBase + (tid < cur.rows ? tid : cur.rows - 1)];
-    }
-    // the first stage has landed (the row scales' load makes that only stricter)
+    // the first stage has landed
     if (forWeights) WaitVmcnt<(Cfg::kStagesB - 1) * Cfg::kSlotsB>();
     else WaitVmcnt<(Cfg::kStagesA - 1) * Cfg::kSlotsA>();
     __syncthreads();
@@ -1078,9 +1213,34 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         }
     };
 
+    // The scales of a tile travel with its first k-step, by DMA into LDS (4 bytes a lane: the wave rows' waves take 64 channels, or rows,
+    // each): loaded in the epilogue they would come behind every stage in flight.  The k loop certifies them with the stages it requests
+    // itself, where it is as long as the ring.
+    const bool rowScalesByDma = kSteps >= Cfg::kStagesB && reinterpret_cast<uintptr_t>(a.rowScale) % 4 == 0;
+    const bool channelScalesByDma = kEpi != Epilogue::kInt32 && kSteps >= Cfg::kStagesB && a.scaleDtype == 0 && reinterpret_cast<uintptr_t>(a.scale) % 4 == 0;
+    auto requestScales = [&]() __attribute__((always_inline)) {
+        const int lane = Opaque(tid) & 63;
+        if (forWeights) {
+            if (channelScalesByDma) {
+                const int c = 64 * waveN + lane;  // of the tile
+                const int32_t col = kSwiglu ? (waveN >= 2 ? min(a.halfN + cur.colBase + c - kTileN / 2, a.N - 1) : min(cur.colBase + c, a.halfN - 1))
+                                            : min(cur.colBase + c, a.N - 1);
+                DmaToLdsAddr4(static_cast<const char*>(a.scale) + static_cast<int64_t>(cur.group) * a.N * 4, static_cast<uint32_t>(col) * 4u,
+                              LdsAddress(reinterpret_cast<const char*>(ldsChannelScale + 64 * waveN)));
+            }
+        } else if (a.rowScale != nullptr && rowScalesByDma && 64 * waveN < kRows) {
+            DmaToLdsAddr4(reinterpret_cast<const char*>(a.rowScale) + static_cast<int64_t>(cur.rowBase) * 4,
+                          static_cast<uint32_t>(min(64 * waveN + lane, cur.rows - 1)) * 4u,
+                          LdsAddress(reinterpret_cast<const char*>(ldsRowScale + 64 * waveN)));
+        } else if (a.rowScale != nullptr && !rowScalesByDma && tid - kThreads / 2 < kRows) {
+            ldsRowScale[tid - kThreads / 2] = a.rowScale[cur.rowBase + min(tid - kThreads / 2, cur.rows - 1)];
+        }
+    };
+
     v4i acc[Blocks::kAll][4];
     while (true) {
         const TileInfo following = tileAt(curNo + 1);
+        if (kEpi != Epilogue::kInt32) requestScales();
 #pragma unroll
         for (int m = 0; m < Blocks::kAll; ++m) {
 #pragma unroll
@@ -1159,7 +1319,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                 multiply(SecondHalf{}, 0, true, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 WaitLds();
-                if (forWeights) WaitVmcnt<Cfg::kYoungerB>();
+                if (forWeights) WaitVmcnt<Cfg::kYoungerB>();  // (stores of the tile before, still under way, make it only stricter)
                 else WaitVmcnt<Cfg::kYoungerA>();
                 PhaseBarrier();
                 if (kMy > 0 && !last) {
@@ -1183,47 +1343,76 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         auto runOne = [&](auto myTag) __attribute__((always_inline)) { runTile(myTag); };
         ForCount<Blocks::kAll>((active + 1 - waveM) >> 1, runOne);
 
-        // The next tile's per-row scale travels in a register until this tile's epilogue has read the LDS copy.  (Not across the k
-        // loop: the tallest tiles have no register left there.)
-        float followingRowScale = 0.0f;
-        if (following.valid && kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kRows) {
-            followingRowScale = a.rowScale[following.rowBase + (tid < following.rows ? tid : following.rows - 1)];
+        // Between the k loop and the next tile's a workgroup asks for nothing, its ring being full, so nothing in here waits for memory
+        // but once, when it has had the tile's arithmetic to answer:
+        //   * the draw for the tile after the next, an atomic that is settled at the memory side, goes out first.  (In front of the k
+        //     loop it would hold up the count of every operand part issued after it: loads return in issue order.)
+        //   * the arithmetic, on scales that are in LDS.
+        //   * every DMA in flight and the draw have landed.  What the ring holds is then certified for the next tile's first steps,
+        //     which need no count of their own, so that the stores may still be under way in them.
+        //   * the drawn tile's entry of the table: one wave, through the scalar cache, while the others store.
+        // us, scales and arguments loaded here, stores drained, draw and entry as two round trips in a row -> this, gate/up / down, two tiles
+        // of a workgroup dealt out on both sides: 128 experts of 128 rows, 4096, 1536 336 / 208 -> 334 / 204; 256, 7168, 2048 1431 / 786 ->
+        // 1425 / 772; 16 of 2000, 4224, 896 216 / 175 -> 208 / 167; 8 of 155, 4096, 14336 215 / 148 -> 211 / 147.
+        v4i next = v4i{0, 0, 0, 0};  // wave 0: the tile that it finds for the ring
+        int32_t drawCounter = -1, drawValue = 0, seatLeft = 0;
+        if (wave == 0 && pull && following.valid) {
+            seatLeft = __builtin_amdgcn_readfirstlane(ldsSeq[kSeqSeatLeft]);
+            if (seatLeft <= 0) {
+                drawCounter = __builtin_amdgcn_readfirstlane(
+                    QueueFirstOpen(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(ldsSeq[kSeqUsedUp])), xcd, prefer, kOneRun));
+                if (drawCounter >= 0 && tid == 0) drawValue = QueueTake(a.queueCounters, drawCounter);
+            }
         }
-
-        // The draw for the tile after the next goes out inside the epilogue and is looked at behind it.  A wave's memory
-        // requests are counted back in issue order and the draw, an atomic that is settled at the memory side, takes
-        // microseconds on a loaded machine: in front of the k loop it would hold up the count of every operand part
-        // issued after it.  During the epilogue the ring is full and nothing is issued.
-        // A share's next tile is asked for there as well, on small tiles, whose epilogue is short beside the table's round trip.
-        int32_t drawValue = 0;
-        int4 sharesNext = make_int4(0, 0, 0, 0);
-        auto draw = [&]() __attribute__((always_inline)) {
-            if (kSmallTile && !pull && tid == 0) sharesNext = shareTile(curNo + kTilesAhead);
-            if (pull && following.valid && tid == 0) {
-                const int c = QueueFirstOpen(static_cast<uint32_t>(ldsSeq[kSeqUsedUp]), xcd, prefer, kOneRun);
-                ldsSeq[kSeqDrawCounter] = c;
-                if (c >= 0) drawValue = QueueTake(a.queueCounters, c);
+        const KernelArgs epilogueArgs = ReloadArgs();
+        auto beforeStores = [&]() __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
+            WaitVmcnt<0>();
+            __builtin_amdgcn_sched_barrier(0);
+            if (wave == 0 && following.valid) {
+                const RunTable runs = ReadRunTable(sched);
+                if (!pull) {
+                    next = shareTile(epilogueArgs, runs, curNo + kTilesAhead);
+                } else if (seatLeft > 0) {
+                    const int32_t logical = __builtin_amdgcn_readfirstlane(ldsSeq[kSeqSeatNext]);
+                    next = decodeTile(epilogueArgs, runs, prefer, logical);
+                    if (tid == 0) {
+                        ldsSeq[kSeqSeatNext] = logical + ldsSeq[kSeqSeatStride];
+                        ldsSeq[kSeqSeatLeft] = seatLeft - 1;
+                    }
+                } else if (drawCounter >= 0) {
+                    const int32_t v = __builtin_amdgcn_readfirstlane(drawValue);
+                    const QueueLists lists{runs.countBig * epilogueArgs.tilesN, runs.countSmall * epilogueArgs.tilesN,
+                                           __builtin_amdgcn_readfirstlane(ldsSeq[kSeqSeated]), __builtin_amdgcn_readfirstlane(ldsSeq[kSeqSeated + 1])};
+                    int32_t first, size;
+                    QueueShare(lists, drawCounter, &first, &size);
+                    int32_t list = drawCounter & 1, logical = first + v;
+                    if (v >= size) {
+                        if (tid == 0) {
+                            const QueueDraw d = QueueResolve(lists, a.queueCounters, xcd, prefer, static_cast<uint32_t>(ldsSeq[kSeqUsedUp]),
+                                                             drawCounter, v, kOneRun);
+                            ldsSeq[kSeqUsedUp] = static_cast<int32_t>(d.usedUp);
+                            list = d.list;
+                            logical = d.logical;
+                        }
+                        list = __builtin_amdgcn_readfirstlane(list);
+                        logical = __builtin_amdgcn_readfirstlane(logical);
+                    }
+                    next = decodeTile(epilogueArgs, runs, list, logical);
+                }
             }
         };
-        const KernelArgs epilogueArgs = ReloadArgs();
-        TileEpilogueWave<kRows, kEpi, kOrderOf<kNz, kNMajor>>(epilogueArgs, cur, acc, waveM, waveN, Opaque(tid) & 15, (Opaque(tid) >> 4) & 3, ldsRowScale,
-                                                              ldsRowMax, draw);
-        if constexpr (kSwiglu) TileEpilogueFoldMax<kRows>(epilogueArgs, cur, Opaque(tid), ldsRowMax);
-        // Loads and stores may retire out of order with respect to each other, so drain everything (the epilogue's
-        // stores and the DMAs in flight, which had the whole epilogue to land) before counting DMAs again.
-        WaitVmcnt<0>();
+        TileEpilogueWave<kRows, kEpi, kOrderOf<kNz, kNMajor>>(epilogueArgs, cur, acc, waveM, waveN, Opaque(tid) & 15, (Opaque(tid) >> 4) & 3,
+                                                              channelScalesByDma ? ldsChannelScale : nullptr, ldsRowScale, ldsRowMax, beforeStores);
+        if (tid == 0 && following.valid) leaveTile(curNo + (pull ? 2 : kTilesAhead), next);
         ++spanTiles;
-        if (!following.valid) break;
-        if (pull && tid == 0) {
-            const QueueDraw d = QueueResolve(bigTiles, totalTiles - bigTiles, a.queueCounters, xcd, prefer,
-                                             static_cast<uint32_t>(ldsSeq[kSeqUsedUp]), ldsSeq[kSeqDrawCounter], drawValue, kOneRun);
-            leaveTile(curNo + 2, decodeTile(d.list, d.logical));
-            ldsSeq[kSeqUsedUp] = static_cast<int32_t>(d.usedUp);
-        }
-        if (!pull && tid == 0) leaveTile(curNo + kTilesAhead, kSmallTile ? sharesNext : shareTile(curNo + kTilesAhead));
-        __syncthreads();  // the epilogue's reads of ldsRowScale / ldsRowMax are done; the drawn tile is in the ring
-        if (kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kRows) ldsRowScale[Opaque(tid)] = followingRowScale;
+        if (!kSwiglu && !following.valid) break;
         WaitLds();
+        PhaseBarrier();  // the reads of the scales are done, the row maxima are complete and the drawn tile is in the ring
+        if constexpr (kSwiglu) {
+            TileEpilogueStoreMax<kRows>(epilogueArgs, cur, Opaque(tid), ldsRowMax);
+            if (!following.valid) break;
+        }
         cur = following;
         ++curNo;
     }
@@ -1268,18 +1457,16 @@ __global__ __launch_bounds__(kThreads) void MixedGemmKernel(KernelArgs a, const 
         WriteSpan(a, spanStart, spanTiles, kLowTileM);
         return;
     }
-    const int64_t costSmall = sched[2], costAll = costSmall + sched[3];
     const int32_t slots = gridDim.x / kXcds, slot = blockIdx.x / kXcds;
-    int64_t forSmall = costAll > 0 ? (slots * costSmall + costAll / 2) / costAll : 0;
-    if (forSmall == 0 && sched[1] > 0 && slots > 1) forSmall = 1;
+    const int32_t forSmall = sched[0] == 0 ? slots : SlotsForSmall(sched, slots);
     if (slot < forSmall) {
         StreamGemmBody<kSmallRows, kEpi, kNz, kNMajor, kSmallRun, kTail>(a, sched, lds, spanTiles);
         __syncthreads();  // the other geometry lays LDS out anew
-        StreamGemmBody<kRows, kEpi, kNz, kNMajor, kBigRun, kTail>(a, sched, lds, spanTiles);
+        StreamGemmBody<kRows, kEpi, kNz, kNMajor, kBigRun, kTail>(a, sched, lds, spanTiles, false);
     } else {
         StreamGemmBody<kRows, kEpi, kNz, kNMajor, kBigRun, kTail>(a, sched, lds, spanTiles);
         __syncthreads();
-        StreamGemmBody<kSmallRows, kEpi, kNz, kNMajor, kSmallRun, kTail>(a, sched, lds, spanTiles);
+        StreamGemmBody<kSmallRows, kEpi, kNz, kNMajor, kSmallRun, kTail>(a, sched, lds, spanTiles, false);
     }
     WriteSpan(a, spanStart, spanTiles);
 }
@@ -1296,7 +1483,7 @@ __global__ __launch_bounds__(kThreads) void GenericGemmKernel(KernelArgs a, cons
     __shared__ __attribute__((aligned(16))) char ldsA[kRows * kStep];
     __shared__ __attribute__((aligned(16))) char ldsB[kTileN * kStep];
     __shared__ __attribute__((aligned(16))) float ldsRowScale[kRows];
-    __shared__ float ldsRowMax[kWavesN * kRows];
+    __shared__ uint32_t ldsRowMax[kRows];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -1320,6 +1507,7 @@ __global__ __launch_bounds__(kThreads) void GenericGemmKernel(KernelArgs a, cons
     if (kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kRows) {
         ldsRowScale[tid] = a.rowScale[t.rowBase + (tid < t.rows ? tid : t.rows - 1)];
     }
+    if (kSwiglu && tid < kRows) ldsRowMax[tid] = 0;
     const int8_t* const wGroup = a.w + static_cast<int64_t>(t.group) * a.wGroupStride;
 
     v4i acc[Blocks::kAll][4];
@@ -1374,8 +1562,11 @@ __global__ __launch_bounds__(kThreads) void GenericGemmKernel(KernelArgs a, cons
         }
         __syncthreads();
     }
-    TileEpilogueWave<kRows, kEpi, kOrderBlock>(a, t, acc, waveM, waveN, l16, quad, ldsRowScale, ldsRowMax);
-    if constexpr (kSwiglu) TileEpilogueFoldMax<kRows>(a, t, tid, ldsRowMax);
+    TileEpilogueWave<kRows, kEpi, kOrderBlock>(a, t, acc, waveM, waveN, l16, quad, nullptr, ldsRowScale, ldsRowMax);
+    if constexpr (kSwiglu) {
+        __syncthreads();
+        TileEpilogueStoreMax<kRows>(a, t, tid, ldsRowMax);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------- launchers

@@ -55,13 +55,6 @@ struct SlimCfg {
     static_assert(kLdsBytes <= kLdsBudget, "LDS of one workgroup");
 };
 
-// 4 bytes per lane from (uniform base + lane offset) into LDS at ldsAddr + lane * 4 (see DmaToLdsAddr16).
-__device__ __forceinline__ void DmaToLdsAddr4(const char* base, uint32_t laneOffset, uint32_t ldsAddr) {
-    const uint32_t m0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(ldsAddr)));
-    const char* const sbase = UniformPtr(base);
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(m0), "v"(laneOffset), "s"(sbase) : "memory");
-}
-
 // Relative cost of a tile of 16, 32 or 64 rows: its weights are the same, but a taller one leaves the ring fewer stages (64
 // tokens evenly over 128 experts, hidden 4096, intermediate 1536: 247 / 251 / 262 us gate/up).  A launch costs its rounds of
 // tiles times that.  What speaks for a taller tile is groups that need several of the lower ones; how many there are is known

@@ -112,6 +112,16 @@ def test_shares_of_more_tiles_than_the_ring_holds(aclnn, monkeypatch, height, gr
     assert torch.equal(got, want)
 
 
+# Groups alike, one m-tile each, eight n-tiles: whole rounds of tiles dealt out, with nothing behind them, one group's tiles, and a part of
+# a round that is drawn; one group in twelve of other rows, more than a tile's, and all rounds but two are drawn
+@pytest.mark.parametrize("height", [96, 192])
+@pytest.mark.parametrize("groups,odd", [(96, 70), (97, 70), (131, 70), (131, 260)])
+def test_even_groups_and_uneven_ones(aclnn, monkeypatch, groups, odd, height):
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", str(height))
+    got, want = _run(aclnn, [odd if e % 12 == 5 else 70 for e in range(groups)], 2048, 1024, "k", torch.bfloat16, groups)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("groups,height", [(128, 256), (129, 256), (192, 192)])
 def test_one_round_of_pulled_tiles_and_one_more(aclnn, monkeypatch, groups, height):
     """Two n-tiles per group: 256 and 258 tiles of 256 rows (256 workgroups), and 384 of 192."""
