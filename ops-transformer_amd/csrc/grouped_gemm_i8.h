@@ -65,7 +65,9 @@ constexpr int64_t kSlimMaxTilesN = 16384;
 struct Plan {
     int tileM = 0;          // rows per workgroup tile (multiple of 32; slim: 16, 32 or 64, the lowest that the kernel may take)
     int lowTileM = 0;       // a lower height that the scheduling kernel may choose instead (0: none)
-    bool lowForRounds = false;  // it chooses by rounds of the machine, else by the rows that groups leave over
+    bool lowForRounds = false;  // it chooses by rounds of the machine,
+    bool lowBySizes = false;    // by how many groups are small or have several m-tiles, else by the rows that groups leave over
+    bool lowIsWide = false;     // those tiles are 512 channels wide
     int64_t maxTiles = 0;   // launch bound on workgroups
     int32_t maxMTiles = 0;  // upper bound on m-tiles of a launch over all groups (its rows / tileM + groups)
     int32_t tilesN = 0;

@@ -49,7 +49,9 @@ struct SchedArgs {
     int32_t isCount;  // 0 cumsum, 1 counts, 2 sparse (expert id, count) pairs
     int32_t tileM;
     int32_t mayLower;  // 1: m-tiles of kLowTileM rows instead where they leave at most an eighth of the groups a small last one;
+                       // 3: for means below those, by how many groups are small or have several m-tiles;
                        // 2: where they fill at most two rounds of the machine, and no more of them than the tall ones
+    int32_t lowIsWide;  // with mayLower 3: the tiles of the lower m-tiles are two 256-channel units wide
     int32_t cus, tilesN;
     int32_t maxMTiles;
     int64_t M;
@@ -157,6 +159,8 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
     end = end < a.rowBegin ? a.rowBegin : (end > a.rowEnd ? a.rowEnd : end);
     const int32_t rows = t < a.groups ? static_cast<int32_t>(end - begin) : 0;
     int32_t tileM = a.tileM, cut = tileM;  // cut: rows per m-tile of this group
+    int32_t wide = 0;
+    bool oneList = false;  // small m-tiles among the big ones
     if (a.mayLower == 2) {
         // Whole rounds of the machine, one of low tiles costing 0.7 to 0.85 of one of tall ones: their ring is a stage deeper, and
         // the launch ends with its tallest tile.  Low tiles where they are one round; where they are two, only if the tall ones
@@ -191,7 +195,37 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
         }
     } else if (a.mayLower) {
         const int32_t last = rows % kLowTileM;
-        if (__syncthreads_count(last > 0 && last <= kSmallRows) * 8 <= a.groups) tileM = cut = kLowTileM;
+        const bool smallLast = last > 0 && last <= kSmallRows;
+        bool lower;
+        if (a.mayLower == 1) {
+            lower = __syncthreads_count(smallLast) * 8 <= a.groups;
+        } else {
+            // Groups of at most kSmallRows rows, nearly all of them: the two-geometry kernel's small run.  us, one geometry / that: 256
+            // experts of 50 rows, hidden 7168, intermediate 2048 1285 (wide) and 736 / 1170 and 708.  Half of them, beside groups of
+            // several m-tiles: that too, 80 rows at rank^-0.6 875 / 808 (down).  Otherwise one geometry, wide only where no group needs a
+            // second m-tile, which costs at least one tile of twice the length at the launch's end: 128 experts, 4096, 1536, 80 rows at
+            // rank^-0.3 332 / 316 with two of them; 60 and 72 rows even 302 / 325 and 299 / 314, down 185 / 199.
+            // (Counted by ballots and one round of LDS: four __syncthreads_count took 3 us.)
+            __shared__ int4 waveCounts[16];
+            const int4 mine = make_int4(__popcll(__ballot(rows > 0)), __popcll(__ballot(rows > 0 && rows <= kSmallRows)),
+                                        __popcll(__ballot(rows > kLowTileM)), __popcll(__ballot(rows > kLowTileM && smallLast)));
+            if ((t & 63) == 0) waveCounts[t >> 6] = mine;
+            __syncthreads();
+            int32_t some = 0, small = 0, over = 0, loses = 0;
+#pragma unroll
+            for (int w = 0; w < 16; ++w) {
+                some += waveCounts[w].x;
+                small += waveCounts[w].y;
+                over += waveCounts[w].z;
+                loses += waveCounts[w].w;
+            }
+            lower = small * 8 < some * 7 && (a.lowIsWide ? over == 0 : loses * 8 <= a.groups && (small * 2 < some || over * 32 < a.groups));
+        }
+        if (lower) {
+            tileM = cut = kLowTileM;
+            wide = a.lowIsWide;
+            oneList = a.mayLower == 3;
+        }
     }
     const int32_t tiles = (rows + cut - 1) / cut;
     // big and small m-tiles of this group (with tiles of at most kSmallRows rows every m-tile is small; otherwise only
@@ -199,7 +233,7 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
     // group the positions of its m-tiles in the two runs of the table, and the launch the totals
     const bool allSmall = tileM <= kSmallRows;
     const int32_t lastRows = tiles > 0 ? rows - (tiles - 1) * cut : 0;
-    const int32_t smallCount = allSmall ? tiles : (tiles > 0 && lastRows <= kSmallRows ? 1 : 0);
+    const int32_t smallCount = allSmall ? tiles : (!oneList && tiles > 0 && lastRows <= kSmallRows ? 1 : 0);
     const int32_t bigCount = tiles - smallCount;
     int32_t bigCost = 0;
     if (bigCount > 0) {
@@ -256,7 +290,8 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
     if (t < kQueueHeaderInts) {
         a.sched[t] = t == 0 ? nBig : t == 1 ? nSmall : t == 2 ? nSmall * kSmallCost : t == 3 ? totals[2] : t == 4 ? wideBands
                    : t == 5 ? (allSmall ? wideBands : 1) : t == kHdrCoveredRows ? sCovered : t == kHdrTileM ? tileM
-                   : t == kHdrEven ? (totalMTiles * 8 <= totals[3] * 9 && nSmall * 8 <= totals[3] ? 1 : 0) : 0;
+                   : t == kHdrWide ? wide
+                   : t == kHdrEven ? (totalMTiles * 8 <= totals[3] * 9 && (nSmall * 8 <= totals[3] || nBig == 0) ? 1 : 0) : 0;
     }
     int4* const mTileTable = reinterpret_cast<int4*>(a.sched + kQueueHeaderInts + kQueueCounterInts);
     for (int32_t m = t; m < totalMTiles; m += 1024) {
@@ -267,7 +302,7 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
         }
         const int32_t inGroup = m - (hi > 0 ? scan[hi - 1] : 0);
         const int32_t tileRows = min(sCut[hi], sRows[hi] - inGroup * sCut[hi]);
-        const bool small = allSmall || tileRows <= kSmallRows;
+        const bool small = allSmall || (!oneList && tileRows <= kSmallRows);
         const int32_t pos = small ? nBig + sSmallBefore[hi] + (allSmall ? inGroup : 0) : sBigBefore[hi] + inGroup;
         const int32_t limit = small ? nBig + nSmall : nBig;
         if (pos < limit) mTileTable[pos] = make_int4(hi, sRowStart[hi] + inGroup * sCut[hi], tileRows, 0);
@@ -541,6 +576,37 @@ Plan MakePlan(const Problem& p) {
         plan.lowTileM = kLowTileM;
         plan.lowForRounds = true;
     }
+    // The SwiGLU operator on groups that 160 rows hold nearly all: tiles of 512 channels instead of 256, where that costs no round of the
+    // machine, on the two-geometry kernel, which takes the lists that turn out uneven (and did so better than one geometry of 96 to 160
+    // rows).  Such launches are bound by what a CU has under way, some 32 KB of lines however deep its ring; wide tiles read the
+    // activations half as often.  us, before -> this: 256 experts of 128 rows, 7168 x 2 x 2048 1417 -> 1340; 128 of 128, 4096 x 2 x 1536
+    // 325 -> 313; 8 of 110, 4096 x 2 x 14336 204 -> 186; 32 of 120, 2880 x 2 x 1440 90 -> 78; 128 of 80, 4096 x 2 x 1536, popularity
+    // rank^-0.6 357 -> 326, rank^-1.2 362 -> 335.  Where they leave a round emptier: 60 of 90, 2816 x 2 x 1408 110 -> 122; 16 of
+    // 100, 5440 x 2 x 10080 369 -> 395; where a workgroup walks a few short tiles: 32 of 60, 1344 x 2 x 1280, rank^-1.2 39 -> 51.  The down
+    // projection, whose tiles are shorter: 1 % either way.
+    if (p.epilogue == Epilogue::kSwiglu && StreamOk(p) && kSteps >= 8 && meanRows >= 16.0 && plan.tileM >= kSmallRows && plan.lowTileM == 0 &&
+        plan.tilesN > 1 && rounds * kSteps >= 40.0 && RowsOfNearlyEveryGroup(meanRows) <= kLowTileM && std::getenv("OPAPI_GEMM_TILE_M") == nullptr &&
+        std::getenv("OPAPI_GEMM_PULL") == nullptr) {
+        const int64_t tiles = groups * plan.tilesN, wideTiles = groups * ((plan.tilesN + 1) / 2), cus = DeviceCuCount();
+        const double used = static_cast<double>(tiles) / 2 / static_cast<double>((wideTiles + cus - 1) / cus * cus);
+        if (used >= 0.97 * RoundEfficiency(tiles)) {
+            plan.tileM = 192;
+            plan.pullTiles = true;
+            plan.lowTileM = kLowTileM;
+            plan.lowBySizes = plan.lowIsWide = true;
+        }
+    }
+    // The others on such groups: 160 rows in one geometry are as good as 96 or 128 where the groups are alike, and the two-geometry kernel
+    // better where they are not, if a workgroup walks more than a few tiles.  us, down, before -> this: 256 experts, 7168, 2048: 50 rows
+    // 736 -> 708, at rank^-1.2 892 -> 750, 80 at rank^-0.6 875 -> 808; 128, 4096, 1536: 50 rows at rank^-1.2 202 -> 185.  Few tiles each,
+    // left alone: 32 of 60, 2880, 1440, rank^-0.6 49 / 62; 60 of 90, 2816, 1408 69 / 74.
+    if (p.epilogue != Epilogue::kSwiglu && StreamOk(p) && kSteps >= 8 && meanRows >= 16.0 && plan.tileM >= kSmallRows && plan.tileM <= kLowTileM &&
+        plan.lowTileM == 0 && !lowHolds && rounds > 4.0 && std::getenv("OPAPI_GEMM_TILE_M") == nullptr && std::getenv("OPAPI_GEMM_PULL") == nullptr) {
+        plan.tileM = 192;
+        plan.pullTiles = true;
+        plan.lowTileM = kLowTileM;
+        plan.lowBySizes = true;
+    }
     const int64_t lowest = plan.lowTileM > 0 ? plan.lowTileM : plan.tileM;
     // The LDS-ring kernels number the tiles of a launch in 32 bits.  More than kMaxTiles of them (the scatter-add alone can ask for so
     // many: its output has few rows) run as several launches, each over a band of rows.  One expert's weights stay below 2 GB
@@ -595,7 +661,8 @@ hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStrea
     sa.groupListIsInt64 = p.groupListIsInt64 ? 1 : 0;
     sa.isCount = static_cast<int32_t>(p.groupListKind);
     sa.tileM = plan.tileM;
-    sa.mayLower = plan.lowForRounds ? 2 : plan.lowTileM > 0 ? 1 : 0;
+    sa.mayLower = plan.lowForRounds ? 2 : plan.lowBySizes ? 3 : plan.lowTileM > 0 ? 1 : 0;
+    sa.lowIsWide = plan.lowIsWide ? 1 : 0;
     sa.cus = DeviceCuCount();
     sa.tilesN = plan.tilesN;
     sa.maxMTiles = plan.maxMTiles;

@@ -108,7 +108,7 @@ constexpr int kLdsBudget = 160 * 1024;
 // ---------------------------------------------------------------------------------------------- scheduling table
 // int32 layout, all written by the scheduling kernel:
 //   header, 32 ints: [0] big m-tiles, [1] small m-tiles, [2] cost of the small ones, [3] cost of the big ones (see below),
-//                    [4] / [5] band width of the big / small run, [6] total rows covered by the groups, [7] rows per m-tile, [8] 1: nearly every group is one big m-tile;
+//                    [4] / [5] band width of the big / small run, [6] total rows covered by the groups, [7] rows per m-tile, [8] 1: nearly every group is one m-tile, of one kind, [9] 1: tiles are 512 channels wide;
 //   16 tile counters in one 128-byte line (32 ints): counter [2 * xcd + list], zeroed;
 //   the m-tile table, 4 ints per m-tile {group, first row, rows, 0} (at most maxMTiles of them): the big m-tiles in group
 //   order, then the small ones.  A GEMM kernel finds everything about a tile with one 16-byte load.
@@ -126,7 +126,8 @@ constexpr int kQueueCounterInts = 32;
 constexpr int kHdrCoveredRows = 6;
 constexpr int kHdrTileM = 7;
 constexpr int kHdrEven = 8;
-// A height that the scheduling kernel may choose instead of 192 or 256 rows (Plan::lowTileM).
+constexpr int kHdrWide = 9;
+// A height that the scheduling kernel may choose instead of 192 or 256 rows (Plan::lowTileM), maybe with wide tiles (Plan::lowIsWide).
 constexpr int kLowTileM = 160;
 __host__ __device__ inline int SchedTotalInts(int maxMTiles) { return kQueueHeaderInts + kQueueCounterInts + 4 * maxMTiles; }
 
@@ -166,10 +167,10 @@ __device__ __forceinline__ RunTable ReadRunTable(const int32_t* sched) {
 // Tile `logical` of one run of the m-tile table (`count` m-tiles from entry `first` on).  Bands of bandWidth m-tiles walk
 // the n-tiles together: consecutive tiles are the band's m-tiles at one n-tile, then the next n-tile.
 template <bool kSwiglu>
-__device__ __forceinline__ TileInfo DecodeListTile(const KernelArgs& a, const int4* __restrict__ table, int32_t first,
+__device__ __forceinline__ TileInfo DecodeListTile(int32_t tilesN, const int4* __restrict__ table, int32_t first,
                                                    int32_t count, int32_t bandWidth, int32_t logical) {
     TileInfo t{};
-    const int32_t perBand = bandWidth * a.tilesN;
+    const int32_t perBand = bandWidth * tilesN;
     const int32_t band = logical / perBand;
     const int32_t rem = logical - band * perBand;
     const int32_t bandTiles = min(bandWidth, count - bandWidth * band);
@@ -395,7 +396,10 @@ struct RowBlocks {
 // Epilogue of one tile.  acc[m][n][v] is C[row, col] with row = RowOf(m) + 4 * quad + v and col = ColumnInTile(n) of lane l16.
 // ldsRowScale holds the tile's per-row scales, ldsChannelScale those of its 256 channels by their place in the tile (null: they are
 // loaded here).  kSwiglu: ldsRowMax, zero before, takes the tile's row maxima of |S| as float bits (TileEpilogueStoreMax).
-// beforeStores() is called between the arithmetic and the stores of whole column blocks, in front of both elsewhere (256 rows: see there).
+// beforeStores() is called between the arithmetic and the stores of whole column blocks, in front of both elsewhere.  Not so without
+// kAllAtOnce: a block's results are stored before the next one's are worked out, and beforeStores() comes behind them all, where the DMAs
+// have landed.  The tallest and the wide tiles have no registers for all results beside the accumulators of those to come (and the SwiGLU
+// of 256 rows, which has, is slower for them on short K: 64 groups of 2000 rows, K 1024 x 2 x 512, 187 / 181 us).
 // Row checks are made per 16-row block, wave-uniformly: a block wholly inside the expert's rows takes a copy of the code
 // without checks, a block wholly outside is skipped, and only the one that straddles the last row tests every lane.  (A
 // per-lane test makes every element a predicated basic block of its own, and their independent chains no longer interleave.)
@@ -410,7 +414,7 @@ __device__ __forceinline__ void SettleLoads(float (&v)[kCount]) {
 struct NoHook {
     __device__ __forceinline__ void operator()() const {}
 };
-template <int kRows, Epilogue kEpi, int kOrder, typename Hook = NoHook>
+template <int kRows, Epilogue kEpi, int kOrder, bool kAllAtOnce = (kRows < 256), typename Hook = NoHook>
 __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const TileInfo& t, v4i (&acc)[RowBlocks<kRows>::kAll][4], int waveM,
                                                  int waveN, int l16, int quad, const float* ldsChannelScale, const float* ldsRowScale,
                                                  uint32_t* ldsRowMax, Hook beforeStores = NoHook{}) {
@@ -454,9 +458,6 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
         // + 32-bit lane offset) address.  Past the caches: nothing reads them back before they have left these.
         const bool halves = kEpi == Epilogue::kDequant && (a.outDtype == 27 || a.outDtype == 1) && whole && pairs;
         const bool toBf16 = a.outDtype == 27;  // wave-uniform: bf16, else fp16
-        // The tallest tiles have no registers for the results of all blocks beside the accumulators of those to come: a block's are stored
-        // before the next one's are worked out, and beforeStores() comes behind them all, where the DMAs have landed.
-        constexpr bool kAllAtOnce = kRows < 256;
         uint32_t word[kAllAtOnce ? Blocks::kAll : 1][4][2];
         auto results = [&](int m, uint32_t (&w)[4][2], auto bf16Tag) __attribute__((always_inline)) {
             constexpr bool kToBf16 = decltype(bf16Tag)::value;  // compile-time: a run-time choice per element splits the block
@@ -619,36 +620,39 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
         };
         // wave-uniform: every column of the wave exists, and S rows start on a lane's pair
         const bool whole = t.colBase + 32 * waveN + 32 <= a.halfN && (kOrder != kOrderLane || (a.halfN & 1) == 0);
-        Float2 s[Blocks::kAll][4];
-        if (whole) {
-            auto results = [&](int m, auto fullTag) __attribute__((always_inline)) {
-                constexpr bool kFull = decltype(fullTag)::value;
-                const int rTop = Blocks::RowOf(m, waveM);
-                const float4 xs4 = *reinterpret_cast<const float4*>(ldsRowScale + rTop + 4 * quad);
-                const float xs[4] = {xs4.x, xs4.y, xs4.z, xs4.w};
-                float top[4];
+        Float2 s[kAllAtOnce ? Blocks::kAll : 1][4];
+        auto results = [&](int m, Float2 (&out)[4], auto fullTag) __attribute__((always_inline)) {
+            constexpr bool kFull = decltype(fullTag)::value;
+            const int rTop = Blocks::RowOf(m, waveM);
+            const float4 xs4 = *reinterpret_cast<const float4*>(ldsRowScale + rTop + 4 * quad);
+            const float xs[4] = {xs4.x, xs4.y, xs4.z, xs4.w};
+            float top[4];
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    s[m][v] = Float2{activated(m, 0, v, xs[v]), activated(m, 1, v, xs[v])};
-                    const bool ok = kFull || rTop + 4 * quad + v < rows;
-                    top[v] = ok ? fmaxf(fabsf(s[m][v][0]), fabsf(s[m][v][1])) : 0.0f;
-                }
-                const float m16 = FourMaxOver16(top, l16);
-                if ((l16 & 3) == 0) RaiseRowMax(ldsRowMax + rTop + 4 * quad + (l16 >> 2), m16);
-            };
+            for (int v = 0; v < 4; ++v) {
+                out[v] = Float2{activated(m, 0, v, xs[v]), activated(m, 1, v, xs[v])};
+                const bool ok = kFull || rTop + 4 * quad + v < rows;
+                top[v] = ok ? fmaxf(fabsf(out[v][0]), fabsf(out[v][1])) : 0.0f;
+            }
+            const float m16 = FourMaxOver16(top, l16);
+            if ((l16 & 3) == 0) RaiseRowMax(ldsRowMax + rTop + 4 * quad + (l16 >> 2), m16);
+        };
+        auto forBlocks = [&](auto f) __attribute__((always_inline)) {
 #pragma unroll
             for (int m = 0; m < Blocks::kAll; ++m) {
                 const int rTop = Blocks::RowOf(m, waveM);
                 if (rTop >= rows) continue;
-                if (rTop + 16 <= rows) results(m, std::true_type{});
-                else results(m, std::false_type{});
+                if (rTop + 16 <= rows) f(m, std::true_type{});
+                else f(m, std::false_type{});
             }
+        };
+        if constexpr (kAllAtOnce) {
+            if (whole) forBlocks([&](int m, auto fullTag) __attribute__((always_inline)) { results(m, s[m], fullTag); });
+            beforeStores();
         }
-        beforeStores();
         if (whole) {
             float* const sTile = a.sOut + static_cast<int64_t>(rowBase) * a.halfN;
             const int32_t laneOff = 4 * quad * a.halfN + col[0];
-            auto store = [&](int m, auto fullTag) __attribute__((always_inline)) {
+            auto store = [&](int m, const Float2 (&v2)[4], auto fullTag) __attribute__((always_inline)) {
                 constexpr bool kFull = decltype(fullTag)::value;
                 const int rTop = Blocks::RowOf(m, waveM);
 #pragma unroll
@@ -656,22 +660,21 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
                     float* const sRow = sTile + static_cast<int64_t>(rTop + v) * a.halfN;
                     const bool ok = kFull || rTop + 4 * quad + v < rows;
                     if constexpr (kOrder == kOrderLane) {
-                        if (ok) __builtin_nontemporal_store(s[m][v], reinterpret_cast<Float2*>(sRow + laneOff));
+                        if (ok) __builtin_nontemporal_store(v2[v], reinterpret_cast<Float2*>(sRow + laneOff));
                     } else {
-                        if (ok) __builtin_nontemporal_store(s[m][v][0], sRow + laneOff);
-                        if (ok) __builtin_nontemporal_store(s[m][v][1], sRow + laneOff + 16);
+                        if (ok) __builtin_nontemporal_store(v2[v][0], sRow + laneOff);
+                        if (ok) __builtin_nontemporal_store(v2[v][1], sRow + laneOff + 16);
                     }
                 }
             };
-#pragma unroll
-            for (int m = 0; m < Blocks::kAll; ++m) {
-                const int rTop = Blocks::RowOf(m, waveM);
-                if (rTop >= rows) continue;
-                if (rTop + 16 <= rows) store(m, std::true_type{});
-                else store(m, std::false_type{});
-            }
+            forBlocks([&](int m, auto fullTag) __attribute__((always_inline)) {
+                if constexpr (!kAllAtOnce) results(m, s[0], fullTag);
+                store(m, s[kAllAtOnce ? m : 0], fullTag);
+            });
+            if constexpr (!kAllAtOnce) beforeStores();
             return;
         }
+        if constexpr (!kAllAtOnce) beforeStores();
 #pragma unroll
         for (int m = 0; m < Blocks::kAll; ++m) {
             const int rTop = Blocks::RowOf(m, waveM);
@@ -695,12 +698,13 @@ __device__ __forceinline__ void TileEpilogueWave(const KernelArgs& a, const Tile
     }
 }
 
-// The part of the kSwiglu epilogue behind a barrier: one partial maximum per (n-tile, row) goes to memory -- no atomics there and
+// The part of the kSwiglu epilogue behind a barrier: one partial maximum per (256 channels, row) goes to memory -- no atomics there and
 // nothing to pre-zero; the requantisation folds them -- and the LDS copies start at zero again.  (The workgroup has at least kRows threads.)
 template <int kRows>
-__device__ __forceinline__ void TileEpilogueStoreMax(const KernelArgs& a, const TileInfo& t, int tid, uint32_t* ldsRowMax) {
+__device__ __forceinline__ void TileEpilogueStoreMax(const KernelArgs& a, const TileInfo& t, int32_t unit, int32_t units, int tid, uint32_t* ldsRowMax) {
     if (tid < t.rows) {
-        a.rowMax[static_cast<int64_t>(t.tileN) * a.M + t.rowBase + tid] = __uint_as_float(ldsRowMax[tid]);
+        const float m = __uint_as_float(ldsRowMax[tid]);
+        for (int32_t u = unit; u < unit + units; ++u) a.rowMax[static_cast<int64_t>(u) * a.M + t.rowBase + tid] = m;
         ldsRowMax[tid] = 0;
     }
 }
@@ -747,7 +751,7 @@ constexpr int kStep = 128;
 //
 // One DMA instruction moves 64 lanes x 16 bytes = 8 rows of 128 k-bytes.  Slot q of wave column w is instruction w + 4 q of
 // its kind, i.e. 32 rows per slot: even slots of the activation rows are the first half of the wave rows' blocks.
-template <int kRows>
+template <int kRows, int kUnits = 1>
 struct StreamCfg {
     using Blocks = RowBlocks<kRows>;
     static constexpr int kStageBytesA = kRows * kStep;
@@ -755,7 +759,7 @@ struct StreamCfg {
     static constexpr int kHalfBytesB = kStageBytesB / 2;
     static constexpr int kQueueLdsInts = 40;  // the workgroup's next eight tiles and how it comes by them
     static constexpr int kRowScales = (kRows + 63) / 64 * 64;  // in whole DMA instructions
-    static constexpr int kScratchBytes = (kTileN + kRowScales + kRows + kQueueLdsInts) * 4;  // channel scales, row scales, row maxima, tiles
+    static constexpr int kScratchBytes = (kUnits * kTileN + kRowScales + kRows + kQueueLdsInts) * 4;  // channel scales, row scales, row maxima, tiles
     static constexpr int kRingBytes = kLdsBudget - kScratchBytes;
     // as many weight stages as leave room for two of activation rows, then as many of those as fit
     static constexpr int kFitB = (kRingBytes - 2 * kStageBytesA) / kStageBytesB;
@@ -906,6 +910,10 @@ __device__ __forceinline__ void PhaseBarrier() {
 // kSmallRun: that run only, pulled, until its counters are used up on every XCD -- the form in which MixedGemmKernel
 // calls the body twice, once per run with a stage geometry of that run's own; `begins` says for which of them.
 //
+// kUnits: how many times 256 channels a tile is wide.  With two, a k-step is one stage of activation rows and two of weights, multiplied in
+// turn, and the ring of the rows moves on at every other stage of the weights'.  The accumulators of 160 rows and the fragments are what
+// the registers hold.
+//
 // kTail: K is a multiple of 16 and at least one k-step, but no multiple of a k-step.  The last k-step then starts kStep
 // bytes before the end of K instead of behind the step before it: every DMA stays inside its row and is as wide as any
 // other, and the k that the step before has already covered are multiplied by zero (the weight fragments of that one
@@ -913,15 +921,16 @@ __device__ __forceinline__ void PhaseBarrier() {
 // Before, such K went through the byte-wise kernel: a 301-token pass over 32 experts with hidden 2880 and intermediate
 // 1440 took 1.396 ms and takes 0.126 ms (its 398 MB of weights alone are 0.06 ms at the HBM's streaming rate).
 constexpr int kBigRun = 0, kSmallRun = 1, kBothRuns = 2;
-template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, int kRun, bool kTail>
+template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, int kRun, bool kTail, int kUnits = 1>
 __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_t* __restrict__ sched, char* const lds,
                                                uint64_t& spanTiles, bool begins = true) {
     static_assert(!(kNz && kNMajor), "one weight layout at a time");
-    using Cfg = StreamCfg<kRows>;
+    using Cfg = StreamCfg<kRows, kUnits>;
     using Blocks = RowBlocks<kRows>;
     constexpr bool kSwiglu = kEpi == Epilogue::kSwiglu;
-    float* const ldsChannelScale = reinterpret_cast<float*>(lds + Cfg::kFirstB + Cfg::kStagesB * Cfg::kStageBytesB);  // [kTileN]
-    float* const ldsRowScale = ldsChannelScale + kTileN;                                     // [kRowScales]
+    constexpr int kUnitCols = kSwiglu ? kTileN / 2 : kTileN;  // output columns of 256 channels
+    float* const ldsChannelScale = reinterpret_cast<float*>(lds + Cfg::kFirstB + Cfg::kStagesB * Cfg::kStageBytesB);  // [kUnits][kTileN]
+    float* const ldsRowScale = ldsChannelScale + kUnits * kTileN;                            // [kRowScales]
     uint32_t* const ldsRowMax = reinterpret_cast<uint32_t*>(ldsRowScale + Cfg::kRowScales);  // [kRows]
 
     const int tid = threadIdx.x;
@@ -948,16 +957,17 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     // Which list this workgroup draws from first.
     const int32_t forSmall = sched[0] == 0 ? slots : SlotsForSmall(sched, slots);
     const int prefer = kOneRun ? kRun : (slot < forSmall ? 1 : 0);
+    auto tilesAcross = [](const KernelArgs& args) __attribute__((always_inline)) { return (args.tilesN + kUnits - 1) / kUnits; };
     // tile `logical` of a run (list < 0: none), decoded
     auto decodeTile = [&](const KernelArgs& args, const RunTable& r, int32_t list, int32_t logical) __attribute__((always_inline)) -> v4i {
         if (list < 0) return v4i{0, 0, 0, 0};
-        const TileInfo t = DecodeListTile<kSwiglu>(args, r.entries, list ? r.countBig : 0, list ? r.countSmall : r.countBig,
+        const TileInfo t = DecodeListTile<kSwiglu>(tilesAcross(args), r.entries, list ? r.countBig : 0, list ? r.countSmall : r.countBig,
                                                    list ? r.bandSmall : r.bandBig, logical);
         return v4i{t.group, t.rowBase, t.rows, t.tileN};
     };
     // the n-th tile of this workgroup in fixed shares
     auto shareTile = [&](const KernelArgs& args, const RunTable& r, int32_t n) __attribute__((always_inline)) -> v4i {
-        const int32_t big = r.countBig * args.tilesN, total = big + r.countSmall * args.tilesN;
+        const int32_t big = r.countBig * tilesAcross(args), total = big + r.countSmall * tilesAcross(args);
         const int32_t perXcd = (total + kXcds - 1) / kXcds, local = slot + n * slots, logical = xcd * perXcd + local;
         const bool none = local >= perXcd || logical >= total;
         return decodeTile(args, r, none ? -1 : logical < big ? 0 : 1, logical < big ? logical : logical - big);
@@ -972,9 +982,13 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         t.rows = __builtin_amdgcn_readfirstlane(e.z);
         t.tileN = __builtin_amdgcn_readfirstlane(e.w);
         t.valid = t.rows > 0;
-        t.colBase = kSwiglu ? t.tileN * (kTileN / 2) : t.tileN * kTileN;
+        t.colBase = t.tileN * kUnits * kUnitCols;
         return t;
     };
+    // 256-channel units of a tile, and the first column of its second: where that would end behind the last column it begins earlier, over
+    // columns of the first, which then are computed, and stored, twice
+    auto unitsOf = [&](const TileInfo& t) __attribute__((always_inline)) { return min(kUnits, a.tilesN - kUnits * t.tileN); };
+    auto secondUnit = [&](const TileInfo& t) __attribute__((always_inline)) { return min(t.colBase + kUnitCols, (kSwiglu ? a.halfN : a.N) - kUnitCols); };
     // Side by side: their table entries are one round trip (0.3 to 1.2 us of a launch of shares, as one thread's loop).
     if (!pull && tid < kTilesAhead) leaveTile(tid, shareTile(a, ReadRunTable(sched), tid));
     if (kSwiglu && tid < kRows) ldsRowMax[tid] = 0;
@@ -993,12 +1007,15 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     // N 2048, 216 big and 104 small tiles 67 -> 52; the other way round 830 -> 858 at most (of sixty launches).
     if (wave == 0 && pull) {
         const RunTable runs = ReadRunTable(sched);
-        const int32_t bigTiles = runs.countBig * a.tilesN, smallTiles = runs.countSmall * a.tilesN;
-        auto eachOf = [&](int32_t tiles, int32_t seats) __attribute__((always_inline)) {
-            return (kOneRun ? tiles : bigTiles + smallTiles) <= static_cast<int32_t>(gridDim.x) ? 1
-                   : max(2, sched[kHdrEven] != 0 && seats > 0 ? tiles / kXcds / seats : 0);
+        const int32_t bigTiles = runs.countBig * tilesAcross(a), smallTiles = runs.countSmall * tilesAcross(a);
+        auto eachOf = [&](int32_t tiles) __attribute__((always_inline)) {
+            return (kOneRun ? tiles : bigTiles + smallTiles) <= static_cast<int32_t>(gridDim.x) ? 1 : 2;
         };
-        const int32_t eachBig = eachOf(bigTiles, slots - forSmall), eachSmall = eachOf(smallTiles, forSmall);
+        int32_t eachBig = eachOf(bigTiles), eachSmall = eachOf(smallTiles);
+        if (sched[kHdrEven] != 0) {
+            if (eachBig > 1 && slots > forSmall) eachBig = max(eachBig, bigTiles / kXcds / (slots - forSmall));
+            if (eachSmall > 1 && bigTiles == 0) eachSmall = max(eachSmall, smallTiles / kXcds / slots);
+        }
         const QueueLists lists{bigTiles, smallTiles, eachBig * (slots - forSmall), eachSmall * forSmall};
         const int32_t seats = prefer ? forSmall : slots - forSmall, seat = prefer ? slot : slot - forSmall;
         const int32_t each = prefer ? eachSmall : eachBig;
@@ -1080,6 +1097,8 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     uint32_t issAddr = issFirst;
     const char* issBase = nullptr;  // the tile's activation rows, or its expert's weights
     uint32_t laneOff[Cfg::kSlotsB];
+    int32_t issUnit = 0, issUnits = 1;  // weights: unit of the k-step that goes out next
+    int64_t issUnitShift = 0;           // from the first unit's weights to the second's, bytes
 
     // The lambdas below are forced inline: left to the inliner's size heuristics, one of them staying a real call puts
     // the whole issue state (captured by reference) into scratch memory and the kernel runs three times slower.
@@ -1100,6 +1119,10 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
             return;
         }
         issBase = UniformPtr(reinterpret_cast<const char*>(a.w) + static_cast<int64_t>(t.group) * a.wGroupStride);
+        if constexpr (kUnits > 1) {
+            issUnits = unitsOf(t);
+            issUnitShift = static_cast<int64_t>(secondUnit(t) - t.colBase) * (kNMajor ? 1 : a.K);  // (blocked: 32 channels, K x 32 bytes)
+        }
 #pragma unroll
         for (int q = 0; q < Cfg::kSlotsB; ++q) {
             constexpr int kPerHalf = Cfg::kSlotsB / 2;
@@ -1127,9 +1150,16 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
             }
         }
     };
-    // Moves the cursor to the next k-step.
+    // Moves the cursor to the next k-step (or, with two units, the weights' to the other one).
     auto advance = [&]() __attribute__((always_inline)) {
         issAddr = issAddr + issStride == issEnd ? issFirst : issAddr + issStride;
+        if constexpr (kUnits > 1) {
+            if (issUnit + 1 < issUnits) {
+                ++issUnit;
+                return;
+            }
+            issUnit = 0;
+        }
         if (__builtin_expect(++issStep == kSteps, 0)) {
             // move to this workgroup's next tile.  Past the last one the issue slots still go out (that keeps the number
             // of outstanding DMAs per stage, hence the vmcnt arithmetic, constant) into ring buffers nobody reads -- but
@@ -1144,6 +1174,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                 setupIssue(issTile);
             } else if (!issDrained) {
                 issDrained = true;
+                issUnitShift = 0;
                 // any mapped, 16-byte aligned kilobyte will do: the start of the last tile's expert's weights
                 issBase = UniformPtr(reinterpret_cast<const char*>(a.w) + static_cast<int64_t>(issTile.group) * a.wGroupStride);
 #pragma unroll
@@ -1158,7 +1189,8 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         const int kIdx = issStep + issRotate;
         const int kOff = issDrained ? 0 : kTail ? min(kIdx * kStep, a.K - kStep) : (kIdx >= kSteps ? kIdx - kSteps : kIdx) * kStep;
         // weights -- blocked layout: one k is 32 bytes further; row-major: N bytes
-        const char* const base = issBase + ((kNz || kNMajor) && forWeights ? static_cast<int64_t>(kOff) * (kNz ? 32 : a.N) : kOff);
+        const char* const base = issBase + ((kNz || kNMajor) && forWeights ? static_cast<int64_t>(kOff) * (kNz ? 32 : a.N) : kOff) +
+                                 (kUnits > 1 && issUnit != 0 ? issUnitShift : 0);
         const uint32_t dst = issAddr + 1024 * kWavesN * q;
         if constexpr (kSmallTile) {
             if (forWeights) DmaToLdsAddr16<true>(base, laneOff[q], dst);
@@ -1222,11 +1254,15 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         const int lane = Opaque(tid) & 63;
         if (forWeights) {
             if (channelScalesByDma) {
-                const int c = 64 * waveN + lane;  // of the tile
-                const int32_t col = kSwiglu ? (waveN >= 2 ? min(a.halfN + cur.colBase + c - kTileN / 2, a.N - 1) : min(cur.colBase + c, a.halfN - 1))
-                                            : min(cur.colBase + c, a.N - 1);
-                DmaToLdsAddr4(static_cast<const char*>(a.scale) + static_cast<int64_t>(cur.group) * a.N * 4, static_cast<uint32_t>(col) * 4u,
-                              LdsAddress(reinterpret_cast<const char*>(ldsChannelScale + 64 * waveN)));
+#pragma unroll
+                for (int u = 0; u < kUnits; ++u) {
+                    if (u > 0 && unitsOf(cur) == 1) break;
+                    const int c = 64 * waveN + lane, base = u ? secondUnit(cur) : cur.colBase;  // of the unit; the unit's
+                    const int32_t col = kSwiglu ? (waveN >= 2 ? min(a.halfN + base + c - kTileN / 2, a.N - 1) : min(base + c, a.halfN - 1))
+                                                : min(base + c, a.N - 1);
+                    DmaToLdsAddr4(static_cast<const char*>(a.scale) + static_cast<int64_t>(cur.group) * a.N * 4, static_cast<uint32_t>(col) * 4u,
+                                  LdsAddress(reinterpret_cast<const char*>(ldsChannelScale + u * kTileN + 64 * waveN)));
+                }
             }
         } else if (a.rowScale != nullptr && rowScalesByDma && 64 * waveN < kRows) {
             DmaToLdsAddr4(reinterpret_cast<const char*>(a.rowScale) + static_cast<int64_t>(cur.rowBase) * 4,
@@ -1237,15 +1273,19 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         }
     };
 
-    v4i acc[Blocks::kAll][4];
+    v4i acc[kUnits][Blocks::kAll][4];
     while (true) {
         const TileInfo following = tileAt(curNo + 1);
         if (kEpi != Epilogue::kInt32) requestScales();
 #pragma unroll
-        for (int m = 0; m < Blocks::kAll; ++m) {
+        for (int u = 0; u < kUnits; ++u) {
 #pragma unroll
-            for (int n = 0; n < 4; ++n) acc[m][n] = v4i{0, 0, 0, 0};
+            for (int m = 0; m < Blocks::kAll; ++m) {
+#pragma unroll
+                for (int n = 0; n < 4; ++n) acc[u][m][n] = v4i{0, 0, 0, 0};
+            }
         }
+        const int32_t units = unitsOf(cur);
 
         // The k loop of a wave with kMy row blocks (the loop is instantiated once per count, so that its body stays
         // straight-line code: blocks that hold no real row are never multiplied -- on the memory-bound shapes the matrix
@@ -1263,7 +1303,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
             // The product of one half of the rows with one slice, and between its instructions, if asked for, the requests of the even
             // or the odd slots.  From one row block to the next the weight blocks are walked back and forth: consecutive instructions
             // share an operand, which costs the matrix unit 2 to 3 % less power.
-            auto multiply = [&](auto halfTag, int ks, bool requests, int odd = 0) __attribute__((always_inline)) {
+            auto multiply = [&](auto unitTag, auto halfTag, int ks, bool requests, int odd = 0) __attribute__((always_inline)) {
                 constexpr int kHalf = decltype(halfTag)::value;
                 constexpr int kCount = kHalf ? kMy1 : kMy0, kOnes = kCount > 0 ? kCount : 1;
 #pragma unroll
@@ -1272,7 +1312,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
 #pragma unroll
                         for (int step = 0; step < 4; ++step) {
                             const int n = i & 1 ? 3 - step : step;
-                            v4i& c = acc[kHalf * Blocks::kFirst + i][n];
+                            v4i& c = acc[decltype(unitTag)::value][kHalf * Blocks::kFirst + i][n];
                             c = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[ks][i], bf[ks][n], c, 0, 0, 0);
                         }
                     }
@@ -1294,20 +1334,22 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                     }
                 }
             };
-            auto kStepOf = [&](bool last) __attribute__((always_inline)) {
-                const uint32_t nextA = ringA + Cfg::kStageBytesA == ldsBase + Cfg::kFirstB ? ldsBase : ringA + Cfg::kStageBytesA;
+            auto kStepOf = [&](auto unit, bool last, bool lastUnit) __attribute__((always_inline)) {
+                const uint32_t nextA = !lastUnit ? ringA : ringA + Cfg::kStageBytesA == ldsBase + Cfg::kFirstB ? ldsBase : ringA + Cfg::kStageBytesA;
+                // a stage of activation rows is read once per unit, and refilled with the last
+                const bool refills = forWeights || lastUnit;
                 const uint32_t nextB = ringB + Cfg::kStageBytesB == ldsBase + Cfg::kFirstB + Cfg::kStagesB * Cfg::kStageBytesB
                                            ? ldsBase + Cfg::kFirstB : ringB + Cfg::kStageBytesB;
                 if (kMy > 0) readB(bf[1], ringB, 1);
                 readA(af[1], ringA, FirstHalf{}, 1);
                 __builtin_amdgcn_sched_barrier(0);
                 maskB(0, last);
-                multiply(FirstHalf{}, 0, false);
+                multiply(unit, FirstHalf{}, 0, false);
                 __builtin_amdgcn_sched_barrier(0);
                 readA(af[0], ringA, SecondHalf{}, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 maskB(1, last);
-                multiply(FirstHalf{}, 1, false);
+                multiply(unit, FirstHalf{}, 1, false);
                 // This wave's reads of weights and first half have returned: the products above used them, so the compiler has
                 // waited for them already.  But nothing orders those register instructions against the barrier, behind which DMAs
                 // that the compiler does not see overwrite what was read.  The kMy1 reads of the second half may be outstanding.
@@ -1316,20 +1358,20 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                 PhaseBarrier();
                 readA(af[1], ringA, SecondHalf{}, 1);
                 __builtin_amdgcn_sched_barrier(0);
-                multiply(SecondHalf{}, 0, true, 0);
+                multiply(unit, SecondHalf{}, 0, refills, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 WaitLds();
                 if (forWeights) WaitVmcnt<Cfg::kYoungerB>();  // (stores of the tile before, still under way, make it only stricter)
-                else WaitVmcnt<Cfg::kYoungerA>();
+                else if (refills) WaitVmcnt<Cfg::kYoungerA>();
                 PhaseBarrier();
-                if (kMy > 0 && !last) {
+                if (kMy > 0 && !(last && lastUnit)) {
                     readB(bf[0], nextB, 0);
                     readA(af[0], nextA, FirstHalf{}, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                multiply(SecondHalf{}, 1, true, 1);
+                multiply(unit, SecondHalf{}, 1, refills, 1);
                 __builtin_amdgcn_sched_barrier(0);
-                advance();
+                if (refills) advance();
                 ringA = nextA;
                 ringB = nextB;
             };
@@ -1337,7 +1379,12 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
             if (kMy > 0) readB(bf[0], ringB, 0);
             readA(af[0], ringA, FirstHalf{}, 0);
 #pragma unroll 1
-            for (int step = 0; step < kSteps; ++step) kStepOf(step + 1 == kSteps);
+            for (int step = 0; step < kSteps; ++step) {
+                kStepOf(std::integral_constant<int, 0>{}, step + 1 == kSteps, kUnits == 1 || units == 1);
+                if constexpr (kUnits > 1) {
+                    if (units > 1) kStepOf(std::integral_constant<int, 1>{}, step + 1 == kSteps, true);
+                }
+            }
         };
         const int active = (cur.rows + 15) >> 4;  // blocks with real rows
         auto runOne = [&](auto myTag) __attribute__((always_inline)) { runTile(myTag); };
@@ -1382,7 +1429,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                     }
                 } else if (drawCounter >= 0) {
                     const int32_t v = __builtin_amdgcn_readfirstlane(drawValue);
-                    const QueueLists lists{runs.countBig * epilogueArgs.tilesN, runs.countSmall * epilogueArgs.tilesN,
+                    const QueueLists lists{runs.countBig * tilesAcross(epilogueArgs), runs.countSmall * tilesAcross(epilogueArgs),
                                            __builtin_amdgcn_readfirstlane(ldsSeq[kSeqSeated]), __builtin_amdgcn_readfirstlane(ldsSeq[kSeqSeated + 1])};
                     int32_t first, size;
                     QueueShare(lists, drawCounter, &first, &size);
@@ -1402,15 +1449,29 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                 }
             }
         };
-        TileEpilogueWave<kRows, kEpi, kOrderOf<kNz, kNMajor>>(epilogueArgs, cur, acc, waveM, waveN, Opaque(tid) & 15, (Opaque(tid) >> 4) & 3,
-                                                              channelScalesByDma ? ldsChannelScale : nullptr, ldsRowScale, ldsRowMax, beforeStores);
+        constexpr int kOrder = kOrderOf<kNz, kNMajor>;
+        const float* const channelScales = channelScalesByDma ? ldsChannelScale : nullptr;
+        if constexpr (kUnits == 1) {
+            TileEpilogueWave<kRows, kEpi, kOrder>(epilogueArgs, cur, acc[0], waveM, waveN, Opaque(tid) & 15, (Opaque(tid) >> 4) & 3, channelScales,
+                                                  ldsRowScale, ldsRowMax, beforeStores);
+        } else {  // two units' accumulators leave no room for the results of one
+            TileEpilogueWave<kRows, kEpi, kOrder, false>(epilogueArgs, cur, acc[0], waveM, waveN, Opaque(tid) & 15, (Opaque(tid) >> 4) & 3, channelScales,
+                                                         ldsRowScale, ldsRowMax);
+            beforeStores();
+            if (units > 1) {
+                TileInfo second = cur;
+                second.colBase = secondUnit(cur);
+                TileEpilogueWave<kRows, kEpi, kOrder, false>(epilogueArgs, second, acc[1], waveM, waveN, Opaque(tid) & 15, (Opaque(tid) >> 4) & 3,
+                                                             channelScalesByDma ? ldsChannelScale + kTileN : nullptr, ldsRowScale, ldsRowMax);
+            }
+        }
         if (tid == 0 && following.valid) leaveTile(curNo + (pull ? 2 : kTilesAhead), next);
         ++spanTiles;
         if (!kSwiglu && !following.valid) break;
         WaitLds();
         PhaseBarrier();  // the reads of the scales are done, the row maxima are complete and the drawn tile is in the ring
         if constexpr (kSwiglu) {
-            TileEpilogueStoreMax<kRows>(epilogueArgs, cur, Opaque(tid), ldsRowMax);
+            TileEpilogueStoreMax<kRows>(epilogueArgs, cur, kUnits * cur.tileN, units, Opaque(tid), ldsRowMax);
             if (!following.valid) break;
         }
         cur = following;
@@ -1445,13 +1506,21 @@ __global__ __launch_bounds__(kThreads) void StreamGemmKernel(KernelArgs a, const
 // of each XCD's workgroups that its cost is of the whole) until that run's counters are used up on every XCD, lets its
 // ring drain, and serves the other; a launch without small m-tiles costs the workgroups that looked for them one draw.
 //
-// The scheduling kernel may have cut the groups into m-tiles of at most kLowTileM rows instead; these run in one geometry.
+// The scheduling kernel may have cut the groups into m-tiles of at most kLowTileM rows instead; these run in one geometry, in tiles of 256
+// or of 512 channels.
 
 template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
 __global__ __launch_bounds__(kThreads) void MixedGemmKernel(KernelArgs a, const int32_t* __restrict__ sched) {
     extern __shared__ __attribute__((aligned(128))) char lds[];
     const uint64_t spanStart = a.wgSpans != nullptr ? __builtin_amdgcn_s_memrealtime() : 0;
     uint64_t spanTiles = 0;
+    if constexpr (kEpi == Epilogue::kSwiglu) {
+        if (sched[kHdrWide] != 0) {
+            StreamGemmBody<kLowTileM, kEpi, kNz, kNMajor, kBothRuns, kTail, 2>(a, sched, lds, spanTiles);
+            WriteSpan(a, spanStart, spanTiles, kLowTileM);
+            return;
+        }
+    }
     if (sched[kHdrTileM] == kLowTileM) {
         StreamGemmBody<kLowTileM, kEpi, kNz, kNMajor, kBothRuns, kTail>(a, sched, lds, spanTiles);
         WriteSpan(a, spanStart, spanTiles, kLowTileM);
@@ -1461,12 +1530,16 @@ __global__ __launch_bounds__(kThreads) void MixedGemmKernel(KernelArgs a, const 
     const int32_t forSmall = sched[0] == 0 ? slots : SlotsForSmall(sched, slots);
     if (slot < forSmall) {
         StreamGemmBody<kSmallRows, kEpi, kNz, kNMajor, kSmallRun, kTail>(a, sched, lds, spanTiles);
-        __syncthreads();  // the other geometry lays LDS out anew
-        StreamGemmBody<kRows, kEpi, kNz, kNMajor, kBigRun, kTail>(a, sched, lds, spanTiles, false);
+        if (sched[0] != 0) {
+            __syncthreads();  // the other geometry lays LDS out anew
+            StreamGemmBody<kRows, kEpi, kNz, kNMajor, kBigRun, kTail>(a, sched, lds, spanTiles, false);
+        }
     } else {
         StreamGemmBody<kRows, kEpi, kNz, kNMajor, kBigRun, kTail>(a, sched, lds, spanTiles);
-        __syncthreads();
-        StreamGemmBody<kSmallRows, kEpi, kNz, kNMajor, kSmallRun, kTail>(a, sched, lds, spanTiles, false);
+        if (sched[1] != 0) {
+            __syncthreads();
+            StreamGemmBody<kSmallRows, kEpi, kNz, kNMajor, kSmallRun, kTail>(a, sched, lds, spanTiles, false);
+        }
     }
     WriteSpan(a, spanStart, spanTiles);
 }
@@ -1502,8 +1575,8 @@ __global__ __launch_bounds__(kThreads) void GenericGemmKernel(KernelArgs a, cons
     const int32_t logical = static_cast<int32_t>(blockIdx.x % kXcds) * perXcd + local;
     if (local >= perXcd || logical >= totalTiles) return;
     const TileInfo t = logical < bigTiles
-        ? DecodeListTile<kSwiglu>(a, mTileTable, 0, countBig, queueHdr[4], logical)
-        : DecodeListTile<kSwiglu>(a, mTileTable, countBig, countSmall, queueHdr[5], logical - bigTiles);
+        ? DecodeListTile<kSwiglu>(a.tilesN, mTileTable, 0, countBig, queueHdr[4], logical)
+        : DecodeListTile<kSwiglu>(a.tilesN, mTileTable, countBig, countSmall, queueHdr[5], logical - bigTiles);
     if (kEpi != Epilogue::kInt32 && a.rowScale != nullptr && tid < kRows) {
         ldsRowScale[tid] = a.rowScale[t.rowBase + (tid < t.rows ? tid : t.rows - 1)];
     }
@@ -1565,7 +1638,7 @@ __global__ __launch_bounds__(kThreads) void GenericGemmKernel(KernelArgs a, cons
     TileEpilogueWave<kRows, kEpi, kOrderBlock>(a, t, acc, waveM, waveN, l16, quad, nullptr, ldsRowScale, ldsRowMax);
     if constexpr (kSwiglu) {
         __syncthreads();
-        TileEpilogueStoreMax<kRows>(a, t, tid, ldsRowMax);
+        TileEpilogueStoreMax<kRows>(a, t, t.tileN, 1, tid, ldsRowMax);
     }
 }
 
@@ -1590,7 +1663,7 @@ hipError_t LaunchStream(const KernelArgs& args, const int32_t* sched, int64_t ma
 
 template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
 hipError_t LaunchMixed(const KernelArgs& args, const int32_t* sched, int64_t maxTiles, hipStream_t stream) {
-    constexpr int kLdsBytes = std::max({StreamCfg<kRows>::kLdsBytes, StreamCfg<kSmallRows>::kLdsBytes, StreamCfg<kLowTileM>::kLdsBytes});
+    constexpr int kLdsBytes = std::max({StreamCfg<kRows>::kLdsBytes, StreamCfg<kSmallRows>::kLdsBytes, StreamCfg<kLowTileM>::kLdsBytes, StreamCfg<kLowTileM, 2>::kLdsBytes});
     auto kernel = MixedGemmKernel<kRows, kEpi, kNz, kNMajor, kTail>;
     static std::atomic<uint64_t> optedIn{0};
     const hipError_t attr = opapi::EnsureDynamicLds(reinterpret_cast<const void*>(kernel), kLdsBytes, optedIn);

@@ -207,3 +207,45 @@ def test_few_tiles_swiglu_equals_a_forced_height(aclnn, oracle, dev, monkeypatch
     diff = np.abs(y.cpu().numpy()[sample].astype(np.int32) - h.astype(np.int32))
     assert diff.max() <= 1 and (diff != 0).mean() < 1e-3  # an LSB where exp and division round differently
     np.testing.assert_allclose(ys.cpu().numpy()[sample], hs, rtol=1e-5)
+
+
+# Groups whose sizes the scheduling kernel looks at: alike (one geometry: for SwiGLU tiles of two times 256 channels), one that needs a
+# second m-tile (no wide tiles), and nearly all of at most 64 rows (two geometries).  N: whole pairs of 256 channels, a second 256
+# that begin over the first's, a last tile of 256.
+SIZES = {"alike": ([65, 80, 96, 97, 128, 129, 159, 160, 1, 0, 64, 100, 112, 144, 145, 81] * 8, 160),
+         "over": ([65, 80, 96, 97, 70, 81, 112, 160] * 15 + [0, 100, 100, 100, 100, 100, 161, 100], 192),
+         "small": ([60, 64, 63, 49, 48, 33, 64, 64] * 15 + [60, 64, 64, 64, 160, 160, 159, 250], 192)}
+
+
+@pytest.mark.parametrize("layout,K,columns", [("k", 1280, 1024), ("k", 1296, 1001), ("k", 1536, 880), ("nd", 1280, 1008), ("nz", 1296, 992)])
+@pytest.mark.parametrize("name", sorted(SIZES))
+def test_tiles_by_sizes_swiglu_equals_a_forced_height(aclnn, dev, monkeypatch, name, layout, K, columns):
+    sizes, want_rows = SIZES[name]
+    E, M = len(sizes), sum(sizes)
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.empty((M, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    w = torch.empty((E, 2 * columns, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    view, nz = _weights(w, layout)
+    scale, x_scale = torch.rand((E, 2 * columns), device=dev, generator=g) * 1e-3, torch.rand((M,), device=dev, generator=g) * 1e-2
+    cumsum = torch.cumsum(torch.tensor(sizes), 0).to(dev)
+
+    def call():
+        out = (torch.full((M, columns), 7, dtype=torch.int8, device=dev), torch.full((M,), 7.0, device=dev))
+        return aclnn.grouped_matmul_swiglu_quant(x, view, cumsum, scale, x_scale, out=out, weight_nz=nz)
+
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    (y, ys), rows = _spanned(aclnn, call)
+    assert rows == want_rows
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", "96")
+    (y96, ys96), rows = _spanned(aclnn, call)
+    assert rows == 96 and torch.equal(y, y96) and torch.equal(ys, ys96)
+
+
+@pytest.mark.parametrize("layout,K", [("k", 1024), ("nd", 1040), ("nz", 1152)])
+@pytest.mark.parametrize("name", sorted(SIZES))
+def test_tiles_by_sizes_down(aclnn, monkeypatch, name, layout, K):
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    sizes, want_rows = SIZES[name]
+    (got, want), rows = _spanned(aclnn, lambda: _run(aclnn, sizes, 2208, K, layout, torch.bfloat16, K))
+    assert rows == (160 if name == "over" else want_rows)  # (one group in 128 with a small second m-tile)
+    assert torch.equal(got, want)
