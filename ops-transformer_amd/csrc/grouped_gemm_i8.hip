@@ -576,6 +576,8 @@ Plan MakePlan(const Problem& p) {
         plan.lowTileM = kLowTileM;
         plan.lowForRounds = true;
     }
+    // Workspaces are sized, and S is held, for the height chosen so far: the two choices below change neither.
+    const int sizedFor = plan.lowTileM > 0 ? plan.lowTileM : plan.tileM, bandHeight = plan.tileM;
     // The SwiGLU operator on groups that 160 rows hold nearly all: tiles of 512 channels instead of 256, where that costs no round of the
     // machine, on the two-geometry kernel, which takes the lists that turn out uneven (and did so better than one geometry of 96 to 160
     // rows).  Such launches are bound by what a CU has under way, some 32 KB of lines however deep its ring; wide tiles read the
@@ -607,13 +609,13 @@ Plan MakePlan(const Problem& p) {
         plan.lowTileM = kLowTileM;
         plan.lowBySizes = true;
     }
-    const int64_t lowest = plan.lowTileM > 0 ? plan.lowTileM : plan.tileM;
+    const int64_t lowest = sizedFor;
     // The LDS-ring kernels number the tiles of a launch in 32 bits.  More than kMaxTiles of them (the scatter-add alone can ask for so
     // many: its output has few rows) run as several launches, each over a band of rows.  One expert's weights stay below 2 GB
     // (StreamOk), so that every group's last m-tile is a small part of the limit: 1024 groups x 65536 n-tiles.
     int64_t bandRows = p.M;
     if (StreamOk(p) && (p.M / lowest + groups) * plan.tilesN > kMaxTiles) {
-        bandRows = (kMaxTiles / plan.tilesN - groups) * lowest / plan.tileM * plan.tileM;
+        bandRows = (kMaxTiles / plan.tilesN - groups) * lowest / bandHeight * bandHeight;
     }
     const int64_t maxMTiles = bandRows / lowest + groups;
     plan.maxMTiles = static_cast<int32_t>(maxMTiles);
@@ -631,8 +633,8 @@ Plan MakePlan(const Problem& p) {
         // costs nothing (halving the limit twice costs 2 % and 7 % of the pass).
         const uint64_t capBytes = SwigluWorkspaceCap();
         const uint64_t rowBytes = static_cast<uint64_t>(p.N / 2) * 4;
-        int64_t capRows = rowBytes > 0 ? static_cast<int64_t>(capBytes / rowBytes) / plan.tileM * plan.tileM : p.M;
-        if (capRows < plan.tileM) capRows = plan.tileM;
+        int64_t capRows = rowBytes > 0 ? static_cast<int64_t>(capBytes / rowBytes) / bandHeight * bandHeight : p.M;
+        if (capRows < bandHeight) capRows = bandHeight;
         if (capRows < bandRows) bandRows = capRows;
         plan.offS = off;
         off += Align256(static_cast<uint64_t>(bandRows) * rowBytes);
