@@ -16,6 +16,13 @@ ACL_API aclTensor* opapiCreateTensorPacked(const int64_t* packed);
 
 ACL_API void opapiDestroyTensors(const aclTensor* const* tensors, uint64_t count);
 
+// The first phase of an operator on descriptors that exist for the call only.  packed: the operator's number (0 aclnnMoeGatingTopKSoftmaxV2,
+// 1 aclnnMoeInitRoutingV2, 2 aclnnMoeInitRoutingQuantV2, 3 aclnnMoeInitRoutingV3 on all experts, 4 aclnnGroupedMatmulSwigluQuant,
+// 5 aclnnGroupedMatmulV4 on lists of one tensor, 6 aclnnMoeFinalizeRoutingV2), its scalars, then its tensors as above, both in the order of
+// its first phase, absent tensors with no dimensions and no address.  Left out: offset and activeExpertRange of 3, outputOffset of 4, the
+// lists of 5 other than x, weight, bias, scale, perTokenScale and out (the group list stands before out).
+ACL_API aclnnStatus opapiPlanPacked(const int64_t* packed, uint64_t length, uint64_t* workspaceSize, aclOpExecutor** executor);
+
 #ifdef __cplusplus
 }
 #endif

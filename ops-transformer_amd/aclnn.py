@@ -119,6 +119,8 @@ def lib():
         l.opapiCreateTensorPacked.restype = _VP
         l.opapiDestroyTensors.argtypes = [ctypes.c_char_p, ctypes.c_uint64]
         l.opapiDestroyTensors.restype = None
+        l.opapiPlanPacked.argtypes = [ctypes.c_char_p, ctypes.c_uint64, _VP, _VP]
+        l.opapiPlanPacked.restype = ctypes.c_int32
         l.opapiMoeFfnForward.argtypes = [ctypes.c_char_p, ctypes.c_uint64, _VP, ctypes.c_uint64, _VP, _U64P,
                                          ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_char_p)]
         l.opapiMoeFfnForward.restype = ctypes.c_int32
@@ -278,6 +280,48 @@ def _run_two_phase(api, args, device, workspace=None, static_workspace_api=None)
     return ws_keepalive
 
 
+# Operators of opapiPlanPacked (include/opapi_descriptor.h), by number.
+_PLANNED = ("aclnnMoeGatingTopKSoftmaxV2", "aclnnMoeInitRoutingV2", "aclnnMoeInitRoutingQuantV2", "aclnnMoeInitRoutingV3",
+            "aclnnGroupedMatmulSwigluQuant", "aclnnGroupedMatmulV4", "aclnnMoeFinalizeRoutingV2")
+(_GATING, _ROUTING_V2, _ROUTING_QUANT_V2, _ROUTING_V3, _SWIGLU_QUANT, _GROUPED_MATMUL_V4, _FINALIZE_V2) = range(7)
+
+
+def _packed(t):
+    if t is None:
+        return _PACK[0](0, 0, 0)
+    shape = t.shape
+    n = len(shape)
+    if n > 8:
+        raise MemoryError("aclCreateTensor failed")
+    return _PACK[n](n, _DTYPE_CODE[t.dtype], t.data_ptr(), *shape, *t.stride())
+
+
+def _run_packed(op, scalars, tensors, device, workspace=None):
+    """Both phases of an operator: the first in one foreign call on descriptors packed into one array.
+
+    A call on a few rows is bound by the host, and its descriptors, a foreign call each to make and a handle to drop, were a part of
+    that.  us, before -> this: a MoE layer of five operators on 5 tokens, 160 experts, hidden 3840, intermediate 576 86 -> 63; on 4
+    tokens, 160 experts, 2880, 1984 91 -> 78; permutation and combine of 46 tokens of 1024 37 -> 31."""
+    l = lib()
+    packed = struct.pack("%dq" % (1 + len(scalars)), op, *scalars) + b"".join([_packed(t) for t in tensors])
+    planned = (ctypes.c_uint64 * 2)()  # workspace bytes, executor
+    where = ctypes.addressof(planned)
+    api = _PLANNED[op]
+    st = l.opapiPlanPacked(packed, len(packed) >> 3, where, where + 8)
+    if st != ACLNN_SUCCESS:
+        raise AclnnError(api + "GetWorkspaceSize", st, last_error())
+    nbytes, executor = planned
+    ws_ptr = None
+    if workspace is not None:
+        workspace.requested[api] = max(workspace.requested.get(api, 0), nbytes)
+    if nbytes > 0:
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=device) if workspace is None else workspace.reserve(nbytes, device)
+        ws_ptr = ws.data_ptr()
+    st = getattr(l, api)(ws_ptr, nbytes, executor, _stream_ptr())
+    if st != ACLNN_SUCCESS:
+        raise AclnnError(api, st, last_error())
+
+
 def workspace_size(api, args):
     """Phase 1 only: returns the workspace byte count and releases the executor."""
     l = lib()
@@ -315,13 +359,18 @@ def moe_init_routing_v2(x, expert_idx, active_num=0, expert_capacity=0, expert_n
                      if (drop_pad_mode == 0 and expert_tokens_count_or_cumsum_flag > 0) else None)
         before_out = (torch.empty((expert_num,), dtype=torch.int32, device=dev)
                       if (drop_pad_mode == 1 and expert_tokens_before_capacity_flag) else None)
+    if not static_workspace:
+        _run_packed(_ROUTING_V2, (active_num, expert_capacity, expert_num, drop_pad_mode, expert_tokens_count_or_cumsum_flag,
+                                  bool(expert_tokens_before_capacity_flag)),
+                    (x, expert_idx, expanded_x, expanded_row_idx, count_out, before_out), dev, workspace)
+        return expanded_x, expanded_row_idx, count_out, before_out
     h = _Handles()
     try:
         args = [h.tensor(x), h.tensor(expert_idx), active_num, expert_capacity, expert_num, drop_pad_mode,
                 expert_tokens_count_or_cumsum_flag, bool(expert_tokens_before_capacity_flag), h.tensor(expanded_x),
                 h.tensor(expanded_row_idx), h.tensor(count_out), h.tensor(before_out)]
         _run_two_phase("aclnnMoeInitRoutingV2", args, dev, workspace,
-                       static_workspace_api="aclnnMoeInitRoutingV2StaticWorkspace" if static_workspace else None)
+                       static_workspace_api="aclnnMoeInitRoutingV2StaticWorkspace")
     finally:
         h.close()
     return expanded_x, expanded_row_idx, count_out, before_out
@@ -352,14 +401,9 @@ def moe_init_routing_quant_v2(x, expert_idx, quant_mode, scale=None, offset=None
     counts = fresh((expert_num,), dtype=torch.int32, device=dev) if count_flag else None
     before = fresh((expert_num,), dtype=torch.int32, device=dev) if before_flag else None
     dyn = fresh((rows,), dtype=torch.float32, device=dev) if quant_mode == 1 else None
-    h = _Handles()
-    try:
-        args = [h.tensor(x), h.tensor(expert_idx), h.tensor(scale), h.tensor(offset), active_num, expert_capacity,
-                expert_num, drop_pad_mode, expert_tokens_count_or_cumsum_flag, expert_tokens_before_capacity_flag,
-                quant_mode, h.tensor(expanded_x), h.tensor(row_idx), h.tensor(counts), h.tensor(before), h.tensor(dyn)]
-        _run_two_phase("aclnnMoeInitRoutingQuantV2", args, dev, workspace)
-    finally:
-        h.close()
+    _run_packed(_ROUTING_QUANT_V2, (active_num, expert_capacity, expert_num, drop_pad_mode, expert_tokens_count_or_cumsum_flag,
+                                    bool(expert_tokens_before_capacity_flag), quant_mode),
+                (x, expert_idx, scale, offset, expanded_x, row_idx, counts, before, dyn), dev, workspace)
     return expanded_x, row_idx, counts, before, dyn
 
 
@@ -373,12 +417,7 @@ def moe_gating_top_k_softmax_v2(x, k, renorm=0, finished=None, output_softmax=Fa
         y = torch.empty(lead + (k,), dtype=x.dtype, device=dev)
         idx = torch.empty(lead + (k,), dtype=torch.int32, device=dev)
         sm = torch.empty(tuple(x.shape), dtype=torch.float32, device=dev) if (output_softmax and renorm == 0) else None
-    h = _Handles()
-    try:
-        args = [h.tensor(x), h.tensor(finished), k, renorm, bool(output_softmax), h.tensor(y), h.tensor(idx), h.tensor(sm)]
-        _run_two_phase("aclnnMoeGatingTopKSoftmaxV2", args, dev, None)
-    finally:
-        h.close()
+    _run_packed(_GATING, (k, renorm, bool(output_softmax)), (x, finished, y, idx, sm), dev)
     return y, idx, sm
 
 
@@ -403,11 +442,15 @@ def moe_init_routing_v3(x, expert_idx, scale=None, expert_num=0, expert_tokens_n
         counts = fresh((expert_num, 2) if expert_tokens_num_type == 2 else (end - start,), dtype=torch.int64, device=dev)
         expanded_scale = (fresh((T * K,), dtype=torch.float32, device=dev)
                           if (scale is not None or quant_mode == 1) else None)
+    if active_expert_range is None:
+        _run_packed(_ROUTING_V3, (active_num, 0, expert_num, 0, expert_tokens_num_type, True, quant_mode, row_idx_type),
+                    (x, expert_idx, scale, expanded_x, row_idx, counts, expanded_scale), dev, workspace)
+        return expanded_x, row_idx, counts, expanded_scale
     h = _Handles()
     try:
         args = [h.tensor(x), h.tensor(expert_idx), h.tensor(scale), None, active_num, 0, expert_num, 0,
                 expert_tokens_num_type, True, quant_mode,
-                None if active_expert_range is None else h.int_array(list(active_expert_range)), row_idx_type,
+                h.int_array(list(active_expert_range)), row_idx_type,
                 h.tensor(expanded_x), h.tensor(row_idx), h.tensor(counts), h.tensor(expanded_scale)]
         _run_two_phase("aclnnMoeInitRoutingV3", args, dev, workspace)
     finally:
@@ -439,18 +482,18 @@ def grouped_matmul_swiglu_quant(x, weight, group_list, weight_scale, x_scale, bi
     else:
         output = torch.empty((M, N // 2), dtype=torch.int8, device=dev)
         output_scale = torch.empty((M,), dtype=torch.float32, device=dev)
+    if weight is not None:
+        _run_packed(_SWIGLU_QUANT, (), (x, weight, bias, offset, weight_scale, x_scale, group_list, output, output_scale), dev, workspace)
+        return output, output_scale
     h = _Handles()
     try:
         api = "aclnnGroupedMatmulSwigluQuant"
-        if weight is not None:
-            wh = h.tensor(weight)
+        tensor, how = weight_nz
+        if how == "nz5d":
+            wh = h.raw(nz_weight_handle(tensor))
         else:
-            tensor, how = weight_nz
-            if how == "nz5d":
-                wh = h.raw(nz_weight_handle(tensor))
-            else:
-                api = "aclnnGroupedMatmulSwigluQuantWeightNZ"
-                wh = h.raw(nz_weight_handle(tensor, view_3d=(how == "entry3d"), fmt=ACL_FORMAT_ND))
+            api = "aclnnGroupedMatmulSwigluQuantWeightNZ"
+            wh = h.raw(nz_weight_handle(tensor, view_3d=(how == "entry3d"), fmt=ACL_FORMAT_ND))
         args = [h.tensor(x), wh, h.tensor(bias), h.tensor(offset), h.tensor(weight_scale),
                 h.tensor(x_scale), h.tensor(group_list), h.tensor(output), h.tensor(output_scale), None]
         _run_two_phase(api, args, dev, workspace)
@@ -475,6 +518,14 @@ def grouped_matmul_v4(x, weight, bias=None, scale=None, offset=None, antiquant_s
             output_dtype = torch.int32 if scale is None else (
                 torch.bfloat16 if scale[0].dtype == torch.bfloat16 else torch.float16)
         out = [torch.empty((x[0].shape[0], n_out), dtype=output_dtype, device=dev)]
+    one = lambda ts: ts is None or len(ts) == 1 and ts[0] is not None
+    if (weight is not None and tuning_config is None and all(map(one, (x, weight, bias, scale, per_token_scale, out))) and
+            all(ts is None for ts in (offset, antiquant_scale, antiquant_offset, activation_input, activation_quant_scale,
+                                      activation_quant_offset))):
+        first = lambda ts: None if ts is None else ts[0]
+        _run_packed(_GROUPED_MATMUL_V4, (split_item, group_type, group_list_type, act_type),
+                    (x[0], weight[0], first(bias), first(scale), first(per_token_scale), group_list, out[0]), dev, workspace)
+        return out
     h = _Handles()
     try:
         api = "aclnnGroupedMatmulV5" if tuning_config is not None else "aclnnGroupedMatmulV4"
@@ -557,22 +608,8 @@ def moe_finalize_routing_v2(expanded_x, expanded_row_idx, x1=None, x2=None, bias
     dev = expanded_x.device
     if out is None:
         out = torch.empty((T, H), dtype=expanded_x.dtype, device=dev)
-    h = _Handles()
-    try:
-        args = [h.tensor(expanded_x), h.tensor(expanded_row_idx), h.tensor(x1), h.tensor(x2), h.tensor(bias),
-                h.tensor(scales), h.tensor(expert_idx), drop_pad_mode, h.tensor(out)]
-        _run_two_phase("aclnnMoeFinalizeRoutingV2", args, dev)
-    finally:
-        h.close()
+    _run_packed(_FINALIZE_V2, (drop_pad_mode,), (expanded_x, expanded_row_idx, x1, x2, bias, scales, expert_idx, out), dev)
     return out
-
-
-def _packed(t):
-    if t is None:
-        return _PACK[0](0, 0, 0)
-    shape = t.shape
-    n = len(shape)
-    return _PACK[n](n, _DTYPE_CODE[t.dtype], t.data_ptr(), *shape, *t.stride())
 
 
 _FFN_OPERATORS = (("aclnnMoeInitRoutingV2", "aclnnGroupedMatmulSwigluQuant", "aclnnGroupedMatmulV4"),

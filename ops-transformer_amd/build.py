@@ -37,6 +37,7 @@ SOURCES = [
     "grouped_matmul_finalize_routing.hip",
     "moe_finalize_routing_v2.hip",
     "moe_ffn_forward.hip",
+    "packed_operators.hip",
     "calibration_copy.hip",
 ]
 

@@ -10,6 +10,7 @@ import ctypes
 import glob
 import os
 import re
+import struct
 
 import pytest
 import torch
@@ -772,3 +773,21 @@ def test_ring_tiles_are_numbered_in_32_bits(aclnn, monkeypatch, M, N, E):
     assert E <= m_tiles and m_tiles * ((N + 255) // 256) < 1 << 31
     code, ws = _status(aclnn, *_combine_args(aclnn, M=65536, K=128, N=N, E=E, batch=16))
     assert code == 0 and (ws - 4 * 65536) // 16 - 16 >= 256  # one launch: every row has its place in the table
+
+
+@pytest.mark.parametrize("packed,code", [
+    (None, 161001),                                     # no array
+    ([], 161002), ([7], 161002), ([-1], 161002),        # no operator of that number
+    ([0, 8, 0], 161002),                                # gating without its last scalar
+    ([6, 0] + [0, 0, 0] * 7, 161002),                   # seven of eight tensors
+    ([6, 0] + [0, 0, 0] * 9, 161002),                   # nine
+    ([6, 0] + [9, 0, 0] + [1] * 18 + [0, 0, 0] * 7, 161002),  # nine dimensions
+    ([6, 0] + [2, 0, 0, 4], 161002),                    # an extent short
+    ([6, 0] + [0, 0, 0] * 8, 161001),                   # the operator's own check: no expandedX
+])
+def test_packed_plans_check_their_array(aclnn, packed, code):
+    planned = (ctypes.c_uint64 * 2)()
+    where = ctypes.addressof(planned)
+    data = None if packed is None else struct.pack("%dq" % len(packed), *packed)
+    assert aclnn.lib().opapiPlanPacked(data, 0 if packed is None else len(packed), where, where + 8) == code
+    assert planned[1] == 0
