@@ -80,7 +80,19 @@ struct Plan {
 
 Plan MakePlan(const Problem& p);
 
+// Scheduling shared by two problems on the same group list, one launch for both: the first one's names the second (next...) and where its
+// table goes, the second's names that table.  Both as SchedulesOnce says.
+struct SharedSchedule {
+    const Problem* nextProblem = nullptr;
+    const Plan* nextPlan = nullptr;
+    int32_t* nextTable = nullptr;
+    int32_t* table = nullptr;
+};
+// The plan has one scheduling launch and no second band; its table's bytes.
+bool SchedulesOnce(const Problem& p, const Plan& plan);
+uint64_t ScheduleBytes(const Plan& plan);
+
 // Enqueues scheduling, GEMM and (kSwiglu) requantisation kernels on `stream`.  Returns hipSuccess or the launch error.
-hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStream_t stream);
+hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStream_t stream, const SharedSchedule& shared = SharedSchedule());
 
 }  // namespace gemm

@@ -58,7 +58,9 @@ struct SchedArgs {
     int64_t rowBegin, rowEnd;  // only rows in [rowBegin, rowEnd) get tiles (one band of a launch that runs in row bands)
 };
 
-__global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs a) {
+// One workgroup a table: two problems on one group list share a launch (SharedSchedule).
+__global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs first, SchedArgs second) {
+    const SchedArgs a = blockIdx.x == 0 ? first : second;
     __shared__ int32_t scan[1024];
     const int t = threadIdx.x;
     auto at = [&](int i) -> int64_t {
@@ -623,7 +625,7 @@ Plan MakePlan(const Problem& p) {
     plan.maxTiles = (maxMTiles * plan.tilesN + kXcds - 1) / kXcds * kXcds;
     uint64_t off = 0;
     plan.offSched = off;
-    off += Align256(static_cast<uint64_t>(SchedTotalInts(plan.maxMTiles)) * 4);
+    off += ScheduleBytes(plan);
     if (p.epilogue == Epilogue::kSwiglu) {
         plan.offRowMax = off;
         off += Align256(static_cast<uint64_t>(p.M) * 4 * static_cast<uint64_t>(plan.tilesN));
@@ -644,21 +646,11 @@ Plan MakePlan(const Problem& p) {
     return plan;
 }
 
-hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStream_t stream) {
-    if (p.M == 0 || p.N == 0 || p.groups == 0) return hipSuccess;
-    if (p.groups > kMaxGroups) return hipErrorInvalidValue;
-    // K = 0 leaves the other epilogues nothing to do; with kSwiglu it would leave the requantisation an unwritten S
-    // (the operator's first phase refuses K = 0, so this is a guard, not a path)
-    if (p.K <= 0 && p.epilogue == Epilogue::kSwiglu) return hipErrorInvalidValue;
-    char* ws = static_cast<char*>(workspace);
-    int32_t* sched = reinterpret_cast<int32_t*>(ws + plan.offSched);
-    const bool swiglu = p.epilogue == Epilogue::kSwiglu;
-    float* rowMax = swiglu ? reinterpret_cast<float*>(ws + plan.offRowMax) : nullptr;
-    float* sBuf = swiglu ? reinterpret_cast<float*>(ws + plan.offS) : nullptr;
-
+namespace {
+SchedArgs ScheduleArgsOf(const Problem& p, const Plan& plan, int32_t* table) {
     SchedArgs sa{};
     sa.groupList = p.groupList;
-    sa.sched = sched;
+    sa.sched = table;
     sa.groups = p.groups;
     sa.groupListIsInt64 = p.groupListIsInt64 ? 1 : 0;
     sa.isCount = static_cast<int32_t>(p.groupListKind);
@@ -669,6 +661,30 @@ hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStrea
     sa.tilesN = plan.tilesN;
     sa.maxMTiles = plan.maxMTiles;
     sa.M = p.M;
+    sa.rowEnd = p.M;
+    return sa;
+}
+}  // namespace
+
+bool SchedulesOnce(const Problem& p, const Plan& plan) {
+    return !plan.slim && p.M > 0 && p.N > 0 && p.K > 0 && p.groups > 0 && p.groups <= kMaxGroups && (plan.bandRows == 0 || plan.bandRows >= p.M);
+}
+
+uint64_t ScheduleBytes(const Plan& plan) { return Align256(static_cast<uint64_t>(SchedTotalInts(plan.maxMTiles)) * 4); }
+
+hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStream_t stream, const SharedSchedule& shared) {
+    if (p.M == 0 || p.N == 0 || p.groups == 0) return hipSuccess;
+    if (p.groups > kMaxGroups) return hipErrorInvalidValue;
+    // K = 0 leaves the other epilogues nothing to do; with kSwiglu it would leave the requantisation an unwritten S
+    // (the operator's first phase refuses K = 0, so this is a guard, not a path)
+    if (p.K <= 0 && p.epilogue == Epilogue::kSwiglu) return hipErrorInvalidValue;
+    char* ws = static_cast<char*>(workspace);
+    int32_t* sched = shared.table != nullptr ? shared.table : reinterpret_cast<int32_t*>(ws + plan.offSched);
+    const bool swiglu = p.epilogue == Epilogue::kSwiglu;
+    float* rowMax = swiglu ? reinterpret_cast<float*>(ws + plan.offRowMax) : nullptr;
+    float* sBuf = swiglu ? reinterpret_cast<float*>(ws + plan.offS) : nullptr;
+
+    SchedArgs sa = ScheduleArgsOf(p, plan, sched);
 
     KernelArgs ka{};
     ka.x = p.x;
@@ -710,9 +726,11 @@ hipError_t Enqueue(const Problem& p, const Plan& plan, void* workspace, hipStrea
         const int64_t rowEnd = rowBegin + bandRows < p.M ? rowBegin + bandRows : p.M;
         sa.rowBegin = rowBegin;
         sa.rowEnd = rowEnd;
-        if (!plan.slim) {
+        if (!plan.slim && shared.table == nullptr) {
             opapi::KernelTimer timer("gmm_schedule", stream);
-            hipLaunchKernelGGL(ScheduleKernel, dim3(1), dim3(1024), 0, stream, sa);
+            const bool both = shared.nextTable != nullptr;
+            hipLaunchKernelGGL(ScheduleKernel, dim3(both ? 2 : 1), dim3(1024), 0, stream, sa,
+                               both ? ScheduleArgsOf(*shared.nextProblem, *shared.nextPlan, shared.nextTable) : sa);
         }
         if (swiglu) {
             ka.sOut = reinterpret_cast<float*>(reinterpret_cast<uintptr_t>(sBuf) -

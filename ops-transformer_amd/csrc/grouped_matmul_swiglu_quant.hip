@@ -14,8 +14,7 @@
 
 #include <new>
 
-#include "grouped_gemm_i8.h"
-#include "opapi_common.h"
+#include "gemm_executor.h"
 
 namespace {
 
@@ -24,12 +23,10 @@ class NoOpExecutor : public aclOpExecutor {
     aclnnStatus Run(void*, hipStream_t) override { return ACLNN_SUCCESS; }
 };
 
-class SwigluQuantExecutor : public aclOpExecutor {
+class SwigluQuantExecutor : public GemmExecutor {
    public:
-    gemm::Problem problem;
-    gemm::Plan plan;
     aclnnStatus Run(void* workspace, hipStream_t stream) override {
-        const hipError_t e = gemm::Enqueue(problem, plan, workspace, stream);
+        const hipError_t e = gemm::Enqueue(problem, plan, workspace, stream, shared);
         if (e != hipSuccess) {
             opapi::SetError("aclnnGroupedMatmulSwigluQuant: launch failed: %s", hipGetErrorString(e));
             return ACLNN_ERR_RUNTIME_ERROR;

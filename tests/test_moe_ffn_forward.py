@@ -38,6 +38,17 @@ def test_too_small_a_workspace_enqueues_nothing(aclnn, routing):
     assert sizes[0] > 0 and sizes[1] > 0 and sizes[4] == max(sizes[:4])
 
 
+@pytest.mark.parametrize("cap_mb,shared", [(None, True), (1, False)])  # 1 MB: the SwiGLU operator runs in bands, each with its schedule
+def test_one_schedule_adds_the_second_table(aclnn, monkeypatch, cap_mb, shared):
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    monkeypatch.delenv("OPAPI_SWIGLU_WORKSPACE_MB", raising=False)
+    if cap_mb:
+        monkeypatch.setenv("OPAPI_SWIGLU_WORKSPACE_MB", str(cap_mb))
+    st, sizes, enqueued, _ = _call(aclnn, _pack(aclnn, 2, _tensors(2000, 1024, 512, 4, 2, False)))
+    assert st == 0 and enqueued == 0
+    assert (sizes[4] > max(sizes[:4])) == shared and sizes[4] - max(sizes[:4]) <= sizes[2] + 256
+
+
 @pytest.mark.parametrize("routing", [2, 3])
 def test_a_pass_that_was_not_enqueued_is_an_error(aclnn, monkeypatch, routing):
     """The outputs are reused from pass to pass: returning without having enqueued one would hand out the last one's."""
