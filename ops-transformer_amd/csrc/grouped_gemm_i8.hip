@@ -279,7 +279,8 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs first, SchedArg
     scan[t] = t < a.groups ? tileInc : 0x7fffffff;
     __syncthreads();
     const int32_t totalMTiles = scan[a.groups - 1];
-    // A well-formed list never needs more than maxMTiles m-tiles (M / tileM + groups).  A malformed one whose groups
+    // A well-formed list never needs more than maxMTiles m-tiles: the rows of the launch by the lowest height that MakePlan sizes the table
+    // for, and one more per group (wide tiles are lower only where every group is one).  A malformed one whose groups
     // overlap could: the m-tiles beyond the table are dropped, so no kernel indexes past it.
     const int32_t nBig = min(totals[0], a.maxMTiles);
     const int32_t nSmall = min(totals[1], a.maxMTiles - nBig);
@@ -578,7 +579,8 @@ Plan MakePlan(const Problem& p) {
         plan.lowTileM = kLowTileM;
         plan.lowForRounds = true;
     }
-    // Workspaces are sized, and S is held, for the height chosen so far: the two choices below change neither.
+    // The bands that S is held for are cut at the height chosen so far: the two choices below do not change them.  The table is sized
+    // for the lowest height that a list of more m-tiles than groups may be cut at: this one, or what those put in its place.
     const int sizedFor = plan.lowTileM > 0 ? plan.lowTileM : plan.tileM, bandHeight = plan.tileM;
     // The SwiGLU operator on groups that 160 rows hold nearly all: tiles of 512 channels instead of 256, where that costs no round of the
     // machine, on the two-geometry kernel, which takes the lists that turn out uneven (and did so better than one geometry of 96 to 160
@@ -611,7 +613,7 @@ Plan MakePlan(const Problem& p) {
         plan.lowTileM = kLowTileM;
         plan.lowBySizes = true;
     }
-    const int64_t lowest = sizedFor;
+    const int64_t lowest = std::min(sizedFor, plan.tileM);
     // The LDS-ring kernels number the tiles of a launch in 32 bits.  More than kMaxTiles of them (the scatter-add alone can ask for so
     // many: its output has few rows) run as several launches, each over a band of rows.  One expert's weights stay below 2 GB
     // (StreamOk), so that every group's last m-tile is a small part of the limit: 1024 groups x 65536 n-tiles.

@@ -751,6 +751,23 @@ def test_tile_height_leaves_room_for_uneven_groups(aclnn, monkeypatch):
     assert chosen == of_height[96] != of_height[64]
 
 
+@pytest.mark.parametrize("E,K,N", [(128, 4096, 3072), (256, 7168, 4096), (64, 4096, 28672), (128, 1280, 2048), (128, 2880, 2880)])
+@pytest.mark.parametrize("api", ["aclnnGroupedMatmulSwigluQuant", "aclnnGroupedMatmulV4"])
+def test_table_holds_the_worst_list(aclnn, monkeypatch, api, E, K, N):
+    """32 to 130 rows per group, where the scheduling kernel chooses the height by the sizes it finds: the workspace has sixteen bytes
+    for every m-tile of the list that needs the most (no group empty, as many groups as possible a row past a cut), at the lowest height that
+    such a list may be cut at: 192 rows, or 160 without the SwiGLU epilogue."""
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    monkeypatch.delenv("OPAPI_GEMM_PULL", raising=False)
+    align = lambda n: (n + 255) // 256 * 256
+    swiglu = api == "aclnnGroupedMatmulSwigluQuant"
+    for M in range(32 * E, 1304 * E // 10 + 1, E // 2):
+        code, ws = _status(aclnn, api, _swiglu_args(aclnn, M=M, K=K, N=N, E=E) if swiglu else _gmm_args(aclnn, M=M, K=K, N=N, E=E))
+        assert code == 0
+        table = ws - align(M * 4 * ((N // 2 + 127) // 128)) - align(M * (N // 2) * 4) if swiglu else ws
+        assert table // 16 - 16 >= E + (M - E) // (192 if swiglu else 160), M / E
+
+
 def test_slim_tiles_are_numbered_in_32_bits(aclnn):
     """Two million channels are the widest that the kernels for a handful of rows take (their workspace is a header alone); beyond,
     65535 m-tiles of a malformed list times the tiles side by side would not fit a tile number, and the ring kernels run."""

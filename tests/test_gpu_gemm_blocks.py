@@ -249,3 +249,26 @@ def test_tiles_by_sizes_down(aclnn, monkeypatch, name, layout, K):
     (got, want), rows = _spanned(aclnn, lambda: _run(aclnn, sizes, 2208, K, layout, torch.bfloat16, K))
     assert rows == (160 if name == "over" else want_rows)  # (one group in 128 with a small second m-tile)
     assert torch.equal(got, want)
+
+
+# 130 rows per group: even ones take wide tiles of 160 rows, uneven ones 192, of which these lists need more than M / 256 beyond one per group
+@pytest.mark.parametrize("sizes", [[193] * 86 + [1] * 42, [2080] * 7 + [17] * 98 + [18] * 23])
+def test_table_holds_lists_of_many_second_tiles(aclnn, dev, monkeypatch, sizes):
+    K, columns, E, M = 1280, 1024, len(sizes), sum(sizes)
+    assert (E, M) == (128, 130 * 128) and sum((r + 191) // 192 for r in sizes) > M // 256 + E
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.empty((M, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    w = torch.empty((E, 2 * columns, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    scale, x_scale = torch.rand((E, 2 * columns), device=dev, generator=g) * 1e-3, torch.rand((M,), device=dev, generator=g) * 1e-2
+    cumsum = torch.cumsum(torch.tensor(sizes), 0).to(dev)
+
+    def call():
+        out = (torch.full((M, columns), 7, dtype=torch.int8, device=dev), torch.full((M,), 7.0, device=dev))
+        return aclnn.grouped_matmul_swiglu_quant(x, w.transpose(1, 2), cumsum, scale, x_scale, out=out)
+
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    (y, ys), rows = _spanned(aclnn, call)
+    assert rows == 192
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", "96")
+    (y96, ys96), rows = _spanned(aclnn, call)
+    assert rows == 96 and torch.equal(y, y96) and torch.equal(ys, ys96)
