@@ -21,8 +21,10 @@ extern "C" {
 //   x int8 [T, H], xScale fp32 [T], expertIdx int32 [T, K], weights of the combine [T, K] (no dimensions at address 0: none, K 1),
 //   w13 [E, H, 2I], w13Scale [E, 2I], w2 [E, I, H], w2Scale [E, H]  (a five-dimensional weight is FRACTAL_NZ),
 //   expandedX, expandedRowIdx, cumsum, expandedScale, h, hScale, y, out.
-// count: values in the array.  workspaceSizes[5]: what each operator asks for, and the largest of them.  When that is more
-// than workspaceSize nothing is enqueued and ACLNN_SUCCESS is returned with *enqueued 0: call again with as much.
+// count: values in the array.  workspaceSizes[5]: what each operator asks for, and what the pass makes use of, which is the largest of
+// these and, where one launch can schedule both GEMMs, room behind it for the second one's table.  When the largest is more
+// than workspaceSize nothing is enqueued and ACLNN_SUCCESS is returned with *enqueued 0: call again with workspaceSizes[4] bytes.  With
+// the largest but less than those every GEMM is scheduled by a launch of its own, with the same results.
 // On failure *failedOperator names the entry point that returned the status (its message: aclGetRecentErrMsg).
 ACL_API aclnnStatus opapiMoeFfnForward(const int64_t* packed, uint64_t count, void* workspace, uint64_t workspaceSize, aclrtStream stream,
                                        uint64_t* workspaceSizes, int32_t* enqueued, const char** failedOperator);

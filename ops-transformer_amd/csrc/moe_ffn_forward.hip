@@ -94,17 +94,17 @@ extern "C" aclnnStatus opapiMoeFfnForward(const int64_t* packed, uint64_t count,
                                                    weighted ? &t[kTopKWeight] : nullptr, nullptr, 2,
                                                    &t[kOut], &workspaceSizes[3], &ex.of[3]);
     if (st != ACLNN_SUCCESS) return st;
-    workspaceSizes[4] = *std::max_element(workspaceSizes, workspaceSizes + 4);
+    const uint64_t largest = *std::max_element(workspaceSizes, workspaceSizes + 4);
     // One launch schedules both GEMMs where each has one: the down projection's table then waits behind everybody's workspace.  (A launch
     // of 4 us less: 1303 tokens top-2 of 8 experts, hidden and intermediate 1024, 67 -> 64 us; 1000 of these, 4096, 14336, 505 -> 500.)
     auto* const up = dynamic_cast<GemmExecutor*>(ex.of[1]);
     auto* const down = dynamic_cast<GemmExecutor*>(ex.of[2]);
-    const uint64_t tableAt = AlignUp(workspaceSizes[4], 256);
-    const bool oneSchedule = up != nullptr && down != nullptr && up->stagingBytes == 0 && down->stagingBytes == 0 &&
+    const uint64_t tableAt = AlignUp(largest, 256);
+    const bool mayShare = up != nullptr && down != nullptr && up->stagingBytes == 0 && down->stagingBytes == 0 &&
                              gemm::SchedulesOnce(up->problem, up->plan) && gemm::SchedulesOnce(down->problem, down->plan);
-    if (oneSchedule) workspaceSizes[4] = tableAt + gemm::ScheduleBytes(down->plan);
-    if (workspaceSizes[4] > workspaceSize) return ACLNN_SUCCESS;
-    if (oneSchedule) {  // (the second executor outlives the first one's run)
+    workspaceSizes[4] = mayShare ? tableAt + gemm::ScheduleBytes(down->plan) : largest;
+    if (largest > workspaceSize) return ACLNN_SUCCESS;
+    if (mayShare && workspaceSizes[4] <= workspaceSize) {  // (the second executor outlives the first one's run)
         down->shared.table = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + tableAt);
         up->shared.nextProblem = &down->problem;
         up->shared.nextPlan = &down->plan;

@@ -176,3 +176,31 @@ def test_equals_the_operators_one_by_one(pkg, aclnn, dev, tokens, routing):
                                 group_type=0, group_list_type=0, output_dtype=torch.bfloat16)[0]
     want = aclnn.moe_finalize_routing_v2(y, row_idx, scales=wgt, drop_pad_mode=2)
     assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_a_workspace_without_room_for_the_second_table(aclnn, dev):
+    """The largest of the operators' sizes is enough: the pass is enqueued, with the results of one that has room for both tables."""
+    T, H, I, E, K = 2000, 1024, 512, 4, 2
+    tensors = _tensors(T, H, I, E, K, dev=dev)
+    g = torch.Generator(device=dev).manual_seed(2)
+    for t in tensors[:8]:
+        if t.dtype == torch.int8:
+            t.random_(-127, 128, generator=g)
+        elif t.dtype == torch.float32:
+            t.uniform_(1e-3, 1e-2, generator=g)
+    tensors[2].copy_(torch.rand((T, E), device=dev, generator=g).topk(K, dim=1)[1])
+    data = _pack(aclnn, 2, tensors)
+    sizes = _call(aclnn, data)[1]
+    assert sizes[4] > max(sizes[:4])
+    outs = []
+    for nbytes in (sizes[4], sizes[4] - 1, max(sizes[:4])):
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        tensors[15].zero_()
+        torch.cuda.synchronize()
+        st, _, enqueued, name = _call(aclnn, data, workspace.data_ptr(), nbytes)
+        torch.cuda.synchronize()
+        assert st == 0 and enqueued == 1, name
+        outs.append(tensors[15].clone())
+    assert outs[0].any() and torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    assert _call(aclnn, data, 0x1000, max(sizes[:4]) - 1)[1:3] == (sizes, 0)
