@@ -1184,7 +1184,9 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     };
     // This wave's DMA instruction of slot q of the stage at the cursor.  Activation rows always stay cacheable (the
     // n-tiles of a group re-read them from L2); on small tiles (every weight byte is used exactly once) the weights stream
-    // past the caches.  On large tiles the m-tiles of a group share their weight columns through L2 and must not.
+    // past the caches.  On large tiles the m-tiles of a group share their weight columns through L2 and must not, nor must K-contiguous rows
+    // with K off the 128 grid: a k-step of such a row ends inside a line, and the next one asks for that again.  us, past the caches ->
+    // this: 256 experts of 20 rows, 2880 x 2 x 1440 511 -> 446, down 312 -> 245; of 25, rank^-0.8 577 -> 476, 353 -> 269.
     auto request = [&](int q) __attribute__((always_inline)) {
         const int kIdx = issStep + issRotate;
         const int kOff = issDrained ? 0 : kTail ? min(kIdx * kStep, a.K - kStep) : (kIdx >= kSteps ? kIdx - kSteps : kIdx) * kStep;
@@ -1193,7 +1195,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                                  (kUnits > 1 && issUnit != 0 ? issUnitShift : 0);
         const uint32_t dst = issAddr + 1024 * kWavesN * q;
         if constexpr (kSmallTile) {
-            if (forWeights) DmaToLdsAddr16<true>(base, laneOff[q], dst);
+            if (forWeights) DmaToLdsAddr16<!kTail || kNz || kNMajor>(base, laneOff[q], dst);
             else if (q < Cfg::kSlotsA) DmaToLdsAddr16<false>(base, laneOff[q], dst);
         } else {
             if (q < Cfg::kSlotsA || forWeights) DmaToLdsAddr16<false>(base, laneOff[q], dst);
