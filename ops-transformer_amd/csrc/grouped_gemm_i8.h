@@ -61,6 +61,9 @@ constexpr int kSlimMaxGroups = 512;
 constexpr int64_t kSlimMaxRows = 65535;
 constexpr int64_t kSlimMaxTilesN = 16384;
 
+// Plan::offGrid: weights whose rows begin inside cache lines, in launches of few and of many k-steps a workgroup.
+constexpr int kOffGridShort = 1, kOffGridLong = 2;
+
 // Tile shape chosen from the static shape (M, groups); fixed for the lifetime of a plan.
 struct Plan {
     int tileM = 0;          // rows per workgroup tile (multiple of 32; slim: 16, 32 or 64, the lowest that the kernel may take)
@@ -68,6 +71,8 @@ struct Plan {
     bool lowForRounds = false;  // it chooses by rounds of the machine,
     bool lowBySizes = false;    // by how many groups are small or have several m-tiles, else by the rows that groups leave over
     bool lowIsWide = false;     // those tiles are 512 channels wide
+    int offGrid = 0;            // with lowBySizes: small m-tiles cost more than they are taken for (kOffGridShort, kOffGridLong)
+    bool maySmall = false;      // with lowBySizes: or 64 rows for all, the height by the mean
     int64_t maxTiles = 0;   // launch bound on workgroups
     int32_t maxMTiles = 0;  // upper bound on m-tiles of a launch over all groups (its rows / tileM + groups)
     int32_t tilesN = 0;

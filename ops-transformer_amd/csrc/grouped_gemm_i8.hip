@@ -51,12 +51,32 @@ struct SchedArgs {
     int32_t mayLower;  // 1: m-tiles of kLowTileM rows instead where they leave at most an eighth of the groups a small last one;
                        // 3: for means below those, by how many groups are small or have several m-tiles;
                        // 2: where they fill at most two rounds of the machine, and no more of them than the tall ones
-    int32_t lowIsWide;  // with mayLower 3: the tiles of the lower m-tiles are two 256-channel units wide
+    // with mayLower 3:
+    int32_t lowIsWide;   // the tiles of the lower m-tiles are two 256-channel units wide
+    int32_t offGrid;     // weights whose rows begin inside cache lines (Plan::offGrid)
+    int32_t maySmall;    // or all m-tiles of kSmallRows rows
+    int32_t kSteps;
     int32_t cus, tilesN;
     int32_t maxMTiles;
     int64_t M;
     int64_t rowBegin, rowEnd;  // only rows in [rowBegin, rowEnd) get tiles (one band of a launch that runs in row bands)
 };
+
+// A group's m-tiles of at most `cut` rows, and the cost of the big ones.
+struct Cut {
+    int32_t big, small, bigCost;
+};
+__device__ __forceinline__ Cut CutOf(int32_t rows, int32_t cut, bool allSmall, bool oneList) {
+    const int32_t tiles = (rows + cut - 1) / cut, lastRows = tiles > 0 ? rows - (tiles - 1) * cut : 0;
+    Cut c{};
+    c.small = allSmall ? tiles : (!oneList && tiles > 0 && lastRows <= kSmallRows ? 1 : 0);
+    c.big = tiles - c.small;
+    if (c.big > 0) {
+        const bool lastIsBig = c.small == 0;
+        c.bigCost = (c.big - (lastIsBig ? 1 : 0)) * max(cut >> 5, kSmallCost) + (lastIsBig ? max((lastRows + 31) >> 5, kSmallCost) : 0);
+    }
+    return c;
+}
 
 // One workgroup a table: two problems on one group list share a launch (SharedSchedule).
 __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs first, SchedArgs second) {
@@ -163,6 +183,7 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs first, SchedArg
     int32_t tileM = a.tileM, cut = tileM;  // cut: rows per m-tile of this group
     int32_t wide = 0;
     bool oneList = false;  // small m-tiles among the big ones
+    bool dealt = false;    // every tile belongs to a workgroup from the start
     if (a.mayLower == 2) {
         // Whole rounds of the machine, one of low tiles costing 0.7 to 0.85 of one of tall ones: their ring is a stage deeper, and
         // the launch ends with its tallest tile.  Low tiles where they are one round; where they are two, only if the tall ones
@@ -198,15 +219,19 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs first, SchedArg
     } else if (a.mayLower) {
         const int32_t last = rows % kLowTileM;
         const bool smallLast = last > 0 && last <= kSmallRows;
-        bool lower;
+        bool lower, narrow = false;
         if (a.mayLower == 1) {
             lower = __syncthreads_count(smallLast) * 8 <= a.groups;
         } else {
-            // Groups of at most kSmallRows rows, nearly all of them: the two-geometry kernel's small run.  us, one geometry / that: 256
-            // experts of 50 rows, hidden 7168, intermediate 2048 1285 (wide) and 736 / 1170 and 708.  Half of them, beside groups of
-            // several m-tiles: that too, 80 rows at rank^-0.6 875 / 808 (down).  Otherwise one geometry, wide only where no group needs a
-            // second m-tile, which costs at least one tile of twice the length at the launch's end: 128 experts, 4096, 1536, 80 rows at
-            // rank^-0.3 332 / 316 with two of them; 60 and 72 rows even 302 / 325 and 299 / 314, down 185 / 199.
+            // us; experts, rows each on average at popularity rank^-s, sizes of the launch.
+            // Groups of at most kSmallRows rows, nearly all of them: the two-geometry kernel's small run.  One geometry / that: 256
+            // of 50, 7168 x 2 x 2048 1285 (wide), 2048 x 7168 736 / 1170, 708.  Half of them, beside groups of
+            // several m-tiles: that too, of 80 at s 0.6 875 / 808 (down).  Otherwise one geometry.
+            // Wide tiles are half as many, and a launch of a part of a round ends with a tile of twice the length: beside second m-tiles of
+            // more than a few groups they are taken where few groups are small and there are four rounds of them, two geometries / that:
+            // 7168 x 2 x 2048, 256 of 100 at s 0.4 1541 / 1440; 1024 x 2 x 1024 170 / 147; not 7168 x 2 x 2048, 256 of 128 even, one of
+            // 161 rows 1440 / 1463, nor 32 of 100 at s 0.4 245 / 267; and where they fill at most two rounds of the machine well:
+            // 4096 x 2 x 1536, 32 of 80 at s 1.2 121 / 88.
             // (Counted by ballots and one round of LDS: four __syncthreads_count took 3 us.)
             __shared__ int4 waveCounts[16];
             const int4 mine = make_int4(__popcll(__ballot(rows > 0)), __popcll(__ballot(rows > 0 && rows <= kSmallRows)),
@@ -221,28 +246,70 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs first, SchedArg
                 over += waveCounts[w].z;
                 loses += waveCounts[w].w;
             }
-            lower = small * 8 < some * 7 && (a.lowIsWide ? over == 0 : loses * 8 <= a.groups && (small * 2 < some || over * 32 < a.groups));
+            const bool fewSmall = small * 8 < some * 7, manyOver = over * 16 > some;
+            const bool offGridOver = a.offGrid != 0 && over > 0, oneOrTwo = a.lowIsWide && !a.maySmall && fewSmall && manyOver;
+            if (a.lowIsWide) lower = over == 0 && (fewSmall || a.offGrid);
+            else lower = a.offGrid == kOffGridLong || (fewSmall && loses * 8 <= a.groups && (small * 2 < some || over * 32 < a.groups));
+            // What asks for sums over the groups asks once more (1.7 us): the m-tiles of the lowest height, and in two geometries the big
+            // ones and the cost of all.
+            if (!lower && (a.maySmall || offGridOver || oneOrTwo)) {
+                __shared__ uint2 waveSums[16];
+                const Cut planned = CutOf(rows, tileM, false, false);
+                const int32_t lowestHeight = a.maySmall ? kSmallRows : kLowTileM;
+                // (the two counts in one register, where a wave's sums stay below 2^16)
+                uint32_t countSum = min((rows + lowestHeight - 1) / lowestHeight, 1023) | min(planned.big, 1023) << 16;
+                uint32_t costSum = planned.bigCost + planned.small * kSmallCost;
+#pragma unroll
+                for (int d = 1; d < 64; d <<= 1) {
+                    countSum += __shfl_xor(countSum, d, 64);
+                    costSum += __shfl_xor(costSum, d, 64);
+                }
+                if ((t & 63) == 0) waveSums[t >> 6] = make_uint2(countSum, costSum);
+                __syncthreads();
+                uint32_t lowestSum = 0, bigSum = 0;
+                costSum = 0;
+#pragma unroll
+                for (int w = 0; w < 16; ++w) {
+                    lowestSum += waveSums[w].x & 0xffffu;
+                    bigSum += waveSums[w].x >> 16;
+                    costSum += waveSums[w].y;
+                }
+                const float perCu = static_cast<float>(a.tilesN) / static_cast<float>(a.cus);  // rounds of the machine that an m-tile's tiles are
+                const float wideRounds = static_cast<float>(lowestSum) * static_cast<float>((a.tilesN + 1) / 2) / static_cast<float>(a.cus);
+                if (a.maySmall) {
+                    // Means that 64-row tiles hold: those for every group, dealt out whole, where the weights that groups of several of them
+                    // read again cost less than the change of geometry, 8 k-steps' time, or 12 with more big tiles than workgroups begin
+                    // with.  A round that has begun is half a one at least (a quarter behind tiles that are drawn).  64-row tiles / two
+                    // geometries: 2048 x 2 x 2048, 64 of 25 at s 0.4 104 / 108, of 32 at s 1.2 119 / 110; 7168 x 2 x 2048, 64 of 25 at
+                    // s 0.4 327 / 298.  (The ones of a fixed share took 104 too, drawn ones 111.)
+                    auto begun = [](float r, float least) { return floorf(r) + (r > floorf(r) ? fmaxf(r - floorf(r), least) : 0.0f); };
+                    const float kSteps = static_cast<float>(a.kSteps), change = static_cast<float>(bigSum) * perCu * 8.0f <= 7.0f ? 8.0f : 12.0f;
+                    if (begun(static_cast<float>(lowestSum) * perCu, 0.5f) * kSteps <
+                        begun(static_cast<float>(costSum) * perCu * (1.0f / kSmallCost), 0.25f) * kSteps + change) {
+                        tileM = cut = kSmallRows;
+                        dealt = true;
+                    }
+                } else if (a.offGrid == kOffGridLong) {
+                    lower = true;
+                    narrow = wideRounds < 4.0f;
+                } else {
+                    lower = oneOrTwo && (wideRounds <= 2.0f ? wideRounds * 6.0f >= ceilf(wideRounds) * 5.0f : small * 4 < some && wideRounds >= 4.0f);
+                    if (!lower && offGridOver && fewSmall && manyOver) lower = narrow = true;
+                }
+            }
         }
         if (lower) {
             tileM = cut = kLowTileM;
-            wide = a.lowIsWide;
+            wide = a.lowIsWide && !narrow;
             oneList = a.mayLower == 3;
         }
     }
-    const int32_t tiles = (rows + cut - 1) / cut;
     // big and small m-tiles of this group (with tiles of at most kSmallRows rows every m-tile is small; otherwise only
     // a group's last, partly filled m-tile can be) and the cost of the big ones; two packed prefix sums give every
     // group the positions of its m-tiles in the two runs of the table, and the launch the totals
     const bool allSmall = tileM <= kSmallRows;
-    const int32_t lastRows = tiles > 0 ? rows - (tiles - 1) * cut : 0;
-    const int32_t smallCount = allSmall ? tiles : (!oneList && tiles > 0 && lastRows <= kSmallRows ? 1 : 0);
-    const int32_t bigCount = tiles - smallCount;
-    int32_t bigCost = 0;
-    if (bigCount > 0) {
-        const bool lastIsBig = smallCount == 0;
-        const int32_t lastSub = (lastRows + 31) >> 5;
-        bigCost = (bigCount - (lastIsBig ? 1 : 0)) * max(cut >> 5, kSmallCost) + (lastIsBig ? max(lastSub, kSmallCost) : 0);
-    }
+    const Cut own = CutOf(rows, cut, allSmall, oneList);
+    const int32_t tiles = own.big + own.small, smallCount = own.small, bigCount = own.big, bigCost = own.bigCost;
     uint64_t countsInc = static_cast<uint64_t>(tiles) | (static_cast<uint64_t>(bigCount) << 32);
     uint64_t costInc = static_cast<uint64_t>(bigCost) | (static_cast<uint64_t>(tiles > 0 ? 1 : 0) << 32);
     inclusiveScan64(countsInc, costInc);
@@ -280,7 +347,7 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs first, SchedArg
     __syncthreads();
     const int32_t totalMTiles = scan[a.groups - 1];
     // A well-formed list never needs more than maxMTiles m-tiles: the rows of the launch by the lowest height that MakePlan sizes the table
-    // for, and one more per group (wide tiles are lower only where every group is one).  A malformed one whose groups
+    // for, and one more per group.  A malformed one whose groups
     // overlap could: the m-tiles beyond the table are dropped, so no kernel indexes past it.
     const int32_t nBig = min(totals[0], a.maxMTiles);
     const int32_t nSmall = min(totals[1], a.maxMTiles - nBig);
@@ -294,7 +361,7 @@ __global__ __launch_bounds__(1024) void ScheduleKernel(SchedArgs first, SchedArg
         a.sched[t] = t == 0 ? nBig : t == 1 ? nSmall : t == 2 ? nSmall * kSmallCost : t == 3 ? totals[2] : t == 4 ? wideBands
                    : t == 5 ? (allSmall ? wideBands : 1) : t == kHdrCoveredRows ? sCovered : t == kHdrTileM ? tileM
                    : t == kHdrWide ? wide
-                   : t == kHdrEven ? (totalMTiles * 8 <= totals[3] * 9 && (nSmall * 8 <= totals[3] || nBig == 0) ? 1 : 0) : 0;
+                   : t == kHdrEven ? dealt ? 2 : (totalMTiles * 8 <= totals[3] * 9 && (nSmall * 8 <= totals[3] || nBig == 0) ? 1 : 0) : 0;
     }
     int4* const mTileTable = reinterpret_cast<int4*>(a.sched + kQueueHeaderInts + kQueueCounterInts);
     for (int32_t m = t; m < totalMTiles; m += 1024) {
@@ -580,8 +647,11 @@ Plan MakePlan(const Problem& p) {
         plan.lowForRounds = true;
     }
     // The bands that S is held for are cut at the height chosen so far: the two choices below do not change them.  The table is sized
-    // for the lowest height that a list of more m-tiles than groups may be cut at: this one, or what those put in its place.
+    // for the lowest height that a list may be cut at: this one, or what those put in its place.
     const int sizedFor = plan.lowTileM > 0 ? plan.lowTileM : plan.tileM, bandHeight = plan.tileM;
+    // (Row-major weights: two geometries beat 64-row tiles on nearly every uneven list, gate/up 2048 x 2 x 2048, 256 experts of 20 at
+    // rank^-0.4 378 / 463 us.)
+    const bool maySmall = plan.tileM == kSmallRows && (p.wKMajor || p.wNz);
     // The SwiGLU operator on groups that 160 rows hold nearly all: tiles of 512 channels instead of 256, where that costs no round of the
     // machine, on the two-geometry kernel, which takes the lists that turn out uneven (and did so better than one geometry of 96 to 160
     // rows).  Such launches are bound by what a CU has under way, some 32 KB of lines however deep its ring; wide tiles read the
@@ -600,6 +670,7 @@ Plan MakePlan(const Problem& p) {
             plan.pullTiles = true;
             plan.lowTileM = kLowTileM;
             plan.lowBySizes = plan.lowIsWide = true;
+            plan.maySmall = maySmall;
         }
     }
     // The others on such groups: 160 rows in one geometry are as good as 96 or 128 where the groups are alike, and the two-geometry kernel
@@ -612,8 +683,18 @@ Plan MakePlan(const Problem& p) {
         plan.pullTiles = true;
         plan.lowTileM = kLowTileM;
         plan.lowBySizes = true;
+        plan.maySmall = maySmall;
     }
-    const int64_t lowest = std::min(sizedFor, plan.tileM);
+    // Weights whose rows begin inside cache lines -- K-contiguous ones with K off the 128 grid, the two halves of row-major ones for SwiGLU with N
+    // off it -- on taller plans than 64 rows: tiles of few rows pay for the lines at the ends of theirs, and one geometry is better for more
+    // lists.  Long: a workgroup walks sixty k-steps and more.  us, two geometries / one: 2880 x 2 x 1440, 256 experts of 50 rows even 480 / 439
+    // (wide), at rank^-0.4 492 / 476, 128 of these, 277 / 252 (268 wide); down 272 / 263, of 60 296 / 271; 1296 x 2 x 1024, 128 of 60 at
+    // rank^-0.8 120 / 112 (125 wide).  Row-major: 2880 x 2 x 1440, 256 of 50 even 553 / 437, of 100 at rank^-0.8 667 / 558; not 1344 x 2 x 1280, of 50 at
+    // rank^-0.4 191 / 213 (wide).
+    if (plan.lowBySizes && !plan.maySmall && !p.wNz && (p.wKMajor ? p.K : p.epilogue == Epilogue::kSwiglu ? p.N : 0) % 128 != 0) {
+        plan.offGrid = rounds * kSteps >= 60.0 ? kOffGridLong : kOffGridShort;
+    }
+    const int64_t lowest = plan.lowBySizes ? std::min(sizedFor, kLowTileM) : sizedFor;
     // The LDS-ring kernels number the tiles of a launch in 32 bits.  More than kMaxTiles of them (the scatter-add alone can ask for so
     // many: its output has few rows) run as several launches, each over a band of rows.  One expert's weights stay below 2 GB
     // (StreamOk), so that every group's last m-tile is a small part of the limit: 1024 groups x 65536 n-tiles.
@@ -659,6 +740,9 @@ SchedArgs ScheduleArgsOf(const Problem& p, const Plan& plan, int32_t* table) {
     sa.tileM = plan.tileM;
     sa.mayLower = plan.lowForRounds ? 2 : plan.lowBySizes ? 3 : plan.lowTileM > 0 ? 1 : 0;
     sa.lowIsWide = plan.lowIsWide ? 1 : 0;
+    sa.offGrid = plan.offGrid;
+    sa.maySmall = plan.maySmall ? 1 : 0;
+    sa.kSteps = static_cast<int32_t>((p.K + 127) / 128);
     sa.cus = DeviceCuCount();
     sa.tilesN = plan.tilesN;
     sa.maxMTiles = plan.maxMTiles;

@@ -108,7 +108,7 @@ constexpr int kLdsBudget = 160 * 1024;
 // ---------------------------------------------------------------------------------------------- scheduling table
 // int32 layout, all written by the scheduling kernel:
 //   header, 32 ints: [0] big m-tiles, [1] small m-tiles, [2] cost of the small ones, [3] cost of the big ones (see below),
-//                    [4] / [5] band width of the big / small run, [6] total rows covered by the groups, [7] rows per m-tile, [8] 1: nearly every group is one m-tile, of one kind, [9] 1: tiles are 512 channels wide;
+//                    [4] / [5] band width of the big / small run, [6] total rows covered by the groups, [7] rows per m-tile, [8] 1: nearly every group is one m-tile, of one kind, 2: every tile is dealt out, [9] 1: tiles are 512 channels wide;
 //   16 tile counters in one 128-byte line (32 ints): counter [2 * xcd + list], zeroed;
 //   the m-tile table, 4 ints per m-tile {group, first row, rows, 0} (at most maxMTiles of them): the big m-tiles in group
 //   order, then the small ones.  A GEMM kernel finds everything about a tile with one 16-byte load.
@@ -1022,7 +1022,9 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         int32_t eachBig = eachOf(bigTiles), eachSmall = eachOf(smallTiles);
         if (sched[kHdrEven] != 0) {
             if (eachBig > 1 && slots > forSmall) eachBig = max(eachBig, bigTiles / kXcds / (slots - forSmall));
-            if (eachSmall > 1 && bigTiles == 0) eachSmall = max(eachSmall, smallTiles / kXcds / slots);
+            // (2: the part of a round that is left too; drawn, it would cost every workgroup a draw that finds nothing, some 6 us)
+            const int32_t lastRound = sched[kHdrEven] == 2 ? kXcds * slots - 1 : 0;
+            if (eachSmall > 1 && bigTiles == 0) eachSmall = max(eachSmall, (smallTiles + lastRound) / kXcds / slots);
         }
         const QueueLists lists{bigTiles, smallTiles, eachBig * (slots - forSmall), eachSmall * forSmall};
         const int32_t seats = prefer ? forSmall : slots - forSmall, seat = prefer ? slot : slot - forSmall;
@@ -1550,7 +1552,7 @@ __global__ __launch_bounds__(kThreads) void MixedGemmKernel(KernelArgs a, const 
             StreamGemmBody<kSmallRows, kEpi, kNz, kNMajor, kSmallRun, kTail>(a, sched, lds, spanTiles, false);
         }
     }
-    WriteSpan(a, spanStart, spanTiles);
+    WriteSpan(a, spanStart, spanTiles, sched[kHdrTileM]);
 }
 
 // ---------------------------------------------------------------------------------------------- generic path

@@ -756,7 +756,7 @@ def test_tile_height_leaves_room_for_uneven_groups(aclnn, monkeypatch):
 def test_table_holds_the_worst_list(aclnn, monkeypatch, api, E, K, N):
     """32 to 130 rows per group, where the scheduling kernel chooses the height by the sizes it finds: the workspace has sixteen bytes
     for every m-tile of the list that needs the most (no group empty, as many groups as possible a row past a cut), at the lowest height that
-    such a list may be cut at: 192 rows, or 160 without the SwiGLU epilogue."""
+    such a list may be cut at: 160 rows."""
     monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
     monkeypatch.delenv("OPAPI_GEMM_PULL", raising=False)
     align = lambda n: (n + 255) // 256 * 256
@@ -765,7 +765,7 @@ def test_table_holds_the_worst_list(aclnn, monkeypatch, api, E, K, N):
         code, ws = _status(aclnn, api, _swiglu_args(aclnn, M=M, K=K, N=N, E=E) if swiglu else _gmm_args(aclnn, M=M, K=K, N=N, E=E))
         assert code == 0
         table = ws - align(M * 4 * ((N // 2 + 127) // 128)) - align(M * (N // 2) * 4) if swiglu else ws
-        assert table // 16 - 16 >= E + (M - E) // (192 if swiglu else 160), M / E
+        assert table // 16 - 16 >= E + (M - E) // 160, M / E
 
 
 def test_slim_tiles_are_numbered_in_32_bits(aclnn):

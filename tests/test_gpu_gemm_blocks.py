@@ -272,3 +272,50 @@ def test_table_holds_lists_of_many_second_tiles(aclnn, dev, monkeypatch, sizes):
     monkeypatch.setenv("OPAPI_GEMM_TILE_M", "96")
     (y96, ys96), rows = _spanned(aclnn, call)
     assert rows == 96 and torch.equal(y, y96) and torch.equal(ys, ys96)
+
+
+# What else the sizes decide: 64-row tiles for all, dealt out with a part of a round; the big tiles of two geometries, 96 and 192 of them all begun
+# with and 304 that are not; wide tiles beside second m-tiles, in more than four rounds and in most of one; rows of weights that begin inside
+# cache lines, K-contiguous and row-major, in launches of few and of many k-steps a workgroup
+FORMS = {"dealt": ([30, 29, 33, 64, 1, 28, 35, 31] * 15 + [65, 70, 129, 0, 30, 30, 17, 30], "k", 1280, 1024, 64),
+         "dealt_blocked": ([30, 29, 33, 64, 1, 28, 35, 31] * 15 + [65, 70, 129, 0, 30, 30, 17, 30], "nz", 1280, 1024, 64),
+         "begun": ([25] * 120 + [64, 0, 1, 1] + [1150] * 4, "k", 1280, 1024, 192),
+         "begun_long": ([14] * 120 + [64, 0, 1, 1] + [575] * 4, "k", 4096, 1024, 192),
+         "some_begun": ([13] * 120 + [192 * 4, 300, 700, 192 * 5, 192 * 5, 192 * 5, 1100, 1300], "k", 1280, 1024, 192),
+         "wide_over": ([100] * 230 + [161, 200, 320, 321, 65] * 5, "k", 1024, 1024, 160),
+         "wide_round": ([80] * 26 + [200, 161, 170, 180, 190, 320], "k", 4096, 1536, 160),
+         "short": ([50] * 100 + [161, 200] * 6 + [70] * 16, "k", 1296, 1024, 160),
+         "long": ([50] * 100 + [161, 200] * 6 + [70] * 16, "k", 2064, 1001, 160),
+         "long_small": ([64] * 64 + [45] * 63 + [1], "k", 2064, 1024, 160),
+         "long_row_major": ([50] * 100 + [161, 200] * 6 + [70] * 16, "nd", 2048, 1008, 160)}
+
+
+@pytest.mark.parametrize("name", sorted(FORMS))
+def test_forms_by_sizes_swiglu_equal_a_forced_height(aclnn, dev, monkeypatch, name):
+    sizes, layout, K, columns, want_rows = FORMS[name]
+    E, M = len(sizes), sum(sizes)
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.empty((M, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    w = torch.empty((E, 2 * columns, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    view, nz = _weights(w, layout)
+    scale, x_scale = torch.rand((E, 2 * columns), device=dev, generator=g) * 1e-3, torch.rand((M,), device=dev, generator=g) * 1e-2
+    cumsum = torch.cumsum(torch.tensor(sizes), 0).to(dev)
+
+    def call():
+        out = (torch.full((M, columns), 7, dtype=torch.int8, device=dev), torch.full((M,), 7.0, device=dev))
+        return aclnn.grouped_matmul_swiglu_quant(x, view, cumsum, scale, x_scale, out=out, weight_nz=nz)
+
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    (y, ys), rows = _spanned(aclnn, call)
+    assert rows == want_rows
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", "96")
+    (y96, ys96), rows = _spanned(aclnn, call)
+    assert rows == 96 and torch.equal(y, y96) and torch.equal(ys, ys96)
+
+
+@pytest.mark.parametrize("name,K,N,want_rows", [("dealt", 1280, 2208, 64), ("begun", 1280, 2208, 192), ("some_begun", 1024, 2208, 192), ("long_small", 2064, 2208, 160)])
+def test_forms_by_sizes_down(aclnn, monkeypatch, name, K, N, want_rows):
+    monkeypatch.delenv("OPAPI_GEMM_TILE_M", raising=False)
+    (got, want), rows = _spanned(aclnn, lambda: _run(aclnn, FORMS[name][0], N, K, "k", torch.bfloat16, K))
+    assert rows == want_rows
+    assert torch.equal(got, want)
