@@ -767,7 +767,10 @@ struct StreamCfg {
     static constexpr int kHalfBytesB = kStageBytesB / 2;
     static constexpr int kQueueLdsInts = 40;  // the workgroup's next eight tiles and how it comes by them
     static constexpr int kRowScales = (kRows + 63) / 64 * 64;  // in whole DMA instructions
-    static constexpr int kScratchBytes = (kUnits * kTileN + kRowScales + kRows + kQueueLdsInts) * 4;  // channel scales, row scales, row maxima, tiles
+    // Tiles of 256 rows, whose rings are two stages deep, hold the next tile's scales too (see requestScales).
+    static constexpr int kScaleSets = kRows == 256 ? 2 : 1;
+    // channel scales, row scales, row maxima, tiles
+    static constexpr int kScratchBytes = (kScaleSets * (kUnits * kTileN + kRowScales) + kRows + kQueueLdsInts) * 4;
     static constexpr int kRingBytes = kLdsBudget - kScratchBytes;
     // as many weight stages as leave room for two of activation rows, then as many of those as fit
     static constexpr int kFitB = (kRingBytes - 2 * kStageBytesA) / kStageBytesB;
@@ -937,9 +940,9 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     using Blocks = RowBlocks<kRows>;
     constexpr bool kSwiglu = kEpi == Epilogue::kSwiglu;
     constexpr int kUnitCols = kSwiglu ? kTileN / 2 : kTileN;  // output columns of 256 channels
-    float* const ldsChannelScale = reinterpret_cast<float*>(lds + Cfg::kFirstB + Cfg::kStagesB * Cfg::kStageBytesB);  // [kUnits][kTileN]
-    float* const ldsRowScale = ldsChannelScale + kUnits * kTileN;                            // [kRowScales]
-    uint32_t* const ldsRowMax = reinterpret_cast<uint32_t*>(ldsRowScale + Cfg::kRowScales);  // [kRows]
+    float* const ldsScales = reinterpret_cast<float*>(lds + Cfg::kFirstB + Cfg::kStagesB * Cfg::kStageBytesB);
+    constexpr int kScaleSet = kUnits * kTileN + Cfg::kRowScales;  // of a tile: [kUnits][kTileN] of channels, [kRowScales] of rows
+    uint32_t* const ldsRowMax = reinterpret_cast<uint32_t*>(ldsScales + Cfg::kScaleSets * kScaleSet);  // [kRows]
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1214,6 +1217,45 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     using FirstHalf = std::integral_constant<int, 0>;
     using SecondHalf = std::integral_constant<int, 1>;
 
+    // The scales of a tile come by DMA into LDS (4 bytes a lane: the wave rows' waves take 64 channels, or rows, each): loaded in the
+    // epilogue they would come behind every stage in flight.  They travel with the tile's first k-step, and the k loop certifies them with
+    // the stages it requests itself, where it is as long as the ring.  Where that is two stages deep, the wait of the first k-step is for
+    // them, and it shows on tiles of a few: there they are asked for behind the k loop of the tile before, with its draw, and settled with
+    // it.  us, loaded in the epilogue / with the first k-step / this: gate/up, 64 groups of 500 rows, K x 2 x 1024: K 128 40.6 / 42.9 / 41.1,
+    // 256 44.8 / 45.9 / 45.6, 384 49.9 / 50.4 / 50.1, 768 63.2 / 63.9 / 63.6, 1024 87.4 / 77.2 / 76.7 (what is left of the loss is the wait for
+    // the stores of the tile before); down 41.6 / 41.0 / 40.9 at K 256 x 2048; 8 groups of 4000, K 4096 x 2 x 2048 421 / 417 / 414.
+    constexpr bool kScalesAhead = Cfg::kScaleSets == 2;
+    const bool scalesByDma = kScalesAhead || kSteps >= Cfg::kStagesB;
+    const bool rowScalesByDma = scalesByDma && reinterpret_cast<uintptr_t>(a.rowScale) % 4 == 0;
+    const bool channelScalesByDma = kEpi != Epilogue::kInt32 && scalesByDma && a.scaleDtype == 0 && reinterpret_cast<uintptr_t>(a.scale) % 4 == 0;
+    // those of the n-th tile of this workgroup
+    auto scalesOf = [&](int32_t n) __attribute__((always_inline)) -> float* { return kScalesAhead ? ldsScales + (n & 1) * kScaleSet : ldsScales; };
+    auto requestScales = [&](const TileInfo& t, int32_t n) __attribute__((always_inline)) {
+        const int lane = Opaque(tid) & 63;
+        float* const channelScales = scalesOf(n);
+        float* const rowScales = channelScales + kUnits * kTileN;
+        if (forWeights) {
+            if (channelScalesByDma) {
+#pragma unroll
+                for (int u = 0; u < kUnits; ++u) {
+                    if (u > 0 && unitsOf(t) == 1) break;
+                    const int c = 64 * waveN + lane, base = u ? secondUnit(t) : t.colBase;  // of the unit; the unit's
+                    const int32_t col = kSwiglu ? (waveN >= 2 ? min(a.halfN + base + c - kTileN / 2, a.N - 1) : min(base + c, a.halfN - 1))
+                                                : min(base + c, a.N - 1);
+                    DmaToLdsAddr4(static_cast<const char*>(a.scale) + static_cast<int64_t>(t.group) * a.N * 4, static_cast<uint32_t>(col) * 4u,
+                                  LdsAddress(reinterpret_cast<const char*>(channelScales + u * kTileN + 64 * waveN)));
+                }
+            }
+        } else if (a.rowScale != nullptr && rowScalesByDma && 64 * waveN < kRows) {
+            DmaToLdsAddr4(reinterpret_cast<const char*>(a.rowScale) + static_cast<int64_t>(t.rowBase) * 4,
+                          static_cast<uint32_t>(min(64 * waveN + lane, t.rows - 1)) * 4u,
+                          LdsAddress(reinterpret_cast<const char*>(rowScales + 64 * waveN)));
+        } else if (a.rowScale != nullptr && !rowScalesByDma && tid - kThreads / 2 < kRows) {
+            rowScales[tid - kThreads / 2] = a.rowScale[t.rowBase + min(tid - kThreads / 2, t.rows - 1)];
+        }
+    };
+
+    if (kScalesAhead && kEpi != Epilogue::kInt32) requestScales(cur, 0);
     setupIssue(cur);
 #pragma unroll 1
     for (int s = 0; s < (forWeights ? Cfg::kStagesB : Cfg::kStagesA); ++s) {
@@ -1257,38 +1299,10 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         }
     };
 
-    // The scales of a tile travel with its first k-step, by DMA into LDS (4 bytes a lane: the wave rows' waves take 64 channels, or rows,
-    // each): loaded in the epilogue they would come behind every stage in flight.  The k loop certifies them with the stages it requests
-    // itself, where it is as long as the ring.
-    const bool rowScalesByDma = kSteps >= Cfg::kStagesB && reinterpret_cast<uintptr_t>(a.rowScale) % 4 == 0;
-    const bool channelScalesByDma = kEpi != Epilogue::kInt32 && kSteps >= Cfg::kStagesB && a.scaleDtype == 0 && reinterpret_cast<uintptr_t>(a.scale) % 4 == 0;
-    auto requestScales = [&]() __attribute__((always_inline)) {
-        const int lane = Opaque(tid) & 63;
-        if (forWeights) {
-            if (channelScalesByDma) {
-#pragma unroll
-                for (int u = 0; u < kUnits; ++u) {
-                    if (u > 0 && unitsOf(cur) == 1) break;
-                    const int c = 64 * waveN + lane, base = u ? secondUnit(cur) : cur.colBase;  // of the unit; the unit's
-                    const int32_t col = kSwiglu ? (waveN >= 2 ? min(a.halfN + base + c - kTileN / 2, a.N - 1) : min(base + c, a.halfN - 1))
-                                                : min(base + c, a.N - 1);
-                    DmaToLdsAddr4(static_cast<const char*>(a.scale) + static_cast<int64_t>(cur.group) * a.N * 4, static_cast<uint32_t>(col) * 4u,
-                                  LdsAddress(reinterpret_cast<const char*>(ldsChannelScale + u * kTileN + 64 * waveN)));
-                }
-            }
-        } else if (a.rowScale != nullptr && rowScalesByDma && 64 * waveN < kRows) {
-            DmaToLdsAddr4(reinterpret_cast<const char*>(a.rowScale) + static_cast<int64_t>(cur.rowBase) * 4,
-                          static_cast<uint32_t>(min(64 * waveN + lane, cur.rows - 1)) * 4u,
-                          LdsAddress(reinterpret_cast<const char*>(ldsRowScale + 64 * waveN)));
-        } else if (a.rowScale != nullptr && !rowScalesByDma && tid - kThreads / 2 < kRows) {
-            ldsRowScale[tid - kThreads / 2] = a.rowScale[cur.rowBase + min(tid - kThreads / 2, cur.rows - 1)];
-        }
-    };
-
     v4i acc[kUnits][Blocks::kAll][4];
     while (true) {
         const TileInfo following = tileAt(curNo + 1);
-        if (kEpi != Epilogue::kInt32) requestScales();
+        if (!kScalesAhead && kEpi != Epilogue::kInt32) requestScales(cur, curNo);
 #pragma unroll
         for (int u = 0; u < kUnits; ++u) {
 #pragma unroll
@@ -1423,6 +1437,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                 if (drawCounter >= 0 && tid == 0) drawValue = QueueTake(a.queueCounters, drawCounter);
             }
         }
+        if (kScalesAhead && kEpi != Epilogue::kInt32 && following.valid) requestScales(following, curNo + 1);
         const KernelArgs epilogueArgs = ReloadArgs();
         auto beforeStores = [&]() __attribute__((always_inline)) {
             __builtin_amdgcn_sched_barrier(0);
@@ -1462,7 +1477,8 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
             }
         };
         constexpr int kOrder = kOrderOf<kNz, kNMajor>;
-        const float* const channelScales = channelScalesByDma ? ldsChannelScale : nullptr;
+        const float* const channelScales = channelScalesByDma ? scalesOf(curNo) : nullptr;
+        const float* const ldsRowScale = scalesOf(curNo) + kUnits * kTileN;
         if constexpr (kUnits == 1) {
             TileEpilogueWave<kRows, kEpi, kOrder>(epilogueArgs, cur, acc[0], waveM, waveN, Opaque(tid) & 15, (Opaque(tid) >> 4) & 3, channelScales,
                                                   ldsRowScale, ldsRowMax, beforeStores);
@@ -1474,7 +1490,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                 TileInfo second = cur;
                 second.colBase = secondUnit(cur);
                 TileEpilogueWave<kRows, kEpi, kOrder, false>(epilogueArgs, second, acc[1], waveM, waveN, Opaque(tid) & 15, (Opaque(tid) >> 4) & 3,
-                                                             channelScalesByDma ? ldsChannelScale + kTileN : nullptr, ldsRowScale, ldsRowMax);
+                                                             channelScalesByDma ? channelScales + kTileN : nullptr, ldsRowScale, ldsRowMax);
             }
         }
         if (tid == 0 && following.valid) leaveTile(curNo + (pull ? 2 : kTilesAhead), next);

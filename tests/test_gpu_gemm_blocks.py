@@ -319,3 +319,27 @@ def test_forms_by_sizes_down(aclnn, monkeypatch, name, K, N, want_rows):
     (got, want), rows = _spanned(aclnn, lambda: _run(aclnn, FORMS[name][0], N, K, "k", torch.bfloat16, K))
     assert rows == want_rows
     assert torch.equal(got, want)
+
+
+# 256-row tiles ask for a tile's scales behind the one before, into two places in turn: three and more tiles a workgroup, of one k-step and
+# more, from shares (K below 1024) and drawn
+@pytest.mark.parametrize("K", [128, 272, 1024])
+def test_scales_of_tiles_in_a_row(aclnn, dev, monkeypatch, K):
+    sizes, columns = [300, 256, 0, 299, 301] * 20, 512
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", "256")
+    got, want = _run(aclnn, sizes, 2 * columns, K, "k", torch.bfloat16, K)
+    assert torch.equal(got, want)
+    E, M = len(sizes), sum(sizes)
+    g = torch.Generator(device=dev).manual_seed(K)
+    x = torch.empty((M, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    w = torch.empty((E, 2 * columns, K), dtype=torch.int8, device=dev).random_(-127, 128, generator=g)
+    scale, x_scale = torch.rand((E, 2 * columns), device=dev, generator=g) * 1e-3, torch.rand((M + 1,), device=dev, generator=g) * 1e-2
+    cumsum = torch.cumsum(torch.tensor(sizes), 0).to(dev)
+
+    def call():
+        return aclnn.grouped_matmul_swiglu_quant(x, w.transpose(1, 2), cumsum, scale, x_scale[1:])
+
+    y, ys = call()
+    monkeypatch.setenv("OPAPI_GEMM_TILE_M", "96")
+    y96, ys96 = call()
+    assert torch.equal(y, y96) and torch.equal(ys, ys96)
