@@ -148,8 +148,8 @@ def check_ring_barrier_waits(asm_path):
     not see, so the wave's reads of them have to have been waited for.  In the device assembly of StreamGemmKernel and
     MixedGemmKernel, going back from every s_barrier inside a basic block that multiplies, a wait for LDS (lgkmcnt of at most four:
     the reads of the rows' second half, which the barrier does not free) has to come before any LDS read.  Nor may such a block wait for
-    every memory request (vmcnt(0) or a counter past it): the compiler does so where it believes a register's load still pending, and
-    the DMAs in flight are then drained in every k-step.
+    every memory request (vmcnt(0)): the compiler does so where it believes a register's load still pending, and the DMAs in flight are
+    then drained in every k-step.
     Returns the number of barriers checked."""
     checked = 0
     for body in open(asm_path).read().split("; -- Begin function ")[1:]:

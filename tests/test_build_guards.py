@@ -1,7 +1,8 @@
 """The build-time guards of ops-transformer_amd/build.py around the LDS-DMA kernels: the compiler pin, the check that, in
 the device assembly, m0 is written only as the first half of an (s_mov_b32 m0, global_load_lds_dwordx4) pair, and the
 check of the generated code for scratch use, generic memory instructions and merged multiply-convert instructions, and the
-check that a barrier among matrix instructions comes behind a wait for the LDS reads of what it frees."""
+check that a barrier among matrix instructions comes behind a wait for the LDS reads of what it frees and that no memory wait there
+drains the loads in flight."""
 import importlib.util
 import os
 
@@ -132,3 +133,14 @@ def test_barrier_guard_refuses(build, tmp_path, bad):
 
 def test_barrier_guard_checks_ring_kernels_only(build, tmp_path):
     assert build.check_ring_barrier_waits(_write(tmp_path, BARRIER_GOOD.replace("StreamGemm", "GenericGemm"))) == 0
+
+
+@pytest.mark.parametrize("wait", ["vmcnt(0) lgkmcnt(1)", "vmcnt(0) expcnt(0) lgkmcnt(1)"])
+def test_barrier_guard_refuses_a_wait_for_all_requests_among_products(build, tmp_path, wait):
+    with pytest.raises(RuntimeError, match="drains its DMAs"):
+        build.check_ring_barrier_waits(_write(tmp_path, BARRIER_GOOD.replace("vmcnt(3) lgkmcnt(1)", wait)))
+
+
+def test_barrier_guard_accepts_a_wait_for_all_requests_elsewhere(build, tmp_path):
+    for kept in ("\ts_endpgm", ".LBB0_1:"):  # behind the loop and in front of it
+        assert build.check_ring_barrier_waits(_write(tmp_path, BARRIER_GOOD.replace(kept, "\ts_waitcnt vmcnt(0)\n" + kept))) == 1
