@@ -952,14 +952,14 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     // ---- this workgroup's sequence of tiles ----
     // Workgroup b serves XCD b % 8 as its slot b / 8.  Wave 0 finds the tiles and leaves them, decoded, in an eight-entry ring
     // in LDS.  With a.pullTiles the first ones are its seat's and the others come out of the tile counters (see QueueShare): tile n + 2 is
-    // drawn while tile n's epilogue runs, because the issue side already reads tile n + 1's operands during tile n.  Otherwise the two runs of the m-tile table are one list cut into eight fixed
+    // drawn while tile n's epilogue runs, because the issue side already reads tile n + 1's operands during tile n.  Otherwise (tiles of 256 channels only) the two runs of the m-tile table are one list cut into eight fixed
     // shares, which the workgroups of an XCD walk with stride gridDim / 8, and the ring holds six tiles (tiles of one k-step
     // have the issue side five tiles ahead).
     const int xcd = blockIdx.x % kXcds;
     const int32_t slots = gridDim.x / kXcds;
     const int32_t slot = blockIdx.x / kXcds;
     constexpr bool kOneRun = kRun != kBothRuns;
-    const bool pull = kOneRun || a.pullTiles != 0;
+    const bool pull = kOneRun || kUnits > 1 || a.pullTiles != 0;
     int32_t* const ldsSeq = reinterpret_cast<int32_t*>(ldsRowMax + kRows);
     // wave 0's state, behind the ring: used-up counters, tiles of a share that are dealt out (big, small), this workgroup's next tile of those,
     // how many it has left, and how far apart they are
@@ -978,7 +978,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     };
     // the n-th tile of this workgroup in fixed shares
     auto shareTile = [&](const KernelArgs& args, const RunTable& r, int32_t n) __attribute__((always_inline)) -> v4i {
-        const int32_t big = r.countBig * tilesAcross(args), total = big + r.countSmall * tilesAcross(args);
+        const int32_t big = r.countBig * args.tilesN, total = big + r.countSmall * args.tilesN;
         const int32_t perXcd = (total + kXcds - 1) / kXcds, local = slot + n * slots, logical = xcd * perXcd + local;
         const bool none = local >= perXcd || logical >= total;
         return decodeTile(args, r, none ? -1 : logical < big ? 0 : 1, logical < big ? logical : logical - big);
