@@ -208,18 +208,19 @@ __device__ __forceinline__ void QueueShare(const QueueLists q, int counter, int3
 }
 // Workgroups of an XCD's `slots` that begin with the small m-tiles: the share that their cost is of the whole, so that lists of many
 // rounds run dry at about the same time; until then a part of the machine streams weights for a handful of rows each while
-// the rest multiplies.  But where the tiles of the big ones are no more than seven eighths of the workgroups, all of these begin with: those
+// the rest multiplies.  But in two geometries, where the tiles of the big ones are no more than seven eighths of the workgroups, all of these begin with: those
 // left over would each be a whole tile behind the last small one.  us, by cost -> this: gate/up 2048 x 2 x 2048, 64 experts of 25 rows on average,
 // popularity rank^-0.8 (112 big tiles) 127 -> 108; 7168 x 2 x 2048, 32 of 80, rank^-1.2 (224) 238 -> 197; down 1536 x 4096, 128 of 20,
 // rank^-0.4 (16) 167 -> 155.  With 240 and 256 of them, which leaves the small ones' weights for a round of their own: 64 of 60,
 // rank^-0.4 115 -> 125, 256 of 50, 2048 x 2 x 768 161 -> 172.  Row-major weights for SwiGLU are left with the share of the cost (7168 x 2 x 2048,
-// 32 of 25, rank^-0.4 176 against 192 us).
-template <Epilogue kEpi, bool kNMajor>
+// 32 of 25, rank^-0.4 176 against 192 us), and so is one geometry for both (int32, 59 experts of 68 rows, rank^-0.4, 1536 x 2048 51 against 59 us;
+// bf16, 99 of 62 even, 1024 x 1024 36 against 40).
+template <Epilogue kEpi, bool kNMajor, bool kTwoGeometries>
 __device__ __forceinline__ int32_t SlotsForSmall(const int32_t* __restrict__ hdr, int32_t slots, int32_t tilesN) {
     const int64_t costSmall = hdr[2], costAll = costSmall + hdr[3];
     int32_t forSmall = static_cast<int32_t>(costAll > 0 ? (slots * costSmall + costAll / 2) / costAll : 0);
     if (forSmall == 0 && hdr[1] > 0 && slots > 1) forSmall = 1;
-    if (kNMajor && kEpi == Epilogue::kSwiglu) return forSmall;
+    if (!kTwoGeometries || (kNMajor && kEpi == Epilogue::kSwiglu)) return forSmall;
     const int32_t forBig = (hdr[0] * tilesN + kXcds - 1) / kXcds;
     return 8 * forBig <= 7 * slots ? min(forSmall, slots - forBig) : forSmall;
 }
@@ -966,7 +967,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     constexpr int kSeqUsedUp = 32, kSeqSeated = 33, kSeqSeatNext = 35, kSeqSeatLeft = 36, kSeqSeatStride = 37;
     constexpr int kTilesAhead = 6;
     // Which list this workgroup draws from first.
-    const int32_t forSmall = sched[0] == 0 ? slots : SlotsForSmall<kEpi, kNMajor>(sched, slots, a.tilesN);
+    const int32_t forSmall = sched[0] == 0 ? slots : SlotsForSmall<kEpi, kNMajor, kOneRun>(sched, slots, a.tilesN);
     const int prefer = kOneRun ? kRun : (slot < forSmall ? 1 : 0);
     auto tilesAcross = [](const KernelArgs& args) __attribute__((always_inline)) { return (args.tilesN + kUnits - 1) / kUnits; };
     // tile `logical` of a run (list < 0: none), decoded
@@ -1554,7 +1555,7 @@ __global__ __launch_bounds__(kThreads) void MixedGemmKernel(KernelArgs a, const 
         return;
     }
     const int32_t slots = gridDim.x / kXcds, slot = blockIdx.x / kXcds;
-    const int32_t forSmall = sched[0] == 0 ? slots : SlotsForSmall<kEpi, kNMajor>(sched, slots, a.tilesN);
+    const int32_t forSmall = sched[0] == 0 ? slots : SlotsForSmall<kEpi, kNMajor, true>(sched, slots, a.tilesN);
     if (slot < forSmall) {
         StreamGemmBody<kSmallRows, kEpi, kNz, kNMajor, kSmallRun, kTail>(a, sched, lds, spanTiles);
         if (sched[0] != 0) {
