@@ -760,7 +760,7 @@ constexpr int kStep = 128;
 //
 // One DMA instruction moves 64 lanes x 16 bytes = 8 rows of 128 k-bytes.  Slot q of wave column w is instruction w + 4 q of
 // its kind, i.e. 32 rows per slot: even slots of the activation rows are the first half of the wave rows' blocks.
-template <int kRows, int kUnits = 1>
+template <int kRows, Epilogue kEpi, int kUnits = 1>
 struct StreamCfg {
     using Blocks = RowBlocks<kRows>;
     static constexpr int kStageBytesA = kRows * kStep;
@@ -768,8 +768,8 @@ struct StreamCfg {
     static constexpr int kHalfBytesB = kStageBytesB / 2;
     static constexpr int kQueueLdsInts = 40;  // the workgroup's next eight tiles and how it comes by them
     static constexpr int kRowScales = (kRows + 63) / 64 * 64;  // in whole DMA instructions
-    // Tiles of 256 rows, whose rings are two stages deep, hold the next tile's scales too (see requestScales).
-    static constexpr int kScaleSets = kRows == 256 ? 2 : 1;
+    // SwiGLU tiles of 256 rows, whose rings are two stages deep, hold the next tile's scales too (see requestScales).
+    static constexpr int kScaleSets = kRows == 256 && kEpi == Epilogue::kSwiglu ? 2 : 1;
     // channel scales, row scales, row maxima, tiles
     static constexpr int kScratchBytes = (kScaleSets * (kUnits * kTileN + kRowScales) + kRows + kQueueLdsInts) * 4;
     static constexpr int kRingBytes = kLdsBudget - kScratchBytes;
@@ -937,7 +937,7 @@ template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, int kRun, bool kTail
 __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_t* __restrict__ sched, char* const lds,
                                                uint64_t& spanTiles, bool begins = true) {
     static_assert(!(kNz && kNMajor), "one weight layout at a time");
-    using Cfg = StreamCfg<kRows, kUnits>;
+    using Cfg = StreamCfg<kRows, kEpi, kUnits>;
     using Blocks = RowBlocks<kRows>;
     constexpr bool kSwiglu = kEpi == Epilogue::kSwiglu;
     constexpr int kUnitCols = kSwiglu ? kTileN / 2 : kTileN;  // output columns of 256 channels
@@ -1221,10 +1221,11 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
     // The scales of a tile come by DMA into LDS (4 bytes a lane: the wave rows' waves take 64 channels, or rows, each): loaded in the
     // epilogue they would come behind every stage in flight.  They travel with the tile's first k-step, and the k loop certifies them with
     // the stages it requests itself, where it is as long as the ring.  Where that is two stages deep, the wait of the first k-step is for
-    // them, and it shows on tiles of a few: there they are asked for behind the k loop of the tile before, with its draw, and settled with
-    // it.  us, loaded in the epilogue / with the first k-step / this: gate/up, 64 groups of 500 rows, K x 2 x 1024: K 128 40.6 / 42.9 / 41.1,
+    // them, and it shows on SwiGLU tiles of a few: there they are asked for behind the k loop of the tile before, with its draw, and settled
+    // with it.  us, loaded in the epilogue / with the first k-step / this: gate/up, 64 groups of 500 rows, K x 2 x 1024: K 128 40.6 / 42.9 / 41.1,
     // 256 44.8 / 45.9 / 45.6, 384 49.9 / 50.4 / 50.1, 768 63.2 / 63.9 / 63.6, 1024 87.4 / 77.2 / 76.7 (what is left of the loss is the wait for
-    // the stores of the tile before); down 41.6 / 41.0 / 40.9 at K 256 x 2048; 8 groups of 4000, K 4096 x 2 x 2048 421 / 417 / 414.
+    // the stores of the tile before); 8 groups of 4000, K 4096 x 2 x 2048 421 / 417 / 414.  16-bit results
+    // gain nothing by it: 29 groups of 1212 rows, 1024 x 4096 185 / 184 / 191; 8 of 4000, 2048 x 4096 228 / 220 / 222.
     constexpr bool kScalesAhead = Cfg::kScaleSets == 2;
     const bool scalesByDma = kScalesAhead || kSteps >= Cfg::kStagesB;
     const bool rowScalesByDma = scalesByDma && reinterpret_cast<uintptr_t>(a.rowScale) % 4 == 0;
@@ -1256,7 +1257,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
         }
     };
 
-    if (kScalesAhead && kEpi != Epilogue::kInt32) requestScales(cur, 0);
+    if (kScalesAhead) requestScales(cur, 0);
     setupIssue(cur);
 #pragma unroll 1
     for (int s = 0; s < (forWeights ? Cfg::kStagesB : Cfg::kStagesA); ++s) {
@@ -1438,7 +1439,7 @@ __device__ __forceinline__ void StreamGemmBody(const KernelArgs& a, const int32_
                 if (drawCounter >= 0 && tid == 0) drawValue = QueueTake(a.queueCounters, drawCounter);
             }
         }
-        if (kScalesAhead && kEpi != Epilogue::kInt32 && following.valid) requestScales(following, curNo + 1);
+        if (kScalesAhead && following.valid) requestScales(following, curNo + 1);
         const KernelArgs epilogueArgs = ReloadArgs();
         auto beforeStores = [&]() __attribute__((always_inline)) {
             __builtin_amdgcn_sched_barrier(0);
@@ -1673,7 +1674,7 @@ __global__ __launch_bounds__(kThreads) void GenericGemmKernel(KernelArgs a, cons
 // ---------------------------------------------------------------------------------------------- launchers
 template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
 hipError_t LaunchStream(const KernelArgs& args, const int32_t* sched, int64_t maxTiles, hipStream_t stream) {
-    using Cfg = StreamCfg<kRows>;
+    using Cfg = StreamCfg<kRows, kEpi>;
     auto kernel = StreamGemmKernel<kRows, kEpi, kNz, kNMajor, kTail>;
     static std::atomic<uint64_t> optedIn{0};
     const hipError_t attr = opapi::EnsureDynamicLds(reinterpret_cast<const void*>(kernel), Cfg::kLdsBytes, optedIn);
@@ -1691,7 +1692,8 @@ hipError_t LaunchStream(const KernelArgs& args, const int32_t* sched, int64_t ma
 
 template <int kRows, Epilogue kEpi, bool kNz, bool kNMajor, bool kTail>
 hipError_t LaunchMixed(const KernelArgs& args, const int32_t* sched, int64_t maxTiles, hipStream_t stream) {
-    constexpr int kLdsBytes = std::max({StreamCfg<kRows>::kLdsBytes, StreamCfg<kSmallRows>::kLdsBytes, StreamCfg<kLowTileM>::kLdsBytes, StreamCfg<kLowTileM, 2>::kLdsBytes});
+    constexpr int kLdsBytes = std::max({StreamCfg<kRows, kEpi>::kLdsBytes, StreamCfg<kSmallRows, kEpi>::kLdsBytes, StreamCfg<kLowTileM, kEpi>::kLdsBytes,
+                                        StreamCfg<kLowTileM, kEpi, 2>::kLdsBytes});
     auto kernel = MixedGemmKernel<kRows, kEpi, kNz, kNMajor, kTail>;
     static std::atomic<uint64_t> optedIn{0};
     const hipError_t attr = opapi::EnsureDynamicLds(reinterpret_cast<const void*>(kernel), kLdsBytes, optedIn);
