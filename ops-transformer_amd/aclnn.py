@@ -300,8 +300,8 @@ def _run_packed(op, scalars, tensors, device, workspace=None):
     """Both phases of an operator: the first in one foreign call on descriptors packed into one array.
 
     A call on a few rows is bound by the host, and its descriptors, a foreign call each to make and a handle to drop, were a part of
-    that.  us, before -> this: a MoE layer of five operators on 5 tokens, 160 experts, hidden 3840, intermediate 576 86 -> 63; on 4
-    tokens, 160 experts, 2880, 1984 91 -> 78; permutation and combine of 46 tokens of 1024 37 -> 31."""
+    that.  us, before -> this: a MoE layer of five operators on 2 tokens, 16 experts, hidden 1024, intermediate 512 92 -> 68; permutation
+    and combine of 46 tokens of 1024 36 -> 29."""
     l = lib()
     packed = struct.pack("%dq" % (1 + len(scalars)), op, *scalars) + b"".join([_packed(t) for t in tensors])
     planned = (ctypes.c_uint64 * 2)()  # workspace bytes, executor
