@@ -321,7 +321,7 @@ def test_forms_by_sizes_down(aclnn, monkeypatch, name, K, N, want_rows):
     assert torch.equal(got, want)
 
 
-# 256-row tiles ask for a tile's scales behind the one before, into two places in turn: three and more tiles a workgroup, of one k-step and
+# 256-row SwiGLU tiles ask for a tile's scales behind the one before, into two places in turn: three and more tiles a workgroup, of one k-step and
 # more, from shares (K below 1024) and drawn
 @pytest.mark.parametrize("K", [128, 272, 1024])
 def test_scales_of_tiles_in_a_row(aclnn, dev, monkeypatch, K):
